@@ -32,7 +32,7 @@ class EngineConfig:
     # the plain kernels in bfloat16 too, which splits a mismatch into "tuned kernel" or "bfloat16
     # rounding" (the reference picks its math provider in the same place:
     # core/src/main/java/io/teknek/deliverance/benchmark/InferenceBenchmark.java:1067,1139).
-    # 32-bit always runs the plain kernels.
+    # In 32-bit "tuned" puts the products on the matrix cores' 32-bit instructions; nothing is rounded to fewer bits.
     kernels: str = "tuned"
     page_size: int = 16                # tokens per KV page: 16, 32 or 64 (what every attention kernel takes)
     max_cached_tokens: Optional[int] = None   # pool size in tokens; None: sized from free memory

@@ -79,6 +79,7 @@ _ARGTYPES = {
     "da_state_scatter": [_VP, _VP, _VP, _VP, _I, _I, _I, _VP],
     "da_layernorm": [_VP, _VP, _VP, _I, _VP, _I, _F, _VP, _I, _I, _I, _VP],
     "da_gemm_ref": [_VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP],
+    "da_gemm_f32": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _VP],
     "da_gemm_bf16": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_few_rows": [_I, _I],
     "da_gemm_bf16_kv_split": [_VP, _I, _VP, _I, _VP, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
@@ -763,8 +764,8 @@ def top_logprobs(logits: torch.Tensor, params: torch.Tensor, n: int, out_idx: to
 
 # ------------------------------------------------------------------------------- dispatch
 # "tuned": MFMA products and the prefill/decode attention kernels in bfloat16;
-# "reference": the plain kernels everywhere (for A/B checks).  32-bit always runs the plain
-# kernels: they are its product path.
+# "reference": the plain kernels everywhere (for A/B checks).  32-bit runs its products on the matrix
+# cores' 32-bit instructions in "tuned" (csrc/gemm_f32.hip), everything else on the plain kernels.
 _MODE = "tuned"
 
 
@@ -943,6 +944,49 @@ def _mfma_ok(a: torch.Tensor, w: torch.Tensor) -> bool:
             and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def _f32_ok(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    return (a.dtype == torch.float32 and w.dtype == torch.float32 and out.dtype == torch.float32 and a.shape[1] % 4 == 0
+            and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+F32_FORMS = {"auto": 0, "rows": 1, "64x64": 2, "32x32": 3}
+
+
+def linear_f32(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
+               act: Optional[str] = None, accumulate: bool = False, kv_cache: Optional[torch.Tensor] = None,
+               slot_map: Optional[torch.Tensor] = None, q_cols: int = 0, form: str = "auto") -> torch.Tensor:
+    """out (+)= act(a @ w.T + bias) in 32-bit on the matrix cores; K a multiple of 4.  With ``kv_cache`` the columns from
+    ``q_cols`` on (k | v) also go to the cache rows ``slot_map``.  ``form``: "auto" lets the library choose by shape; the
+    others ask for one kernel (tests and timing)."""
+    _dev(a, w, bias, out, kv_cache, slot_map)
+    _rows_2d(a, "a"); _rows_2d(w, "w"); _rows_2d(out, "out")
+    M, K = a.shape
+    N = w.shape[0]
+    _need(a.dtype == w.dtype == out.dtype == torch.float32, "linear_f32: a, w and out must be float32")
+    if not (w.shape[1] == K):
+        raise KernelError(f"linear: a is [{M},{K}] but w is {list(w.shape)}")
+    if not (out.shape[0] == M and out.shape[1] == N):
+        raise KernelError(f"linear: out is {list(out.shape)}, expected [{M},{N}]")
+    _need(bias is None or bias.numel() == N, "linear: bias length differs from N")
+    if not (act in ACTIVATIONS):
+        raise KernelError(f"linear: unknown activation {act!r}")
+    if form not in F32_FORMS:
+        raise KernelError(f"linear_f32: unknown form {form!r}")
+    kvp = (None, None, 0, 0, 0, 0, 0)
+    if kv_cache is not None:
+        _need(not accumulate, "linear: a cache scatter goes with a plain store")
+        _need(kv_cache.dim() == 5 and kv_cache.is_contiguous() and kv_cache.dtype == torch.float32,
+              "linear_f32: cache slot must be contiguous float32 [pages,2,Hkv,page,D]")
+        _, _, Hkv, page, D = kv_cache.shape
+        _need(slot_map is not None and slot_map.dtype == torch.int32 and slot_map.numel() >= M, "linear_f32: slot_map must be int32 [rows]")
+        _need(q_cols + 2 * Hkv * D == N, "linear_f32: q|k|v columns do not add up to N")
+        kvp = (_ptr(kv_cache), _ptr(slot_map), q_cols, Hkv * D, Hkv, D, page)
+    with _timed("product_f32", _product_bytes(a, w, bias, out, accumulate), 2 * M * N * K, "fp32"):
+        _check(_lib().da_gemm_f32(_ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(bias), _dt(bias) if bias is not None else 0,
+                                  ACTIVATIONS[act], int(accumulate), _ptr(out), out.stride(0), M, N, K, *kvp, F32_FORMS[form], _stream()))
+    return out
+
+
 # Measured on MI355X (q|k|v of 768 to 1,600 wide, 128 to 2,048 rows): the cache write in the product's
 # epilogue adds 1.3 to 3.4 us where the rows' places are runs of consecutive cache rows (a prompt
 # portion: keys and values both go over in 16-byte pieces), the write kernel after the product 3.7 to
@@ -953,11 +997,13 @@ def linear(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: 
            act: Optional[str] = None, accumulate: bool = False, kv_cache: Optional[torch.Tensor] = None,
            slot_map: Optional[torch.Tensor] = None, q_cols: int = 0) -> torch.Tensor:
     """out (+)= act(a @ w.T + bias); picks the kernel by dtype and mode.  Shapes the matrix-core
-    kernel does not take (K not a multiple of 8) go to the plain kernel, which takes any.  With
+    kernels do not take (K not a multiple of 8, in 32-bit of 4) go to the plain kernel, which takes any.  With
     ``kv_cache`` the k | v columns (from ``q_cols`` on) are also written to the cache rows
     ``slot_map``: in the product's epilogue on the matrix cores, by the write kernel otherwise."""
     if _MODE == "tuned" and _mfma_ok(a, w):
         return linear_mfma(a, w, bias, out, act, accumulate, kv_cache, slot_map, q_cols)
+    if _MODE == "tuned" and _f32_ok(a, w, out):
+        return linear_f32(a, w, bias, out, act, accumulate, kv_cache, slot_map, q_cols)
     linear_ref(a, w, bias, out, act, accumulate)
     if kv_cache is not None:
         _, _, Hkv, _, D = kv_cache.shape

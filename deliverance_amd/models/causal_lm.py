@@ -72,7 +72,7 @@ class CausalLM:
 
     def kernel_units(self) -> List[str]:
         """The kernel units that the model's steps call: what a first call in a fresh checkout compiles, side by side."""
-        names = ["rowwise", "dispatch"] + (["gemm_mfma", "gemm_wide", "gemm_fused"] if self.dtype == torch.bfloat16 else ["gemm_ref"])
+        names = ["rowwise", "dispatch"] + (["gemm_mfma", "gemm_wide", "gemm_fused"] if self.dtype == torch.bfloat16 else ["gemm_ref", "gemm_f32"])
         norms = [self.final_norm, self.embed_norm]
         for b in self.blocks:
             norms += [b.pre_mixer_norm, b.post_mixer_norm, b.pre_ff_norm, b.post_ff_norm, b.post_block_norm]

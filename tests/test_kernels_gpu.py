@@ -130,6 +130,46 @@ def test_gemm_plain_32bit(ops, M, N, K):
         assert (out - ref).abs().max() < 2e-5 * max(1.0, ref.abs().max().item())
 
 
+@pytest.mark.parametrize("form", ["auto", "rows", "64x64", "32x32"])
+@pytest.mark.parametrize("M,N,K", [(1, 50, 24), helpers.quick(5, 1000, 96), (16, 64, 128), helpers.quick(17, 33, 132), (65, 200, 772),
+                                   (130, 77, 200), (300, 1100, 640), (16, 2100, 3072)])
+def test_gemm_32bit_on_the_matrix_cores(ops, M, N, K, form):
+    """Every kernel form behind ``linear_f32``: K below a group, below a chunk, cut and whole chunks; edges in M and N; a
+    row has the same bits in every form and beside any other rows.  Bound: a sum in chunks of 128 loses at most
+    (128 + K / 128) roundings of 2^-24 of the sum of magnitudes, which is below sqrt(K) times the operands' scale here."""
+    helpers.skip_in_simulation_if(M * N * K > 4e6)
+    g = torch.Generator().manual_seed(M * 1000 + N)
+    fn = lambda a, w, b, out, act, acc: ops.linear_f32(a, w, b, out, act, acc, form=form)
+    for act, acc, bias in ((None, False, True), ("gelu_new", False, True), (None, True, True), ("silu", False, False)):
+        out, ref = _gemm_case(ops, fn, M, N, K, torch.float32, act, acc, bias, torch.float32, g)
+        assert (out - ref).abs().max() < 2e-5 * max(1.0, ref.abs().max().item())
+    a = (torch.randn(M, K, generator=g)).to(DEV)
+    w = (torch.randn(N, K, generator=g)).to(DEV)
+    o1, o2, o3 = (torch.empty(M, N, device=DEV) for _ in range(3))
+    ops.linear_f32(a, w, None, o1, form=form)
+    ops.linear_f32(a, w, None, o2, form="32x32")
+    ops.linear_f32(a[M // 2:M // 2 + 1], w, None, o3[:1])
+    assert torch.equal(o1, o2) and torch.equal(o1[M // 2], o3[0])
+
+
+def test_gemm_32bit_writes_keys_and_values(ops):
+    g = torch.Generator().manual_seed(7)
+    Hq, Hkv, D, page, K = 5, 3, 20, 16, 132
+    N = (Hq + 2 * Hkv) * D
+    for M in (3, 70):
+        n_pages = (M + page - 1) // page + 2
+        a, w, bias = (torch.randn(*s, generator=g).to(DEV) for s in ((M, K), (N, K), (N,)))
+        slots = torch.randperm(n_pages * page, generator=g)[:M].to(torch.int32)
+        slots[M // 2] = -1
+        slots = slots.to(DEV)
+        c1 = torch.zeros(n_pages, 2, Hkv, page, D, device=DEV)
+        c2 = torch.zeros_like(c1)
+        out = torch.empty(M, N, device=DEV)
+        ops.linear_f32(a, w, bias, out, kv_cache=c1, slot_map=slots, q_cols=Hq * D)
+        ops.kv_write(out, Hq * D, (Hq + Hkv) * D, c2, slots, Hkv, D)
+        assert torch.equal(c1, c2) and c1.abs().sum() > 0
+
+
 @pytest.mark.parametrize("M", [1, helpers.quick(3, mark="simt_a"), 5, 8, 12, 16, helpers.quick(17, mark="simt_a"), 40, 64,
                                helpers.quick(65, mark="simt_a"), 128, helpers.quick(200, mark="simt_a"), 513, 1100, 2048])
 @pytest.mark.parametrize("N,K", [helpers.quick(96, 200, mark="simt_b"), helpers.quick(1000, 96, mark="simt_b"), (2304, 768),
