@@ -1,0 +1,226 @@
+// Paged attention in 32-bit on the matrix cores (v_mfma_f32_16x16x4_f32): portions of prompts and one-token sequences alike.
+//
+// One workgroup per (sequence, query head, 16 query rows); 8 wavefronts share out the keys in aligned chunks of 64:
+// wavefront v takes the chunks whose number is v modulo 8, in ascending order, with a running maximum and sum per row,
+// and the wavefronts' partial results are merged in LDS in order.  Every sum's order so depends on a row's own position
+// and the window only, never on how the step was cut or what else is in the batch; a chunk that a row does not see
+// changes nothing in its sums.
+//   scores : S[row, key] = Q . K^T, 4 pieces of 16 keys; a lane's 16-byte piece of a key row is 4 of the inner sum's
+//            terms (an instruction takes the dimensions with d % 4 = j; see gemm_f32.hip for the fragments);
+//   softmax: a lane holds 4 rows of one key column, so a row's maximum and sum are exchanges among 16 lanes;
+//   values : stored dimension-major, so a lane's 16-byte piece is 4 consecutive keys of its dimension, which is the
+//            right operand as it lies in memory; the weights turn from columns into rows through LDS.
+// All key and value loads of a chunk are asked for before any is used (for head sizes up to 64; above, the values once
+// the scores are done).  Bound by two trips to memory and 16 D / 4 instructions of 32 cycles a chunk.
+// Formulas: core/src/main/java/io/teknek/deliverance/generator/CausalSelfAttention.java:481-491,512-527.
+#include "gemm_common.h"
+
+#define AF_WAVES 8
+#define AF_CHUNK 64
+#define AF_PLD (AF_CHUNK + 4)        // padded row of weights in LDS, floats
+
+__device__ __forceinline__ floatx4 af_group(const float4& a, const float4& b, floatx4 c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+}
+__device__ __forceinline__ float af_max16(float v) {          // the maximum over 16 consecutive lanes, in all of them
+  v = fmaxf(v, dpp_move<0xB1, 0xF>(v, v));
+  v = fmaxf(v, dpp_move<0x4E, 0xF>(v, v));
+  v = fmaxf(v, dpp_move<0x141, 0xF>(v, v));
+  return fmaxf(v, dpp_move<0x140, 0xF>(v, v));
+}
+
+template <int D16>
+__global__ void __launch_bounds__(AF_WAVES * DA_WAVE)
+attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__ cache, const int* __restrict__ block_table,
+                int max_blocks, const int* __restrict__ q_start, const int* __restrict__ seq_lens, int Hq, int Hkv, int page,
+                float scale, int window, float* __restrict__ out, int out_ld) {
+  constexpr int D = D16 * 16;
+  constexpr int OLD = D + 4;                                   // padded row of a partial result
+  constexpr int P_FLOATS = AF_WAVES * 16 * AF_PLD, O_FLOATS = AF_WAVES * 16 * OLD;
+  __shared__ __attribute__((aligned(16))) float smem[P_FLOATS > O_FLOATS ? P_FLOATS : O_FLOATS];   // weights, then partial results
+  __shared__ float part_m[AF_WAVES][16], part_l[AF_WAVES][16];
+
+  const int s = (int)blockIdx.x / Hq, h = (int)blockIdx.x % Hq, hk = h / (Hq / Hkv);
+  const int row0 = q_start[s], T = q_start[s + 1] - row0;
+  const int i0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * 16;  // (the rows with the most keys are launched first)
+  if (i0 >= T) return;
+  const int past = seq_lens[s] - T;
+  const int t = threadIdx.x, lane = t % DA_WAVE, wave = __builtin_amdgcn_readfirstlane(t / DA_WAVE);
+  const int col = lane % 16, quad = lane / 16;
+  const int last_row = i0 + 15 < T ? i0 + 15 : T - 1;
+  const int p_max = past + last_row;                           // the last key that any of the rows sees (-1: a padding row)
+  const int lo_min = (window > 0 && past + i0 - window + 1 > 0) ? past + i0 - window + 1 : 0;
+  const int* bt = block_table + (size_t)s * max_blocks;
+  const int lg = 31 - __builtin_clz(page), pmask = page - 1;   // (a power of two, checked on the host)
+  const long long page_elems = 2LL * Hkv * page * D;
+  const float* kbase = cache + (long long)hk * page * D;
+  const float* vbase = cache + (long long)(Hkv + hk) * page * D;
+
+  float4 qf[D16];
+  {
+    const int qi = i0 + col < T ? i0 + col : T - 1;
+    const float* qr = q + (size_t)(row0 + qi) * q_ld + h * D + quad * 4;
+#pragma unroll
+    for (int g = 0; g < D16; ++g) qf[g] = *(const float4*)(qr + g * 16);
+  }
+  floatx4 o[D16];
+#pragma unroll
+  for (int d = 0; d < D16; ++d) o[d] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float m[4], l[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) { m[r] = -INFINITY; l[r] = 0.f; }
+  float* const ps = smem + wave * 16 * AF_PLD;
+
+  const int first_chunk = lo_min / AF_CHUNK;
+  for (int ci = first_chunk + (wave + AF_WAVES - first_chunk % AF_WAVES) % AF_WAVES; ci * AF_CHUNK <= p_max; ci += AF_WAVES) {
+    const int c0 = ci * AF_CHUNK;
+    // The pages of the chunk's 4 pieces of 16 keys (a piece lies in one page), the same for the whole wavefront.  A piece
+    // that no row sees, or whose page was given back, reads page 0 and is dropped.
+    bool seen[4];
+    const float* kp[4];
+    const float* vp[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int k0 = c0 + j * 16;
+      const bool in = k0 <= p_max && k0 + 15 >= lo_min;
+      const int pg = in ? __builtin_amdgcn_readfirstlane(bt[k0 >> lg]) : -1;
+      seen[j] = pg >= 0;
+      const long long off = (long long)(pg >= 0 ? pg : 0) * page_elems;
+      kp[j] = kbase + off + (k0 & pmask) * D;
+      vp[j] = vbase + off + (k0 & pmask);
+    }
+    float4 kf[4][D16], vf[4][D16];
+    constexpr bool EARLY_V = D16 <= 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int g = 0; g < D16; ++g) kf[j][g] = *(const float4*)(kp[j] + col * D + g * 16 + quad * 4);
+    if (EARLY_V) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int d = 0; d < D16; ++d) vf[j][d] = *(const float4*)(vp[j] + (d * 16 + col) * page + quad * 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);                          // (the loads stay ahead of the arithmetic)
+    floatx4 sc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int g = 0; g < D16; ++g) sc[j] = af_group(qf[g], kf[j][g], sc[j]);
+    }
+    float alpha[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + quad * 4 + r, p = past + i;
+      const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
+      bool ok[4];
+      float top = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int key = c0 + j * 16 + col;
+        ok[j] = seen[j] && i < T && key <= p && key >= lo;
+        sc[j][r] = ok[j] ? sc[j][r] * scale : -INFINITY;        // (a select: an unseen key's row may hold anything)
+        top = fmaxf(top, sc[j][r]);
+      }
+      const float m_new = fmaxf(m[r], af_max16(top));
+      alpha[r] = m_new == -INFINITY ? 1.f : expf(m[r] - m_new);
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float e = ok[j] ? expf(sc[j][r] - m_new) : 0.f;
+        ps[(quad * 4 + r) * AF_PLD + j * 16 + col] = e;
+        sum += e;
+      }
+      l[r] = l[r] * alpha[r] + group_sum<16>(sum);
+      m[r] = m_new;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+    for (int d = 0; d < D16; ++d)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[d][r] *= alpha[r];
+    if (!EARLY_V) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int d = 0; d < D16; ++d) vf[j][d] = *(const float4*)(vp[j] + (d * 16 + col) * page + quad * 4);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 w = *(const float4*)&ps[col * AF_PLD + j * 16 + quad * 4];
+      // keys past the last seen one were never written and keys in front of a window may be anybody's: zeros in their
+      // place (their weights are zero, but zero times an infinity is not)
+      const int k0 = c0 + j * 16 + quad * 4;
+#pragma unroll
+      for (int d = 0; d < D16; ++d) {
+        float4 v = vf[j][d];
+        v.x = seen[j] && k0 <= p_max && k0 >= lo_min ? v.x : 0.f;
+        v.y = seen[j] && k0 + 1 <= p_max && k0 + 1 >= lo_min ? v.y : 0.f;
+        v.z = seen[j] && k0 + 2 <= p_max && k0 + 2 >= lo_min ? v.z : 0.f;
+        v.w = seen[j] && k0 + 3 <= p_max && k0 + 3 >= lo_min ? v.w : 0.f;
+        o[d] = af_group(w, v, o[d]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  }
+  __syncthreads();                                              // the weights' place takes the partial results
+#pragma unroll
+  for (int d = 0; d < D16; ++d)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) smem[(wave * 16 + quad * 4 + r) * OLD + d * 16 + col] = o[d][r];
+  if (col == 0) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { part_m[wave][quad * 4 + r] = m[r]; part_l[wave][quad * 4 + r] = l[r]; }
+  }
+  __syncthreads();
+  for (int e = t; e < 16 * D; e += AF_WAVES * DA_WAVE) {
+    const int row = e / D, d = e % D;
+    if (i0 + row >= T) continue;
+    float mm = part_m[0][row];
+#pragma unroll
+    for (int w = 1; w < AF_WAVES; ++w) mm = fmaxf(mm, part_m[w][row]);
+    float ll = 0.f, v = 0.f;
+#pragma unroll
+    for (int w = 0; w < AF_WAVES; ++w) {
+      const float f = part_m[w][row] == -INFINITY ? 0.f : expf(part_m[w][row] - mm);
+      ll += part_l[w][row] * f;
+      v += smem[(w * 16 + row) * OLD + d] * f;
+    }
+    out[(size_t)(row0 + i0 + row) * out_ld + h * D + d] = ll > 0.f ? v / ll : 0.f;      // (a padding row: zeros)
+  }
+}
+
+// Attention of every row of a step (sequence s has the rows q_start[s] .. q_start[s + 1] - 1, the last of which sits at
+// position seq_lens[s] - 1; at most max_query_len rows) over its sequence's pages.
+extern "C" int da_attn_f32(const float* q, int q_ld, const float* cache, const int* block_table, int max_blocks, const int* q_start,
+                           const int* seq_lens, int n_seqs, int max_query_len, int Hq, int Hkv, int D, int page, float scale, int window,
+                           float* out, int out_ld, void* stream) {
+  DA_REQUIRE(n_seqs >= 0 && max_query_len > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0, "attn_f32: bad sizes (%d sequences, %d rows, %d and %d heads)",
+             n_seqs, max_query_len, Hq, Hkv);
+  DA_REQUIRE(D % 16 == 0 && D >= 16 && D <= 128, "attn_f32: head size %d is not a multiple of 16 up to 128", D);
+  DA_REQUIRE(page % 16 == 0 && (page & (page - 1)) == 0, "attn_f32: page size %d must be a power of two from 16 on", page);
+  DA_REQUIRE(q_ld >= Hq * D && out_ld >= Hq * D && q_ld % 4 == 0, "attn_f32: row lengths (q %d, out %d)", q_ld, out_ld);
+  DA_REQUIRE((uintptr_t)q % 16 == 0 && (uintptr_t)cache % 16 == 0, "attn_f32: q and the cache must be 16-byte aligned");
+  DA_REQUIRE(window >= 0 && max_blocks > 0, "attn_f32: bad window or block table");
+  if (n_seqs == 0) return 0;
+  const dim3 grid(n_seqs * Hq, da_ceil_div(max_query_len, 16)), block(AF_WAVES * DA_WAVE);
+#define AF_LAUNCH(X)                                                                                                            \
+  case X: hipLaunchKernelGGL(attn_f32_kernel<X>, grid, block, 0, (hipStream_t)stream, q, q_ld, cache, block_table, max_blocks, \
+                             q_start, seq_lens, Hq, Hkv, page, scale, window, out, out_ld); break
+  switch (D / 16) {
+    AF_LAUNCH(1); AF_LAUNCH(2); AF_LAUNCH(3); AF_LAUNCH(4); AF_LAUNCH(5); AF_LAUNCH(6); AF_LAUNCH(7);
+    default: hipLaunchKernelGGL(attn_f32_kernel<8>, grid, block, 0, (hipStream_t)stream, q, q_ld, cache, block_table, max_blocks,
+                                q_start, seq_lens, Hq, Hkv, page, scale, window, out, out_ld); break;
+  }
+#undef AF_LAUNCH
+  DA_CHECK_LAUNCH("attn_f32");
+  return 0;
+}

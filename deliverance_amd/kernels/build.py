@@ -35,7 +35,8 @@ HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
 EXTRA_FLAGS = {"attn_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_prefill_rel": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_latent_mfma": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-               "attn_window": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+               "attn_window": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+               "attn_f32": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 # The unit that holds the error message every entry point may leave; every other unit needs it.
 BASE_UNIT = "rowwise"
 # Units whose functions a unit calls.

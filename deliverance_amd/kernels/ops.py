@@ -91,6 +91,7 @@ _ARGTYPES = {
                          _I, _I, _I, _I, _I, _VP],
     "da_kv_write": [_VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _VP],
     "da_attn_ref": [_VP, _I, _VP, _I, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
+    "da_attn_f32": [_VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
     "da_attn_decode": [_VP, _I, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
     "da_attn_decode_split": [_VP, _I, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _I, _VP, ctypes.c_long, _VP],
     "da_attn_prefill": [_VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _I, _VP],
@@ -656,6 +657,26 @@ def attention_ref(q: torch.Tensor, cache_slot: torch.Tensor, block_table: torch.
     return out
 
 
+def attention_f32_takes(head_dim: int, page: int) -> bool:
+    """Whether ``attention_f32`` takes these sizes (the plain kernel takes the others)."""
+    return head_dim % 16 == 0 and 16 <= head_dim <= 128 and page % 16 == 0 and page & (page - 1) == 0
+
+
+def attention_f32(q: torch.Tensor, cache_slot: torch.Tensor, block_table: torch.Tensor, q_start: torch.Tensor,
+                  seq_lens: torch.Tensor, n_seqs: int, max_query_len: int, n_heads: int, scale: float,
+                  window: Optional[int], out: torch.Tensor) -> torch.Tensor:
+    """Paged attention in 32-bit on the matrix cores for the rows of ``n_seqs`` sequences, portions and one-token sequences
+    alike: sequence s has the rows q_start[s] .. q_start[s + 1] - 1, the last at position seq_lens[s] - 1."""
+    _dev(q, cache_slot, block_table, q_start, seq_lens, out)
+    Hkv, page, D = _attn_common(q, cache_slot, block_table, n_heads, out, "attention_f32", torch.float32)
+    _need(q_start.dtype == torch.int32 and q_start.numel() >= n_seqs + 1 and seq_lens.dtype == torch.int32
+          and seq_lens.numel() >= n_seqs and block_table.shape[0] >= n_seqs, "attention_f32: q_start int32 [S + 1], seq_lens int32 [S]")
+    _check(_lib().da_attn_f32(_ptr(q), q.stride(0), _ptr(cache_slot), _ptr(block_table), block_table.shape[1], _ptr(q_start),
+                              _ptr(seq_lens), n_seqs, max_query_len, n_heads, Hkv, D, page, scale, int(window or 0), _ptr(out),
+                              out.stride(0), _stream()))
+    return out
+
+
 def cache_page_elems(cache_slot: torch.Tensor) -> int:
     return cache_slot[0].numel()
 
@@ -765,7 +786,7 @@ def top_logprobs(logits: torch.Tensor, params: torch.Tensor, n: int, out_idx: to
 # ------------------------------------------------------------------------------- dispatch
 # "tuned": MFMA products and the prefill/decode attention kernels in bfloat16;
 # "reference": the plain kernels everywhere (for A/B checks).  32-bit runs its products on the matrix
-# cores' 32-bit instructions in "tuned" (csrc/gemm_f32.hip), everything else on the plain kernels.
+# cores' 32-bit instructions in "tuned" (csrc/gemm_f32.hip), and plain attention too (csrc/attn_f32.hip).
 _MODE = "tuned"
 
 
@@ -1038,7 +1059,7 @@ def linear_kv_split(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
     return out
 
 
-def _attn_common(q, cache_slot, block_table, n_heads, out, name):
+def _attn_common(q, cache_slot, block_table, n_heads, out, name, dtype=torch.bfloat16):
     _dev(q, cache_slot, block_table, out)
     _rows_2d(q, "q"); _rows_2d(out, "out")
     P, two, Hkv, page, D = cache_slot.shape
@@ -1046,8 +1067,7 @@ def _attn_common(q, cache_slot, block_table, n_heads, out, name):
         raise KernelError(f"{name}: cache slot must be contiguous [pages,2,Hkv,page,D]")
     if not (q.shape[1] == n_heads * D and out.shape[1] == n_heads * D):
         raise KernelError(f"{name}: q/out must be [rows, Hq*D]")
-    _need(q.dtype == torch.bfloat16 and cache_slot.dtype == torch.bfloat16 and out.dtype == torch.bfloat16,
-          f"{name}: q, cache and out must be bfloat16")
+    _need(q.dtype == cache_slot.dtype == out.dtype == dtype, f"{name}: q, cache and out must be {str(dtype)[6:]}")
     _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.is_contiguous(),
           f"{name}: block_table must be contiguous int32 [S, max_blocks]")
     return Hkv, page, D
@@ -1116,8 +1136,8 @@ def paged_attention(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: int, 
                     scale: float, window: Optional[int], out: torch.Tensor) -> torch.Tensor:
     """Attention of every row of the step over its sequence's pages.  In bfloat16 the one-token
     sequences (the first ``ctx.n_decode``) go to the decode kernel and the portions to the
-    prefill kernel; 32-bit, the reference mode and head sizes that are no multiple of 16 (which the
-    matrix-core kernels do not take) use the plain kernel for all rows."""
+    prefill kernel, in 32-bit both to one kernel; the reference mode and head sizes that are no multiple of 16
+    (which the matrix-core kernels do not take) use the plain kernel for all rows."""
     bt = ctx.block_tables[group]
     Hkv, page, D = cache_slot.shape[2], cache_slot.shape[3], cache_slot.shape[4]
     el = cache_slot.element_size()
@@ -1152,6 +1172,9 @@ def paged_attention(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: int, 
                 attention_prefill(q, cache_slot, bt, ctx.q_start, ctx.seq_lens, nd, ctx.n_seqs - nd,
                                   ctx.max_query_len, n_heads, scale, window, out)
         return out
+    if _MODE == "tuned" and q.dtype == torch.float32 and attention_f32_takes(D, page) and q.stride(0) % 4 == 0 and q.data_ptr() % 16 == 0:
+        with _timed("attention_f32", *cost(0, ctx.n_seqs), "fp32"):
+            return attention_f32(q, cache_slot, bt, ctx.q_start, ctx.seq_lens, ctx.n_seqs, ctx.max_query_len, n_heads, scale, window, out)
     with _timed("attention_plain", *cost(0, ctx.n_seqs), "fp32" if q.dtype == torch.float32 else "bf16"):
         return attention_ref(q, cache_slot, bt, ctx.seq_of_token, ctx.positions, n_heads, scale, window, out)
 

@@ -160,7 +160,7 @@ class CausalSelfAttention(Mixer):
             out += ("attn_rel",)
         D = self.head_dim
         if dtype != torch.bfloat16:
-            return out + (("attn_rel",) if self.extras else ("attn_ref",))
+            return out + (("attn_rel",) if self.extras else ("attn_ref", "attn_f32"))
         if not self.extras:
             return out + (("attn_decode", "attn_prefill") if D % 16 == 0 else ("attn_ref",))
         scores_only = self.v_head_dim == D and D % 16 == 0 and D <= 128 and self.softcap == 0.0 and not self.keep_first

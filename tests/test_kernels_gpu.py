@@ -390,6 +390,27 @@ def test_attention_plain_kernel(ops, dtype, Hq, Hkv, D, page, window):
 
 
 @pytest.mark.parametrize("Hq,Hkv,D,page,window", [helpers.quick(4, 4, 16, 16, None), (6, 2, 48, 16, None), helpers.quick(2, 1, 80, 32, 37),
+                                                  (3, 3, 128, 64, None), (12, 12, 64, 16, None), (5, 5, 64, 16, 100), (2, 1, 96, 16, 70),
+                                                  (2, 2, 112, 16, None)])
+def test_attention_32bit_on_the_matrix_cores(ops, Hq, Hkv, D, page, window):
+    """Portions and one-token sequences in one launch, chunk edges, a padding sequence; a row has the same bits however its
+    portion is cut."""
+    lens, new = [70, 5, 131, 64, 1, 65, 600, 129], [70, 1, 9, 17, 1, 1, 33, 129]
+    case = PagedCase(lens=lens, new=new, Hq=Hq, Hkv=Hkv, D=D, page=page, dtype=torch.float32, seed=D)
+    scale = 0.7 / math.sqrt(D)
+    out = torch.full_like(case.qcat, 7.0)
+    ops.attention_f32(case.qcat, case.cache, case.bt, case.q_start, case.seq_lens, len(lens), max(new), Hq, scale, window, out)
+    assert np.abs(out.double().cpu().numpy() - case.plain(scale, window)).max() < ATT_TOL[torch.float32]
+    # the last 5 rows of the last sequence alone, then a sequence of length 0
+    one = torch.full((6, Hq * D), 7.0, device=DEV)
+    q = torch.cat([case.qcat[-5:], case.qcat[:1]])
+    bt = torch.cat([case.bt[-1:], torch.full_like(case.bt[:1], -1)])
+    ops.attention_f32(q, case.cache, bt, torch.tensor([0, 5, 6], dtype=torch.int32, device=DEV),
+                      torch.tensor([129, 0], dtype=torch.int32, device=DEV), 2, 5, Hq, scale, window, one)
+    assert torch.equal(one[:5], out[-5:]) and not bool(one[5].any())
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,page,window", [helpers.quick(4, 4, 16, 16, None), (6, 2, 48, 16, None), helpers.quick(2, 1, 80, 32, 37),
                                                   (3, 3, 128, 64, None), (12, 12, 64, 16, None), (5, 5, 64, 16, 100),
                                                   helpers.quick(2, 2, 256, 16, None), (25, 25, 64, 32, 70)])
 def test_attention_decode_kernel(ops, Hq, Hkv, D, page, window):
