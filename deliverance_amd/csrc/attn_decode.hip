@@ -1,16 +1,23 @@
 // Paged attention for decode rows in bfloat16: one query row per sequence.
 //
-// One workgroup of 8 wavefronts per (sequence, query head).  The keys lo..p of the sequence
-// are walked in aligned chunks of 64; wavefront v takes chunks v, v+8, ... (two each at a
-// context of 1,024).  All loads of a phase are issued before any is used, so a chunk costs two
-// memory round trips.
-//   scores : CPR lanes share a key, each holding a 16-byte piece of the key row and the matching
-//            piece of q in registers; their partial dot products are added by lane exchange.
-//            One load instruction so covers 64 / CPR whole key rows that lie next to each other.
-//   softmax: every lane ends up with one key's score; running maximum and sum per wavefront
+// One workgroup of 8 or 16 wavefronts per (sequence, query head).  The keys lo..p of the sequence
+// are walked in aligned chunks of 64; wavefront v takes chunks v, v + 8 (16), ...  All loads of a chunk are
+// issued before any is used, so a chunk costs two memory round trips: the block table's entries, then keys
+// and values.  The arithmetic is on the matrix cores (MFMA 16x16x32), with one useful column in the first
+// product and three in the second: a single wavefront's chain of instructions, not the chip's rate, is what a
+// step of few requests waits for, and a chunk takes 16 instructions of 16 cycles here where it took about 700
+// of the vector unit (one head of 64, 512 keys: 6.0 -> 5.7 us a launch in a recorded chain, of which 1.6 are
+// the launch and about 2 the 130 KB that one compute unit pulls in; 64 sequences of 25 heads: 42.5 -> 40.7 us, 5.4 TB/s).
+//   scores : S[key, *] = K . q, 4 pieces of 16 keys (a lane holds row l % 16 and 8 dimensions, 16 bytes of the key
+//            row as it lies in the page; q is the same in all 16 columns).  Products of bfloat16 are exact and
+//            their sums 32-bit; the scale comes after.
+//   softmax: every lane of a quarter-wavefront holds the same 4 keys of each piece; it keeps the piece l % 4.
+//            Running maximum and sum per wavefront
 //            (the recurrence of native/src/main/resources/decode_paged_attention_f32.wgsl:31-65).
-//   values : values are stored dimension-major, so lane d reads 8 consecutive keys of its own
-//            dimension in 16 bytes and keeps one accumulator; no exchange between lanes.
+//   values : O[d, part] += V^T[d, key] . P[key, part]; values are stored dimension-major, so the left operand is
+//            16 bytes as they lie in the page.  The 32-bit weights lose nothing: column 0 takes a weight rounded to
+//            bfloat16, column 1 what is left rounded again, column 2 what is left of that (3 x 8 bits hold a 32-bit
+//            number's 24), and the three columns' sums are added at the end.
 // The wavefronts' partial results are merged in LDS in a fixed order.  Every sum's order
 // depends on p and lo only, never on the batch.
 //
@@ -24,7 +31,7 @@
 // whose exponential joins the softmax's denominator, without a key or a value and not scaled; and a gate, rows like out,
 // of which o is multiplied with the logistic function.  The last two act once, after everything has been merged.  The
 // plain build has none of that code.
-#include "common.h"
+#include "gemm_common.h"
 
 #define DEC_MAX_D 256
 
@@ -74,53 +81,53 @@ __device__ __forceinline__ float dec_gate(float z) {
 // of j.  The split depends on the step's shape only (pairs, widest block table), never on the
 // sequences' lengths, so a recorded graph can hold it.
 //
-// CPR: 16-byte pieces per key row, rounded up to a power of two (2..32)
-template <int CPR, int DEC_WAVES, bool SPLIT>
+// DK: dimensions in steps of 32, rounded up to a power of two (1, 2, 4, 8)
+template <int DK, int DEC_WAVES, bool SPLIT>
 // (registers are held to 128 for head sizes up to 64, so that two workgroups share a compute unit)
-__global__ void __launch_bounds__(DEC_WAVES * DA_WAVE, (CPR <= 8 || DEC_WAVES == 16) ? 4 : 2)
+__global__ void __launch_bounds__(DEC_WAVES * DA_WAVE, (DK <= 2 || DEC_WAVES == 16) ? 4 : 2)
 DEC_KERNEL(const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
            const int* __restrict__ block_table, int max_blocks,
            const int* __restrict__ seq_lens, int Hq, int Hkv, int D, int page, float scale,
            int window, bf16_t* __restrict__ out, int out_ld, int span, float* __restrict__ partial DEC_REL_PARAMS) {
-  constexpr int G = DA_WAVE / CPR;            // keys scored side by side
-  constexpr int DPL = CPR <= 8 ? 1 : CPR / 8; // value dimensions per lane: D <= 8 * CPR <= 64 * DPL
-  __shared__ __attribute__((aligned(16))) float ps[DEC_WAVES][DA_WAVE];
-  __shared__ float part_acc[DEC_WAVES][DPL * DA_WAVE];
+  constexpr int DV = 2 * DK;                  // pieces of 16 value dimensions
+  constexpr int DMAX = 32 * DK;
+  __shared__ __attribute__((aligned(16))) bf16_t ps[DEC_WAVES][4][DA_WAVE];     // a chunk's weights in three parts; part 3: zeros
+  __shared__ __attribute__((aligned(16))) float part_acc[DEC_WAVES][DMAX];
   __shared__ float part_m[DEC_WAVES], part_l[DEC_WAVES];
 
   const int s = blockIdx.x / Hq, h = blockIdx.x % Hq;
   const int hk = h / (Hq / Hkv);
-  const int t = threadIdx.x, lane = t % DA_WAVE, wave = t / DA_WAVE;
+  const int t = threadIdx.x, lane = t % DA_WAVE, wave = __builtin_amdgcn_readfirstlane(t / DA_WAVE);
+  const int col = lane % 16, quad = lane / 16;
   const int* bt = block_table + (size_t)s * max_blocks;
   // addressing by shifts: the page size is a power of two (checked on the host)
   const int lg = 31 - __builtin_clz(page), pmask = page - 1;
-  const long long page_elems = 2LL * Hkv * page * D;
-  const bf16_t* kbase = cache + (long long)hk * page * D;
-  const bf16_t* vbase = cache + (long long)(Hkv + hk) * page * D;
-  const int piece = lane % CPR, sub = lane / CPR;
-  const bool piece_ok = piece * 8 < D;
+  const uint32_t page_bytes = 4u * (uint32_t)(Hkv * page * D);
+  const char* kbase = (const char*)(cache + (long long)hk * page * D);
+  const char* vbase = (const char*)(cache + (long long)(Hkv + hk) * page * D);
 
-  // Asked for before the sequence's length is known, so that they travel beside it: the query (as
-  // raw bits; converted where it is used) and the block-table entries of the chunk this wavefront
-  // starts with when nothing is cut off by a window (keys wave*64 ..).  Entries past the
-  // sequence's pages are read (the table has max_blocks of them) and never used.
-  const uint4 qraw = *(const uint4*)(q + (size_t)s * q_ld + h * D + (piece_ok ? piece * 8 : 0));
+  // Asked for before the sequence's length is known, so that they travel beside it: the query and the
+  // block-table entries of the chunk this wavefront starts with when nothing is cut off by a window
+  // (keys wave*64 ..).  Entries past the sequence's pages are read (the table has max_blocks of them) and
+  // never used.  A lane's dimensions past D (a head size that is no multiple of 32) meet zeros of q.
+  uint4 qf[DK];
+#pragma unroll
+  for (int k = 0; k < DK; ++k) {
+    const int d = 32 * k + 8 * quad;
+    qf[k] = *(const uint4*)(q + (size_t)s * q_ld + h * D + (d < D ? d : 0));
+  }
   const int split0 = SPLIT ? (int)blockIdx.y * span : 0;          // the first key of this workgroup's share
   const int c0_guess = split0 + wave * DA_WAVE;
-  // (head sizes above 128 have no registers to spare for them and read the table chunk by chunk)
-  constexpr bool EARLY_BT = CPR <= 16;
-  int btk0[EARLY_BT ? CPR : 1], btv0[EARLY_BT ? 8 : 1];
-  if (EARLY_BT) {
+  int btk0[4], btv0[2];
 #pragma unroll
-    for (int i = 0; i < (EARLY_BT ? CPR : 1); ++i) {
-      const int pg = (c0_guess + i * G + sub) >> lg;
-      btk0[i] = bt[pg < max_blocks ? pg : max_blocks - 1];
-    }
+  for (int j = 0; j < 4; ++j) {
+    const int pg = (c0_guess + 16 * j + col) >> lg;
+    btk0[j] = bt[pg < max_blocks ? pg : max_blocks - 1];
+  }
 #pragma unroll
-    for (int g = 0; g < (EARLY_BT ? 8 : 1); ++g) {
-      const int pg = (c0_guess + g * 8) >> lg;
-      btv0[g] = bt[pg < max_blocks ? pg : max_blocks - 1];
-    }
+  for (int g = 0; g < 2; ++g) {
+    const int pg = (c0_guess + 32 * g + 8 * quad) >> lg;
+    btv0[g] = bt[pg < max_blocks ? pg : max_blocks - 1];
   }
 #ifdef DEC_REL
   // asked for here, used at the end
@@ -145,196 +152,190 @@ DEC_KERNEL(const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ ca
 #else
   const float qscale = scale;
 #endif
-
-  float acc[DPL];
 #pragma unroll
-  for (int i = 0; i < DPL; ++i) acc[i] = 0.f;
+  for (int k = 0; k < DK; ++k)
+    if (32 * k + 8 * quad >= D) qf[k] = make_uint4(0, 0, 0, 0);
+
+  floatx4 acc[DV];
+#pragma unroll
+  for (int i = 0; i < DV; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
 
   for (int c0 = (lo / DA_WAVE) * DA_WAVE + wave * DA_WAVE; c0 <= p; c0 += DEC_WAVES * DA_WAVE) {
-    // ---- all loads of the chunk first: the key pieces of the score phase and the value groups
-    // of the weighted sum (both need only the block table), then the arithmetic
-    float mine = -INFINITY;      // one key's score per lane, once the loop is done
-    uint4 kv[CPR];
     const int first = c0 > lo ? c0 : lo;                 // valid keys of the chunk: first..last
     const int last = c0 + DA_WAVE - 1 < p ? c0 + DA_WAVE - 1 : p;
     // the pages of the chunk's keys and value groups: those asked for at the start, or read now
-    int btk[CPR], btv[8], bt_safe;
-    if (EARLY_BT && c0 == c0_guess && first == c0) {     // the same for the whole wavefront
+    int btk[4], btv[2], bt_safe;
+    if (c0 == c0_guess && first == c0) {                 // the same for the whole wavefront
 #pragma unroll
-      for (int i = 0; i < CPR; ++i) btk[i] = btk0[EARLY_BT ? i : 0];
-#pragma unroll
-      for (int g = 0; g < 8; ++g) btv[g] = btv0[EARLY_BT ? g : 0];
+      for (int j = 0; j < 4; ++j) btk[j] = btk0[j];
+      btv[0] = btv0[0];
+      btv[1] = btv0[1];
       bt_safe = __builtin_amdgcn_readfirstlane(btk0[0]); // lane 0 holds the page of key c0
-    } else if (CPR == 32) {
-      // Two keys a load, both in one page (a page has 8 rows at least), and the chunk is the same for
-      // the whole wavefront: the table entries are read by the scalar unit and take no vector registers,
-      // which this head size has none to spare of.
-      const int c0u = __builtin_amdgcn_readfirstlane(c0), fu = __builtin_amdgcn_readfirstlane(first),
-                lu = __builtin_amdgcn_readfirstlane(last);
-      bt_safe = __builtin_amdgcn_readfirstlane(bt[fu >> lg]);
-#pragma unroll
-      for (int i = 0; i < CPR; ++i) {
-        const int k0 = c0u + i * G;                      // the load's first key; G = 2
-        btk[i] = __builtin_amdgcn_readfirstlane(bt[((k0 + G - 1 >= fu && k0 <= lu) ? k0 : fu) >> lg]);
-      }
-#pragma unroll
-      for (int g = 0; g < 8; ++g) {
-        const int g0 = c0u + g * 8;
-        btv[g] = __builtin_amdgcn_readfirstlane(bt[((g0 + 7 >= fu && g0 <= lu) ? g0 : fu) >> lg]);
-      }
     } else {
       bt_safe = bt[first >> lg];
 #pragma unroll
-      for (int i = 0; i < CPR; ++i) {
-        const int key = c0 + i * G + sub;
-        btk[i] = bt[((key >= first && key <= last) ? key : first) >> lg];
+      for (int j = 0; j < 4; ++j) {
+        const int key = c0 + 16 * j + col;
+        btk[j] = bt[((key >= first && key <= last) ? key : first) >> lg];
       }
 #pragma unroll
-      for (int g = 0; g < 8; ++g) {
-        const int g0 = c0 + g * 8;
+      for (int g = 0; g < 2; ++g) {
+        const int g0 = c0 + 32 * g + 8 * quad;
         btv[g] = bt[((g0 + 7 >= first && g0 <= last) ? g0 : first) >> lg];
       }
     }
-    // a key that is not seen reads `first` instead, a row that surely exists
+    // ---- all loads of the chunk, then the arithmetic.  A key that is not seen reads `first` instead, a row that
+    // surely exists; of the values, a group of 8 keys (which never crosses a page) without a seen key reads the group
+    // of `first` instead.  Both are dropped.
+    // (head sizes above 128 have no registers for all of it: two pieces of keys at a time, the values once the scores
+    // are done, half of the chunk at a time)
+    constexpr bool EARLY_V = DK <= 4;
+    constexpr int KJ = EARLY_V ? 4 : 2, VG = EARLY_V ? 2 : 1;
+    uint4 kf[KJ][DK], vf[VG][DV];
+    floatx4 sc[4];
+    auto load_k = [&](int j0) {
 #pragma unroll
-    for (int i = 0; i < CPR; ++i) {
-      const int key = c0 + i * G + sub;
-      const bool valid = key >= lo && key <= p;
-      // (CPR 32: btk[i] is the pair's page, or the page of `first` if neither key is seen, the same for every
-      // lane: the page's address stays with the scalar unit; a lane whose own key is not seen reads some row of it)
-      const long long pg = CPR == 32 ? btk[i] : (valid ? btk[i] : bt_safe);
-      const int kk = valid ? key : first;
-      kv[i] = *(const uint4*)(kbase + pg * page_elems + (kk & pmask) * D + (piece_ok ? piece * 8 : 0));
-    }
-    // the chunk's 8 groups of 8 keys (a group never crosses a page) of this lane's first dimension;
-    // groups with no seen key read the group of `first` instead and are dropped
-    // (head sizes above 128 hold 128 registers of keys at this point: their values are asked for once the
-    // scores are done, all dimensions at once)
-    constexpr bool EARLY_V = CPR <= 16;
-    uint4 vv0[8];
-    if (EARLY_V) {
-      const int d = lane < D ? lane : 0;
+      for (int j = 0; j < KJ; ++j) {
+        const int key = c0 + 16 * (j0 + j) + col;
+        const bool valid = key >= first && key <= last;
+        const char* kp = kbase + (uint64_t)(uint32_t)(valid ? btk[j0 + j] : bt_safe) * page_bytes +
+                         (uint32_t)(2 * (((valid ? key : first) & pmask) * D + (DK > 1 || 8 * quad < D ? 8 * quad : 0)));
 #pragma unroll
-      for (int g = 0; g < 8; ++g) {
-        const int g0 = c0 + g * 8;
-        const bool any = g0 + 7 >= first && g0 <= last;
-        const int gs = any ? g0 : (first / 8) * 8;
-        const long long pg = any ? btv[g] : bt_safe;
-        vv0[g] = *(const uint4*)(vbase + pg * page_elems + d * page + (gs & pmask));
+        for (int k = 0; k < DK; ++k)         // (D > 16 DK: only the upper half of the steps can lie past D; there the first step is read)
+          kf[j][k] = *(const uint4*)(kp + (2 * k + 1 < DK || 32 * k + 8 * quad < D ? 64 * k : 0));
       }
-    }
+    };
+    auto scores = [&](int j0) {
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) sc[j0 + j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < DK; ++k)
+#pragma unroll
+        for (int j = 0; j < KJ; ++j)
+          sc[j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[j][k]), __builtin_bit_cast(bf16x8_t, qf[k]), sc[j0 + j], 0, 0, 0);
+    };
+    auto load_v = [&](int g0_) {
+#pragma unroll
+      for (int g = 0; g < VG; ++g) {
+        const int g0 = c0 + 32 * (g0_ + g) + 8 * quad;
+        const bool any = g0 + 7 >= first && g0 <= last;
+        const int gs = any ? g0 : (first & ~7);
+        const char* vp = vbase + (uint64_t)(uint32_t)(any ? btv[g0_ + g] : bt_safe) * page_bytes + (uint32_t)(2 * ((gs & pmask) + col * page));
+#pragma unroll
+        for (int i = 0; i < DV; ++i) {
+          vf[g][i] = *(const uint4*)vp;
+          vp += 16 * (i + 1) < D ? 32 * page : 0;        // (a whole piece past D reads the last one again and is dropped)
+        }
+      }
+    };
 #ifdef DEC_REL
-    // the bias of the key whose score this lane will keep, asked for beside the keys and values (a key past the
+    // the biases of the keys whose scores this lane will keep, asked for in front of the keys and values (a key past the
     // row's own position has no distance: it reads entry 0 and is dropped with its score)
-    float brel = 0.f;
-    if (slopes) brel = -slope * (float)(p_row - (c0 + piece * G + sub));
-    if (brow) {
-      const int dist = p_row - (c0 + piece * G + sub);
-      brel += brow[dist < 0 ? 0 : (dist < n_dist ? dist : n_dist - 1)];
+    float brel[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int dist = p_row - (c0 + 16 * (col % 4) + 4 * quad + r);
+      brel[r] = slopes ? -slope * (float)dist : 0.f;
+      if (brow) brel[r] += brow[dist < 0 ? 0 : (dist < n_dist ? dist : n_dist - 1)];
     }
 #endif
+    load_k(0);
+    if (EARLY_V) load_v(0);
     // nothing moves across this line: the compiler would otherwise push the value loads down behind
     // the scores to save registers, and a chunk would cost a third memory round trip
     __builtin_amdgcn_sched_barrier(0);
-    float qf[8];
-    {
-      const uint32_t u[4] = {qraw.x, qraw.y, qraw.z, qraw.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        qf[2 * e] = piece_ok ? __uint_as_float(u[e] << 16) * qscale : 0.f;
-        qf[2 * e + 1] = piece_ok ? __uint_as_float(u[e] & 0xffff0000u) * qscale : 0.f;
-      }
+    scores(0);
+    if (!EARLY_V) {
+      load_k(EARLY_V ? 0 : 2);
+      scores(EARLY_V ? 0 : 2);
     }
+    // this lane's 4 keys: rows 4 * quad + r of piece col % 4
+    const int key0 = c0 + 16 * (col % 4) + 4 * quad;
+    float sv[4], e[4];
 #pragma unroll
-    for (int i = 0; i < CPR; ++i) {
-      const int key = c0 + i * G + sub;
-      const bool valid = key >= lo && key <= p;
-      const uint32_t u[4] = {kv[i].x, kv[i].y, kv[i].z, kv[i].w};
-      float dot = 0.f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        dot = fmaf(qf[2 * e], __uint_as_float(u[e] << 16), dot);
-        dot = fmaf(qf[2 * e + 1], __uint_as_float(u[e] & 0xffff0000u), dot);
-      }
-      dot = group_sum<CPR>(dot);
-      // all CPR lanes of the group now hold the score; the lane whose piece number is i keeps it
-      if (piece == i) mine = valid ? dot : -INFINITY;
-    }
-    const int kidx = piece * G + sub;                 // which key of the chunk this lane kept
-    const int key = c0 + kidx;
-    const bool valid = key >= lo && key <= p;
+    for (int r = 0; r < 4; ++r) {
+      const float s01 = col & 1 ? sc[1][r] : sc[0][r], s23 = col & 1 ? sc[3][r] : sc[2][r];
+      sv[r] = (col & 2 ? s23 : s01) * qscale;
 #ifdef DEC_REL
-    mine += brel;                                     // (-inf stays -inf)
+      sv[r] += brel[r];
 #endif
-    const float m_new = fmaxf(m, wave_max(mine));
-    const float e = valid ? dec_exp(mine - m_new) : 0.f;
-    const float alpha = dec_exp(m - m_new);
-    l = l * alpha + wave_sum(e);
+      sv[r] = key0 + r >= first && key0 + r <= last ? sv[r] : -INFINITY;
+    }
+    const float m_new = fmaxf(m, wave_max(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]))));
+    const float alpha = dec_exp(m - m_new);              // (a chunk that is walked has a seen key: m_new is finite)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) e[r] = dec_exp(sv[r] - m_new);
+    l = l * alpha + 0.25f * wave_sum((e[0] + e[1]) + (e[2] + e[3]));      // (four lanes hold each key)
     m = m_new;
-    ps[wave][kidx] = e;
+    {
+      // lane group col / 4 = 0, 1, 2 parks the first, second, third part of its 4 weights, group 3 zeros
+      const int part = col / 4;
+      uint32_t w2[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float a = e[2 * i], b = e[2 * i + 1];
+        const uint32_t p0 = pack2_bf16(a, b);
+        const float a1 = a - __uint_as_float(p0 << 16), b1 = b - __uint_as_float(p0 & 0xffff0000u);
+        const uint32_t p1 = pack2_bf16(a1, b1);
+        const uint32_t p2 = pack2_bf16(a1 - __uint_as_float(p1 << 16), b1 - __uint_as_float(p1 & 0xffff0000u));
+        w2[i] = part == 0 ? p0 : (part == 1 ? p1 : (part == 2 ? p2 : 0u));
+      }
+      *(uint2*)&ps[wave][part][16 * (col % 4) + 4 * quad] = make_uint2(w2[0], w2[1]);
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");   // LDS only: the value loads stay in flight
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    // ---- values: lane owns dimensions lane, lane + 64, ...; what was not asked for ahead of the scores is
-    // asked for now, every dimension's loads before any is used
-    uint4 vall[DPL][8];
-    if (!EARLY_V) __builtin_amdgcn_sched_barrier(0);    // (not moved up among the scores: the keys' registers are free only now)
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) {
-      if (EARLY_V && i == 0) {
+    for (int i = 0; i < DV; ++i)
 #pragma unroll
-        for (int g = 0; g < 8; ++g) vall[0][g] = vv0[g];
-      } else {
-        const int di = lane + i * DA_WAVE, d = di < D ? di : 0;
+      for (int r = 0; r < 4; ++r) acc[i][r] *= alpha;
+    const bool cut = first != c0 || last != c0 + DA_WAVE - 1;         // the same for the whole wavefront
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-          const int g0 = c0 + g * 8;
-          const bool any = g0 + 7 >= first && g0 <= last;
-          const int gs = any ? g0 : (first / 8) * 8;
-          const long long pg = any ? btv[g] : bt_safe;
-          vall[i][g] = *(const uint4*)(vbase + pg * page_elems + d * page + (gs & pmask));
-        }
+    for (int g = 0; g < 2; ++g) {
+      uint4 (&v)[DV] = vf[EARLY_V ? g : 0];
+      if (!EARLY_V) {
+        __builtin_amdgcn_sched_barrier(0);               // (not moved up among the scores: the keys' registers are free only now)
+        load_v(EARLY_V ? 0 : g);
       }
-    }
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) {
-      const int d = lane + i * DA_WAVE;
-      if (DPL > 1 && d >= D) break;
-      float a = acc[i] * alpha;
-      const uint4* vv = vall[i];
-#pragma unroll
-      for (int g = 0; g < 8; ++g) {
+      const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, *(const uint4*)&ps[wave][col < 3 ? col : 3][32 * g + 8 * quad]);
+      if (cut) {
         // Rows outside first..last were never written (or belong to someone else) and may hold anything:
-        // their bits are cleared.  The seen rows of a group are g0+lo8 .. g0+hi8; the masks are the same
-        // for every lane, so the scalar unit builds them.
-        const int g0 = c0 + g * 8;
-        const int lo8 = first - g0 > 0 ? first - g0 : 0, hi8 = last - g0 < 7 ? last - g0 : 7;
+        // their bits are cleared.  The seen rows of the lane's group are g0 + lo8 .. g0 + hi8.
+        const int g0 = c0 + 32 * g + 8 * quad;
+        const int lo8 = first - g0, hi8 = last - g0;
         uint32_t msk[4];
 #pragma unroll
-        for (int e2 = 0; e2 < 4; ++e2)
-          msk[e2] = ((2 * e2 >= lo8 && 2 * e2 <= hi8) ? 0x0000ffffu : 0u) |
-                    ((2 * e2 + 1 >= lo8 && 2 * e2 + 1 <= hi8) ? 0xffff0000u : 0u);
-        const uint32_t u[4] = {vv[g].x & msk[0], vv[g].y & msk[1], vv[g].z & msk[2], vv[g].w & msk[3]};
-        const float4 w0 = *(const float4*)&ps[wave][g * 8];
-        const float4 w1 = *(const float4*)&ps[wave][g * 8 + 4];
-        const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+        for (int w = 0; w < 4; ++w)
+          msk[w] = ((2 * w >= lo8 && 2 * w <= hi8) ? 0x0000ffffu : 0u) | ((2 * w + 1 >= lo8 && 2 * w + 1 <= hi8) ? 0xffff0000u : 0u);
 #pragma unroll
-        for (int e2 = 0; e2 < 4; ++e2) {
-          a = fmaf(w[2 * e2], __uint_as_float(u[e2] << 16), a);
-          a = fmaf(w[2 * e2 + 1], __uint_as_float(u[e2] & 0xffff0000u), a);
+        for (int i = 0; i < DV; ++i) {
+          v[i].x &= msk[0];
+          v[i].y &= msk[1];
+          v[i].z &= msk[2];
+          v[i].w &= msk[3];
         }
       }
-      acc[i] = a;
+#pragma unroll
+      for (int i = 0; i < DV; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, v[i]), pf, acc[i], 0, 0, 0);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");   // LDS only: the value loads stay in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   }
+  // a lane holds dimensions 16 i + 4 * quad + r of part col; parts 0..2 (and the zeros of column 3) are added.  (An
+  // infinite value stays what the first part makes of it: the other parts may be zero or of the other sign.)
 #pragma unroll
-  for (int i = 0; i < DPL; ++i) {
-    const int d = lane + i * DA_WAVE;
-    if (d < D) part_acc[wave][d] = acc[i];
+  for (int i = 0; i < DV; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float sum = group_sum<4>(acc[i][r]);
+      acc[i][r] = fabsf(acc[i][r]) < INFINITY ? sum : acc[i][r];
+    }
+  if (col == 0) {
+#pragma unroll
+    for (int i = 0; i < DV; ++i) *(floatx4*)&part_acc[wave][16 * i + 4 * quad] = acc[i];
   }
   if (lane == 0) { part_m[wave] = m; part_l[wave] = l; }
   __syncthreads();
@@ -432,10 +433,9 @@ static int decode_checks(const void* q, int q_ld, const void* cache, int max_blo
 static int decode_launch(const void* q, int q_ld, const void* cache, const int* block_table, int max_blocks,
                          const int* seq_lens, int S, int Hq, int Hkv, int D, int page, float scale, int window,
                          void* out, int out_ld, int n_splits, int span, float* partial, hipStream_t st DEC_REL_DECL) {
-  const int pieces = D / 8;
   // 8 wavefronts; 16 where the workgroups are no more than the compute units (a context above 512 is then
   // still one chunk a wavefront, and the larger workgroup's start is paid once per compute unit)
-  const bool wide = (long)S * Hq * n_splits <= 256 && pieces <= 8;     // larger heads need the registers of 8 wavefronts
+  const bool wide = (long)S * Hq * n_splits <= 256 && D <= 64;         // larger heads need the registers of 8 wavefronts
   dim3 grid(S * Hq, n_splits);
 #define LAUNCH3(C, W, SP)                                                                                   \
   hipLaunchKernelGGL((DEC_KERNEL<C, W, SP>), grid, dim3(W * DA_WAVE), 0, st, (const bf16_t*)q, q_ld, \
@@ -443,11 +443,10 @@ static int decode_launch(const void* q, int q_ld, const void* cache, const int* 
                      (bf16_t*)out, out_ld, span, partial DEC_REL_ARGS)
 #define LAUNCH2(C, W) do { if (n_splits > 1) LAUNCH3(C, W, true); else LAUNCH3(C, W, false); } while (0)
 #define LAUNCH(C) do { if (wide) LAUNCH2(C, 16); else LAUNCH2(C, 8); } while (0)
-  if (pieces <= 2) LAUNCH(2);
-  else if (pieces <= 4) LAUNCH(4);
-  else if (pieces <= 8) LAUNCH(8);
-  else if (pieces <= 16) LAUNCH2(16, 8);
-  else LAUNCH2(32, 8);
+  if (D <= 32) LAUNCH(1);
+  else if (D <= 64) LAUNCH(2);
+  else if (D <= 128) LAUNCH2(4, 8);
+  else LAUNCH2(8, 8);
 #undef LAUNCH
 #undef LAUNCH2
 #undef LAUNCH3
