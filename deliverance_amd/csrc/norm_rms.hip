@@ -2,9 +2,10 @@
 //
 //   rms(x)[i] = x[i] / sqrt(mean(x^2) + eps) * (offset + w[i])
 //
-// `offset` is 0 for a gain stored as it is applied and 1 for a gain stored around zero.  One wavefront
-// owns a row; where the width allows it the whole row sits in registers, so every load is in flight at
-// once and the row is read once.
+// `offset` is 0 for a gain stored as it is applied and 1 for a gain stored around zero.  A workgroup of
+// four wavefronts owns a row; where the width allows it the whole row sits in registers, so every load is in flight
+// at once and the row is read once.  (Four wavefronts a row and not one: with few rows the chain of instructions
+// behind the loads is what the kernel takes.)
 //
 //   da_rmsnorm      y = rms(x[rows[r]] or x[r])                       (32-bit or bfloat16 out)
 //   da_rmsnorm_add  x += rms_a(src);  h = rms_b(x), or x itself converted (optional)   the norm behind a part, the residual
@@ -28,46 +29,52 @@ __device__ __forceinline__ void rms_store4(void* y, int y_dtype, size_t at, floa
   }
 }
 
-// VPL float4 a lane: E a multiple of 4, E <= 256 * VPL.  ADD: src is normalised with (wa), added into x,
+#define RMS_WAVES 4
+
+// the sum over the row's wavefronts, in every lane; `red` is used once
+__device__ __forceinline__ float rms_row_sum(float v, float* red) {
+  v = wave_sum(v);
+  if (threadIdx.x % DA_WAVE == 0) red[threadIdx.x / DA_WAVE] = v;
+  lds_barrier();
+  return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// VPL float4 a lane: E a multiple of 4, E <= 1024 * VPL.  ADD: src is normalised with (wa), added into x,
 // and (if h) the new x is normalised with (wb) into h.  !ADD: y = rms(x) with wa.
 template <int VPL, bool ADD>
-__global__ void __launch_bounds__(4 * DA_WAVE)
+__global__ void __launch_bounds__(RMS_WAVES * DA_WAVE)
 rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, const void* __restrict__ wa, int wa_dtype,
                    float* __restrict__ x, const void* __restrict__ wb, int wb_dtype, float offset, float eps,
-                   void* __restrict__ y, int y_dtype, int R, int E) {
-  const int lane = threadIdx.x % DA_WAVE;
-  const int r = blockIdx.x * (blockDim.x / DA_WAVE) + threadIdx.x / DA_WAVE;
-  if (r >= R) return;
+                   void* __restrict__ y, int y_dtype, int E) {
+  __shared__ float red[2][RMS_WAVES];
+  constexpr int STRIDE = 4 * RMS_WAVES * DA_WAVE;
+  const int r = blockIdx.x, c0 = (int)threadIdx.x * 4;
   const float* sr = src + (size_t)(rows ? rows[r] : r) * E;
-  // Up to a width of 1,024 the gains are asked for beside the rows, so that the kernel costs one round trip
-  // to memory and not one per norm; wider rows have no registers to spare for that and read them when needed.
-  constexpr bool EARLY = VPL <= 4;
-  float4 v[VPL], xv[VPL], ga[EARLY ? VPL : 1], gb[EARLY ? VPL : 1];
+  // the gains are asked for beside the rows, so that the kernel costs one round trip to memory and not one per norm
+  float4 v[VPL], xv[VPL], ga[VPL], gb[VPL];
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
-    const int c = (lane + i * DA_WAVE) * 4;
+    const int c = c0 + i * STRIDE;
     v[i] = *(const float4*)(sr + (c < E ? c : 0));
     if (ADD) xv[i] = *(const float4*)(x + (size_t)r * E + (c < E ? c : 0));
   }
-  if (EARLY) {
 #pragma unroll
-    for (int i = 0; i < (EARLY ? VPL : 1); ++i) {
-      const int c = (lane + i * DA_WAVE) * 4, cc = c < E ? c : 0;
-      ga[i] = rms_param4(wa, wa_dtype, cc);
-      if (ADD && y && wb) gb[i] = rms_param4(wb, wb_dtype, cc);
-    }
+  for (int i = 0; i < VPL; ++i) {
+    const int c = c0 + i * STRIDE, cc = c < E ? c : 0;
+    ga[i] = rms_param4(wa, wa_dtype, cc);
+    if (ADD && y && wb) gb[i] = rms_param4(wb, wb_dtype, cc);
   }
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL; ++i)
-    q += ((lane + i * DA_WAVE) * 4 < E ? 1.f : 0.f) * ((v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w));
-  const float inv = 1.0f / sqrtf(wave_sum(q) / (float)E + eps);
+    if (c0 + i * STRIDE < E) q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+  const float inv = 1.0f / sqrtf(rms_row_sum(q, red[0]) / (float)E + eps);
   float q2 = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
-    const int c = (lane + i * DA_WAVE) * 4;
+    const int c = c0 + i * STRIDE;
     if (c < E) {
-      const float4 g = EARLY ? ga[EARLY ? i : 0] : rms_param4(wa, wa_dtype, c);
+      const float4 g = ga[i];
       float4 o = make_float4(v[i].x * inv * (offset + g.x), v[i].y * inv * (offset + g.y),
                              v[i].z * inv * (offset + g.z), v[i].w * inv * (offset + g.w));
       if (ADD) {
@@ -83,16 +90,16 @@ rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, 
   if (ADD && y && !wb) {                               // no second norm: the new x itself, converted
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      const int c = (lane + i * DA_WAVE) * 4;
+      const int c = c0 + i * STRIDE;
       if (c < E) rms_store4(y, y_dtype, (size_t)r * E + c, xv[i]);
     }
   } else if (ADD && y) {
-    const float inv2 = 1.0f / sqrtf(wave_sum(q2) / (float)E + eps);
+    const float inv2 = 1.0f / sqrtf(rms_row_sum(q2, red[1]) / (float)E + eps);
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      const int c = (lane + i * DA_WAVE) * 4;
+      const int c = c0 + i * STRIDE;
       if (c < E) {
-        const float4 g = EARLY ? gb[EARLY ? i : 0] : rms_param4(wb, wb_dtype, c);
+        const float4 g = gb[i];
         rms_store4(y, y_dtype, (size_t)r * E + c,
                    make_float4(xv[i].x * inv2 * (offset + g.x), xv[i].y * inv2 * (offset + g.y),
                                xv[i].z * inv2 * (offset + g.z), xv[i].w * inv2 * (offset + g.w)));
@@ -138,16 +145,13 @@ static void rms_launch(const float* src, const int* rows, const void* wa, int wa
                        int wb_dtype, float offset, float eps, void* y, int y_dtype, int R, int E, hipStream_t st) {
   const bool aligned = ((uintptr_t)src % 16 == 0) && ((uintptr_t)y % 16 == 0) && ((uintptr_t)wa % 16 == 0) &&
                        ((uintptr_t)wb % 16 == 0) && ((uintptr_t)x % 16 == 0);
-  const int wpb = R >= 512 ? 4 : 1;
-#define RMS_LAUNCH(V)                                                                                                  \
-  hipLaunchKernelGGL((rmsnorm_row_kernel<V, ADD>), dim3(da_ceil_div(R, wpb)), dim3(wpb * DA_WAVE), 0, st, src, rows, wa, \
-                     wa_dtype, x, wb, wb_dtype, offset, eps, y, y_dtype, R, E)
+#define RMS_LAUNCH(V)                                                                                              \
+  hipLaunchKernelGGL((rmsnorm_row_kernel<V, ADD>), dim3(R), dim3(RMS_WAVES * DA_WAVE), 0, st, src, rows, wa, wa_dtype, x, \
+                     wb, wb_dtype, offset, eps, y, y_dtype, E)
   if (E % 4 == 0 && E <= 4096 && aligned) {
-    if (E <= 256) RMS_LAUNCH(1);
-    else if (E <= 512) RMS_LAUNCH(2);
-    else if (E <= 1024) RMS_LAUNCH(4);
-    else if (E <= 2048) RMS_LAUNCH(8);
-    else RMS_LAUNCH(16);
+    if (E <= 1024) RMS_LAUNCH(1);
+    else if (E <= 2048) RMS_LAUNCH(2);
+    else RMS_LAUNCH(4);
   } else {
     hipLaunchKernelGGL((rmsnorm_any_kernel<ADD>), dim3(da_ceil_div(R, 4)), dim3(4 * DA_WAVE), 0, st, src, rows, wa,
                        wa_dtype, x, wb, wb_dtype, offset, eps, y, y_dtype, R, E);

@@ -205,35 +205,47 @@ __device__ __forceinline__ float4 load_param4(const void* p, int dtype, int i) {
 }
 
 // The same norm with the whole row held in registers: every load of the row is in flight at
-// once, which is what counts when a step has a handful of rows.  E a multiple of 4, E <= 256*VPL.
-// A workgroup is one wavefront (few rows: as many compute units as rows) or four (many rows: fewer,
-// fuller workgroups).
+// once, which is what counts when a step has a handful of rows.  E a multiple of 4, E <= 1024 * VPL.
+// A workgroup of four wavefronts is one row, a float4 a lane (two above a width of 1,024): the chain of
+// instructions behind the loads, not the bytes, is what the kernel takes (measured in a recorded chain
+// behind the kernel that writes x, one wavefront a row -> four: 64 rows of 768 2.4 -> 2.2 us, of 1,024 2.5 -> 2.1,
+// of 1,600 3.1 -> 2.5; 2,048 rows of 1,600 9.4 -> 8.9, of 1,024 level), whatever the rows, so that a row's sums keep
+// their order.
 // Loads come back in the order they were asked for: the row first, then gain and bias, as raw bits
 // that are converted where they are used (a conversion right after its load, or a load inside a
-// branch, is waited for on the spot).  PBF16: gain and bias are bfloat16 (else 32-bit).
-template <int VPL, bool PBF16>
-__global__ void __launch_bounds__(4 * DA_WAVE)
+// branch, is waited for on the spot).  PBF16: gain and bias are bfloat16 (else 32-bit); YBF16: y is.
+#define LN_WAVES 4
+
+// the sum over the row's wavefronts, in every lane; `red` is used once
+__device__ __forceinline__ float ln_row_sum(float v, float* red) {
+  v = wave_sum(v);
+  if (threadIdx.x % DA_WAVE == 0) red[threadIdx.x / DA_WAVE] = v;
+  lds_barrier();
+  return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+template <int VPL, bool PBF16, bool YBF16>
+__global__ void __launch_bounds__(LN_WAVES * DA_WAVE)
 layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                      const void* __restrict__ w, const void* __restrict__ b,
-                     float eps, void* __restrict__ y, int y_dtype, int R, int E) {
-  const int lane = threadIdx.x % DA_WAVE;
-  const int r = blockIdx.x * (blockDim.x / DA_WAVE) + threadIdx.x / DA_WAVE;
-  if (r >= R) return;
+                     float eps, void* __restrict__ y, int E) {
+  __shared__ float red[2][LN_WAVES];
+  constexpr int STRIDE = 4 * LN_WAVES * DA_WAVE;
+  const int r = blockIdx.x, c0 = (int)threadIdx.x * 4;
   const float* xr = x + (size_t)(rows ? rows[r] : r) * E;
   // every load of the row, of the gain and of the bias is asked for at once (past the row's end
   // the row's start is read and left out of the sums), before anything is reduced
   float4 v[VPL];
   uint4 graw[VPL], braw[VPL];           // bfloat16: .x and .y hold the four values
-  float s = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
-    const int c = (lane + i * DA_WAVE) * 4;
+    const int c = c0 + i * STRIDE;
     v[i] = *(const float4*)(xr + (c < E ? c : 0));
   }
   const void* bsrc = b ? b : w;         // without a bias the gain is read twice and dropped
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
-    const int c = (lane + i * DA_WAVE) * 4, cc = c < E ? c : 0;
+    const int c = c0 + i * STRIDE, cc = c < E ? c : 0;
     if (PBF16) {
       const uint2 g2 = *(const uint2*)((const bf16_t*)w + cc), b2 = *(const uint2*)((const bf16_t*)bsrc + cc);
       graw[i] = make_uint4(g2.x, g2.y, 0, 0);
@@ -244,46 +256,37 @@ layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
     }
   }
   __builtin_amdgcn_sched_barrier(0);
+  float s = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL; ++i)
-    s += ((lane + i * DA_WAVE) * 4 < E ? 1.f : 0.f) * ((v[i].x + v[i].y) + (v[i].z + v[i].w));
-  const float mean = wave_sum(s) / (float)E;
+    if (c0 + i * STRIDE < E) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+  const float mean = ln_row_sum(s, red[0]) / (float)E;
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
-    const int c = (lane + i * DA_WAVE) * 4;
-    if (c < E) {
-      const float d0 = v[i].x - mean, d1 = v[i].y - mean, d2 = v[i].z - mean, d3 = v[i].w - mean;
-      q += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
-    }
+    v[i].x -= mean; v[i].y -= mean; v[i].z -= mean; v[i].w -= mean;
+    if (c0 + i * STRIDE < E) q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
   }
-  const float inv = 1.0f / sqrtf(wave_sum(q) / (float)E + eps);
+  const float inv = 1.0f / sqrtf(ln_row_sum(q, red[1]) / (float)E + eps);
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
-    const int c = (lane + i * DA_WAVE) * 4;
-    if (c < E) {
-      float4 g, bb;
-      if (PBF16) {
-        g = make_float4(__uint_as_float(graw[i].x << 16), __uint_as_float(graw[i].x & 0xffff0000u),
-                        __uint_as_float(graw[i].y << 16), __uint_as_float(graw[i].y & 0xffff0000u));
-        bb = make_float4(__uint_as_float(braw[i].x << 16), __uint_as_float(braw[i].x & 0xffff0000u),
-                         __uint_as_float(braw[i].y << 16), __uint_as_float(braw[i].y & 0xffff0000u));
-      } else {
-        g = make_float4(__uint_as_float(graw[i].x), __uint_as_float(graw[i].y), __uint_as_float(graw[i].z), __uint_as_float(graw[i].w));
-        bb = make_float4(__uint_as_float(braw[i].x), __uint_as_float(braw[i].y), __uint_as_float(braw[i].z), __uint_as_float(braw[i].w));
-      }
-      if (!b) bb = make_float4(0.f, 0.f, 0.f, 0.f);
-      const float4 o = make_float4((v[i].x - mean) * inv * g.x + bb.x, (v[i].y - mean) * inv * g.y + bb.y,
-                                   (v[i].z - mean) * inv * g.z + bb.z, (v[i].w - mean) * inv * g.w + bb.w);
-      if (y_dtype == DA_BF16) {
-        uint2 u;
-        u.x = (uint32_t)f32_to_bf16(o.x) | ((uint32_t)f32_to_bf16(o.y) << 16);
-        u.y = (uint32_t)f32_to_bf16(o.z) | ((uint32_t)f32_to_bf16(o.w) << 16);
-        *(uint2*)((bf16_t*)y + (size_t)r * E + c) = u;
-      } else {
-        *(float4*)((float*)y + (size_t)r * E + c) = o;
-      }
+    const int c = c0 + i * STRIDE;
+    if (c >= E) continue;
+    float4 g, bb;
+    if (PBF16) {
+      g = make_float4(__uint_as_float(graw[i].x << 16), __uint_as_float(graw[i].x & 0xffff0000u),
+                      __uint_as_float(graw[i].y << 16), __uint_as_float(graw[i].y & 0xffff0000u));
+      bb = make_float4(__uint_as_float(braw[i].x << 16), __uint_as_float(braw[i].x & 0xffff0000u),
+                       __uint_as_float(braw[i].y << 16), __uint_as_float(braw[i].y & 0xffff0000u));
+    } else {
+      g = make_float4(__uint_as_float(graw[i].x), __uint_as_float(graw[i].y), __uint_as_float(graw[i].z), __uint_as_float(graw[i].w));
+      bb = make_float4(__uint_as_float(braw[i].x), __uint_as_float(braw[i].y), __uint_as_float(braw[i].z), __uint_as_float(braw[i].w));
     }
+    if (!b) bb = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 o = make_float4(v[i].x * inv * g.x + bb.x, v[i].y * inv * g.y + bb.y,
+                                 v[i].z * inv * g.z + bb.z, v[i].w * inv * g.w + bb.w);
+    if (YBF16) *(uint2*)((bf16_t*)y + (size_t)r * E + c) = make_uint2(pack2_bf16(o.x, o.y), pack2_bf16(o.z, o.w));
+    else *(float4*)((float*)y + (size_t)r * E + c) = o;
   }
 }
 
@@ -296,22 +299,15 @@ extern "C" int da_layernorm(const float* x, const int* rows, const void* w, int 
   hipStream_t st = (hipStream_t)stream;
   const bool aligned = ((uintptr_t)x % 16 == 0) && ((uintptr_t)y % 16 == 0) && ((uintptr_t)w % 16 == 0) &&
                        (!b || (uintptr_t)b % 16 == 0);
-  const int wpb = R >= 512 ? 4 : 1;      // wavefronts (rows) per workgroup
   const bool same = (!b || b_dtype == w_dtype) && (w_dtype == DA_BF16 || w_dtype == DA_F32);   // gain and bias alike
   if (E % 4 == 0 && E <= 2048 && aligned && same) {
-#define LN_LAUNCH(V)                                                                                                \
-  do {                                                                                                              \
-    if (w_dtype == DA_BF16)                                                                                         \
-      hipLaunchKernelGGL((layernorm_row_kernel<V, true>), dim3(da_ceil_div(R, wpb)), dim3(wpb * DA_WAVE), 0, st, x, \
-                         rows, w, b, eps, y, y_dtype, R, E);                                                        \
-    else                                                                                                            \
-      hipLaunchKernelGGL((layernorm_row_kernel<V, false>), dim3(da_ceil_div(R, wpb)), dim3(wpb * DA_WAVE), 0, st, x, \
-                         rows, w, b, eps, y, y_dtype, R, E);                                                        \
-  } while (0)
-    if (E <= 256) LN_LAUNCH(1);
-    else if (E <= 512) LN_LAUNCH(2);
-    else if (E <= 1024) LN_LAUNCH(4);
-    else LN_LAUNCH(8);
+#define LN_LAUNCH(V, P, Y) hipLaunchKernelGGL((layernorm_row_kernel<V, P, Y>), dim3(R), dim3(LN_WAVES * DA_WAVE), 0, st, x, rows, w, b, eps, y, E)
+#define LN_LAUNCH_Y(V, P) do { if (y_dtype == DA_BF16) LN_LAUNCH(V, P, true); else LN_LAUNCH(V, P, false); } while (0)
+#define LN_LAUNCH_P(V) do { if (w_dtype == DA_BF16) LN_LAUNCH_Y(V, true); else LN_LAUNCH_Y(V, false); } while (0)
+    if (E <= 4 * LN_WAVES * DA_WAVE) LN_LAUNCH_P(1);
+    else LN_LAUNCH_P(2);
+#undef LN_LAUNCH_P
+#undef LN_LAUNCH_Y
 #undef LN_LAUNCH
   } else {
     const int waves = 4;
