@@ -190,6 +190,45 @@ def test_gemm_matrix_cores(ops, M, N, K):
         assert (out - ref).abs().max() < tol, (act, acc, bias, od)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 4100, 2600), (8, 4800, 1600), helpers.quick(3, 4112, 40), (16, 8192, 72), (17, 6401, 648),
+                                   (48, 8190, 1160), (64, 4800, 4616)])
+def test_gemm_one_workgroup_a_compute_unit(ops, M, N, K):
+    """Between 4,097 and 8,192 columns: up to 32 columns a workgroup (17 to 32 here), several rounds of steps in flight, a
+    last step that K cuts; a row has the same bits beside any other rows; keys and values in the epilogue."""
+    g = torch.Generator().manual_seed(M + N)
+    for act, acc, bias, od in ((None, False, True, torch.bfloat16), ("gelu_new", False, False, torch.bfloat16), (None, True, True, torch.float32)):
+        out, ref = _gemm_case(ops, ops.linear_mfma, M, N, K, torch.bfloat16, act, acc, bias, od, g)
+        tol = (1e-2 if od == torch.bfloat16 else 1e-4) * max(1.0, ref.abs().max().item())
+        assert (out - ref).abs().max() < tol, (act, acc, bias, od)
+    a, w = bf(torch.randn(64, K, generator=g)).to(DEV), bf(torch.randn(N, K, generator=g) * 0.1).to(DEV)
+    rows = lambda lo, hi: ops.linear_mfma(a[lo:hi], w, None, torch.empty(hi - lo, N, device=DEV))
+    assert torch.equal(rows(5, 10)[2], rows(0, 64)[7]) and torch.equal(rows(0, 33)[7], rows(4, 20)[3])
+    page, D, Hkv = 16, N // 4 // 16 * 4, 2
+    if N % 4 == 0 and D % 4 == 0:
+        slots = torch.randperm(5 * page, generator=g)[:M].to(torch.int32).to(DEV)
+        c1, c2 = (torch.zeros(5, 2, Hkv, page, D, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+        ops.linear_mfma(a[:M], w, None, out, kv_cache=c1, slot_map=slots, q_cols=N - 2 * Hkv * D)
+        ops.kv_write(out, N - 2 * Hkv * D, N - Hkv * D, c2, slots, Hkv, D)
+        assert torch.equal(c1, c2) and bool(c1.any())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4800, 1600), (3, 6400, 1600), helpers.quick(2, 4100, 72), (8, 8192, 1304), (16, 4801, 1000), (9, 6000, 768)])
+def test_fused_norm_product_one_workgroup_a_compute_unit(ops, M, N, K):
+    """The fused norm and product with up to 32 columns a workgroup, parameters in bfloat16 and in 32-bit."""
+    g = torch.Generator().manual_seed(M + N)
+    x = (torch.randn(M, K, generator=g) * 2 + 1).to(DEV)
+    w = bf(torch.randn(N, K, generator=g) * 0.1).to(DEV)
+    for dt in (torch.bfloat16, torch.float32):
+        gw, gb, bias = (torch.randn(n, generator=g).to(dt).to(DEV) for n in (K, K, N))
+        out = torch.empty(M, N, device=DEV)
+        ops.linear_ln(x, None, M, gw, gb, 1e-5, w, bias, out)
+        a = F.layer_norm(x.double(), (K,), gw.double(), gb.double(), 1e-5).to(torch.bfloat16).double()
+        ref = a @ w.double().t() + bias.double()
+        # (the norm's 32-bit rounding may move an entry of a to the next bfloat16: 2^-8 of one product among K)
+        assert (out.double() - ref).abs().max() < 2e-2 * max(1.0, ref.abs().max().item())
+
+
 @pytest.mark.parametrize("M,N,K", [(1600, 2000, 200), (1555, 1999, 320), (2048, 1600, 1600), (1536, 2304, 768), (2048, 2304, 768),
                                    (4096, 768, 3072), (2500, 1600, 2112), (2048, 1600, 6400)])
 def test_gemm_tiles_alone_on_their_compute_units(ops, M, N, K):
