@@ -58,6 +58,82 @@ __device__ __forceinline__ void kv_scatter_store(const KvScatter& kv, int slot, 
   else if (cv < kv.Hkv * kv.Dv) base[(long long)kv.Hkv * kv.page * kv.D + (long long)cv * kv.page + row] = f32_to_bf16(v);
 }
 
+// The values of 32 rows of a product whose k and v columns go to the cache.  Values are dimension-major: 4 rows whose places
+// are 4 consecutive ones from a multiple of 4 on are 8 consecutive bytes.  kv_run_offset: which row such groups begin
+// with (0 .. 3), or -1 where some are not such groups (rows of several sequences, places in any order, rows without a
+// place); `slot` is the place of row `lane % 32` (-1: none).  The answer is the same for the whole
+// wavefront.
+// kv_all_runs: whether the groups begin with row 0 and all rows that have a place are in such groups (what one prompt
+// portion's rows are, and what is asked first: lane moves inside a quad and a sum, against two exchanges through LDS), or
+// the product has so few rows that it does not matter: up to 512 rows fewer tiles than compute units store their values
+// entry by entry in less time than the chain through LDS takes (prompts of odd lengths, K = 768, N = 2,304: 552 rows 12.2 us
+// against 11.7, 300 rows with one group a turn 8.9 against 10.3; K = 1,600, N = 4,800: 23.0 against 18.6, 17.0 against 16.7).
+__device__ __forceinline__ bool kv_all_runs(int slot, int lane, long long M) {
+  const int first = dpp_move_i<0x00, 0xF>(slot, slot);      // quad_perm [0, 0, 0, 0]
+  const bool ok = slot < 0 || ((first & 3) == 0 && slot == first + (lane & 3));
+  return M <= 512 || wave_sum_i(ok ? 0 : 1) == 0;
+}
+// 4 consecutive rows' values of one column (in w): su holds the rows' places
+__device__ __forceinline__ void kv_store_run(bf16_t* col, const uint4& su, uint2 w, bool vwide, long long page_stride, int lgp, int pmask) {
+  const struct { int x, y, z, w; } sl = {(int)su.x, (int)su.y, (int)su.z, (int)su.w};
+  if (vwide && sl.x >= 0 && (sl.x & 3) == 0 && sl.y == sl.x + 1 && sl.z == sl.x + 2 && sl.w == sl.x + 3) {
+    *(uint2*)(col + (long long)(sl.x >> lgp) * page_stride + (sl.x & pmask)) = w;
+    return;
+  }
+  const int s4[4] = {sl.x, sl.y, sl.z, sl.w};
+  const uint32_t w2[2] = {w.x, w.y};
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (s4[e] >= 0) col[(long long)(s4[e] >> lgp) * page_stride + (s4[e] & pmask)] = (bf16_t)(w2[e / 2] >> (16 * (e % 2)));
+}
+__device__ __forceinline__ int kv_run_offset(int slot, int lane) {
+  const int r = lane % 32, o = (4 - (__builtin_amdgcn_readlane(slot, 0) & 3)) & 3;
+  const int base = o + ((r - o) & ~3);                  // (arithmetic: rows before the first group have a base below 0)
+  const bool whole = base >= 0 && base + 3 < 32;
+  const int first = __shfl(slot, whole ? base : r, DA_WAVE);
+  const bool off = whole && (slot < 0 || (first & 3) != 0 || slot != first + (r - base));
+  return wave_sum_i(off ? 1 : 0) == 0 ? o : -1;
+}
+
+// A column a lane: `park` is the lane's entry of the first row in LDS (rows LDT entries apart), `dst` the lane's column's
+// run in page 0 (null: not a value column).  Two groups a turn are read and stored, 8 bytes each; the at most 4 rows outside of
+// groups, and all rows where `offset` is -1, are stored one by one.  (A prompt behind another one of odd length begins
+// anywhere in a tile: stored entry by entry from the accumulators its values took half as long as the product, 1,624 rows,
+// N = 3,072, K = 1,024 32.0 us against 23.8; the same rows in whole groups of 4 21.9.  The loops stay loops: with
+// every offset written out the code is so long that also prompts that never run it wait, 2,048 rows, N = 4,800, K = 1,600
+// between a step's other kernels 48.9 -> 52.0.)
+template <int LDT>
+__device__ __forceinline__ void kv_store_values32(const bf16_t* park, int slot, int offset, bf16_t* dst, long long page_stride, int lgp, int pmask) {
+  const int groups = offset < 0 ? 0 : offset == 0 ? 8 : 7;
+#pragma unroll 1
+  for (int g = 0; g < groups; g += 2) {                 // (two groups a turn; the last of 7 is stored twice)
+    const int r0 = offset + 4 * g, r1 = offset + 4 * min(g + 1, groups - 1);
+    const bf16_t *const p = park + r0 * LDT, *const q = park + r1 * LDT;
+    const uint32_t p0 = p[0], p1 = p[LDT], p2 = p[2 * LDT], p3 = p[3 * LDT], q0 = q[0], q1 = q[LDT], q2 = q[2 * LDT], q3 = q[3 * LDT];
+    const int s0 = __builtin_amdgcn_readlane(slot, r0), s1 = __builtin_amdgcn_readlane(slot, r1);
+    if (dst) {
+      *(uint2*)(dst + (long long)(s0 >> lgp) * page_stride + (s0 & pmask)) = make_uint2(p0 | (p1 << 16), p2 | (p3 << 16));
+      *(uint2*)(dst + (long long)(s1 >> lgp) * page_stride + (s1 & pmask)) = make_uint2(q0 | (q1 << 16), q2 | (q3 << 16));
+    }
+  }
+  const int singles = 32 - 4 * groups;                  // 0, 4 or 32
+#pragma unroll 1
+  for (int i = 0; i < singles; i += 4) {
+    int sl[4];
+    bf16_t v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = i + e < offset || offset < 0 ? i + e : 4 * groups + i + e;
+      sl[e] = __builtin_amdgcn_readlane(slot, r);
+      v[e] = park[r * LDT];
+    }
+    if (dst)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (sl[e] >= 0) dst[(long long)(sl[e] >> lgp) * page_stride + (sl[e] & pmask)] = v[e];
+  }
+}
+
 __device__ __forceinline__ uint4 load16(const bf16_t* p) { return *(const uint4*)p; }
 
 

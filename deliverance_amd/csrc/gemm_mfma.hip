@@ -155,40 +155,41 @@ tile_epilogue(floatx16 (&acc)[BM / WM / 32][BN / WN / 32], const float (&bias)[B
         if (nn[k] + e >= kv.q_cols && nn[k] + e < v0)
           kv_scatter_bits(kv, pg, prow, nn[k] + e, (bf16_t)(words[e / 2] >> (16 * (e % 2))));
     }
-    // Values, straight from the accumulators: a lane holds 4 consecutive rows of its column (r % 4), which are 8
-    // consecutive bytes of the dimension-major page when the rows' places are 4 consecutive ones from a multiple
-    // of 4 on (a prompt portion's are); the lane of the other half holds the 4 rows beside them.
+    // Values: where all groups of 4 rows of a piece of 32 have places that are runs from a multiple of 4 on (one prompt
+    // portion's are), straight from the accumulators: a lane holds 4 consecutive rows of its column (r % 4); the lane
+    // of the other half holds the 4 rows beside them.  Else from the parked tile, a column a lane.
     const bool vwide = (uintptr_t)kv.cache % 8 == 0 && kv.page % 4 == 0;
     const long long page_stride = 2LL * kv.Hkv * kv.page * kv.D;
     bf16_t* vb = (bf16_t*)kv.cache;
+    if (n0 + wn + BN / WN <= v0 || n0 + wn >= N) return;                // (no value column among the wavefront's)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + wn + j * 32 + fr;
-      if (n < v0 || n >= N) continue;
-      const int cc = n - v0;
-      const int vcol = (kv.Hkv + cc / kv.D) * kv.page * kv.D + (cc % kv.D) * kv.page;   // the column's run in a page
+    for (int i = 0; i < TM; ++i) {
+      const int sl = slots[wm + i * 32 + lane % 32];
+      if (__builtin_expect(kv_all_runs(sl, lane, M), 1)) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+        for (int j = 0; j < TN; ++j) {
+          const int n = n0 + wn + j * 32 + fr;
+          if (n < v0 || n >= N) continue;
+          const int cc = n - v0;
+          const int vcol = (kv.Hkv + cc / kv.D) * kv.page * kv.D + (cc % kv.D) * kv.page;   // the column's run in a page
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int r0 = wm + i * 32 + 8 * q + 4 * (lane / 32);           // the first of the lane's 4 tile rows
-          const uint4 su = *(const uint4*)&slots[r0];
-          const int s4[4] = {(int)su.x, (int)su.y, (int)su.z, (int)su.w};
-          uint32_t w2[2];
+          for (int q = 0; q < 4; ++q) {
+            uint32_t w2[2];
 #pragma unroll
-          for (int e = 0; e < 2; ++e)
-            w2[e] = pack2_bf16(apply_act_bf16(acc[i][j][4 * q + 2 * e] + bias[j], ACT),
-                               apply_act_bf16(acc[i][j][4 * q + 2 * e + 1] + bias[j], ACT));
-          const bool run = vwide && s4[0] >= 0 && (s4[0] & 3) == 0 && s4[1] == s4[0] + 1 && s4[2] == s4[0] + 2 && s4[3] == s4[0] + 3;
-          if (run) {
-            *(uint2*)(vb + (long long)(s4[0] >> lgp) * page_stride + vcol + (s4[0] & pmask)) = make_uint2(w2[0], w2[1]);
-            continue;
+            for (int e = 0; e < 2; ++e)
+              w2[e] = pack2_bf16(apply_act_bf16(acc[i][j][4 * q + 2 * e] + bias[j], ACT),
+                                 apply_act_bf16(acc[i][j][4 * q + 2 * e + 1] + bias[j], ACT));
+            kv_store_run(vb + vcol, *(const uint4*)&slots[wm + i * 32 + 8 * q + 4 * (lane / 32)], make_uint2(w2[0], w2[1]), vwide, page_stride, lgp, pmask);
           }
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (s4[e] >= 0)
-              vb[(long long)(s4[e] >> lgp) * page_stride + vcol + (s4[e] & pmask)] = (bf16_t)(w2[e / 2] >> (16 * (e % 2)));
         }
+        continue;
+      }
+      static_assert(BN / WN <= 64, "a column a lane");
+      const int n = n0 + wn + lane, cc = n - v0;
+      const bool mine = lane < BN / WN && cc >= 0 && n < N;
+      bf16_t* const dst = mine ? vb + (long long)(kv.Hkv + cc / kv.D) * kv.page * kv.D + (cc % kv.D) * kv.page : nullptr;
+      kv_store_values32<LDT>((const bf16_t*)smem + (wm + i * 32) * LDT + wn + lane % (BN / WN), sl,
+                             vwide ? kv_run_offset(sl, lane) : -1, dst, page_stride, lgp, pmask);
     }
   }
 }

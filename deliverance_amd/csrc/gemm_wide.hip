@@ -23,7 +23,7 @@
 // of LDS (bias and activation applied, rounded to the output's type), and leave in 16-byte pieces, whole
 // rows side by side; += adds to 16-byte pieces read the same way; a fused q|k|v projection also writes
 // its k and v columns to the rows' places in the paged cache (keys in 16-byte pieces of their rows,
-// values in 16-byte runs where 8 rows' places are consecutive).
+// values in 8-byte runs where 4 rows' places are consecutive: kv_all_runs, kv_run_offset).
 #include "gemm_common.h"
 #include <da_lds_dma.h>
 #include <type_traits>
@@ -152,34 +152,33 @@ wide_epilogue(floatx16 (&acc)[TM][TN], const float (&bias)[TN], char* region, co
           if (nn[k] + e >= kv.q_cols && nn[k] + e < v0)
             kv_scatter_bits(kv, pg, prow, nn[k] + e, (bf16_t)(words[e / 2] >> (16 * (e % 2))));
       }
-      // values, straight from the accumulators: a lane holds 4 consecutive rows of its column (r % 4), which
-      // are 8 consecutive bytes of the dimension-major page when the rows' places are 4 consecutive ones from
-      // a multiple of 4 on (a prompt portion's are); the lane of the other half holds the 4 rows beside them
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = nw + j * 32 + fr;
-        if (n < v0 || n >= N) continue;
+      // values: where the groups of 4 rows have places that are runs from a multiple of 4 on (one prompt portion's
+      // are), straight from the accumulators: a lane holds 4 consecutive rows of its column (r % 4), which are 8
+      // consecutive bytes of the dimension-major page; the lane of the other half holds the 4 rows beside them.
+      // Else from LDS, a column a lane.
+      if (nw + WC > v0) {
         bf16_t* vb = (bf16_t*)kv.cache;
+        const int sl = slots[lane % 32];
+        if (__builtin_expect(kv_all_runs(sl, lane, M), 1)) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int r0 = 8 * q + 4 * (lane / 32);             // the first of the lane's 4 rows in this pass
-          const uint4 su = *(const uint4*)&slots[r0];
-          const struct { int x, y, z, w; } sl = {(int)su.x, (int)su.y, (int)su.z, (int)su.w};
-          uint32_t w2[2];
+          for (int j = 0; j < TN; ++j) {
+            const int n = nw + j * 32 + fr;
+            if (n < v0 || n >= N) continue;
 #pragma unroll
-          for (int e = 0; e < 2; ++e)
-            w2[e] = pack2_bf16(apply_act_bf16(acc[i][j][4 * q + 2 * e] + bias[j], ACT),
-                               apply_act_bf16(acc[i][j][4 * q + 2 * e + 1] + bias[j], ACT));
-          const bool run = vwide && sl.x >= 0 && (sl.x & 3) == 0 && sl.y == sl.x + 1 && sl.z == sl.x + 2 && sl.w == sl.x + 3;
-          if (run) {
-            *(uint2*)(vb + (long long)(sl.x >> lgp) * page_stride + vcol[j] + (sl.x & pmask)) = make_uint2(w2[0], w2[1]);
-            continue;
+            for (int q = 0; q < 4; ++q) {
+              uint32_t w2[2];
+#pragma unroll
+              for (int e = 0; e < 2; ++e)
+                w2[e] = pack2_bf16(apply_act_bf16(acc[i][j][4 * q + 2 * e] + bias[j], ACT),
+                                   apply_act_bf16(acc[i][j][4 * q + 2 * e + 1] + bias[j], ACT));
+              kv_store_run(vb + vcol[j], *(const uint4*)&slots[8 * q + 4 * (lane / 32)], make_uint2(w2[0], w2[1]), vwide, page_stride, lgp, pmask);
+            }
           }
-          const int s4[4] = {sl.x, sl.y, sl.z, sl.w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (s4[e] >= 0)
-              vb[(long long)(s4[e] >> lgp) * page_stride + vcol[j] + (s4[e] & pmask)] = (bf16_t)(w2[e / 2] >> (16 * (e % 2)));
+        } else {
+          static_assert(WC == 64, "a column a lane");
+          const int n = nw + lane, cc = n - v0;
+          bf16_t* const dst = cc >= 0 && n < N ? vb + (long long)(kv.Hkv + cc / kv.D) * kv.page * kv.D + (cc % kv.D) * kv.page : nullptr;
+          kv_store_values32<LDT>((const bf16_t*)region + lane, sl, vwide ? kv_run_offset(sl, lane) : -1, dst, page_stride, lgp, pmask);
         }
       }
     }

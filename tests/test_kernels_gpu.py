@@ -301,6 +301,36 @@ def test_gemm_wide_tiles_write_keys_and_values(ops, M, form):
 
 
 @pytest.mark.simt_quick
+@pytest.mark.parametrize("form", ["auto", "wide", "wide_256x128", "wide_128x128"])
+@pytest.mark.parametrize("M", [512, 517])
+def test_product_writes_values_of_prompts_of_odd_lengths(ops, M, form):
+    """More than 512 rows of several sequences, each from any place of a page on: groups of 4 places that begin with
+    each row of a piece of 32, pieces with rows of two sequences, and rows without a place at the start, in the middle
+    and at the end of a group.  512 rows take the way of few rows."""
+    g = torch.Generator().manual_seed(M)
+    Hq, Hkv, D, page, K = 1, 2, 24, 16, 64
+    N = (Hq + 2 * Hkv) * D
+    a, w, bias = (bf(torch.randn(*s, generator=g)).to(DEV) for s in ((M, K), (N, K), (N,)))
+    places, page0 = [], 1
+    for first, n in ((0, 64), (1, 95), (2, 97), (3, 94), (5, 33), (0, 2), (6, 70), (0, M - 455)):
+        places += range(page0 * page + first, page0 * page + first + n)
+        page0 += (first + n) // page + 2
+    slots = torch.tensor(places, dtype=torch.int32)
+    assert slots.numel() == M
+    for r in (96, 130, 195, 260, 393, M - 1):
+        slots[r] = -1
+    slots = slots.to(DEV)
+    c1 = torch.zeros(page0 + 1, 2, Hkv, page, D, dtype=torch.bfloat16, device=DEV)
+    c2 = torch.zeros_like(c1)
+    out1, out2 = (torch.empty(M, N, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    ops.linear_mfma(a, w, bias, out1, kv_cache=c1, slot_map=slots, q_cols=Hq * D, form=form)
+    ops.linear_mfma(a, w, bias, out2)
+    ops.kv_write(out2, Hq * D, (Hq + Hkv) * D, c2, slots, Hkv, D)
+    assert torch.equal(out1, out2)
+    assert torch.equal(c1, c2) and c1.abs().sum() > 0
+
+
+@pytest.mark.simt_quick
 @pytest.mark.parametrize("M", [20, 200])
 def test_gemm_into_rows_longer_than_the_result(ops, M):
     """The output's rows are longer than N (a view of a wider matrix): the tile kernel stores whole
