@@ -1010,7 +1010,8 @@ def linear_f32(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], o
 
 # Measured on MI355X (q|k|v of 768 to 1,600 wide, 128 to 2,048 rows): the cache write in the product's
 # epilogue adds 1.3 to 3.4 us where the rows' places are runs of consecutive cache rows (a prompt
-# portion: keys and values both go over in 16-byte pieces), the write kernel after the product 3.7 to
+# portion: keys go over in 16-byte pieces, values in 8-byte ones; behind a prompt of odd length 0.3 to 4 us
+# more), the write kernel after the product 3.7 to
 # 9.2 us; with places in any order the two are level at 2,048 rows and the epilogue is ahead below.
 
 
