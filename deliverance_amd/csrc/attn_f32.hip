@@ -32,6 +32,30 @@ __device__ __forceinline__ float af_max16(float v) {          // the maximum ove
   return fmaxf(v, dpp_move<0x140, 0xF>(v, v));
 }
 
+// What the products cannot give: an entry whose weighted sum is not finite (the 16 rows of a tile share their keys, and a
+// weight of zero times another row's infinite value is no number), or whose row has no weight at all (ll is 0: it sees no
+// key, or only scores of minus infinity).  Key by key in ascending order, a value whose weight is zero is not looked at.
+// Not on any ordinary row's way.  qr: the row's query; kb, vb: the head's keys and the entry's dimension in page 0; mm, ll:
+// the row's maximum and sum.
+__device__ __forceinline__ float af_entry(const float* qr, const float* kb, const float* vb, const int* bt, int lg, int pmask,
+                                          long long page_elems, int D, int lo, int p, float scale, float mm, float ll) {
+  if (ll != ll) return ll;
+  bool any = false;
+  float sum = 0.f;
+  for (int key = lo; key <= p; ++key) {
+    const int pg = bt[key >> lg];
+    if (pg < 0) continue;
+    any = true;
+    if (ll == 0.f) break;
+    const float* kr = kb + pg * page_elems + (key & pmask) * D;
+    float dot = 0.f;
+    for (int d = 0; d < D; ++d) dot = fmaf(qr[d], kr[d], dot);
+    const float e = expf(dot * scale - mm);
+    if (e != 0.f) sum = fmaf(e, vb[pg * page_elems + (key & pmask)], sum);
+  }
+  return ll == 0.f ? (any ? NAN : 0.f) : sum / ll;
+}
+
 template <int D16>
 __global__ void __launch_bounds__(AF_WAVES * DA_WAVE)
 attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__ cache, const int* __restrict__ block_table,
@@ -128,10 +152,11 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
       }
       const float m_new = fmaxf(m[r], af_max16(top));
       alpha[r] = m_new == -INFINITY ? 1.f : expf(m[r] - m_new);
+      const float m_ref = m_new == -INFINITY ? 0.f : m_new;     // (scores of minus infinity alone weigh nothing here: another chunk may hold more)
       float sum = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float e = ok[j] ? expf(sc[j][r] - m_new) : 0.f;
+        const float e = ok[j] ? expf(sc[j][r] - m_ref) : 0.f;
         ps[(quad * 4 + r) * AF_PLD + j * 16 + col] = e;
         sum += e;
       }
@@ -194,7 +219,14 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
       ll += part_l[w][row] * f;
       v += smem[(w * 16 + row) * OLD + d] * f;
     }
-    out[(size_t)(row0 + i0 + row) * out_ld + h * D + d] = ll > 0.f ? v / ll : 0.f;      // (a padding row: zeros)
+    float* const entry = out + (size_t)(row0 + i0 + row) * out_ld + h * D + d;
+    if (ll > 0.f && fabsf(v) < INFINITY) {
+      *entry = v / ll;
+      continue;
+    }
+    const int p = past + i0 + row;
+    *entry = af_entry(q + (size_t)(row0 + i0 + row) * q_ld + h * D, kbase, vbase + (long long)d * page, bt, lg, pmask, page_elems, D,
+                      (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0, p, scale, mm, ll);
   }
 }
 

@@ -479,6 +479,53 @@ def test_attention_32bit_on_the_matrix_cores(ops, Hq, Hkv, D, page, window):
     assert torch.equal(one[:5], out[-5:]) and not bool(one[5].any())
 
 
+def _attention_64(q, k, v, past, scale, window):
+    """One head in 64 bits, row by row: a value whose weight is zero is not looked at, scores without a number or of plus
+    infinity (or of minus infinity alone) leave no number."""
+    out = np.zeros((q.shape[0], v.shape[1]))
+    with np.errstate(all="ignore"):
+        for i in range(q.shape[0]):
+            lo = max(0, past + i - window + 1) if window else 0
+            s = (k[lo:past + i + 1] @ q[i]) * scale
+            e = np.exp(s - s.max())
+            seen = e != 0.0
+            out[i] = (e[seen, None] * v[lo:past + i + 1][seen]).sum(0) / e.sum()
+    return out
+
+
+@pytest.mark.simt_quick
+@pytest.mark.parametrize("window", [None, 20])
+def test_attention_32bit_with_numbers_that_are_not_finite(ops, window):
+    """Infinite and missing numbers in queries, keys and values: they reach the rows that see them with a weight and no
+    other row, though 16 rows and 64 keys share a tile.  (Every row is compared, bound as for finite numbers.)"""
+    inf, nan = float("inf"), float("nan")
+    D, page, T, past = 16, 16, 40, 90
+    n = past + T
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(n, D, generator=g) for _ in range(3))
+    q = q[:T].abs() + 0.1
+    v[past + 9, 3], v[past + 21, 4], v[past + 30, 5] = inf, nan, -inf     # seen by the rows behind them only
+    k[past + 12] = -inf                                                  # a score of minus infinity: no weight
+    v[past + 12] = nan
+    k[past + 35, 2] = nan                                                # rows from 35 on: no number
+    k[64:64 + 20] = -inf                                                 # with the window some rows' first chunk is this alone
+    q[2, 7] = nan
+    cache = torch.full((12, 2, 1, page, D), nan)
+    bt = torch.tensor([[3, 7, 1, 9, 0, 4, 8, 2, 5]], dtype=torch.int32)
+    for j in range(n):
+        cache[bt[0, j // page], 0, 0, j % page] = k[j]
+        cache[bt[0, j // page], 1].view(D, page)[:, j % page] = v[j]
+    out = torch.full((T, D), 7.0, device=DEV)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    ops.attention_f32(q.to(DEV), cache.to(DEV), bt.to(DEV), i32(0, T), i32(n), 1, T, 1, 0.2, window, out)
+    want = _attention_64(q.double().numpy(), k.double().numpy(), v.double().numpy(), past, 0.2, window)
+    got = out.double().cpu().numpy()
+    assert np.isnan(want).any() and np.isposinf(want).any() and np.isfinite(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    fin = np.isfinite(want)
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]) and np.abs(got[fin] - want[fin]).max() < ATT_TOL[torch.float32]
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,page,window", [helpers.quick(4, 4, 16, 16, None), (6, 2, 48, 16, None), helpers.quick(2, 1, 80, 32, 37),
                                                   (3, 3, 128, 64, None), (12, 12, 64, 16, None), (5, 5, 64, 16, 100),
                                                   helpers.quick(2, 2, 256, 16, None), (25, 25, 64, 32, 70)])
