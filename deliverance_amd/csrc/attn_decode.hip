@@ -206,7 +206,22 @@ DEC_KERNEL(const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ ca
           kf[j][k] = *(const uint4*)(kp + (2 * k + 1 < DK || 32 * k + 8 * quad < D ? 64 * k : 0));
       }
     };
+    // Zeros in place of what lanes past D read: q is zero there, but zero times an infinite key is no number.
+    auto clear_k = [&]() {
+#pragma unroll
+      for (int k = DK / 2; k < DK; ++k) {
+        const uint32_t keep = 32 * k + 8 * quad < D ? 0xffffffffu : 0u;
+#pragma unroll
+        for (int j = 0; j < KJ; ++j) {
+          kf[j][k].x &= keep;
+          kf[j][k].y &= keep;
+          kf[j][k].z &= keep;
+          kf[j][k].w &= keep;
+        }
+      }
+    };
     auto scores = [&](int j0) {
+      if (D < DMAX) clear_k();
 #pragma unroll
       for (int j = 0; j < KJ; ++j) sc[j0 + j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -540,6 +540,31 @@ def test_attention_decode_kernel(ops, Hq, Hkv, D, page, window):
     assert np.abs(got - case.plain(scale, window)).max() < ATT_TOL[torch.bfloat16]
 
 
+@pytest.mark.simt_quick
+@pytest.mark.parametrize("D", [16, 48, 80, 144])
+def test_attention_decode_with_infinite_keys_and_values(ops, D):
+    """A key of minus infinity in some dimension has no weight (head sizes that are no multiple of 32 fill the matrix
+    instruction's depth with zeros, which may not meet it), an infinite value stands in the result."""
+    inf, page, n = float("inf"), 16, 100
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (bf(torch.randn(m, D, generator=g)) for m in (1, n, n))
+    q = q.abs() + 0.25
+    k[70, 1] = k[71, 7] = k[3, 0] = k[60, 20 % D] = k[99, D - 1] = k[40, D - 9] = -inf
+    v[50, 2], v[20, D - 1] = -inf, inf
+    cache = torch.full((7, 2, 1, page, D), float("nan"), dtype=torch.bfloat16)
+    for j in range(n):
+        cache[j // page, 0, 0, j % page] = k[j]
+        cache[j // page, 1].view(D, page)[:, j % page] = v[j]
+    out = torch.empty(1, D, dtype=torch.bfloat16, device=DEV)
+    ops.attention_decode(q.to(DEV), cache.to(DEV), torch.arange(7, dtype=torch.int32, device=DEV).view(1, 7),
+                         torch.tensor([n], dtype=torch.int32, device=DEV), 1, 1, 0.2, None, out)
+    want = _attention_64(q.double().numpy(), k.double().numpy(), v.double().numpy(), n - 1, 0.2, None)
+    got = out.double().cpu().numpy()
+    fin = np.isfinite(want)
+    assert fin.sum() == D - 2 and np.array_equal(got[~fin], want[~fin])
+    assert np.abs(got[fin] - want[fin]).max() < ATT_TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("n_splits", [2, helpers.quick(3, mark="simt_a"), 7, 16])
 @pytest.mark.parametrize("Hq,Hkv,D,page,window", [helpers.quick(2, 2, 64, 16, None, mark="simt_b"), (4, 2, 48, 32, None),
                                                   helpers.quick(1, 1, 128, 64, 700, mark="simt_b"), (3, 3, 16, 16, 90)])
