@@ -1025,8 +1025,12 @@ def linear(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: 
     if _MODE == "tuned" and _mfma_ok(a, w):
         return linear_mfma(a, w, bias, out, act, accumulate, kv_cache, slot_map, q_cols)
     if _MODE == "tuned" and _f32_ok(a, w, out):
-        return linear_f32(a, w, bias, out, act, accumulate, kv_cache, slot_map, q_cols)
-    linear_ref(a, w, bias, out, act, accumulate)
+        # (the epilogue writes what a plain store of q | k | v holds; sums added to, and columns behind v, go by the write kernel)
+        if kv_cache is None or (not accumulate and q_cols + 2 * kv_cache.shape[2] * kv_cache.shape[4] == w.shape[0]):
+            return linear_f32(a, w, bias, out, act, accumulate, kv_cache, slot_map, q_cols)
+        linear_f32(a, w, bias, out, act, accumulate)
+    else:
+        linear_ref(a, w, bias, out, act, accumulate)
     if kv_cache is not None:
         _, _, Hkv, _, D = kv_cache.shape
         kv_write(out, q_cols, q_cols + Hkv * D, kv_cache, slot_map, Hkv, D)

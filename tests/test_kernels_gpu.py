@@ -170,6 +170,26 @@ def test_gemm_32bit_writes_keys_and_values(ops):
         assert torch.equal(c1, c2) and c1.abs().sum() > 0
 
 
+@pytest.mark.simt_quick
+@pytest.mark.parametrize("extra,accumulate", [(0, False), (0, True), (12, False), (12, True)])
+def test_product_32bit_keeps_keys_and_values_of_any_call(ops, extra, accumulate):
+    """``linear`` with a cache: columns behind q | k | v, and sums that are added to what was there; the cache holds what
+    the rows hold afterwards."""
+    g = torch.Generator().manual_seed(11)
+    Hq, Hkv, D, page, K, M = 2, 1, 16, 16, 64, 5
+    N = (Hq + 2 * Hkv) * D + extra
+    a, w = (torch.randn(*s, generator=g).to(DEV) for s in ((M, K), (N, K)))
+    base = torch.randn(M, N, generator=g).to(DEV)
+    out = base.clone()
+    slots = torch.tensor([20, 3, -1, 31, 0], dtype=torch.int32, device=DEV)
+    c1, c2 = (torch.zeros(2, 2, Hkv, page, D, device=DEV) for _ in range(2))
+    ops.linear(a, w, None, out, accumulate=accumulate, kv_cache=c1, slot_map=slots, q_cols=Hq * D)
+    ref = a.double() @ w.double().t() + (base.double() if accumulate else 0.0)
+    assert (out.double() - ref).abs().max() < 2e-5 * max(1.0, ref.abs().max().item())
+    ops.kv_write(out, Hq * D, (Hq + Hkv) * D, c2, slots, Hkv, D)
+    assert torch.equal(c1, c2) and bool(c1.any())
+
+
 @pytest.mark.parametrize("M", [1, helpers.quick(3, mark="simt_a"), 5, 8, 12, 16, helpers.quick(17, mark="simt_a"), 40, 64,
                                helpers.quick(65, mark="simt_a"), 128, helpers.quick(200, mark="simt_a"), 513, 1100, 2048])
 @pytest.mark.parametrize("N,K", [helpers.quick(96, 200, mark="simt_b"), helpers.quick(1000, 96, mark="simt_b"), (2304, 768),
