@@ -671,6 +671,7 @@ def attention_f32(q: torch.Tensor, cache_slot: torch.Tensor, block_table: torch.
     Hkv, page, D = _attn_common(q, cache_slot, block_table, n_heads, out, "attention_f32", torch.float32)
     _need(q_start.dtype == torch.int32 and q_start.numel() >= n_seqs + 1 and seq_lens.dtype == torch.int32
           and seq_lens.numel() >= n_seqs and block_table.shape[0] >= n_seqs, "attention_f32: q_start int32 [S + 1], seq_lens int32 [S]")
+    _need(q.shape[0] == out.shape[0], "attention_f32: q and out differ in rows")
     _check(_lib().da_attn_f32(_ptr(q), q.stride(0), _ptr(cache_slot), _ptr(block_table), block_table.shape[1], _ptr(q_start),
                               _ptr(seq_lens), n_seqs, max_query_len, n_heads, Hkv, D, page, scale, int(window or 0), _ptr(out),
                               out.stride(0), _stream()))
@@ -1177,7 +1178,8 @@ def paged_attention(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: int, 
                 attention_prefill(q, cache_slot, bt, ctx.q_start, ctx.seq_lens, nd, ctx.n_seqs - nd,
                                   ctx.max_query_len, n_heads, scale, window, out)
         return out
-    if _MODE == "tuned" and q.dtype == torch.float32 and attention_f32_takes(D, page) and q.stride(0) % 4 == 0 and q.data_ptr() % 16 == 0:
+    if (_MODE == "tuned" and q.dtype == torch.float32 and attention_f32_takes(D, page) and q.stride(0) % 4 == 0
+            and q.data_ptr() % 16 == 0 and cache_slot.data_ptr() % 16 == 0):
         with _timed("attention_f32", *cost(0, ctx.n_seqs), "fp32"):
             return attention_f32(q, cache_slot, bt, ctx.q_start, ctx.seq_lens, ctx.n_seqs, ctx.max_query_len, n_heads, scale, window, out)
     with _timed("attention_plain", *cost(0, ctx.n_seqs), "fp32" if q.dtype == torch.float32 else "bf16"):

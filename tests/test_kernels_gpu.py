@@ -499,6 +499,27 @@ def test_attention_32bit_on_the_matrix_cores(ops, Hq, Hkv, D, page, window):
     assert torch.equal(one[:5], out[-5:]) and not bool(one[5].any())
 
 
+@pytest.mark.simt_quick
+def test_attention_32bit_of_a_cache_that_is_not_aligned(ops):
+    """Rows of q or a cache whose first byte is no multiple of 16: the plain kernel's; fewer rows in out than in q: refused."""
+    from types import SimpleNamespace
+    D, page, Hq = 16, 16, 2
+    case = PagedCase(lens=[33, 5], new=[20, 1], Hq=Hq, Hkv=1, D=D, page=page, dtype=torch.float32, seed=3)
+    ctx = SimpleNamespace(block_tables=[case.bt], n_decode=0, n_seqs=2, max_query_len=20, q_start=case.q_start, seq_lens=case.seq_lens,
+                          seq_of_token=case.seq_of, positions=case.pos, seq_lens_host=[33, 5], q_start_host=[0, 20, 21])
+    cache = torch.empty(case.cache.numel() + 1, device=DEV)[1:].view(case.cache.shape)
+    cache.copy_(case.cache)
+    qs = torch.empty(21, Hq * D + 1, device=DEV)[:, 1:]
+    qs.copy_(case.qcat)
+    want = case.plain(0.3, None)
+    for q, c in ((case.qcat, case.cache), (case.qcat, cache), (qs, case.cache)):
+        out = torch.full_like(case.qcat, 7.0)
+        ops.paged_attention(ctx, q, c, 0, Hq, 0.3, None, out)
+        assert np.abs(out.double().cpu().numpy() - want).max() < ATT_TOL[torch.float32]
+    with pytest.raises(ops.KernelError, match="row|q/out"):
+        ops.paged_attention(ctx, case.qcat, case.cache, 0, Hq, 0.3, None, out[:20])
+
+
 def _attention_64(q, k, v, past, scale, window):
     """One head in 64 bits, row by row: a value whose weight is zero is not looked at, scores without a number or of plus
     infinity (or of minus infinity alone) leave no number."""
