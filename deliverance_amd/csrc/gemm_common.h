@@ -59,19 +59,27 @@ __device__ __forceinline__ void kv_scatter_store(const KvScatter& kv, int slot, 
 }
 
 // The values of 32 rows of a product whose k and v columns go to the cache.  Values are dimension-major: 4 rows whose places
-// are 4 consecutive ones from a multiple of 4 on are 8 consecutive bytes.  kv_run_offset: which row such groups begin
-// with (0 .. 3), or -1 where some are not such groups (rows of several sequences, places in any order, rows without a
-// place); `slot` is the place of row `lane % 32` (-1: none).  The answer is the same for the whole
-// wavefront.
-// kv_all_runs: whether the groups begin with row 0 and all rows that have a place are in such groups (what one prompt
-// portion's rows are, and what is asked first: lane moves inside a quad and a sum, against two exchanges through LDS), or
-// the product has so few rows that it does not matter: up to 512 rows fewer tiles than compute units store their values
-// entry by entry in less time than the chain through LDS takes (prompts of odd lengths, K = 768, N = 2,304: 552 rows 12.2 us
-// against 11.7, 300 rows with one group a turn 8.9 against 10.3; K = 1,600, N = 4,800: 23.0 against 18.6, 17.0 against 16.7).
-__device__ __forceinline__ bool kv_all_runs(int slot, int lane, long long M) {
+// are 4 consecutive ones from a multiple of 4 on are 8 consecutive bytes.  A lane of the accumulators holds the rows 4 i ..
+// 4 i + 3 of its column.  `slot` is the place of row `lane % 32` (-1: none); the answers
+// are the same for each half of the wavefront.
+//  - kv_all_runs: all rows are in such groups and the groups begin with row 0 (what one prompt portion's rows are, asked
+//    first): stored from the accumulators, 8 bytes a group.
+//  - kv_run_offset: all groups begin with row 1, 2 or 3 (a prompt behind another one of odd length): stored from the parked
+//    tile, a column a lane (kv_store_values32).
+//  - else (rows of several sequences, places in any order, rows without a place): from the accumulators again, group by
+//    group, entry by entry where a group is no run (kv_store_run).
+// The first way has code of its own, without a look at each group: inside a step, where another kernel's code has taken the
+// instruction cache, a q|k|v product of 2,048 rows, N = 4,800, K = 1,600 takes 46.7 us with it and 48.7 where the first and
+// the last share theirs.
+// Up to 512 rows the second way is not taken: fewer tiles than compute units store their values entry by entry in less time
+// than the chain through LDS takes (prompts of odd lengths, K = 768, N = 2,304: 552 rows 12.2 us against 11.7, 300 rows
+// with one group a turn 8.9 against 10.3; K = 1,600, N = 4,800: 23.0 against 18.6, 17.0 against 16.7).
+#define KV_WALK_MIN_ROWS 513
+#define KV_WAY_RUNS 4
+__device__ __forceinline__ bool kv_all_runs(int slot, int lane) {
   const int first = dpp_move_i<0x00, 0xF>(slot, slot);      // quad_perm [0, 0, 0, 0]
-  const bool ok = slot < 0 || ((first & 3) == 0 && slot == first + (lane & 3));
-  return M <= 512 || wave_sum_i(ok ? 0 : 1) == 0;
+  const uint64_t off = __builtin_amdgcn_ballot_w64(first < 0 || (first & 3) != 0 || slot != first + (lane & 3));
+  return (uint32_t)(off >> (lane & 32)) == 0;
 }
 // 4 consecutive rows' values of one column (in w): su holds the rows' places
 __device__ __forceinline__ void kv_store_run(bf16_t* col, const uint4& su, uint2 w, bool vwide, long long page_stride, int lgp, int pmask) {
@@ -86,28 +94,30 @@ __device__ __forceinline__ void kv_store_run(bf16_t* col, const uint4& su, uint2
   for (int e = 0; e < 4; ++e)
     if (s4[e] >= 0) col[(long long)(s4[e] >> lgp) * page_stride + (s4[e] & pmask)] = (bf16_t)(w2[e / 2] >> (16 * (e % 2)));
 }
+// Which row the groups begin with: 1 .. 3, or 0 where they do not; the two halves of the wavefront may hold two pieces.
 __device__ __forceinline__ int kv_run_offset(int slot, int lane) {
-  const int r = lane % 32, o = (4 - (__builtin_amdgcn_readlane(slot, 0) & 3)) & 3;
+  const int half = lane & 32, r = lane & 31;
+  const int s0 = half ? __builtin_amdgcn_readlane(slot, 32) : __builtin_amdgcn_readlane(slot, 0), o = (4 - (s0 & 3)) & 3;
   const int base = o + ((r - o) & ~3);                  // (arithmetic: rows before the first group have a base below 0)
   const bool whole = base >= 0 && base + 3 < 32;
-  const int first = __shfl(slot, whole ? base : r, DA_WAVE);
-  const bool off = whole && (slot < 0 || (first & 3) != 0 || slot != first + (r - base));
-  return wave_sum_i(off ? 1 : 0) == 0 ? o : -1;
+  const int first = __shfl(slot, half + (whole ? base : r), DA_WAVE);
+  const uint64_t off = __builtin_amdgcn_ballot_w64(whole && (slot < 0 || (first & 3) != 0 || slot != first + (r - base)));
+  return (uint32_t)(off >> half) ? 0 : o;
 }
 
 // A column a lane: `park` is the lane's entry of the first row in LDS (rows LDT entries apart), `dst` the lane's column's
-// run in page 0 (null: not a value column).  Two groups a turn are read and stored, 8 bytes each; the at most 4 rows outside of
-// groups, and all rows where `offset` is -1, are stored one by one.  (A prompt behind another one of odd length begins
+// run in page 0 (null: not a value column).  Seven groups from row `offset` (1 .. 3) on, two a turn, 8 bytes each; the 4 rows
+// outside of them are stored one by one.  (A prompt behind another one of odd length begins
 // anywhere in a tile: stored entry by entry from the accumulators its values took half as long as the product, 1,624 rows,
-// N = 3,072, K = 1,024 32.0 us against 23.8; the same rows in whole groups of 4 21.9.  The loops stay loops: with
+// N = 3,072, K = 1,024 32.0 us against 23.8; the same rows in whole groups of 4 21.9.  Rows without such groups are no
+// faster from here: 552 rows of prompts of 21 tokens, N = 3,072, K = 1,024 15.2 us against 13.6.  The loop stays a loop: with
 // every offset written out the code is so long that also prompts that never run it wait, 2,048 rows, N = 4,800, K = 1,600
 // between a step's other kernels 48.9 -> 52.0.)
 template <int LDT>
 __device__ __forceinline__ void kv_store_values32(const bf16_t* park, int slot, int offset, bf16_t* dst, long long page_stride, int lgp, int pmask) {
-  const int groups = offset < 0 ? 0 : offset == 0 ? 8 : 7;
 #pragma unroll 1
-  for (int g = 0; g < groups; g += 2) {                 // (two groups a turn; the last of 7 is stored twice)
-    const int r0 = offset + 4 * g, r1 = offset + 4 * min(g + 1, groups - 1);
+  for (int g = 0; g < 7; g += 2) {                      // (the last one is stored twice)
+    const int r0 = offset + 4 * g, r1 = offset + 4 * min(g + 1, 6);
     const bf16_t *const p = park + r0 * LDT, *const q = park + r1 * LDT;
     const uint32_t p0 = p[0], p1 = p[LDT], p2 = p[2 * LDT], p3 = p[3 * LDT], q0 = q[0], q1 = q[LDT], q2 = q[2 * LDT], q3 = q[3 * LDT];
     const int s0 = __builtin_amdgcn_readlane(slot, r0), s1 = __builtin_amdgcn_readlane(slot, r1);
@@ -116,22 +126,18 @@ __device__ __forceinline__ void kv_store_values32(const bf16_t* park, int slot, 
       *(uint2*)(dst + (long long)(s1 >> lgp) * page_stride + (s1 & pmask)) = make_uint2(q0 | (q1 << 16), q2 | (q3 << 16));
     }
   }
-  const int singles = 32 - 4 * groups;                  // 0, 4 or 32
-#pragma unroll 1
-  for (int i = 0; i < singles; i += 4) {
-    int sl[4];
-    bf16_t v[4];
+  int sl[4];
+  bf16_t v[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int r = i + e < offset || offset < 0 ? i + e : 4 * groups + i + e;
-      sl[e] = __builtin_amdgcn_readlane(slot, r);
-      v[e] = park[r * LDT];
-    }
-    if (dst)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (sl[e] >= 0) dst[(long long)(sl[e] >> lgp) * page_stride + (sl[e] & pmask)] = v[e];
+  for (int e = 0; e < 4; ++e) {
+    const int r = e < offset ? e : 28 + e;
+    sl[e] = __builtin_amdgcn_readlane(slot, r);
+    v[e] = park[r * LDT];
   }
+  if (dst)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (sl[e] >= 0) dst[(long long)(sl[e] >> lgp) * page_stride + (sl[e] & pmask)] = v[e];
 }
 
 __device__ __forceinline__ uint4 load16(const bf16_t* p) { return *(const uint4*)p; }

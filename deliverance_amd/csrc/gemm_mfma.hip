@@ -47,14 +47,14 @@ template <int BM, int BN, int OUTMODE>
 constexpr int tile_out_bytes() {
   return BM * (BN + (OUTMODE == 0 ? 8 : 4)) * (OUTMODE == 0 ? 2 : 4);
 }
-// ... and behind it, for a fused q|k|v projection, the tile rows' places in the cache
+// ... and behind it, for a fused q|k|v projection, the tile rows' places in the cache and how the values of each 32 rows go there
 template <int BM, int OUTMODE>
-constexpr int tile_slot_bytes() { return OUTMODE == 0 ? BM * 4 : 0; }
+constexpr int tile_slot_bytes() { return OUTMODE == 0 ? BM * 4 + BM / 32 * 4 : 0; }
 
 template <int BM, int BN, int WM, int WN, int ACT, int OUTMODE>
 __device__ __forceinline__ void
 tile_epilogue(floatx16 (&acc)[BM / WM / 32][BN / WN / 32], const float (&bias)[BN / WN / 32], char* smem, const void* safe,
-              const Epilogue& ep, const KvScatter& kv, int M, int N, int m0, int n0) {
+              const Epilogue& ep, const KvScatter& kv, int slot, int M, int N, int m0, int n0) {
   constexpr int THREADS = WM * WN * 64;
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
   constexpr int ES = OUTMODE == 0 ? 2 : 4, CH = 16 / ES;      // bytes an element; elements a 16-byte piece
@@ -64,6 +64,19 @@ tile_epilogue(floatx16 (&acc)[BM / WM / 32][BN / WN / 32], const float (&bias)[B
   const int t = threadIdx.x, lane = t % 64, wave = t / 64;
   const int wm = (wave % WM) * (BM / WM), wn = (wave / WM) * (BN / WN);
   const int fr = lane % 32;
+  int* slots = (int*)(smem + tile_out_bytes<BM, BN, OUTMODE>());        // the tile rows' places, -1: none
+  int* ways = slots + BM;                                               // of each 32 rows: KV_WAY_RUNS (kv_all_runs) or kv_run_offset
+  const bool vwide = OUTMODE == 0 && kv.cache && (uintptr_t)kv.cache % 8 == 0 && kv.page % 4 == 0;
+  static_assert(BM % 64 == 0 && BM <= THREADS, "whole wavefronts hold the rows' places");
+  if (OUTMODE == 0 && kv.cache && t < BM) {
+    slots[t] = slot;
+    int way = vwide && kv_all_runs(slot, lane) ? KV_WAY_RUNS : 0;
+    if (vwide && M >= KV_WALK_MIN_ROWS) {
+      const int offset = kv_run_offset(slot, lane);
+      way = way ? way : offset;
+    }
+    if (fr == 0) ways[t / 32] = way;
+  }
 
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
@@ -128,13 +141,10 @@ tile_epilogue(floatx16 (&acc)[BM / WM / 32][BN / WN / 32], const float (&bias)[B
 
   // A fused q|k|v projection: the k and v columns also go to the rows' places in the paged cache.
   // Keys are rows there: a piece of 8 columns is a piece of the key's row.  Values are dimension-major
-  // (dimension d of a page's rows side by side): 8 consecutive tile rows of one column are one 16-byte
-  // piece where their places are 8 consecutive rows of one page from a multiple of 8 on (a prompt
+  // (dimension d of a page's rows side by side): 4 consecutive tile rows of one column are one 8-byte
+  // piece where their places are 4 consecutive rows of one page from a multiple of 4 on (a prompt
   // portion mostly is), and go entry by entry otherwise.
   if (OUTMODE == 0 && kv.cache) {
-    int* slots = (int*)(smem + tile_out_bytes<BM, BN, OUTMODE>());      // the tile rows' places, -1: none
-    for (int i = t; i < BM; i += THREADS) slots[i] = m0 + i < M ? kv.slot_map[m0 + i] : -1;
-    lds_barrier();
     // (the page size is a power of two, checked on the host: a place splits into page and row by shift and mask)
     const int lgp = 31 - __builtin_clz(kv.page), pmask = kv.page - 1;
     const bool kwide = (uintptr_t)kv.cache % 16 == 0 && kv.D % 8 == 0 && kv.q_cols % 8 == 0;
@@ -155,17 +165,35 @@ tile_epilogue(floatx16 (&acc)[BM / WM / 32][BN / WN / 32], const float (&bias)[B
         if (nn[k] + e >= kv.q_cols && nn[k] + e < v0)
           kv_scatter_bits(kv, pg, prow, nn[k] + e, (bf16_t)(words[e / 2] >> (16 * (e % 2))));
     }
-    // Values: where all groups of 4 rows of a piece of 32 have places that are runs from a multiple of 4 on (one prompt
-    // portion's are), straight from the accumulators: a lane holds 4 consecutive rows of its column (r % 4); the lane
-    // of the other half holds the 4 rows beside them.  Else from the parked tile, a column a lane.
-    const bool vwide = (uintptr_t)kv.cache % 8 == 0 && kv.page % 4 == 0;
+    // Values: straight from the accumulators (a lane holds 4 consecutive rows of its column, r % 4; the lane of the other
+    // half holds the 4 rows beside them), or from the parked tile, a column a lane; see kv_all_runs.
     const long long page_stride = 2LL * kv.Hkv * kv.page * kv.D;
     bf16_t* vb = (bf16_t*)kv.cache;
     if (n0 + wn + BN / WN <= v0 || n0 + wn >= N) return;                // (no value column among the wavefront's)
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int sl = slots[wm + i * 32 + lane % 32];
-      if (__builtin_expect(kv_all_runs(sl, lane, M), 1)) {
+      const int way = __builtin_amdgcn_readfirstlane(ways[wm / 32 + i]);
+      if (__builtin_expect(way == KV_WAY_RUNS, 1)) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int n = n0 + wn + j * 32 + fr;
+          if (n < v0 || n >= N) continue;
+          const int cc = n - v0;
+          const int vcol = (kv.Hkv + cc / kv.D) * kv.page * kv.D + (cc % kv.D) * kv.page;   // the column's run in a page
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            uint32_t w2[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+              w2[e] = pack2_bf16(apply_act_bf16(acc[i][j][4 * q + 2 * e] + bias[j], ACT),
+                                 apply_act_bf16(acc[i][j][4 * q + 2 * e + 1] + bias[j], ACT));
+            const int s0 = slots[wm + i * 32 + 8 * q + 4 * (lane / 32)];
+            *(uint2*)(vb + vcol + (long long)(s0 >> lgp) * page_stride + (s0 & pmask)) = make_uint2(w2[0], w2[1]);
+          }
+        }
+        continue;
+      }
+      if (way == 0) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           const int n = n0 + wn + j * 32 + fr;
@@ -188,8 +216,8 @@ tile_epilogue(floatx16 (&acc)[BM / WM / 32][BN / WN / 32], const float (&bias)[B
       const int n = n0 + wn + lane, cc = n - v0;
       const bool mine = lane < BN / WN && cc >= 0 && n < N;
       bf16_t* const dst = mine ? vb + (long long)(kv.Hkv + cc / kv.D) * kv.page * kv.D + (cc % kv.D) * kv.page : nullptr;
-      kv_store_values32<LDT>((const bf16_t*)smem + (wm + i * 32) * LDT + wn + lane % (BN / WN), sl,
-                             vwide ? kv_run_offset(sl, lane) : -1, dst, page_stride, lgp, pmask);
+      kv_store_values32<LDT>((const bf16_t*)smem + (wm + i * 32) * LDT + wn + lane % (BN / WN),
+                             slots[wm + i * 32 + lane % 32], way, dst, page_stride, lgp, pmask);
     }
   }
 }
@@ -307,6 +335,13 @@ gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__
     const int idx = has ? n : 0;
     braw[j] = bias_bf16 ? (uint32_t)((const bf16_t*)src)[idx] : ((const uint32_t*)src)[idx];
   }
+  // ... and so is the place in the cache of the tile row that this thread puts into LDS
+  int slot = -1;
+  if (OUTMODE == 0) {
+    const bool has = kv.cache && t < BM && m0 + t < M;
+    const int place = *(has ? kv.slot_map + m0 + t : (const int*)w);
+    slot = has ? place : -1;
+  }
 #pragma unroll
   for (int j = 0; j < PF_SLABS; ++j)
     if (j < nslab) TILE_FETCH(j, j * BKT);
@@ -359,7 +394,7 @@ gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__
   float bias[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) bias[j] = !ep.bias ? 0.f : (bias_bf16 ? __uint_as_float(braw[j] << 16) : __uint_as_float(braw[j]));
-  tile_epilogue<BM, BN, WM, WN, ACT, OUTMODE>(acc, bias, smem, (const void*)w, ep, kv, M, N, m0, n0);
+  tile_epilogue<BM, BN, WM, WN, ACT, OUTMODE>(acc, bias, smem, (const void*)w, ep, kv, slot, M, N, m0, n0);
 }
 
 template <int BM, int BN, int WM, int WN, int PF, int ACT, int OUTMODE>

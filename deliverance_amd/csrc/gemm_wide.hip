@@ -23,7 +23,7 @@
 // of LDS (bias and activation applied, rounded to the output's type), and leave in 16-byte pieces, whole
 // rows side by side; += adds to 16-byte pieces read the same way; a fused q|k|v projection also writes
 // its k and v columns to the rows' places in the paged cache (keys in 16-byte pieces of their rows,
-// values in 8-byte runs where 4 rows' places are consecutive: kv_all_runs, kv_run_offset).
+// values in 8-byte runs where 4 rows' places are consecutive: kv_all_runs).
 #include "gemm_common.h"
 #include <da_lds_dma.h>
 #include <type_traits>
@@ -73,6 +73,15 @@ wide_epilogue(floatx16 (&acc)[TM][TN], const float (&bias)[TN], char* region, co
       vcol[j] = (kv.Hkv + cs / kv.D) * kv.page * kv.D + (cs % kv.D) * kv.page;
     }
   }
+  // the places of every pass's rows (row `lane % 32` of each) are asked for here: a load inside a pass would wait for the
+  // stores of the pass before it
+  int sl[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = mw + i * 32 + fr;
+    sl[i] = OUTMODE == 0 && kv.cache ? *(m < M ? kv.slot_map + m : (const int*)safe) : -1;
+    sl[i] = m < M ? sl[i] : -1;
+  }
   // (a pass per constant i: an index that is not a constant would put the accumulators into memory)
   auto pass = [&](auto ic) {
     constexpr int i = decltype(ic)::value;
@@ -85,7 +94,7 @@ wide_epilogue(floatx16 (&acc)[TM][TN], const float (&bias)[TN], char* region, co
         if (OUTMODE == 0) ((bf16_t*)region)[ml * LDT + nl] = f32_to_bf16(apply_act_bf16(acc[i][j][r] + bias[j], ACT));
         else ((float*)region)[ml * LDT + nl] = apply_act(acc[i][j][r] + bias[j], ACT);
       }
-    if (OUTMODE == 0 && kv.cache && lane < 32) slots[lane] = mp + lane < M ? kv.slot_map[mp + lane] : -1;
+    if (OUTMODE == 0 && kv.cache && lane < 32) slots[lane] = sl[i];
     wave_lds_sync();
 
     uint4 val[NCHK];
@@ -152,14 +161,29 @@ wide_epilogue(floatx16 (&acc)[TM][TN], const float (&bias)[TN], char* region, co
           if (nn[k] + e >= kv.q_cols && nn[k] + e < v0)
             kv_scatter_bits(kv, pg, prow, nn[k] + e, (bf16_t)(words[e / 2] >> (16 * (e % 2))));
       }
-      // values: where the groups of 4 rows have places that are runs from a multiple of 4 on (one prompt portion's
-      // are), straight from the accumulators: a lane holds 4 consecutive rows of its column (r % 4), which are 8
-      // consecutive bytes of the dimension-major page; the lane of the other half holds the 4 rows beside them.
-      // Else from LDS, a column a lane.
+      // values: straight from the accumulators (a lane holds 4 consecutive rows of its column, r % 4; the lane of the
+      // other half holds the 4 rows beside them), or from LDS, a column a lane; see kv_all_runs
       if (nw + WC > v0) {
         bf16_t* vb = (bf16_t*)kv.cache;
-        const int sl = slots[lane % 32];
-        if (__builtin_expect(kv_all_runs(sl, lane, M), 1)) {
+        int offset = 0;
+        const bool runs = vwide && __builtin_amdgcn_readfirstlane(kv_all_runs(sl[i], lane));
+        if (__builtin_expect(runs, 1)) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            const int n = nw + j * 32 + fr;
+            if (n < v0 || n >= N) continue;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              uint32_t w2[2];
+#pragma unroll
+              for (int e = 0; e < 2; ++e)
+                w2[e] = pack2_bf16(apply_act_bf16(acc[i][j][4 * q + 2 * e] + bias[j], ACT),
+                                   apply_act_bf16(acc[i][j][4 * q + 2 * e + 1] + bias[j], ACT));
+              const int s0 = slots[8 * q + 4 * (lane / 32)];
+              *(uint2*)(vb + vcol[j] + (long long)(s0 >> lgp) * page_stride + (s0 & pmask)) = make_uint2(w2[0], w2[1]);
+            }
+          }
+        } else if (!(vwide && M >= KV_WALK_MIN_ROWS && (offset = __builtin_amdgcn_readfirstlane(kv_run_offset(sl[i], lane))) != 0)) {
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
             const int n = nw + j * 32 + fr;
@@ -178,7 +202,7 @@ wide_epilogue(floatx16 (&acc)[TM][TN], const float (&bias)[TN], char* region, co
           static_assert(WC == 64, "a column a lane");
           const int n = nw + lane, cc = n - v0;
           bf16_t* const dst = cc >= 0 && n < N ? vb + (long long)(kv.Hkv + cc / kv.D) * kv.page * kv.D + (cc % kv.D) * kv.page : nullptr;
-          kv_store_values32<LDT>((const bf16_t*)region + lane, sl, vwide ? kv_run_offset(sl, lane) : -1, dst, page_stride, lgp, pmask);
+          kv_store_values32<LDT>((const bf16_t*)region + lane, sl[i], offset, dst, page_stride, lgp, pmask);
         }
       }
     }

@@ -131,6 +131,15 @@ static inline float __shfl_xor(float v, int mask, int) {
 static inline int __shfl_xor(int v, int mask, int) {
   return (int)simt::lane_exchange((uint32_t)v, simt::lane_id() ^ mask, 0u);
 }
+// a bit a lane, for flow that is the same in all lanes
+static inline uint64_t simt_ballot(bool v) {
+  uint32_t half[2] = {0u, 0u};
+  half[simt::lane_id() / 32] = (uint32_t)v << (simt::lane_id() % 32);
+  for (int h = 0; h < 2; ++h)
+    for (int m = 1; m < 64; m *= 2) half[h] |= simt::lane_exchange(half[h], simt::lane_id() ^ m, 0u);
+  return half[0] | (uint64_t)half[1] << 32;
+}
+#define __builtin_amdgcn_ballot_w64(v) simt_ballot(v)
 static inline int __shfl(int v, int src, int) { return (int)simt::lane_exchange((uint32_t)v, src, 0u); }
 static inline float __shfl(float v, int src, int) {
   return __uint_as_float(simt::lane_exchange(__float_as_uint(v), src, 0u));
