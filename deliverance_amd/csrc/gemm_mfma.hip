@@ -8,7 +8,7 @@
 //  * gemm_tile: block tiles of 64x64 to 128x128 (MFMA 32x32x16), operands staged through two LDS
 //    buffers, with the next four slabs already in flight in registers.  For steps with many rows
 //    (prefill).  Products whose sizes suit them go to gemm_wide.hip's tiles instead (da_gemm_wide_choice).
-//  * gemm_skinny: for M <= 64 (decode); gemm_skinny32 where there are more than 4,096 columns (no vocabulary).  A workgroup owns 16 output columns; its wavefronts (4 to 12)
+//  * gemm_skinny: for M <= 64 (decode); gemm_skinny32 where they would be more workgroups than compute units (sk_one_a_unit).  A workgroup owns 16 output columns; its wavefronts (4 to 12)
 //    split K, pull their part of a and w from memory in whole cache lines, pass it through LDS into
 //    MFMA 16x16x32 fragments and add their sums through LDS in a fixed order.  Bound by the bytes of w.
 //  * gemm_skinny4: for M <= 4 and up to 2,048 columns.  MFMA 4x4x4, whose operand layout lets a row
@@ -588,13 +588,14 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restri
 }
 
 // ---------------------------------------------------------------------------------------------
-// M <= 64 where 16 columns a workgroup would give more workgroups than the chip has compute units.  A compute unit
-// pulls in 70 GB/s at best, whatever the pattern (30 to 45 while all of them read from memory), so the bytes of the busiest
-// one are what a product of few rows takes: with two or three workgroups of all rows and 16 columns it pulls the rows of a
-// two or three times.  Here a workgroup owns all rows (row tiles) and `cols` columns, 32 at most, chosen so that every
+// M <= 64 where 16 columns a workgroup would give more workgroups than the chip has compute units (sk_one_a_unit: which
+// sizes).  A compute unit pulls in 70 GB/s at best, whatever the pattern, so the bytes of the busiest
+// one are what a product of few rows takes: with two workgroups of all rows and 16 columns it pulls the rows of a
+// twice.  Here a workgroup owns all rows (row tiles) and `cols` columns, 32 at most, chosen so that every
 // compute unit has one; the rest is as above, except that P steps are in flight in registers at any time: a step's
-// registers take the step P further on as soon as they are parked.
-// Measured on MI355X with cold weights, K = 1,600, N = 4,800 / 6,400 (16 columns -> 19 / 25): 16 rows 7.4 / 7.9 -> 6.4 / 7.2 us,
+// registers take the step P further on as soon as they are parked.  The same sums in the same order as gemm_skinny with 8
+// wavefronts.
+// Measured on MI355X with cold weights, K = 1,600, N = 4,800 / 6,400 (16 columns -> 19 / 25): 16 rows 7.1 / 6.8 -> 6.4 / 6.8 us,
 // 32 rows 10.0 / 10.4 -> 7.8 / 8.4, 48 rows 11.3 / 13.6 -> 8.6 / 9.3, 64 rows 12.4 / 14.6 -> 10.3 / 10.8.
 // ---------------------------------------------------------------------------------------------
 // What one lane of a wavefront leaves in LDS another lane of it reads: LDS serves a wavefront's instructions in order, so
@@ -754,6 +755,21 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
   }
 }
 
+// Whether a product of few rows goes to gemm_skinny32: more than 4,096 columns (fewer give no compute unit two workgroups of
+// 16) and up to 8,192.  More than 16 rows: always (K from 64 to 8,192: 0.55 to 0.98 of the time of 16 columns a
+// workgroup).  Up to 16 rows the rows are few bytes and two workgroups a compute unit hide more latency than one, so it
+// pays only where the busiest compute unit pulls much less of w: with a long K and well below 32 columns a unit.
+// Measured with cold weights, 16 columns against one workgroup a unit, both with 8 wavefronts:
+//    8 rows: K = 1,600, N = 4,800 6.3 against 6.1 us, 8,192 7.0 / 7.8; K = 4,096, N = 4,112 10.6 / 9.2, 6,400 11.9 / 12.1, 8,192 13.1 / 16.3; K = 8,192, N = 6,400 23.8 / 21.7
+//   16 rows: K = 1,600, N = 4,800 7.1 against 6.4 us, 5,888 6.9 / 6.7, 7,168 7.0 / 7.2; K = 3,072, N = 7,168 11.8 / 10.8, 7,680 11.9 / 11.2
+static bool sk_one_a_unit(int M, int N, int K) {
+  const int cols = da_ceil_div(N, 256);              // of the busiest compute unit, where 16 a workgroup give it 32
+  if (cols <= 16 || cols > 32) return false;
+  if (M > 16) return true;
+  if (M > 8) return (K >= 1280 && cols <= 23) || (K >= 3072 && cols <= 28);
+  return (M > 4 && K >= 1280 && cols <= 20) || (K >= 3072 && cols <= 22 + K / 2048);
+}
+
 template <int NW>
 static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw,
                          const Epilogue& ep, const KvScatter& kv, int M, int N, int K) {
@@ -766,12 +782,11 @@ static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* 
     if (M <= 8) DA_SK_GO(1, 8, 4); else DA_SK_GO(2, 8, 4);
     return 0;
   }
-  if (da_ceil_div(N, 16) > 256 && N <= 32 * 256) {
+  if (NW == 8 && sk_one_a_unit(M, N, K)) {
     const int cols = da_ceil_div(N, 256);            // every compute unit one workgroup
     const dim3 grid(da_ceil_div(N, cols));
 #define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, cols)
-    // (8 wavefronts whatever the rows, so that a row's sums keep their order; steps in flight: what the registers of a
-    // workgroup that is alone on its compute unit allow)
+    // (steps in flight: what the registers of a workgroup that is alone on its compute unit allow)
     if (M <= 8) DA_SK32_GO(1, 4);
     else if (mt == 1) DA_SK32_GO(2, 4);
     else if (mt == 2) DA_SK32_GO(4, 3);
@@ -1013,8 +1028,9 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
                   : launch_skinny4<2>(nw, s, A, lda, W, ldw, ep, kv, M, N, K)) return 1;
   } else if (da_gemm_few_rows(M, N)) {
     // The number of wavefronts that split K depends on K and N alone, so a row's sums keep their order:
-    // 4 where the workgroups are many (a vocabulary: several then share a compute unit), else 8, or 12 for a long K.
-    const int nw = da_ceil_div(N, 16) > 1024 ? 4 : (K >= 2048 ? 12 : 8);
+    // 4 where the workgroups are many (a vocabulary: several then share a compute unit), else 8, or 12 for a long K where no compute
+    // unit has two workgroups (between 4,097 and 8,192 columns, K from 2,048 on, up to 16 rows 8 take 0.84 to 0.96 of 12's time).
+    const int nw = da_ceil_div(N, 16) > 1024 ? 4 : (K >= 2048 && (N <= 16 * 256 || N > 32 * 256) ? 12 : 8);
     if (nw == 4 ? launch_skinny<4>(s, A, lda, W, ldw, ep, kv, M, N, K)
                 : (nw == 8 ? launch_skinny<8>(s, A, lda, W, ldw, ep, kv, M, N, K)
                            : launch_skinny<12>(s, A, lda, W, ldw, ep, kv, M, N, K))) return 1;

@@ -211,10 +211,12 @@ def test_gemm_matrix_cores(ops, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 4100, 2600), (8, 4800, 1600), helpers.quick(3, 4112, 40), (16, 8192, 72), (17, 6401, 648),
-                                   (48, 8190, 1160), (64, 4800, 4616)])
+                                   (48, 8190, 1160), (64, 4800, 4616), (9, 5888, 1288), (9, 5889, 1288), (16, 7168, 3080), (16, 7169, 3080),
+                                   (4, 5888, 3080), (4, 5889, 3080), (5, 5120, 1288), (5, 5121, 1288), (5, 8192, 4104)])
 def test_gemm_one_workgroup_a_compute_unit(ops, M, N, K):
-    """Between 4,097 and 8,192 columns: up to 32 columns a workgroup (17 to 32 here), several rounds of steps in flight, a
-    last step that K cuts; a row has the same bits beside any other rows; keys and values in the epilogue."""
+    """Between 4,097 and 8,192 columns: 16 columns a workgroup or up to 32 (17 to 32 here), both sides of the lines between them,
+    several rounds of steps in flight, a last step that K cuts; a row has the same bits beside any other rows, so also in either
+    kernel; keys and values in the epilogue."""
     g = torch.Generator().manual_seed(M + N)
     for act, acc, bias, od in ((None, False, True, torch.bfloat16), ("gelu_new", False, False, torch.bfloat16), (None, True, True, torch.float32)):
         out, ref = _gemm_case(ops, ops.linear_mfma, M, N, K, torch.bfloat16, act, acc, bias, od, g)
