@@ -2,15 +2,15 @@
 //
 //   rms(x)[i] = x[i] / sqrt(mean(x^2) + eps) * (offset + w[i])
 //
-// `offset` is 0 for a gain stored as it is applied and 1 for a gain stored around zero.  A workgroup of
-// four wavefronts owns a row; where the width allows it the whole row sits in registers, so every load is in flight
-// at once and the row is read once.  (Four wavefronts a row and not one: with few rows the chain of instructions
-// behind the loads is what the kernel takes.)
+// `offset` is 0 for a gain stored as it is applied and 1 for a gain stored around zero.  Four wavefronts or one own a
+// row (norm_grid); where the width allows it the whole row sits in registers, so every load is in flight
+// at once and the row is read once.
 //
 //   da_rmsnorm      y = rms(x[rows[r]] or x[r])                       (32-bit or bfloat16 out)
 //   da_rmsnorm_add  x += rms_a(src);  h = rms_b(x), or x itself converted (optional)   the norm behind a part, the residual
 //                   addition and the norm in front of the next part in one pass over the row
-#include "common.h"
+#include "norm_common.h"
+#include <limits.h>
 
 __device__ __forceinline__ float4 rms_param4(const void* p, int dtype, int i) {
   if (dtype == DA_BF16) {
@@ -29,26 +29,18 @@ __device__ __forceinline__ void rms_store4(void* y, int y_dtype, size_t at, floa
   }
 }
 
-#define RMS_WAVES 4
-
-// the sum over the row's wavefronts, in every lane; `red` is used once
-__device__ __forceinline__ float rms_row_sum(float v, float* red) {
-  v = wave_sum(v);
-  if (threadIdx.x % DA_WAVE == 0) red[threadIdx.x / DA_WAVE] = v;
-  lds_barrier();
-  return (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-// VPL float4 a lane: E a multiple of 4, E <= 1024 * VPL.  ADD: src is normalised with (wa), added into x,
+// VPL float4 a lane: W wavefronts a row (4, or 1): E a multiple of 4, E <= 256 * W * VPL.  ADD: src is normalised with (wa), added into x,
 // and (if h) the new x is normalised with (wb) into h.  !ADD: y = rms(x) with wa.
-template <int VPL, bool ADD>
-__global__ void __launch_bounds__(RMS_WAVES * DA_WAVE)
+template <int VPL, int W, bool ADD>
+__global__ void __launch_bounds__(4 * DA_WAVE)
 rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, const void* __restrict__ wa, int wa_dtype,
                    float* __restrict__ x, const void* __restrict__ wb, int wb_dtype, float offset, float eps,
-                   void* __restrict__ y, int y_dtype, int E) {
-  __shared__ float red[2][RMS_WAVES];
-  constexpr int STRIDE = 4 * RMS_WAVES * DA_WAVE;
-  const int r = blockIdx.x, c0 = (int)threadIdx.x * 4;
+                   void* __restrict__ y, int y_dtype, int R, int E) {
+  __shared__ float red[2][4 * DA_WAVE];
+  constexpr int STRIDE = 4 * W * DA_WAVE;
+  const int t = threadIdx.x, c0 = (W == 4 ? t : t % DA_WAVE) * 4;
+  const int r = W == 4 ? (int)blockIdx.x : (int)(blockIdx.x * (blockDim.x / DA_WAVE)) + t / DA_WAVE;
+  if (W == 1 && r >= R) return;
   const float* sr = src + (size_t)(rows ? rows[r] : r) * E;
   // the gains are asked for beside the rows, so that the kernel costs one round trip to memory and not one per norm
   float4 v[VPL], xv[VPL], ga[VPL], gb[VPL];
@@ -64,24 +56,22 @@ rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, 
     ga[i] = rms_param4(wa, wa_dtype, cc);
     if (ADD && y && wb) gb[i] = rms_param4(wb, wb_dtype, cc);
   }
-  float q = 0.f;
+  float part[VPL];
 #pragma unroll
-  for (int i = 0; i < VPL; ++i)
-    if (c0 + i * STRIDE < E) q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
-  const float inv = 1.0f / sqrtf(rms_row_sum(q, red[0]) / (float)E + eps);
-  float q2 = 0.f;
+  for (int i = 0; i < VPL; ++i) part[i] = c0 + i * STRIDE < E ? norm_squares(v[i]) : 0.f;
+  const float inv = 1.0f / sqrtf(norm_row_sum<W>(part, red[0]) / (float)E + eps);
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int c = c0 + i * STRIDE;
     if (c < E) {
       const float4 g = ga[i];
-      float4 o = make_float4(v[i].x * inv * (offset + g.x), v[i].y * inv * (offset + g.y),
-                             v[i].z * inv * (offset + g.z), v[i].w * inv * (offset + g.w));
+      const float4 old = ADD ? xv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 o = make_float4(norm_scaled(v[i].x, inv, offset + g.x, old.x), norm_scaled(v[i].y, inv, offset + g.y, old.y),
+                                   norm_scaled(v[i].z, inv, offset + g.z, old.z), norm_scaled(v[i].w, inv, offset + g.w, old.w));
       if (ADD) {
-        o = make_float4(xv[i].x + o.x, xv[i].y + o.y, xv[i].z + o.z, xv[i].w + o.w);
         *(float4*)(x + (size_t)r * E + c) = o;
         xv[i] = o;
-        q2 += (o.x * o.x + o.y * o.y) + (o.z * o.z + o.w * o.w);
+        part[i] = norm_squares(o);                     // (past the row's end it stays 0)
       } else {
         rms_store4(y, y_dtype, (size_t)r * E + c, o);
       }
@@ -94,7 +84,7 @@ rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, 
       if (c < E) rms_store4(y, y_dtype, (size_t)r * E + c, xv[i]);
     }
   } else if (ADD && y) {
-    const float inv2 = 1.0f / sqrtf(rms_row_sum(q2, red[1]) / (float)E + eps);
+    const float inv2 = 1.0f / sqrtf(norm_row_sum<W>(part, red[1]) / (float)E + eps);
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
       const int c = c0 + i * STRIDE;
@@ -145,13 +135,18 @@ static void rms_launch(const float* src, const int* rows, const void* wa, int wa
                        int wb_dtype, float offset, float eps, void* y, int y_dtype, int R, int E, hipStream_t st) {
   const bool aligned = ((uintptr_t)src % 16 == 0) && ((uintptr_t)y % 16 == 0) && ((uintptr_t)wa % 16 == 0) &&
                        ((uintptr_t)wb % 16 == 0) && ((uintptr_t)x % 16 == 0);
-#define RMS_LAUNCH(V)                                                                                              \
-  hipLaunchKernelGGL((rmsnorm_row_kernel<V, ADD>), dim3(R), dim3(RMS_WAVES * DA_WAVE), 0, st, src, rows, wa, wa_dtype, x, \
-                     wb, wb_dtype, offset, eps, y, y_dtype, E)
+#define RMS_LAUNCH(V, W)                                                                                             \
+  hipLaunchKernelGGL((rmsnorm_row_kernel<V, W, ADD>), dim3(g.blocks), dim3(g.threads), 0, st, src, rows, wa, wa_dtype, x, \
+                     wb, wb_dtype, offset, eps, y, y_dtype, R, E)
   if (E % 4 == 0 && E <= 4096 && aligned) {
-    if (E <= 1024) RMS_LAUNCH(1);
-    else if (E <= 2048) RMS_LAUNCH(2);
-    else RMS_LAUNCH(4);
+    const NormGrid g = norm_grid(R, E, 1536, ADD ? INT_MAX : 4096);
+    if (g.waves == 1) {
+      if (E <= 256) RMS_LAUNCH(1, 1);
+      else if (E <= 512) RMS_LAUNCH(2, 1);
+      else RMS_LAUNCH(4, 1);
+    } else if (E <= 1024) RMS_LAUNCH(1, 4);
+    else if (E <= 2048) RMS_LAUNCH(2, 4);
+    else RMS_LAUNCH(4, 4);
   } else {
     hipLaunchKernelGGL((rmsnorm_any_kernel<ADD>), dim3(da_ceil_div(R, 4)), dim3(4 * DA_WAVE), 0, st, src, rows, wa,
                        wa_dtype, x, wb, wb_dtype, offset, eps, y, y_dtype, R, E);

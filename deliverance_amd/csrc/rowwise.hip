@@ -1,6 +1,6 @@
 // Row-wise kernels: embedding (+ learned positions), LayerNorm (optionally on gathered
 // rows), and the write of new keys and values into the paged cache.
-#include "common.h"
+#include "norm_common.h"
 #include <stdarg.h>
 
 static thread_local char g_error[512] = "";
@@ -205,33 +205,25 @@ __device__ __forceinline__ float4 load_param4(const void* p, int dtype, int i) {
 }
 
 // The same norm with the whole row held in registers: every load of the row is in flight at
-// once, which is what counts when a step has a handful of rows.  E a multiple of 4, E <= 1024 * VPL.
-// A workgroup of four wavefronts is one row, a float4 a lane (two above a width of 1,024): the chain of
+// once, which is what counts when a step has a handful of rows.  E a multiple of 4, E <= 256 * W * VPL.
+// W = 4: a workgroup of four wavefronts is one row, a float4 a lane (two above a width of 1,024): with few rows the chain of
 // instructions behind the loads, not the bytes, is what the kernel takes (measured in a recorded chain
 // behind the kernel that writes x, one wavefront a row -> four: 64 rows of 768 2.4 -> 2.2 us, of 1,024 2.5 -> 2.1,
-// of 1,600 3.1 -> 2.5; 2,048 rows of 1,600 9.4 -> 8.9, of 1,024 level), whatever the rows, so that a row's sums keep
-// their order.
+// of 1,600 3.1 -> 2.5; 2,048 rows of 1,600 9.4 -> 8.9).
+// W = 1: a wavefront a row.  Both give the same bits (norm_row_sum); which one is taken: norm_grid.
 // Loads come back in the order they were asked for: the row first, then gain and bias, as raw bits
 // that are converted where they are used (a conversion right after its load, or a load inside a
 // branch, is waited for on the spot).  PBF16: gain and bias are bfloat16 (else 32-bit); YBF16: y is.
-#define LN_WAVES 4
-
-// the sum over the row's wavefronts, in every lane; `red` is used once
-__device__ __forceinline__ float ln_row_sum(float v, float* red) {
-  v = wave_sum(v);
-  if (threadIdx.x % DA_WAVE == 0) red[threadIdx.x / DA_WAVE] = v;
-  lds_barrier();
-  return (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-template <int VPL, bool PBF16, bool YBF16>
-__global__ void __launch_bounds__(LN_WAVES * DA_WAVE)
+template <int VPL, int W, bool PBF16, bool YBF16>
+__global__ void __launch_bounds__(4 * DA_WAVE)
 layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                      const void* __restrict__ w, const void* __restrict__ b,
-                     float eps, void* __restrict__ y, int E) {
-  __shared__ float red[2][LN_WAVES];
-  constexpr int STRIDE = 4 * LN_WAVES * DA_WAVE;
-  const int r = blockIdx.x, c0 = (int)threadIdx.x * 4;
+                     float eps, void* __restrict__ y, int R, int E) {
+  __shared__ float red[2][4 * DA_WAVE];
+  constexpr int STRIDE = 4 * W * DA_WAVE;
+  const int t = threadIdx.x, c0 = (W == 4 ? t : t % DA_WAVE) * 4;
+  const int r = W == 4 ? (int)blockIdx.x : (int)(blockIdx.x * (blockDim.x / DA_WAVE)) + t / DA_WAVE;
+  if (W == 1 && r >= R) return;
   const float* xr = x + (size_t)(rows ? rows[r] : r) * E;
   // every load of the row, of the gain and of the bias is asked for at once (past the row's end
   // the row's start is read and left out of the sums), before anything is reduced
@@ -256,18 +248,16 @@ layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  float s = 0.f;
+  float part[VPL];
 #pragma unroll
-  for (int i = 0; i < VPL; ++i)
-    if (c0 + i * STRIDE < E) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-  const float mean = ln_row_sum(s, red[0]) / (float)E;
-  float q = 0.f;
+  for (int i = 0; i < VPL; ++i) part[i] = c0 + i * STRIDE < E ? (v[i].x + v[i].y) + (v[i].z + v[i].w) : 0.f;
+  const float mean = norm_row_sum<W>(part, red[0]) / (float)E;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     v[i].x -= mean; v[i].y -= mean; v[i].z -= mean; v[i].w -= mean;
-    if (c0 + i * STRIDE < E) q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    part[i] = c0 + i * STRIDE < E ? norm_squares(v[i]) : 0.f;
   }
-  const float inv = 1.0f / sqrtf(ln_row_sum(q, red[1]) / (float)E + eps);
+  const float inv = 1.0f / sqrtf(norm_row_sum<W>(part, red[1]) / (float)E + eps);
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int c = c0 + i * STRIDE;
@@ -283,8 +273,8 @@ layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
       bb = make_float4(__uint_as_float(braw[i].x), __uint_as_float(braw[i].y), __uint_as_float(braw[i].z), __uint_as_float(braw[i].w));
     }
     if (!b) bb = make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 o = make_float4(v[i].x * inv * g.x + bb.x, v[i].y * inv * g.y + bb.y,
-                                 v[i].z * inv * g.z + bb.z, v[i].w * inv * g.w + bb.w);
+    const float4 o = make_float4(norm_scaled(v[i].x, inv, g.x, bb.x), norm_scaled(v[i].y, inv, g.y, bb.y),
+                                 norm_scaled(v[i].z, inv, g.z, bb.z), norm_scaled(v[i].w, inv, g.w, bb.w));
     if (YBF16) *(uint2*)((bf16_t*)y + (size_t)r * E + c) = make_uint2(pack2_bf16(o.x, o.y), pack2_bf16(o.z, o.w));
     else *(float4*)((float*)y + (size_t)r * E + c) = o;
   }
@@ -301,11 +291,16 @@ extern "C" int da_layernorm(const float* x, const int* rows, const void* w, int 
                        (!b || (uintptr_t)b % 16 == 0);
   const bool same = (!b || b_dtype == w_dtype) && (w_dtype == DA_BF16 || w_dtype == DA_F32);   // gain and bias alike
   if (E % 4 == 0 && E <= 2048 && aligned && same) {
-#define LN_LAUNCH(V, P, Y) hipLaunchKernelGGL((layernorm_row_kernel<V, P, Y>), dim3(R), dim3(LN_WAVES * DA_WAVE), 0, st, x, rows, w, b, eps, y, E)
-#define LN_LAUNCH_Y(V, P) do { if (y_dtype == DA_BF16) LN_LAUNCH(V, P, true); else LN_LAUNCH(V, P, false); } while (0)
-#define LN_LAUNCH_P(V) do { if (w_dtype == DA_BF16) LN_LAUNCH_Y(V, true); else LN_LAUNCH_Y(V, false); } while (0)
-    if (E <= 4 * LN_WAVES * DA_WAVE) LN_LAUNCH_P(1);
-    else LN_LAUNCH_P(2);
+    const NormGrid g = norm_grid(R, E, 1024, 1536);
+#define LN_LAUNCH(V, W, P, Y) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, Y>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, eps, y, R, E)
+#define LN_LAUNCH_Y(V, W, P) do { if (y_dtype == DA_BF16) LN_LAUNCH(V, W, P, true); else LN_LAUNCH(V, W, P, false); } while (0)
+#define LN_LAUNCH_P(V, W) do { if (w_dtype == DA_BF16) LN_LAUNCH_Y(V, W, true); else LN_LAUNCH_Y(V, W, false); } while (0)
+    if (g.waves == 1) {
+      if (E <= 256) LN_LAUNCH_P(1, 1);
+      else if (E <= 512) LN_LAUNCH_P(2, 1);
+      else LN_LAUNCH_P(4, 1);
+    } else if (E <= 1024) LN_LAUNCH_P(1, 4);
+    else LN_LAUNCH_P(2, 4);
 #undef LN_LAUNCH_P
 #undef LN_LAUNCH_Y
 #undef LN_LAUNCH

@@ -96,6 +96,37 @@ def test_layernorm(ops, E, eps):
         assert (o3[0] - want3).abs().max() < 1e-4
 
 
+@pytest.mark.parametrize("E", [helpers.quick(132), helpers.quick(256), 260, helpers.quick(512), 516, 768, 1000, 1024])
+def test_norms_of_many_rows(ops, E):
+    """Rows of up to 1,024 columns take one wavefront or four by their number: the same bits either way, at the lines between
+    the two and beside them."""
+    R = 1537 if E <= 512 else 4097
+    helpers.skip_in_simulation_if(E > 512)
+    g = torch.Generator().manual_seed(E)
+    x, src = ((torch.randn(R, E, generator=g) * 3 + 5).to(DEV) for _ in range(2))
+    w, b = (torch.randn(E, generator=g).to(DEV) for _ in range(2))
+    for y, dt in ((torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)):
+        def norms(lo, hi):
+            n, outs = hi - lo, []
+            outs.append(ops.layernorm(x[lo:hi], w.to(dt), b.to(dt), 1e-5, torch.empty(n, E, dtype=y, device=DEV)))
+            outs.append(ops.rmsnorm(x[lo:hi], w.to(dt), 1.0, 1e-5, torch.empty(n, E, dtype=y, device=DEV)))
+            stream, h = x[lo:hi].clone(), torch.empty(n, E, dtype=y, device=DEV)
+            ops.rmsnorm_add(src[lo:hi], w.to(dt), stream, 1.0, 1e-5, b.to(dt), h)
+            return outs + [stream, h]
+        few = norms(0, 5)
+        for n in (R,) if helpers.SIMT else (511, 513, 1023, 1024, 1535, 1536, R - 1, R):
+            many = norms(0, n)
+            assert all(torch.equal(f, m[:5]) for f, m in zip(few, many)), n
+            if n == R:
+                assert all(torch.equal(f, m[-5:]) for f, m in zip(norms(n - 5, n), many))
+        wd, bd, xd = w.to(dt).double(), b.to(dt).double(), x.double()
+        rms = lambda v, gain: v / (v.square().mean(1, keepdim=True) + 1e-5).sqrt() * (1.0 + gain)
+        new = xd + rms(src.double(), wd)
+        for got, want in zip(many, (F.layer_norm(xd, (E,), wd, bd, 1e-5), rms(xd, wd), new, rms(new, bd))):
+            tol = 2e-5 if got.dtype == torch.float32 else 2.0 ** -8       # (32-bit: as for LayerNorm above; bfloat16: one rounding)
+            assert ((got.double() - want).abs() / want.abs().clamp(min=1.0)).max() < tol
+
+
 # ----------------------------------------------------------------------------- products
 def _gemm_case(ops, fn, M, N, K, dtype, act, accumulate, bias, out_dtype, g):
     a = (torch.randn(M, K, generator=g) * 0.5).to(dtype).to(DEV)
