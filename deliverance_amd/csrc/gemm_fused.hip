@@ -196,9 +196,9 @@ gemm_ln_skinny_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epil
 // share a compute unit and N / 16 workgroups run side by side.
 // ---------------------------------------------------------------------------------------------
 #define FL_LD (64 + 8)       // padded row of a parked step of w, elements
-// A workgroup owns `cols` columns, 16 * CT at most.  16 of them leave some compute units with two workgroups and others
-// with one where there are more than 256: the launch then takes ceil(N / 256) columns (CT 2), one workgroup a compute
-// unit.  A compute unit pulls in about 70 GB/s at best (30 to 45 while all of them read from memory), so its bytes are
+// A workgroup owns `cols` columns, 16 * CT at most.  16 of them leave some compute units with more workgroups than others
+// where there are more than 256: the launch then takes as many columns (CT 2) as give every compute unit one workgroup, or
+// two.  A compute unit pulls in about 70 GB/s at best, so its bytes are
 // what the kernel takes: rows of w, the rows of x, and gain and bias once a wavefront that has a row.
 template <int RV, bool PBF16, bool TWO_ROWS, int CT = 1>
 __global__ void __launch_bounds__(512)
@@ -394,13 +394,18 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
   const int mt = da_ceil_div(M, 16);
   hipStream_t s = (hipStream_t)stream;
   // the kernel with whole-line loads takes one row tile, K up to 2048, and parameters of one dtype
-  // Columns a workgroup: 16, or where that gives more than 256 workgroups (and 32 at most are enough) as many as give
-  // every compute unit one.  Measured on MI355X with cold weights, K = 1,600, N = 4,800 and 6,400
-  // (16 columns -> 19 and 25, with the loads of gain and bias kept to wavefronts that have a row): one row 8.1 and 8.6 us ->
-  // 7.0 and 7.6, 3 rows 8.6 and 8.8 -> 7.4 and 7.9, 8 rows (two groups of 16 columns a workgroup, one after the other) 9.6 and 10.3 ->
-  // 8.8 and 9.8.
-  const bool wide = N > 16 * 256 && N <= 32 * 256;
-  const int cols = wide ? da_ceil_div(N, 256) : FZ_COLS;
+  // Columns a workgroup: 16 up to 4,096 columns and for a vocabulary; up to 8,192 as many as give every compute unit one
+  // workgroup; up to 16,384 as many as give every one two, where two fit side by side (registers: K up to 1,536; LDS: with more than
+  // 8 rows K up to 1,024).  Measured on MI355X with cold weights, 16 columns a workgroup -> this, us:
+  //   K = 1,600, N = 4,800 (19 columns) one row 6.9 -> 6.6, 8 rows 9.6 -> 8.2; N = 6,400 (25) 7.4 -> 7.3, 10.2 -> 9.5
+  //   K =   768, N = 8,320 (17, two a unit) one row 5.5 -> 5.4, 16 rows 10.0 -> 8.6; N = 12,800 (25) 6.4 -> 6.2, 12.2 -> 9.2
+  //   K = 1,536, N = 8,200 (17) one row 7.9 -> 7.6, 8 rows 10.4 -> 10.0; N = 12,800 10.8 -> 9.4, 14.3 -> 11.9; N = 16,384 (32) 11.5 -> 10.9,
+  //              15.0 -> 13.4 (two groups of 16 columns, one after the other: 8 rows 10.4, 13.3 and 14.3)
+  //   K = 1,600, N = 12,800, where only one of 25 fits: one row 11.6 -> 12.4 (so 16 stay; 8 rows: da_can_fuse_ln)
+  const bool one_a_unit = N > 16 * 256 && N <= 32 * 256;
+  const bool two_a_unit = N > 32 * 256 && N <= 64 * 256 && K <= (M <= 8 ? 1536 : 1024);
+  const bool wide = one_a_unit || two_a_unit;
+  const int cols = one_a_unit ? da_ceil_div(N, 256) : (two_a_unit ? da_ceil_div(N, 512) : FZ_COLS);
   const int pdt = g_dtype;
   const bool same = (!b || b_dtype == pdt) && (!bias || bias_dtype == pdt) && (pdt == DA_BF16 || pdt == DA_F32);
 #define LAUNCH_LDS_R(RV, PB, TWO)                                                                                  \

@@ -266,9 +266,12 @@ def test_gemm_one_workgroup_a_compute_unit(ops, M, N, K):
         assert torch.equal(c1, c2) and bool(c1.any())
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 4800, 1600), (3, 6400, 1600), helpers.quick(2, 4100, 72), (8, 8192, 1304), (16, 4801, 1000), (9, 6000, 768)])
+@pytest.mark.parametrize("M,N,K", [(1, 4800, 1600), (3, 6400, 1600), helpers.quick(2, 4100, 72), (8, 8192, 1304), (16, 4801, 1000), (9, 6000, 768),
+                                   helpers.quick(5, 8193, 24), (8, 16384, 1536), (8, 8193, 1544), (1, 8200, 1288), (16, 12800, 1024), (9, 8193, 1032),
+                                   (8, 16385, 264)])
 def test_fused_norm_product_one_workgroup_a_compute_unit(ops, M, N, K):
-    """The fused norm and product with up to 32 columns a workgroup, parameters in bfloat16 and in 32-bit."""
+    """The fused norm and product with up to 32 columns a workgroup, one or two workgroups a compute unit, both sides of the
+    lines to 16 columns; parameters in bfloat16 and in 32-bit.  A column has the same bits among fewer columns."""
     g = torch.Generator().manual_seed(M + N)
     x = (torch.randn(M, K, generator=g) * 2 + 1).to(DEV)
     w = bf(torch.randn(N, K, generator=g) * 0.1).to(DEV)
@@ -276,6 +279,8 @@ def test_fused_norm_product_one_workgroup_a_compute_unit(ops, M, N, K):
         gw, gb, bias = (torch.randn(n, generator=g).to(dt).to(DEV) for n in (K, K, N))
         out = torch.empty(M, N, device=DEV)
         ops.linear_ln(x, None, M, gw, gb, 1e-5, w, bias, out)
+        few = ops.linear_ln(x, None, M, gw, gb, 1e-5, w[:100], bias[:100], torch.empty(M, 100, device=DEV))
+        assert torch.equal(out[:, :100], few)
         a = F.layer_norm(x.double(), (K,), gw.double(), gb.double(), 1e-5).to(torch.bfloat16).double()
         ref = a @ w.double().t() + bias.double()
         # (the norm's 32-bit rounding may move an entry of a to the next bfloat16: 2^-8 of one product among K)
