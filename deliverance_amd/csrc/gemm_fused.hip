@@ -395,14 +395,14 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
   hipStream_t s = (hipStream_t)stream;
   // the kernel with whole-line loads takes one row tile, K up to 2048, and parameters of one dtype
   // Columns a workgroup: 16 up to 4,096 columns and for a vocabulary; up to 8,192 as many as give every compute unit one
-  // workgroup; up to 16,384 as many as give every one two, where two fit side by side (registers: K up to 1,536; LDS: with more than
-  // 8 rows K up to 1,024).  Measured on MI355X with cold weights, 16 columns a workgroup -> this, us:
+  // workgroup; up to 16,384 as many as give every one two, where two fit side by side (registers: K up to 1,536).  With more than
+  // 8 rows only up to K = 1,024 (LDS; no step sends wider ones here).  Measured on MI355X with cold weights, 16 columns a workgroup -> this, us:
   //   K = 1,600, N = 4,800 (19 columns) one row 6.9 -> 6.6, 8 rows 9.6 -> 8.2; N = 6,400 (25) 7.4 -> 7.3, 10.2 -> 9.5
   //   K =   768, N = 8,320 (17, two a unit) one row 5.5 -> 5.4, 16 rows 10.0 -> 8.6; N = 12,800 (25) 6.4 -> 6.2, 12.2 -> 9.2
   //   K = 1,536, N = 8,200 (17) one row 7.9 -> 7.6, 8 rows 10.4 -> 10.0; N = 12,800 10.8 -> 9.4, 14.3 -> 11.9; N = 16,384 (32) 11.5 -> 10.9,
   //              15.0 -> 13.4 (two groups of 16 columns, one after the other: 8 rows 10.4, 13.3 and 14.3)
   //   K = 1,600, N = 12,800, where only one of 25 fits: one row 11.6 -> 12.4 (so 16 stay; 8 rows: da_can_fuse_ln)
-  const bool one_a_unit = N > 16 * 256 && N <= 32 * 256;
+  const bool one_a_unit = N > 16 * 256 && N <= 32 * 256 && (M <= 8 || K <= 1024);
   const bool two_a_unit = N > 32 * 256 && N <= 64 * 256 && K <= (M <= 8 ? 1536 : 1024);
   const bool wide = one_a_unit || two_a_unit;
   const int cols = one_a_unit ? da_ceil_div(N, 256) : (two_a_unit ? da_ceil_div(N, 512) : FZ_COLS);
@@ -412,7 +412,7 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
   do {                                                                                                            \
     const dim3 g2(da_ceil_div(N, cols));                                                                          \
     if (wide)                                                                                                     \
-      hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO, 2>), g2, dim3(512), 0, s, ln, (const bf16_t*)w, ldw, ep, kv, M, N, K, cols); \
+      hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO, (TWO && RV > 4 ? 1 : 2)>), g2, dim3(512), 0, s, ln, (const bf16_t*)w, ldw, ep, kv, M, N, K, cols); \
     else                                                                                                          \
       hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO>), g2, dim3(512), 0, s, ln, (const bf16_t*)w, ldw, ep, kv, M, N, K, cols); \
   } while (0)
