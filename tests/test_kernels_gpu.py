@@ -178,9 +178,23 @@ def test_gemm_32bit_on_the_matrix_cores(ops, M, N, K, form):
     w = (torch.randn(N, K, generator=g)).to(DEV)
     o1, o2, o3 = (torch.empty(M, N, device=DEV) for _ in range(3))
     ops.linear_f32(a, w, None, o1, form=form)
-    ops.linear_f32(a, w, None, o2, form="32x32")
+    ops.linear_f32(a, w, None, o2, form="64x64" if form == "32x32" else "32x32")
     ops.linear_f32(a[M // 2:M // 2 + 1], w, None, o3[:1])
     assert torch.equal(o1, o2) and torch.equal(o1[M // 2], o3[0])
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 40, 4100), helpers.quick(1, 20, 6400), (2, 2100, 6400), (16, 70, 3076), (8, 24, 6404), helpers.quick(1, 9, 6404)])
+def test_gemm_32bit_of_few_rows_and_many_columns_of_a(ops, M, N, K):
+    """The kernel for few rows with its largest room for partial sums (K from 3,073 to 6,400), and above that the tiles; the
+    same bits as the tiles.  Bound as above."""
+    g = torch.Generator().manual_seed(K + N)
+    for act, acc, bias in ((None, True, True), ("gelu_new", False, True)):
+        out, ref = _gemm_case(ops, ops.linear_f32, M, N, K, torch.float32, act, acc, bias, torch.float32, g)
+        assert (out - ref).abs().max() < 2e-5 * max(1.0, ref.abs().max().item())
+    a, w = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV)
+    tiles = ops.linear_f32(a, w, None, torch.empty(M, N, device=DEV), form="32x32")
+    for form in ("auto", "rows", "64x64") if K <= 6400 else ("auto", "64x64"):
+        assert torch.equal(ops.linear_f32(a, w, None, torch.empty(M, N, device=DEV), form=form), tiles), form
 
 
 def test_gemm_32bit_writes_keys_and_values(ops):
@@ -268,7 +282,7 @@ def test_gemm_one_workgroup_a_compute_unit(ops, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(1, 4800, 1600), (3, 6400, 1600), helpers.quick(2, 4100, 72), (8, 8192, 1304), (16, 4801, 1000), (9, 6000, 768),
                                    helpers.quick(5, 8193, 24), (8, 16384, 1536), (8, 8193, 1544), (1, 8200, 1288), (16, 12800, 1024), (9, 8193, 1032),
-                                   (8, 16385, 264)])
+                                   (8, 16385, 264), (9, 4801, 1032)])
 def test_fused_norm_product_one_workgroup_a_compute_unit(ops, M, N, K):
     """The fused norm and product with up to 32 columns a workgroup, one or two workgroups a compute unit, both sides of the
     lines to 16 columns; parameters in bfloat16 and in 32-bit.  A column has the same bits among fewer columns."""
@@ -642,6 +656,40 @@ def test_attention_decode_with_infinite_keys_and_values(ops, D):
     fin = np.isfinite(want)
     assert fin.sum() == D - 2 and np.array_equal(got[~fin], want[~fin])
     assert np.abs(got[fin] - want[fin]).max() < ATT_TOL[torch.bfloat16]
+
+
+@pytest.mark.simt_quick
+@pytest.mark.parametrize("D", [16, 64, 80, 144])
+def test_attention_decode_keeps_the_weights_32_bits(ops, D):
+    """Pairs of keys whose weights differ by 2^-12 and whose values, 65,536 and its negative, nearly cancel: the result is what
+    the weights' low bits say.  Root mean square of the error: the result's rounding to bfloat16 (at most 2^-9 of it) and 2e-3,
+    about six times what the same sums in 32 bits lose; weights of 16 bits lose more than twice the bound, of 8 a
+    thousand times."""
+    A, n, page, scale = 65536.0, 200, 16, 0.125
+    g = torch.Generator().manual_seed(D)
+    q, k = bf(torch.randn(1, D, generator=g)), bf(torch.randn(n, D, generator=g) * 0.5)
+    q[0, 0] = 2.0 ** -6
+    k[1::2] = k[0::2]
+    k[0::2, 0] = 0.0
+    k[1::2, 0] = bf(torch.randn(n // 2, generator=g).sign() * 0.125)
+    v = torch.randn(n // 2, D, generator=g).sign() * A
+    v = bf(torch.stack([v, -v], 1).reshape(n, D))
+    s = (k.double() @ q[0].double()) * scale
+    e = torch.exp(s - s.max())
+    result = lambda weights: (weights @ v.double()) / e.sum()
+    want = result(e)
+    rms = lambda x: x.square().mean().sqrt().item()
+    bound = 2.0 ** -9 * rms(want) + 2e-3
+    high = bf(e).double()
+    assert rms(result(high) - want) > 100 * bound and rms(result(high + bf(e - high).double()) - want) > 2 * bound
+    cache = torch.full((13, 2, 1, page, D), float("nan"), dtype=torch.bfloat16)
+    for j in range(n):
+        cache[j // page, 0, 0, j % page] = k[j]
+        cache[j // page, 1].view(D, page)[:, j % page] = v[j]
+    out = torch.empty(1, D, dtype=torch.bfloat16, device=DEV)
+    ops.attention_decode(q.to(DEV), cache.to(DEV), torch.arange(13, dtype=torch.int32, device=DEV).view(1, 13),
+                         torch.tensor([n], dtype=torch.int32, device=DEV), 1, 1, scale, None, out)
+    assert rms(out[0].double().cpu() - want) < bound
 
 
 @pytest.mark.parametrize("n_splits", [2, helpers.quick(3, mark="simt_a"), 7, 16])
