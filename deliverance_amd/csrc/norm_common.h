@@ -28,7 +28,7 @@ __device__ __forceinline__ float norm_row_sum(const float (&part)[VPL], float* r
 // What the compiler may fuse or not, written out, so that both ways round alike: the sum of four squares, and a * b + c.
 __device__ __forceinline__ float norm_squares(const float4& v) {
 #pragma clang fp contract(off)
-  return fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w)));
+  return fmaf(v.x, v.x, v.y * v.y) + fmaf(v.z, v.z, v.w * v.w);
 }
 __device__ __forceinline__ float norm_scaled(float v, float inv, float gain, float add) {
 #pragma clang fp contract(off)
