@@ -7,7 +7,7 @@
 // product and three in the second: a single wavefront's chain of instructions, not the chip's rate, is what a
 // step of few requests waits for, and a chunk takes 16 instructions of 16 cycles here where it took about 700
 // of the vector unit (one head of 64, 512 keys: 6.0 -> 5.7 us a launch in a recorded chain, of which 1.6 are
-// the launch and about 2 the 130 KB that one compute unit pulls in; 64 sequences of 25 heads: 42.5 -> 40.7 us, 5.4 TB/s).
+// the launch and about 2 the 130 KB that one compute unit pulls in; 64 sequences of 25 heads: 42.5 -> 40.7 us, 5.15 TB/s).
 //   scores : S[key, *] = K . q, 4 pieces of 16 keys (a lane holds row l % 16 and 8 dimensions, 16 bytes of the key
 //            row as it lies in the page; q is the same in all 16 columns).  Products of bfloat16 are exact and
 //            their sums 32-bit; the scale comes after.

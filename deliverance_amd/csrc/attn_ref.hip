@@ -1,6 +1,6 @@
 // Plain paged attention: one wavefront per (token, query head), any mix of prompt rows and
-// decode rows.  It is the attention of the true 32-bit path and the reference beside the
-// MFMA prefill kernel and the split-context decode kernel.
+// decode rows.  It is the reference beside the matrix-core kernels, and the attention of what they do not take (head sizes
+// that are no multiple of 16; in 32-bit also above 128, pages below 16, caches or queries that are not 16-byte aligned).
 //
 // For the token at position p of its sequence, head h:
 //   s_j = (q . k_j) * scale   for j in [lo, p],  lo = 0 or p - window + 1

@@ -16,7 +16,7 @@
 //    from memory into fragments, and the chunks' sums are added through LDS.  Bound by the bytes of w.
 //  * gemm_f32_tile: block tiles of 64 x 64 or 32 x 32 through two LDS buffers, slabs of 32 k, the next four slabs in flight
 //    in registers.  Bound by the matrix cores (157 TFLOP/s in 32-bit) where the tiles fill the chip several times over:
-//    1,000 x 50,257 x 768 in 687 us, 73 % of that rate; below, by the latency of a slab, which small tiles, several of
+//    1,000 x 50,257 x 768 in 687 us, 72 % of that rate; below, by the latency of a slab, which small tiles, several of
 //    them on a compute unit, hide better than large ones (526 x 3,072 x 768: 32 x 32 31 us, 64 x 64 34, 128 x 128 72).
 //
 // Measured on MI355X beside the plain kernel (gemm_ref.hip), which a product of 4 rows walks in 64 x 64 tiles through one

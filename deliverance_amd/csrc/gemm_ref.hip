@@ -1,6 +1,6 @@
-// Plain tiled matrix product with the epilogues a block needs.  This is the whole product
-// path in true 32-bit (no matrix cores, no reduced-precision mode) and the reference beside
-// the MFMA kernel in bfloat16.
+// Plain tiled matrix product with the epilogues a block needs, on the vector unit: the reference beside the matrix-core
+// kernels, and the product of what they do not take (in 32-bit a K that is no multiple of 4 or rows that are not 16-byte
+// aligned, in bfloat16 a K that is no multiple of 8).
 //
 //   out[m, n] (+)= act( sum_k a[m, k] * w[n, k] + bias[n] )
 //

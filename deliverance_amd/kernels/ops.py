@@ -886,7 +886,7 @@ def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
 
 
 # Which steps the fused norm + product kernel takes (few rows, a width it holds; measured limits) is the
-# library's rule, da_can_fuse_ln in csrc/run_step.hip, so that the parts here and the step issued from C++
+# library's rule, da_can_fuse_ln in csrc/dispatch.hip, so that the parts here and the step issued from C++
 # decide alike.
 FUSED_LN_KERNEL_MAX_ROWS = 32
 

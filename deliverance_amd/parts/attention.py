@@ -60,8 +60,8 @@ class CausalSelfAttention(Mixer):
         self.n_heads, self.n_kv_heads, self.head_dim = spec.n_heads, spec.n_kv_heads, spec.head_dim
         if self.n_heads % self.n_kv_heads != 0:
             raise ValueError(f"{self.n_heads} query heads are not a multiple of {self.n_kv_heads} key heads")
-        # Any head size up to 256 runs: multiples of 16 on the matrix-core attention kernels in bfloat16,
-        # the others (and everything in 32-bit) on the plain attention kernel.
+        # Any head size up to 256 runs: multiples of 16 (in 32-bit up to 128) on the matrix-core attention kernels,
+        # the others on the plain attention kernel.
         if not (1 <= self.head_dim <= ops.MAX_HEAD_DIM):
             raise ValueError(f"head size {self.head_dim} is outside 1..{ops.MAX_HEAD_DIM}")
         self.v_head_dim = int(getattr(spec, "v_head_dim", None) or self.head_dim)
