@@ -762,9 +762,10 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
 // Measured with cold weights, 16 columns against one workgroup a unit, both with 8 wavefronts:
 //    8 rows: K = 1,600, N = 4,800 6.3 against 6.1 us, 8,192 7.0 / 7.8; K = 4,096, N = 4,112 10.6 / 9.2, 6,400 11.9 / 12.1, 8,192 13.1 / 16.3; K = 8,192, N = 6,400 23.8 / 21.7
 //   16 rows: K = 1,600, N = 4,800 7.1 against 6.4 us, 5,888 6.9 / 6.7, 7,168 7.0 / 7.2; K = 3,072, N = 7,168 11.8 / 10.8, 7,680 11.9 / 11.2
-static bool sk_one_a_unit(int M, int N, int K) {
+// Its offsets of 64 rows are 32-bit: rows that lie further apart than 2^24 entries stay with 16 columns (the same bits).
+static bool sk_one_a_unit(int M, int N, int K, int lda, int ldw) {
   const int cols = da_ceil_div(N, 256);              // of the busiest compute unit, where 16 a workgroup give it 32
-  if (cols <= 16 || cols > 32) return false;
+  if (cols <= 16 || cols > 32 || lda > (1 << 24) || ldw > (1 << 24)) return false;
   if (M > 16) return true;
   if (M > 8) return (K >= 1280 && cols <= 23) || (K >= 3072 && cols <= 28);
   return (M > 4 && K >= 1280 && cols <= 20) || (K >= 3072 && cols <= 22 + K / 2048);
@@ -782,7 +783,7 @@ static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* 
     if (M <= 8) DA_SK_GO(1, 8, 4); else DA_SK_GO(2, 8, 4);
     return 0;
   }
-  if (NW == 8 && sk_one_a_unit(M, N, K)) {
+  if (NW == 8 && sk_one_a_unit(M, N, K, lda, ldw)) {
     const int cols = da_ceil_div(N, 256);            // every compute unit one workgroup
     const dim3 grid(da_ceil_div(N, cols));
 #define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, cols)

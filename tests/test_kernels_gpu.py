@@ -280,6 +280,17 @@ def test_gemm_one_workgroup_a_compute_unit(ops, M, N, K):
         assert torch.equal(c1, c2) and bool(c1.any())
 
 
+def test_gemm_few_rows_that_lie_far_apart(ops):
+    """17 rows of a with 2^27 entries from one to the next (more than 32-bit offsets hold): the same bits as side by side."""
+    helpers.skip_in_simulation_if(True, "four gigabytes")
+    M, N, K, ld = 17, 4112, 128, (1 << 27) + 64
+    far = torch.empty((M - 1) * ld + K, dtype=torch.bfloat16, device=DEV).as_strided((M, K), (ld, 1))
+    a, w = (bf(torch.randn(n, K, device=DEV)) for n in (M, N))
+    far.copy_(a)
+    outs = [ops.linear_mfma(x, w, None, torch.empty(M, N, device=DEV)) for x in (a, far)]
+    assert torch.equal(*outs) and bool(outs[0].any())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 4800, 1600), (3, 6400, 1600), helpers.quick(2, 4100, 72), (8, 8192, 1304), (16, 4801, 1000), (9, 6000, 768),
                                    helpers.quick(5, 8193, 24), (8, 16384, 1536), (8, 8193, 1544), (1, 8200, 1288), (16, 12800, 1024), (9, 8193, 1032),
                                    (8, 16385, 264), (9, 4801, 1032)])
