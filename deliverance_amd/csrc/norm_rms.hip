@@ -12,13 +12,19 @@
 #include "norm_common.h"
 #include <limits.h>
 
-__device__ __forceinline__ float4 rms_param4(const void* p, int dtype, int i) {
+// Four entries of a gain as raw bits (bfloat16: .x and .y hold them), converted where they are used: a conversion right
+// behind its load would be waited for on the spot.
+__device__ __forceinline__ uint4 rms_raw4(const void* p, int dtype, int i) {
   if (dtype == DA_BF16) {
     const uint2 u = *(const uint2*)((const bf16_t*)p + i);
-    return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u),
-                       __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u));
+    return make_uint4(u.x, u.y, 0, 0);
   }
-  return *(const float4*)((const float*)p + i);
+  return *(const uint4*)((const float*)p + i);
+}
+__device__ __forceinline__ float4 rms_gain4(const uint4& u, int dtype) {
+  const bool h = dtype == DA_BF16;
+  return make_float4(__uint_as_float(h ? u.x << 16 : u.x), __uint_as_float(h ? u.x & 0xffff0000u : u.y),
+                     __uint_as_float(h ? u.y << 16 : u.z), __uint_as_float(h ? u.y & 0xffff0000u : u.w));
 }
 
 __device__ __forceinline__ void rms_store4(void* y, int y_dtype, size_t at, float4 o) {
@@ -36,14 +42,15 @@ __global__ void __launch_bounds__(4 * DA_WAVE)
 rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, const void* __restrict__ wa, int wa_dtype,
                    float* __restrict__ x, const void* __restrict__ wb, int wb_dtype, float offset, float eps,
                    void* __restrict__ y, int y_dtype, int R, int E) {
-  __shared__ float red[2][4 * DA_WAVE];
+  __shared__ float red[2][4];
   constexpr int STRIDE = 4 * W * DA_WAVE;
   const int t = threadIdx.x, c0 = (W == 4 ? t : t % DA_WAVE) * 4;
   const int r = W == 4 ? (int)blockIdx.x : (int)(blockIdx.x * (blockDim.x / DA_WAVE)) + t / DA_WAVE;
   if (W == 1 && r >= R) return;
   const float* sr = src + (size_t)(rows ? rows[r] : r) * E;
   // the gains are asked for beside the rows, so that the kernel costs one round trip to memory and not one per norm
-  float4 v[VPL], xv[VPL], ga[VPL], gb[VPL];
+  float4 v[VPL], xv[VPL];
+  uint4 ga[VPL], gb[VPL];
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int c = c0 + i * STRIDE;
@@ -53,9 +60,10 @@ rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, 
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int c = c0 + i * STRIDE, cc = c < E ? c : 0;
-    ga[i] = rms_param4(wa, wa_dtype, cc);
-    if (ADD && y && wb) gb[i] = rms_param4(wb, wb_dtype, cc);
+    ga[i] = rms_raw4(wa, wa_dtype, cc);
+    if (ADD && y && wb) gb[i] = rms_raw4(wb, wb_dtype, cc);
   }
+  __builtin_amdgcn_sched_barrier(0);                   // the loads stay ahead of the sums
   float part[VPL];
 #pragma unroll
   for (int i = 0; i < VPL; ++i) part[i] = c0 + i * STRIDE < E ? norm_squares(v[i]) : 0.f;
@@ -64,7 +72,7 @@ rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, 
   for (int i = 0; i < VPL; ++i) {
     const int c = c0 + i * STRIDE;
     if (c < E) {
-      const float4 g = ga[i];
+      const float4 g = rms_gain4(ga[i], wa_dtype);
       const float4 old = ADD ? xv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
       const float4 o = make_float4(norm_scaled(v[i].x, inv, offset + g.x, old.x), norm_scaled(v[i].y, inv, offset + g.y, old.y),
                                    norm_scaled(v[i].z, inv, offset + g.z, old.z), norm_scaled(v[i].w, inv, offset + g.w, old.w));
@@ -89,7 +97,7 @@ rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, 
     for (int i = 0; i < VPL; ++i) {
       const int c = c0 + i * STRIDE;
       if (c < E) {
-        const float4 g = gb[i];
+        const float4 g = rms_gain4(gb[i], wb_dtype);
         rms_store4(y, y_dtype, (size_t)r * E + c,
                    make_float4(xv[i].x * inv2 * (offset + g.x), xv[i].y * inv2 * (offset + g.y),
                                xv[i].z * inv2 * (offset + g.z), xv[i].w * inv2 * (offset + g.w)));
@@ -139,7 +147,7 @@ static void rms_launch(const float* src, const int* rows, const void* wa, int wa
   hipLaunchKernelGGL((rmsnorm_row_kernel<V, W, ADD>), dim3(g.blocks), dim3(g.threads), 0, st, src, rows, wa, wa_dtype, x, \
                      wb, wb_dtype, offset, eps, y, y_dtype, R, E)
   if (E % 4 == 0 && E <= 4096 && aligned) {
-    const NormGrid g = norm_grid(R, E, 1536, ADD ? INT_MAX : 4096);
+    const NormGrid g = norm_grid(R, E, 2048, ADD ? INT_MAX : 4096);
     if (g.waves == 1) {
       if (E <= 256) RMS_LAUNCH(1, 1);
       else if (E <= 512) RMS_LAUNCH(2, 1);

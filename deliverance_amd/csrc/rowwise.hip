@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(4 * DA_WAVE)
 layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                      const void* __restrict__ w, const void* __restrict__ b,
                      float eps, void* __restrict__ y, int R, int E) {
-  __shared__ float red[2][4 * DA_WAVE];
+  __shared__ float red[2][4];
   constexpr int STRIDE = 4 * W * DA_WAVE;
   const int t = threadIdx.x, c0 = (W == 4 ? t : t % DA_WAVE) * 4;
   const int r = W == 4 ? (int)blockIdx.x : (int)(blockIdx.x * (blockDim.x / DA_WAVE)) + t / DA_WAVE;
@@ -291,7 +291,7 @@ extern "C" int da_layernorm(const float* x, const int* rows, const void* w, int 
                        (!b || (uintptr_t)b % 16 == 0);
   const bool same = (!b || b_dtype == w_dtype) && (w_dtype == DA_BF16 || w_dtype == DA_F32);   // gain and bias alike
   if (E % 4 == 0 && E <= 2048 && aligned && same) {
-    const NormGrid g = norm_grid(R, E, 1024, 1536);
+    const NormGrid g = norm_grid(R, E, 768, 1024);
 #define LN_LAUNCH(V, W, P, Y) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, Y>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, eps, y, R, E)
 #define LN_LAUNCH_Y(V, W, P) do { if (y_dtype == DA_BF16) LN_LAUNCH(V, W, P, true); else LN_LAUNCH(V, W, P, false); } while (0)
 #define LN_LAUNCH_P(V, W) do { if (w_dtype == DA_BF16) LN_LAUNCH_Y(V, W, true); else LN_LAUNCH_Y(V, W, false); } while (0)

@@ -100,7 +100,7 @@ def test_layernorm(ops, E, eps):
 def test_norms_of_many_rows(ops, E):
     """Rows of up to 1,024 columns take one wavefront or four by their number: the same bits either way, at the lines between
     the two and beside them."""
-    R = 1537 if E <= 512 else 4097
+    R = 2049 if E <= 512 else 4097
     helpers.skip_in_simulation_if(E > 512)
     g = torch.Generator().manual_seed(E)
     x, src = ((torch.randn(R, E, generator=g) * 3 + 5).to(DEV) for _ in range(2))
@@ -114,7 +114,7 @@ def test_norms_of_many_rows(ops, E):
             ops.rmsnorm_add(src[lo:hi], w.to(dt), stream, 1.0, 1e-5, b.to(dt), h)
             return outs + [stream, h]
         few = norms(0, 5)
-        for n in (R,) if helpers.SIMT else (511, 513, 1023, 1024, 1535, 1536, R - 1, R):
+        for n in (R,) if helpers.SIMT else (511, 513, 767, 768, 1023, 1024, 2047, 2048, R - 1, R):
             many = norms(0, n)
             assert all(torch.equal(f, m[:5]) for f, m in zip(few, many)), n
             if n == R:
