@@ -12,29 +12,41 @@
 // sum of a chunk starts from zero and joins the total of the chunks before it.  (Two levels: a long sum into one
 // 32-bit accumulator loses about sqrt(K) roundings, this one sqrt(128) + sqrt(K / 128).)
 //
-//  * gemm_f32_rows: few rows.  A workgroup owns 16 rows and up to 16 columns; its wavefronts take whole chunks, straight
-//    from memory into fragments, and the chunks' sums are added through LDS.  Bound by the bytes of w.
+//  * gemm_f32_rows: few rows.  A workgroup owns 4, 8 or 16 rows and as many columns as give every compute unit one workgroup (16 at
+//    most); its wavefronts take whole chunks, from memory through their own pieces of LDS into fragments, and the chunks' sums are
+//    added through LDS.  Bound by the bytes of w.  gemm_f32_rows16: straight into fragments, where that is ahead.
 //  * gemm_f32_tile: block tiles of 64 x 64 or 32 x 32 through two LDS buffers, slabs of 32 k, the next four slabs in flight
 //    in registers.  Bound by the matrix cores (157 TFLOP/s in 32-bit) where the tiles fill the chip several times over:
 //    1,000 x 50,257 x 768 in 687 us, 72 % of that rate; below, by the latency of a slab, which small tiles, several of
 //    them on a compute unit, hide better than large ones (526 x 3,072 x 768: 32 x 32 31 us, 64 x 64 34, 128 x 128 72).
 //
-// Measured on MI355X beside the plain kernel (gemm_ref.hip), which a product of 4 rows walks in 64 x 64 tiles through one
-// LDS buffer: 4 x 768 x 3,072 226 -> 10 us, 4 x 2,304 x 768 86 -> 4.4, 526 x 768 x 3,072 about 360 -> 37,
-// 526 x 2,304 x 768 128 -> 24, 526 x 50,257 x 768 1,308 -> 384.
+// Measured on MI355X with cold weights, us (before: 16 rows and 16, 8 or 4 columns a workgroup, fragments straight from memory, a
+// chunk a product): 4 rows, K x N 768 x 768 4.5 -> 3.8, 768 x 2,304 5.3 -> 4.7, 768 x 3,072 5.6 -> 5.2, 3,072 x 768 10.8 -> 6.1,
+// 768 x 50,257 39.9 -> 32.1; 8 rows, 3,072 x 768 12.0 -> 7.7; 16 rows 13.8 -> 9.6; 64 rows 14.3 -> 11.4; 32 rows, 768 x 3,072 8.7 -> 7.9.
+// Tiles: 526 x 768 x 3,072 38, 526 x 2,304 x 768 27, 526 x 50,257 x 768 440.
 #include "gemm_common.h"
 #include <type_traits>
 
 #define GF_CHUNK 128
 #define GF_BK 32
+#define GF_ROWS_CAP 50
+#define GF_ROWS_MAX_K (GF_ROWS_CAP * GF_CHUNK)      // the chunks' sums of 16 x 16 outputs fit in 64 KB of LDS
 #define GF_LD (GF_BK + 4)    // padded LDS row, floats (144 bytes): 16 consecutive rows start in different banks
 
 __device__ __forceinline__ float4 gf_load(const float* p) { return *(const float4*)p; }
+
 __device__ __forceinline__ floatx4 gf_group(const float4& a, const float4& w, floatx4 c) {      // the 16 k of a group
   c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, w.x, c, 0, 0, 0);
   c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, w.y, c, 0, 0, 0);
   c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, w.z, c, 0, 0, 0);
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, w.w, c, 0, 0, 0);
+}
+// What one lane of a wavefront leaves in LDS another lane of it reads: LDS serves a wavefront's instructions in order, so
+// it is the compiler alone that must keep them.
+__device__ __forceinline__ void gf_wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // the k and v columns of a q|k|v product (column n >= q_cols of the row whose place in the cache is `slot`)
@@ -48,23 +60,129 @@ __device__ __forceinline__ void gf_scatter(const KvScatter& kv, int slot, int n,
 }
 
 // ---------------------------------------------------------------------------------------------
-// Few rows: blockIdx.x: COLS columns (16, or 8 or 4 where the columns alone would leave compute units idle: the
-// fragment of w then holds them several times and the copies' results are dropped), blockIdx.y: 16 rows.
+// Few rows: blockIdx.x: `cols` columns (4 WL at most), blockIdx.y: 4 AL rows.  A wavefront takes sets of P chunks, v, v + NW,
+// ...; a set's loads (2 rows x 512 bytes each, whole cache lines) are in flight while the set before it is multiplied, and pass
+// through the wavefront's own piece of LDS into fragments.  A product of 16 x 16 holds P chunks side by side: chunk p has the
+// rows and the columns from p * 16 / P on, and what one chunk's rows give with another's columns is dropped.  So 4 rows and 4
+// columns take a quarter of the matrix instructions that a chunk at a time would.
+// Bound by the bytes of w where the columns are many; else by the chain launch, load, products, sums.
 // ---------------------------------------------------------------------------------------------
+// The 16-byte piece kk of a parked row: turned by the row's place in the fragment, so that the writes (32 pieces of a row) and
+// the reads (one piece of 16 rows) both spread over the banks.
+// (the vector type of the language: arrays of HIP's float4, a class, that are only copied stay in memory)
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+__device__ __forceinline__ int gf_place(int row, int kk) { return row * 32 + (kk ^ (row & 15)); }
 // CAP: chunks that the partial sums in LDS have room for.
-template <int COLS, int NW, int CAP>
+template <int WL, int AL, int NW, int CAP>
 __global__ void __launch_bounds__(NW * 64)
 gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w, int ldw, Epilogue ep, KvScatter kv,
+                     int M, int N, int K, int n_chunks, int cols) {
+  constexpr int P = WL == 1 && AL == 1 ? 4 : (WL <= 2 && AL <= 2 ? 2 : 1), S = 16 / P;    // chunks of a product; rows and columns of each
+  constexpr int RA = 4 * AL, CW = 4 * WL, LA = RA / 2, LW = CW / 2;     // rows, columns; loads a chunk
+  static_assert(RA <= S && CW <= S, "a chunk's rows and columns fit their part of the fragments");
+  static_assert(NW * 64 >= RA * CW, "a thread an output");
+  __shared__ __attribute__((aligned(16))) f32x4_t gf_stage[NW][P * (RA + CW) * 32];
+  __shared__ float gf_red[CAP * RA * (CW + 1)];                        // [n_chunks][RA][CW + 1]
+  const int t = threadIdx.x, lane = t % 64, wave = __builtin_amdgcn_readfirstlane(t / 64);
+  const int n0 = blockIdx.x * cols, r0 = blockIdx.y * RA;
+  const int n_end = n0 + cols < N ? n0 + cols : N;
+  const int fr = lane % 16, quad = lane / 16;
+  const int l_row = lane / 32, l_kk = lane % 32;                       // a load: row l_row of 2, piece l_kk
+  f32x4_t* const a_lds = gf_stage[wave];
+  f32x4_t* const w_lds = gf_stage[wave] + P * RA * 32;
+  const float* pa[LA];
+  const float* pw[LW];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) pa[i] = a + (size_t)(r0 + i * 2 + l_row < M ? r0 + i * 2 + l_row : r0) * lda;
+#pragma unroll
+  for (int i = 0; i < LW; ++i) pw[i] = w + (size_t)(n0 + i * 2 + l_row < n_end ? n0 + i * 2 + l_row : n0) * ldw;
+  // what the epilogue needs is asked for first, from places that always exist
+  const int em = r0 + t / CW, en = n0 + t % CW;
+  const bool e_ok = t < RA * CW && em < M && en < n_end;
+  const float e_bias_raw = (e_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, en) : 0.f;
+  const float e_old = *((e_ok && ep.accumulate) ? (const float*)ep.out + (size_t)em * ep.ldo + en : w);
+  const int e_slot = *((e_ok && kv.cache) ? kv.slot_map + em : (const int*)w);
+
+  struct Set { f32x4_t a[P][LA], w[P][LW]; };
+  auto fetch = [&](Set& x, int set) {                                  // (past K: the row's first piece, dropped when it is parked)
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int k = (set * P + p) * GF_CHUNK + l_kk * 4, ks = k < K ? k : 0;
+#pragma unroll
+      for (int i = 0; i < LA; ++i) x.a[p][i] = *(const f32x4_t*)(pa[i] + ks);
+#pragma unroll
+      for (int i = 0; i < LW; ++i) x.w[p][i] = *(const f32x4_t*)(pw[i] + ks);
+    }
+  };
+  // this lane's row of a fragment of a and of w, and the pieces of k group `quad` of it
+  const int fp = fr / S, fs = fr % S;
+  const int row_a = fp * RA + (fs & (RA - 1)), row_w = fp * CW + (fs < CW ? fs : 0);
+  auto products = [&](Set& x, int set) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const bool in = (set * P + p) * GF_CHUNK + l_kk * 4 < K;
+      const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < LA; ++i) a_lds[gf_place(p * RA + i * 2 + l_row, l_kk)] = in ? x.a[p][i] : zero;
+#pragma unroll
+      for (int i = 0; i < LW; ++i) w_lds[gf_place(p * CW + i * 2 + l_row, l_kk)] = in ? x.w[p][i] : zero;
+    }
+    gf_wave_order();
+    floatx4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const f32x4_t fa = a_lds[gf_place(row_a, g * 4 + quad)], fw = w_lds[gf_place(row_w, g * 4 + quad)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fw[e], part, 0, 0, 0);
+    }
+    gf_wave_order();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 4 * quad + r, c = set * P + fp;
+      if (i / S == fp && i % S < RA && fs < CW && c < n_chunks) gf_red[(c * RA + i % S) * (CW + 1) + fs] = part[r];
+    }
+  };
+  const int n_sets = (n_chunks + P - 1) / P;
+  Set x, y;
+  int set = wave;
+  if (set < n_sets) fetch(x, set);
+  for (; set < n_sets; set += 2 * NW) {
+    if (set + NW < n_sets) fetch(y, set + NW);
+    products(x, set);
+    if (set + 2 * NW < n_sets) fetch(x, set + 2 * NW);
+    if (set + NW < n_sets) products(y, set + NW);
+  }
+  lds_barrier();
+  if (!e_ok) return;
+  const float* mine = gf_red + (t / CW) * (CW + 1) + t % CW;
+  float v = mine[0];
+#pragma unroll 4
+  for (int c = 1; c < n_chunks; ++c) v += mine[c * RA * (CW + 1)];
+  v = apply_act(v + e_bias_raw, ep.act);
+  float* o = (float*)ep.out + (size_t)em * ep.ldo + en;
+  *o = ep.accumulate ? e_old + v : v;
+  if (kv.cache && en >= kv.q_cols && e_slot >= 0) gf_scatter(kv, e_slot, en, v);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Up to 16 rows, and either one chunk or 257 to 640 groups of 16 columns: the same products from fragments that come straight from memory (16 rows x
+// 64 bytes a load), a chunk a wavefront.  The loads are half cache lines, but a product starts with its first fragment, and with two
+// workgroups on most compute units that is ahead: K = 768, N = 8,192 4 rows 7.7 us against 8.8, 8 rows 8.5 against 9.6, 16 rows 9.9
+// against 9.4; N = 12,288 4 rows 12.6 against 11.3, N = 2,304 5.3 against 4.7; K = 64, N = 2,304 2.6 against 3.0.
+// ---------------------------------------------------------------------------------------------
+template <int NW, int CAP>
+__global__ void __launch_bounds__(NW * 64)
+gemm_f32_rows16_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w, int ldw, Epilogue ep, KvScatter kv,
                      int M, int N, int K, int n_chunks) {
-  __shared__ float gf_red[CAP * 16 * (COLS + 1)];                      // [n_chunks][16][COLS + 1]
+  __shared__ float gf_red[CAP * 16 * 17];                      // [n_chunks][16][COLS + 1]
   const int t = threadIdx.x, lane = t % 64, wave = t / 64;
-  const int n0 = blockIdx.x * COLS, r0 = blockIdx.y * 16;
+  const int n0 = blockIdx.x * 16, r0 = blockIdx.y * 16;
   const int fr = lane % 16, kq = (lane / 16) * 4;
   const float* pa = a + (size_t)(r0 + fr < M ? r0 + fr : r0) * lda;
-  const float* pw = w + (size_t)(n0 + fr % COLS < N ? n0 + fr % COLS : n0) * ldw;
+  const float* pw = w + (size_t)(n0 + fr < N ? n0 + fr : n0) * ldw;
   // what the epilogue needs is asked for first, from places that always exist
-  const int em = r0 + t / COLS, en = n0 + t % COLS;
-  const bool e_ok = t < 16 * COLS && em < M && en < N;
+  const int em = r0 + t / 16, en = n0 + t % 16;
+  const bool e_ok = t < 256 && em < M && en < N;
   const float e_bias_raw = (e_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, en) : 0.f;
   const float e_old = *((e_ok && ep.accumulate) ? (const float*)ep.out + (size_t)em * ep.ldo + en : w);
   const int e_slot = *((e_ok && kv.cache) ? kv.slot_map + em : (const int*)w);
@@ -84,10 +202,8 @@ gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restri
       if (CUT && c * GF_CHUNK + g * 16 + kq >= K) av[g] = wv[g] = make_float4(0.f, 0.f, 0.f, 0.f);
       part = gf_group(av[g], wv[g], part);
     }
-    if (COLS == 16 || fr < COLS) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) gf_red[(c * 16 + 4 * (lane / 16) + r) * (COLS + 1) + fr] = part[r];
-    }
+    for (int r = 0; r < 4; ++r) gf_red[(c * 16 + 4 * (lane / 16) + r) * 17 + fr] = part[r];
   };
   const int whole = K / GF_CHUNK;
   for (int c = wave; c < n_chunks; c += NW) {
@@ -96,10 +212,10 @@ gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restri
   }
   lds_barrier();
   if (!e_ok) return;
-  const float* mine = gf_red + (t / COLS) * (COLS + 1) + t % COLS;
+  const float* mine = gf_red + (t / 16) * 17 + t % 16;
   float v = mine[0];
 #pragma unroll 4
-  for (int c = 1; c < n_chunks; ++c) v += mine[c * 16 * (COLS + 1)];
+  for (int c = 1; c < n_chunks; ++c) v += mine[c * 16 * 17];
   v = apply_act(v + e_bias_raw, ep.act);
   float* o = (float*)ep.out + (size_t)em * ep.ldo + en;
   *o = ep.accumulate ? e_old + v : v;
@@ -271,21 +387,40 @@ static void launch_f32_tile(hipStream_t s, const float* a, int lda, const float*
                      tiles_n);
 }
 
-template <int COLS, int NW, int CAP>
+template <int WL, int AL, int NW, int CAP>
 static void launch_f32_rows(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
-                            int M, int N, int K) {
-  hipLaunchKernelGGL((gemm_f32_rows_kernel<COLS, NW, CAP>), dim3(da_ceil_div(N, COLS), da_ceil_div(M, 16)), dim3(NW * 64), 0, s, a, lda,
-                     w, ldw, ep, kv, M, N, K, da_ceil_div(K, GF_CHUNK));
+                            int M, int N, int K, int cols) {
+  hipLaunchKernelGGL((gemm_f32_rows_kernel<WL, AL, NW, CAP>), dim3(da_ceil_div(N, cols), da_ceil_div(M, 4 * AL)), dim3(NW * 64), 0, s, a, lda,
+                     w, ldw, ep, kv, M, N, K, da_ceil_div(K, GF_CHUNK), cols);
+}
+// The wavefronts and the room for partial sums, by K.  More workgroups than compute units: few wavefronts each, so that several
+// workgroups share a compute unit's LDS and one's loads run beside another's products (K = 768, N = 50,257: 4 rows 32 us with 3
+// wavefronts, 45 with 6; 8 rows 38 / 51; 32 rows, N = 3,072 7.9 with 4, 8.8 with 6).
+template <int WL, int AL>
+static void launch_f32_rows_k(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
+                              int M, int N, int K, int cols) {
+  const bool many = (long)da_ceil_div(N, cols) * da_ceil_div(M, 4 * AL) > 256;
+  if (many && AL == 4 && K <= 8 * GF_CHUNK) launch_f32_rows<WL, AL, 4, 8>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+  else if (many && AL < 4 && K <= 24 * GF_CHUNK) launch_f32_rows<WL, AL, AL == 4 ? 4 : 3, 24>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+  else if (K <= 6 * GF_CHUNK) launch_f32_rows<WL, AL, 6, 6>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+  else if (K <= 24 * GF_CHUNK) launch_f32_rows<WL, AL, 8, 24>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+  else launch_f32_rows<WL, AL, AL == 4 ? 6 : 8, GF_ROWS_CAP>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+}
+template <int AL>
+static void launch_f32_rows_n(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
+                              int M, int N, int K, int cols) {
+  if (cols <= 4) launch_f32_rows_k<1, AL>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+  else if (cols <= 8) launch_f32_rows_k<2, AL>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+  else if (cols <= 12) launch_f32_rows_k<3, AL>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+  else launch_f32_rows_k<4, AL>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
 }
 
 enum { GF_AUTO = 0, GF_ROWS, GF_64x64, GF_32x32, GF_LAST = GF_32x32 };
-#define GF_ROWS_CAP 50
-#define GF_ROWS_MAX_K (GF_ROWS_CAP * GF_CHUNK)      // the chunks' sums of 16 x 16 outputs fit in 64 KB of LDS
 
 // Which kernel a product goes to.  Measured on MI355X with K from 768 to 4,096:
-//  - the kernel for few rows up to 8 rows (the head: 4 rows 30 against 32 us, 16 rows 39 against 32) and where its
-//    workgroups are at most 512, which is what the chip runs side by side (64 x 768 x 3,072 13 against 26 us, 100 x 768 x 768
-//    7.7 against 9.8, 32 x 3,072 x 768 8.0 against 10.3; with 576 of them 10.5 against 9.8);
+//  - the kernel for few rows up to 8 rows (768 x 50,257: 4 rows 32 us against 38 in tiles of 32 x 32, 8 rows 38.1 against 38.4, 16
+//    rows 46 against 38) and where its products of 16 x 16 are at most 512 (100 x 768 x 768 6.8 us against 9.8, 64 x 768 x 3,072
+//    11.4 against 27, 32 x 3,072 x 768 7.9 against 10.9; with 528 of them, 170 x 768 x 768, 10.9 against 9.7);
 //  - else tiles of 64 x 64 where there are 700 and more, counting what M and N waste of them (1,000 x 3,072 x 768 47 against
 //    51 us, 526 x 50,257 x 768 384 against 401, but 200 x 50,257 x 768 183 against 167);
 //  - else tiles of 32 x 32 (526 x 3,072 x 768, 432 of the larger tiles: 31 against 34 us).
@@ -315,25 +450,28 @@ extern "C" int da_gemm_f32(const float* a, int lda, const float* w, int ldw, con
   const KvScatter kv{kv_cache, slot_map, q_cols, kv_cols, Hkv, D, page};
   hipStream_t s = (hipStream_t)stream;
   if (form == GF_AUTO) form = f32_form(M, N, K);
-#define DA_GF_ROWS(C)                                                                                        \
-  do {                                                                                                       \
-    if (K <= 4 * GF_CHUNK) launch_f32_rows<C, 4, 4>(s, a, lda, w, ldw, ep, kv, M, N, K);                     \
-    else if (K <= 8 * GF_CHUNK) launch_f32_rows<C, 8, 8>(s, a, lda, w, ldw, ep, kv, M, N, K);                \
-    else if (K <= 24 * GF_CHUNK) launch_f32_rows<C, 12, 24>(s, a, lda, w, ldw, ep, kv, M, N, K);             \
-    else launch_f32_rows<C, 12, GF_ROWS_CAP>(s, a, lda, w, ldw, ep, kv, M, N, K);                            \
-  } while (0)
   switch (form) {
     case GF_ROWS: {
-      const long tiles = (long)da_ceil_div(M, 16) * da_ceil_div(N, 16);
-      if (tiles <= 64) DA_GF_ROWS(4);
-      else if (tiles <= 128) DA_GF_ROWS(8);
-      else DA_GF_ROWS(16);
+      const long groups = da_ceil_div(N, 16);
+      if (M <= 16 && (K <= GF_CHUNK || (groups > 256 && groups <= 640 && K <= 24 * GF_CHUNK))) {
+        const dim3 grid(groups);
+        const int n_chunks = da_ceil_div(K, GF_CHUNK);
+        if (K <= 8 * GF_CHUNK) hipLaunchKernelGGL((gemm_f32_rows16_kernel<8, 8>), grid, dim3(512), 0, s, a, lda, w, ldw, ep, kv, M, N, K, n_chunks);
+        else hipLaunchKernelGGL((gemm_f32_rows16_kernel<12, 24>), grid, dim3(768), 0, s, a, lda, w, ldw, ep, kv, M, N, K, n_chunks);
+        break;
+      }
+      const int rows = M <= 4 ? 4 : (M <= 8 ? 8 : 16);
+      // every compute unit a workgroup, 16 columns at most
+      const long share = ((long)N * da_ceil_div(M, rows) + 255) / 256;
+      const int cols = share > 16 ? 16 : (int)share;
+      if (rows == 4) launch_f32_rows_n<1>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+      else if (rows == 8) launch_f32_rows_n<2>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+      else launch_f32_rows_n<4>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
       break;
     }
     case GF_64x64: launch_f32_tile<64, 64>(s, a, lda, w, ldw, ep, kv, M, N, K); break;
     default: launch_f32_tile<32, 32>(s, a, lda, w, ldw, ep, kv, M, N, K); break;
   }
-#undef DA_GF_ROWS
   DA_CHECK_LAUNCH("gemm_f32");
   return 0;
 }

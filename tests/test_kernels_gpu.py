@@ -197,6 +197,22 @@ def test_gemm_32bit_of_few_rows_and_many_columns_of_a(ops, M, N, K):
         assert torch.equal(ops.linear_f32(a, w, None, torch.empty(M, N, device=DEV), form=form), tiles), form
 
 
+@pytest.mark.parametrize("M,N,K", [helpers.quick(3, 700, 772), helpers.quick(4, 1030, 132), (2, 250, 6400), (4, 2100, 1284), (1, 13000, 260),
+                                   helpers.quick(8, 1100, 388), (5, 2050, 644), (7, 10500, 132), (8, 5000, 3072), (8, 10500, 3076),
+                                   helpers.quick(9, 300, 260), (16, 1000, 6400), (33, 3000, 388), (12, 4100, 516), (16, 10240, 1028),
+                                   (13, 4200, 3076), helpers.quick(4, 520, 64)])
+def test_gemm_32bit_of_few_rows_by_columns(ops, M, N, K):
+    """The kernel for few rows with 1 to 16 columns a workgroup, four, two and one chunk a product, few and many workgroups, K cut
+    in every place of a set of chunks, and fragments straight from memory: the bits of the tiles.  Bound as above."""
+    helpers.skip_in_simulation_if(M * N * K > 4e6)
+    g = torch.Generator().manual_seed(M + N + K)
+    out, ref = _gemm_case(ops, ops.linear_f32, M, N, K, torch.float32, None, True, True, torch.float32, g)
+    assert (out - ref).abs().max() < 2e-5 * max(1.0, ref.abs().max().item())
+    a, w = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV)
+    rows = ops.linear_f32(a, w, None, torch.empty(M, N, device=DEV), form="rows")
+    assert torch.equal(rows, ops.linear_f32(a, w, None, torch.empty(M, N, device=DEV), form="32x32"))
+
+
 def test_gemm_32bit_writes_keys_and_values(ops):
     g = torch.Generator().manual_seed(7)
     Hq, Hkv, D, page, K = 5, 3, 20, 16, 132
