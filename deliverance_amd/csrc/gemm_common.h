@@ -25,6 +25,16 @@ __device__ __forceinline__ void epilogue_store(const Epilogue& ep, int m, int n,
   else ((float*)ep.out)[o] = v;
 }
 
+// A product's k shared out over workgroups (blockIdx.y: the share, k_share of K each): share s stores its sums, without bias or
+// activation, in rows of their own behind those of share s - 1; whoever reads the rows next adds them up (da_layernorm_join).
+__device__ __forceinline__ void gemm_take_share(const bf16_t* __restrict__& a, const bf16_t* __restrict__& w, Epilogue& ep, int M, int& K, int k_share) {
+  const int k0 = (int)blockIdx.y * k_share;
+  a += k0;
+  w += k0;
+  ep.out = (float*)ep.out + (size_t)blockIdx.y * M * ep.ldo;
+  K = K - k0 < k_share ? K - k0 : k_share;
+}
+
 // For a fused q|k|v projection: the k and v columns of a row also go to the row's place in the
 // paged cache (keys row-major, values dimension-major; see common.h).
 struct KvScatter {
@@ -149,4 +159,4 @@ enum { DA_WIDE_NONE = -1, DA_WIDE_256x256 = 0, DA_WIDE_256x128 = 1, DA_WIDE_128x
 bool da_gemm_wide_takes(int act, int accumulate, int out_dtype, int K);
 extern "C" int da_gemm_wide_choice(int M, int N, int K);
 void da_gemm_wide_launch(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
-                         const KvScatter& kv, int M, int N, int K, int shape);
+                         const KvScatter& kv, int M, int N, int K, int shape, int k_share = 0);

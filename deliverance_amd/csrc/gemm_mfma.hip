@@ -400,7 +400,8 @@ gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__
 template <int BM, int BN, int WM, int WN, int PF, int ACT, int OUTMODE>
 __global__ void __launch_bounds__(WM * WN * 64)
 gemm_tile_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                 Epilogue ep, KvScatter kv, int M, int N, int K, int tiles_m, int tiles_n, Grouping gr) {
+                 Epilogue ep, KvScatter kv, int M, int N, int K, int tiles_m, int tiles_n, Grouping gr, int k_share) {
+  gemm_take_share(a, w, ep, M, K, k_share);
   // two buffers of a slab of a and of w; the epilogue parks the tile's results in the same memory
   constexpr int SLAB_BYTES = 2 * (BM + BN) * LDS_LD * (int)sizeof(bf16_t);
   constexpr int OUT_BYTES = tile_out_bytes<BM, BN, OUTMODE>() + tile_slot_bytes<BM, OUTMODE>();
@@ -411,27 +412,28 @@ gemm_tile_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict
 
 template <int BM, int BN, int WM, int WN, int PF, int ACT>
 static void launch_tile_act(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
-                            const KvScatter& kv, int M, int N, int K, const Grouping& gr) {
+                            const KvScatter& kv, int M, int N, int K, const Grouping& gr, int k_share) {
   const int tiles_m = da_ceil_div(M, BM), tiles_n = da_ceil_div(N, BN);
-  const dim3 grid(tiles_m * tiles_n), block(WM * WN * 64);
+  const dim3 grid(tiles_m * tiles_n, da_ceil_div(K, k_share)), block(WM * WN * 64);
   if (ep.accumulate)
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 2>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 2>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, k_share);
   else if (ep.out_dtype == DA_F32)
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 1>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 1>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, k_share);
   else
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 0>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 0>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, k_share);
 }
 
 template <int BM, int BN, int WM, int WN, int PF>
 static void launch_tile(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
-                        const KvScatter& kv, int M, int N, int K, const Grouping& gr = Grouping{nullptr, 0, 0}) {
+                        const KvScatter& kv, int M, int N, int K, const Grouping& gr = Grouping{nullptr, 0, 0}, int k_share = 0) {
+  if (k_share <= 0) k_share = K;
   switch (ep.act) {
-    case DA_ACT_GELU_TANH: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_GELU_TANH>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
-    case DA_ACT_GELU_ERF: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_GELU_ERF>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
-    case DA_ACT_RELU: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_RELU>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
-    case DA_ACT_SILU: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_SILU>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
-    case DA_ACT_RELU2: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_RELU2>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
-    default: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_NONE>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
+    case DA_ACT_GELU_TANH: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_GELU_TANH>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
+    case DA_ACT_GELU_ERF: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_GELU_ERF>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
+    case DA_ACT_RELU: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_RELU>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
+    case DA_ACT_SILU: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_SILU>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
+    case DA_ACT_RELU2: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_RELU2>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
+    default: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_NONE>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
   }
 }
 
@@ -636,7 +638,8 @@ __device__ __forceinline__ void sk_park(const u32x4_t (&av)[AL], const u32x4_t (
 template <int AL, int NW, int P>
 __global__ void __launch_bounds__(NW * 64)
 gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                     Epilogue ep, KvScatter kv, int M, int N, int K, int cols) {
+                     Epilogue ep, KvScatter kv, int M, int N, int K, int cols, int k_share) {
+  gemm_take_share(a, w, ep, M, K, k_share);
   constexpr int COLS = 32, MT = (AL + 1) / 2, WL = COLS / 8;    // row tiles of 16; loads of 8 rows that cover w's columns
   constexpr int CT = (COLS + 15) / 16;               // column tiles of 16
   constexpr int AR = MT * 16, TR = AR + COLS;        // rows of a; rows of a step: a's, then w's
@@ -648,7 +651,7 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
   const int t = threadIdx.x, lane = t % 64, wave = __builtin_amdgcn_readfirstlane(t / 64);
   const int n0 = blockIdx.x * cols;
   const int n_end = n0 + cols < N ? n0 + cols : N;   // behind the workgroup's last column
-  const int r0 = blockIdx.y * AR;                    // the workgroup's first row
+  const int r0 = blockIdx.z * AR;                    // the workgroup's first row
   const int lr = lane / 8, lc = (lane % 8) * 8;      // a load: row lr of 8, 16-byte piece lane % 8
   const int fr = lane % 16, fk = (lane / 16) * 8;    // a fragment: row fr of 16, k-group lane / 16
   // byte offsets of the lane's rows behind the workgroup's first row of a and of w (64 rows at most: 32 bits hold them)
@@ -786,7 +789,7 @@ static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* 
   if (NW == 8 && sk_one_a_unit(M, N, K, lda, ldw)) {
     const int cols = da_ceil_div(N, 256);            // every compute unit one workgroup
     const dim3 grid(da_ceil_div(N, cols));
-#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, cols)
+#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, cols, K)
     // (steps in flight: what the registers of a workgroup that is alone on its compute unit allow)
     if (M <= 8) DA_SK32_GO(1, 4);
     else if (mt == 1) DA_SK32_GO(2, 4);
@@ -1056,6 +1059,67 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
     else launch_tile<64, 64, 2, 2, 4>(s, A, lda, W, ldw, ep, kv, M, N, K);
   }
   DA_CHECK_LAUNCH("gemm_bf16");
+  return 0;
+}
+
+// How many shares the k of a product into the residual stream is cut into (1: none; da_gemm_bf16 adds into the stream).  With few
+// tiles and a long K most compute units have no tile; cut, share by share, they have one, and what the shares' sums cost is
+// that the norm behind reads them (da_layernorm_join; never a norm that is fused into its product: more rows than
+// da_can_fuse_ln takes).  Whole slabs of 64 k, 512 k a share at least, 8 shares at most.
+//  - up to 64 rows (32 columns a workgroup, gemm_skinny32), K from 4,096: us, cold weights, += / shares: 64 rows, N = 1,600, K = 6,400
+//    14.1 / 10.2 (5), 32 rows 11.1 / 8.0, 16 rows 10.3 / 7.9; N = 1,024, K = 4,096 64 rows 7.4 / 6.5 (8), 48 rows 7.5 / 5.9.  Not K = 3,072,
+//    N = 768: 64 rows 4.9 / 5.5;
+//  - more rows: tiles of 128 x 128 where they are at most 85, as many shares as bring them to about 256 (552 rows, N = 1,024,
+//    K = 4,096 20.1 / 12.2 (6)).  K from 2,048.  (K = 1,024: 552 rows 7.5 / 6.5, which the norm's reads take up; so do they
+//    with two shares of more rows: 1,624 rows, K = 4,096 29.7 / 23.9, a step of them 2,834 / 2,841.)
+struct GemmShares { int shares, k_share, shape; };     // shape: DA_WIDE_..., or DA_WIDE_NONE for gemm_skinny32
+static GemmShares gemm_shares(int M, int N, int K) {
+  const GemmShares none{1, K, DA_WIDE_NONE};
+  if (M <= 8 || (M <= 16 && N <= 1024) || N % 4 || K % 64 || N > 2048) return none;
+  GemmShares g = none;
+  long tiles;
+  if (M <= 64) {
+    if (K < 4096) return none;
+    tiles = da_ceil_div(N, 32);
+  } else {
+    if (K < 2048) return none;
+    tiles = (long)da_ceil_div(M, 128) * da_ceil_div(N, 128);
+    if (tiles > 85) return none;
+    g.shape = DA_WIDE_128x128;
+  }
+  long n = 256 / tiles;
+  if (n > K / 512) n = K / 512;
+  if (n > 8) n = 8;
+  if (n < 2) return none;
+  g.k_share = da_ceil_div(K / 64, n) * 64;
+  g.shares = da_ceil_div(K, g.k_share);
+  return g;
+}
+extern "C" int da_gemm_shares(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? gemm_shares(M, N, K).shares : 1; }
+
+// partial[s] = a @ w.T over share s of k, [M, N] each, 32-bit; as many shares as da_gemm_shares says (more than one).
+extern "C" int da_gemm_bf16_shares(const void* a, int lda, const void* w, int ldw, float* partial, int M, int N, int K, void* stream) {
+  if (gemm_bf16_checks(a, lda, w, ldw, DA_ACT_NONE, 0, DA_F32, N, M, N, K)) return 1;
+  if (M == 0) return 0;
+  const GemmShares g = gemm_shares(M, N, K);
+  DA_REQUIRE(g.shares > 1, "gemm_bf16_shares: a product of %d rows, N=%d, K=%d is not shared out", M, N, K);
+  DA_REQUIRE(partial && (uintptr_t)partial % 16 == 0, "gemm_bf16_shares: the sums' place must be 16-byte aligned");
+  const Epilogue ep{nullptr, 0, DA_ACT_NONE, 0, partial, DA_F32, N};
+  const KvScatter kv{nullptr, nullptr, 0, 0, 0, 0, 0};
+  hipStream_t s = (hipStream_t)stream;
+  const bf16_t *A = (const bf16_t*)a, *W = (const bf16_t*)w;
+  if (g.shape != DA_WIDE_NONE) da_gemm_wide_launch(s, A, lda, W, ldw, ep, kv, M, N, K, g.shape, g.k_share);
+  else {
+    DA_REQUIRE(lda <= (1 << 24) && ldw <= (1 << 24), "gemm_bf16_shares: rows lie too far apart (lda=%d ldw=%d)", lda, ldw);
+    const dim3 grid(da_ceil_div(N, 32), g.shares);
+#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, 32, g.k_share)
+    if (M <= 16) DA_SK32_GO(2, 4);
+    else if (M <= 32) DA_SK32_GO(4, 3);
+    else if (M <= 48) DA_SK32_GO(6, 2);
+    else DA_SK32_GO(8, 2);
+#undef DA_SK32_GO
+  }
+  DA_CHECK_LAUNCH("gemm_bf16_shares");
   return 0;
 }
 

@@ -223,7 +223,8 @@ wide_epilogue(floatx16 (&acc)[TM][TN], const float (&bias)[TN], char* region, co
 template <int BM, int BN, int WM, int WN, int ACT, int OUTMODE>
 __global__ void __launch_bounds__(WM * WN * 64)
 gemm_wide_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                 Epilogue ep, KvScatter kv, int M, int N, int K, int tiles_m, int tiles_n) {
+                 Epilogue ep, KvScatter kv, int M, int N, int K, int tiles_m, int tiles_n, int k_share) {
+  gemm_take_share(a, w, ep, M, K, k_share);
   // Two stages of a slab of a, three of a slab of w.  The rows of a were written by the kernel before and
   // come from a cache; w comes from memory for the first time and needs the longer way ahead.
   constexpr int A_BYTES = BM * WD_ROW_BYTES, W_BYTES = BN * WD_ROW_BYTES;      // a slab of a, of w, in LDS
@@ -416,27 +417,27 @@ gemm_wide_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict
 
 template <int BM, int BN, int WM, int WN, int ACT>
 static void launch_wide_act(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
-                            const KvScatter& kv, int M, int N, int K) {
+                            const KvScatter& kv, int M, int N, int K, int k_share) {
   const int tiles_m = da_ceil_div(M, BM), tiles_n = da_ceil_div(N, BN);
-  const dim3 grid(tiles_m * tiles_n), block(WM * WN * 64);
+  const dim3 grid(tiles_m * tiles_n, da_ceil_div(K, k_share)), block(WM * WN * 64);
   if (ep.accumulate)
-    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, DA_ACT_NONE, 2>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n);
+    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, DA_ACT_NONE, 2>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, k_share);
   else if (ep.out_dtype == DA_F32)
-    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, DA_ACT_NONE, 1>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n);
+    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, DA_ACT_NONE, 1>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, k_share);
   else
-    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, ACT, 0>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n);
+    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, ACT, 0>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, k_share);
 }
 
 template <int BM, int BN, int WM, int WN>
 static void launch_wide(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
-                        const KvScatter& kv, int M, int N, int K) {
+                        const KvScatter& kv, int M, int N, int K, int k_share) {
   switch (ep.act) {
-    case DA_ACT_GELU_TANH: launch_wide_act<BM, BN, WM, WN, DA_ACT_GELU_TANH>(s, A, lda, W, ldw, ep, kv, M, N, K); break;
-    case DA_ACT_GELU_ERF: launch_wide_act<BM, BN, WM, WN, DA_ACT_GELU_ERF>(s, A, lda, W, ldw, ep, kv, M, N, K); break;
-    case DA_ACT_RELU: launch_wide_act<BM, BN, WM, WN, DA_ACT_RELU>(s, A, lda, W, ldw, ep, kv, M, N, K); break;
-    case DA_ACT_SILU: launch_wide_act<BM, BN, WM, WN, DA_ACT_SILU>(s, A, lda, W, ldw, ep, kv, M, N, K); break;
-    case DA_ACT_RELU2: launch_wide_act<BM, BN, WM, WN, DA_ACT_RELU2>(s, A, lda, W, ldw, ep, kv, M, N, K); break;
-    default: launch_wide_act<BM, BN, WM, WN, DA_ACT_NONE>(s, A, lda, W, ldw, ep, kv, M, N, K); break;
+    case DA_ACT_GELU_TANH: launch_wide_act<BM, BN, WM, WN, DA_ACT_GELU_TANH>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share); break;
+    case DA_ACT_GELU_ERF: launch_wide_act<BM, BN, WM, WN, DA_ACT_GELU_ERF>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share); break;
+    case DA_ACT_RELU: launch_wide_act<BM, BN, WM, WN, DA_ACT_RELU>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share); break;
+    case DA_ACT_SILU: launch_wide_act<BM, BN, WM, WN, DA_ACT_SILU>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share); break;
+    case DA_ACT_RELU2: launch_wide_act<BM, BN, WM, WN, DA_ACT_RELU2>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share); break;
+    default: launch_wide_act<BM, BN, WM, WN, DA_ACT_NONE>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share); break;
   }
 }
 
@@ -472,10 +473,11 @@ int da_gemm_wide_choice(int M, int N, int K) {
 }
 
 void da_gemm_wide_launch(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
-                         const KvScatter& kv, int M, int N, int K, int shape) {
-  if (shape == DA_WIDE_128x128) launch_wide<128, 128, 4, 2>(s, A, lda, W, ldw, ep, kv, M, N, K);
-  else if (shape == DA_WIDE_256x128) launch_wide<256, 128, 4, 2>(s, A, lda, W, ldw, ep, kv, M, N, K);
-  else launch_wide<256, 256, 2, 4>(s, A, lda, W, ldw, ep, kv, M, N, K);
+                         const KvScatter& kv, int M, int N, int K, int shape, int k_share) {
+  if (k_share <= 0) k_share = K;
+  if (shape == DA_WIDE_128x128) launch_wide<128, 128, 4, 2>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share);
+  else if (shape == DA_WIDE_256x128) launch_wide<256, 128, 4, 2>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share);
+  else launch_wide<256, 256, 2, 4>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share);
 }
 
 // These tiles alone, of the shape asked for (DA_WIDE_256x256, DA_WIDE_256x128, DA_WIDE_128x128), whatever the

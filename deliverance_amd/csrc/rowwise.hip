@@ -214,11 +214,53 @@ __device__ __forceinline__ float4 load_param4(const void* p, int dtype, int i) {
 // Loads come back in the order they were asked for: the row first, then gain and bias, as raw bits
 // that are converted where they are used (a conversion right after its load, or a load inside a
 // branch, is waited for on the spot).  PBF16: gain and bias are bfloat16 (else 32-bit); YBF16: y is.
-template <int VPL, int W, bool PBF16, bool YBF16>
+// JOIN: sums that a product left share by share (gemm_take_share) join the row first: x + (((p0 + p1) + ...) + add).
+struct RowJoin {
+  const float* partial;        // [n][stride]: the sums of the stream's rows, share by share
+  long stride;
+  int n;                       // 2 to 8
+  const void* add;             // a bias a column, or null
+  int add_dtype;
+  float* keep;                 // where the new row goes (the stream), or null
+};
+// the sums of 4 columns at entry `at`, the bias of column c
+__device__ __forceinline__ float4 join_sums(const RowJoin& j, size_t at, int c) {
+  float4 p[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    p[s] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (s < j.n) p[s] = *(const float4*)(j.partial + (size_t)s * j.stride + at);      // (the same for all: a scalar branch)
+  }
+  uint4 raw = make_uint4(0, 0, 0, 0);
+  if (j.add) {
+    if (j.add_dtype == DA_BF16) {
+      const uint2 u = *(const uint2*)((const bf16_t*)j.add + c);
+      raw = make_uint4(u.x << 16, u.x & 0xffff0000u, u.y << 16, u.y & 0xffff0000u);
+    } else raw = *(const uint4*)((const float*)j.add + c);
+  }
+  float4 v = p[0];
+#pragma unroll
+  for (int s = 1; s < 8; ++s) {
+    const bool in = s < j.n;
+    v.x = in ? v.x + p[s].x : v.x;
+    v.y = in ? v.y + p[s].y : v.y;
+    v.z = in ? v.z + p[s].z : v.z;
+    v.w = in ? v.w + p[s].w : v.w;
+  }
+  if (j.add) {
+    v.x += __uint_as_float(raw.x);
+    v.y += __uint_as_float(raw.y);
+    v.z += __uint_as_float(raw.z);
+    v.w += __uint_as_float(raw.w);
+  }
+  return v;
+}
+
+template <int VPL, int W, bool PBF16, bool YBF16, bool JOIN = false>
 __global__ void __launch_bounds__(4 * DA_WAVE)
 layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                      const void* __restrict__ w, const void* __restrict__ b,
-                     float eps, void* __restrict__ y, int R, int E) {
+                     float eps, void* __restrict__ y, int R, int E, RowJoin join) {
   __shared__ float red[2][4];
   constexpr int STRIDE = 4 * W * DA_WAVE;
   const int t = threadIdx.x, c0 = (W == 4 ? t : t % DA_WAVE) * 4;
@@ -234,6 +276,14 @@ layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
     const int c = c0 + i * STRIDE;
     v[i] = *(const float4*)(xr + (c < E ? c : 0));
   }
+  float4 sums[VPL];
+  if (JOIN) {
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = c0 + i * STRIDE, cc = c < E ? c : 0;
+      sums[i] = join_sums(join, (size_t)(xr - x) + cc, cc);
+    }
+  }
   const void* bsrc = b ? b : w;         // without a bias the gain is read twice and dropped
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
@@ -248,6 +298,14 @@ layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
     }
   }
   __builtin_amdgcn_sched_barrier(0);
+  if (JOIN) {
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = c0 + i * STRIDE;
+      v[i].x += sums[i].x; v[i].y += sums[i].y; v[i].z += sums[i].z; v[i].w += sums[i].w;
+      if (join.keep && c < E) *(float4*)(join.keep + (size_t)(xr - x) + c) = v[i];
+    }
+  }
   float part[VPL];
 #pragma unroll
   for (int i = 0; i < VPL; ++i) part[i] = c0 + i * STRIDE < E ? (v[i].x + v[i].y) + (v[i].z + v[i].w) : 0.f;
@@ -292,7 +350,7 @@ extern "C" int da_layernorm(const float* x, const int* rows, const void* w, int 
   const bool same = (!b || b_dtype == w_dtype) && (w_dtype == DA_BF16 || w_dtype == DA_F32);   // gain and bias alike
   if (E % 4 == 0 && E <= 2048 && aligned && same) {
     const NormGrid g = norm_grid(R, E, 768, 1024);
-#define LN_LAUNCH(V, W, P, Y) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, Y>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, eps, y, R, E)
+#define LN_LAUNCH(V, W, P, Y) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, Y>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, eps, y, R, E, RowJoin{})
 #define LN_LAUNCH_Y(V, W, P) do { if (y_dtype == DA_BF16) LN_LAUNCH(V, W, P, true); else LN_LAUNCH(V, W, P, false); } while (0)
 #define LN_LAUNCH_P(V, W) do { if (w_dtype == DA_BF16) LN_LAUNCH_Y(V, W, true); else LN_LAUNCH_Y(V, W, false); } while (0)
     if (g.waves == 1) {
@@ -310,6 +368,56 @@ extern "C" int da_layernorm(const float* x, const int* rows, const void* w, int 
                        w_dtype, b, b_dtype, eps, y, y_dtype, R, E);
   }
   DA_CHECK_LAUNCH("layernorm");
+  return 0;
+}
+
+// x[r] <- x[r] + (sums of the shares + add) and y[r] <- LayerNorm of the new row, or, with `rows`, y[r] <- LayerNorm of the new
+// row rows[r] and x stays as it is (the rows may repeat).  partial: [n][stride], row r of the stream at r * E of each.
+static bool join_takes(const void* x, const float* partial, long stride, int n, const void* add, int add_dtype, int E) {
+  return E % 4 == 0 && E <= 2048 && n >= 2 && n <= 8 && stride % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)partial % 16 == 0 &&
+         (!add || ((add_dtype == DA_BF16 || add_dtype == DA_F32) && (uintptr_t)add % 16 == 0));
+}
+extern "C" int da_layernorm_join(float* x, const int* rows, const float* partial, long stride, int n, const void* add, int add_dtype,
+                                 const void* w, int w_dtype, const void* b, int b_dtype, float eps, void* y, int y_dtype, int R, int E,
+                                 void* stream) {
+  DA_REQUIRE(R >= 0 && E > 0 && eps > 0.f, "layernorm_join: bad sizes R=%d E=%d eps=%g", R, E, eps);
+  DA_REQUIRE(join_takes(x, partial, stride, n, add, add_dtype, E), "layernorm_join: %d shares of rows of %d (2 to 8, a multiple of 4 up to 2,048, 16-byte aligned)", n, E);
+  DA_REQUIRE((uintptr_t)y % 16 == 0 && (uintptr_t)w % 16 == 0 && (!b || (uintptr_t)b % 16 == 0) && (!b || b_dtype == w_dtype) &&
+             (w_dtype == DA_BF16 || w_dtype == DA_F32) && y_dtype == DA_BF16, "layernorm_join: gain and bias of one type, a bfloat16 result, all 16-byte aligned");
+  if (R == 0) return 0;
+  hipStream_t st = (hipStream_t)stream;
+  const RowJoin j{partial, stride, n, add, add_dtype, rows ? nullptr : x};
+  const NormGrid g = norm_grid(R, E, 768, 1024);
+#define LN_LAUNCH(V, W, P) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, true, true>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, eps, y, R, E, j)
+#define LN_LAUNCH_P(V, W) do { if (w_dtype == DA_BF16) LN_LAUNCH(V, W, true); else LN_LAUNCH(V, W, false); } while (0)
+  if (g.waves == 1) {
+    if (E <= 256) LN_LAUNCH_P(1, 1);
+    else if (E <= 512) LN_LAUNCH_P(2, 1);
+    else LN_LAUNCH_P(4, 1);
+  } else if (E <= 1024) LN_LAUNCH_P(1, 4);
+  else LN_LAUNCH_P(2, 4);
+#undef LN_LAUNCH_P
+#undef LN_LAUNCH
+  DA_CHECK_LAUNCH("layernorm_join");
+  return 0;
+}
+
+// The addition alone, where no such norm follows.
+__global__ void __launch_bounds__(256) join_rows_kernel(float* __restrict__ x, int R, int E, RowJoin join) {
+  const long c4 = E / 4, i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= R * c4) return;
+  const size_t at = (size_t)i * 4;
+  float4 v = *(const float4*)(x + at);
+  const float4 s = join_sums(join, at, (int)(i % c4) * 4);
+  v.x += s.x; v.y += s.y; v.z += s.z; v.w += s.w;
+  *(float4*)(x + at) = v;
+}
+extern "C" int da_join_rows(float* x, const float* partial, long stride, int n, const void* add, int add_dtype, int R, int E, void* stream) {
+  DA_REQUIRE(R >= 0 && E > 0 && join_takes(x, partial, stride, n, add, add_dtype, E), "join_rows: bad sizes R=%d E=%d, %d shares", R, E, n);
+  if (R == 0) return 0;
+  const RowJoin j{partial, stride, n, add, add_dtype, x};
+  hipLaunchKernelGGL(join_rows_kernel, dim3(da_ceil_div((long)R * (E / 4), 256)), dim3(256), 0, (hipStream_t)stream, x, R, E, j);
+  DA_CHECK_LAUNCH("join_rows");
   return 0;
 }
 

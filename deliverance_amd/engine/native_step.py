@@ -51,7 +51,8 @@ class DaStep(ctypes.Structure):
                 ("want_rows", _VP), ("slot_map", _VP * MAX_GROUPS), ("block_table", _VP * MAX_GROUPS),
                 ("max_blocks", _I * MAX_GROUPS),
                 ("residual", _VP), ("norm", _VP), ("qkv", _VP), ("attn_out", _VP), ("ff_mid", _VP), ("final_norm", _VP),
-                ("logits", _VP), ("decode_partial", _VP), ("decode_partial_floats", _L), ("stream", _VP)]
+                ("logits", _VP), ("decode_partial", _VP), ("decode_partial_floats", _L),
+                ("proj_partial", _VP), ("proj_partial_floats", _L), ("stream", _VP)]
 
 
 def _dt(t: Optional[torch.Tensor]) -> int:
@@ -73,6 +74,8 @@ class NativeStep:
         n = len(cfg.schedule)
         self._calls = (DaCall * n)()
         self.qkv_cols = self.q_cols = self.inner = 0
+        self._inners = set()                          # the feed-forwards' inner sizes
+        self._share_floats = {}                       # rows of a step -> floats of the scratch of their second products
         self._decode_shapes = []                      # (heads, head size, group) of every call, for the decode scratch
         for i, call in enumerate(cfg.schedule):
             blk = model.blocks[call.layer]
@@ -93,6 +96,7 @@ class NativeStep:
                 rec.fc_b_dtype, rec.proj_b_dtype = _dt(ff.fc_bias), _dt(ff.proj_bias)
                 rec.inner, rec.act = ff.inner, ops.ACTIVATIONS[ff.activation]
                 self.inner = max(self.inner, ff.inner)
+                self._inners.add(ff.inner)
             self.qkv_cols, self.q_cols = max(self.qkv_cols, at.qkv_cols), max(self.q_cols, at.q_cols)
             self._decode_shapes.append((at.n_heads, at.head_dim, rec.group))
         pos = model.embed_position.embed_table()
@@ -163,6 +167,11 @@ class NativeStep:
                 self._partial_floats[key] = floats
         st.decode_partial = ctx.buf("decode_partial", 1, floats, torch.float32).data_ptr() if floats else None
         st.decode_partial_floats = floats
+        floats = self._share_floats.get(N)
+        if floats is None:
+            floats = self._share_floats[N] = max([s * N * cfg.width for s in (ops.product_shares(N, cfg.width, k) for k in self._inners) if s > 1], default=0)
+        st.proj_partial = ctx.buf("proj_partial", 1, floats, torch.float32).data_ptr() if floats else None
+        st.proj_partial_floats = floats
         st.stream = ops._stream()
         if self._run(ctypes.byref(self._model), ctypes.byref(st)) != 0:
             raise ops.KernelError(ops._lib().da_last_error().decode())

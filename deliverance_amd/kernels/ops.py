@@ -98,6 +98,10 @@ _ARGTYPES = {
     "da_sample": [_VP, _I, _I, _I, _VP, _VP, _VP],
     "da_decode_splits": [_I, _I, _I, _I],
     "da_can_fuse_ln": [_I, _I, _I],
+    "da_gemm_shares": [_I, _I, _I],
+    "da_gemm_bf16_shares": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP],
+    "da_layernorm_join": [_VP, _VP, _VP, ctypes.c_long, _I, _VP, _I, _VP, _I, _VP, _I, _F, _VP, _I, _I, _I, _VP],
+    "da_join_rows": [_VP, _VP, ctypes.c_long, _I, _VP, _I, _I, _I, _VP],
     "da_run_step": [_VP, _VP],
     "da_top_logprobs": [_VP, _I, _I, _I, _VP, _I, _VP, _VP, _VP],
     "da_attn_decode_rel": [_VP, _I, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP, _F, _I, _I, _VP, _VP, _I, _VP, _I, _I, _VP, ctypes.c_long, _VP],
@@ -882,6 +886,61 @@ def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
             _check(_lib().da_gemm_bf16(*args, _stream()))
         else:
             _check(_lib().da_gemm_bf16_wide(*args, WIDE_TILE_SHAPES[form], _stream()))
+    return out
+
+
+def product_shares(M: int, N: int, K: int) -> int:
+    """How many shares the k of a bfloat16 product of M rows into the residual stream is cut into (1: none)."""
+    return int(_lib().da_gemm_shares(int(M), int(N), int(K)))
+
+
+def shares_ok(a: torch.Tensor, w: torch.Tensor, add: Optional[torch.Tensor]) -> bool:
+    """Whether ``linear_shares`` and what joins its sums to the stream take these operands."""
+    return _MODE == "tuned" and _mfma_ok(a, w) and (add is None or add.data_ptr() % 16 == 0)
+
+
+def linear_shares(a: torch.Tensor, w: torch.Tensor, partial: torch.Tensor) -> torch.Tensor:
+    """partial[s] = a @ w.T over share s of k, for ``product_shares(M, N, K)`` shares (more than one): [shares, M, N] float32."""
+    _dev(a, w, partial)
+    _rows_2d(a, "a"); _rows_2d(w, "w")
+    M, K = a.shape
+    N = w.shape[0]
+    _need(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.shape[1] == K, "linear_shares: a [M, K] and w [N, K] must be bfloat16")
+    n = product_shares(M, N, K)
+    _need(partial.dtype == torch.float32 and partial.is_contiguous() and partial.numel() == n * M * N, "linear_shares: partial must be float32 [shares, M, N]")
+    with _timed("product_shares", _nbytes(a, w, partial), 2 * M * N * K):
+        _check(_lib().da_gemm_bf16_shares(_ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(partial), M, N, K, _stream()))
+    return partial
+
+
+def _join_args(x, partial, add, name):
+    _need(x.dtype == torch.float32 and x.dim() == 2 and x.is_contiguous(), f"{name}: x must be contiguous float32 [N, E]")
+    _need(partial.dtype == torch.float32 and partial.is_contiguous() and partial.numel() % x.numel() == 0, f"{name}: partial must be float32 [shares, N, E]")
+    _need(add is None or (add.numel() == x.shape[1] and add.is_contiguous()), f"{name}: the bias's length differs from E")
+    return _ptr(partial), x.numel(), partial.numel() // max(1, x.numel()), _ptr(add), _dt(add) if add is not None else 0
+
+
+def join_rows(x: torch.Tensor, partial: torch.Tensor, add: Optional[torch.Tensor]) -> torch.Tensor:
+    """x += ((partial[0] + partial[1]) + ...) + add: what ``linear_shares`` left joins the stream."""
+    _dev(x, partial, add)
+    args = _join_args(x, partial, add, "join_rows")
+    with _timed("join_rows", 2 * _nbytes(x) + _nbytes(partial, add), x.numel() * (partial.numel() // max(1, x.numel()) + 1), "fp32"):
+        _check(_lib().da_join_rows(_ptr(x), *args, x.shape[0], x.shape[1], _stream()))
+    return x
+
+
+def layernorm_join(x: torch.Tensor, partial: torch.Tensor, add: Optional[torch.Tensor], weight: torch.Tensor, bias: Optional[torch.Tensor],
+                   eps: float, out: torch.Tensor, rows: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``join_rows`` and the LayerNorm of the new rows (bfloat16) in one pass; with ``rows`` only the rows named are added
+    up, for the norm alone, and x stays as it is."""
+    _dev(x, partial, add, weight, bias, out, rows)
+    args = _join_args(x, partial, add, "layernorm_join")
+    R, E = out.shape
+    _need(out.is_contiguous() and E == x.shape[1] and weight.numel() == E and (bias is None or bias.numel() == E), "layernorm_join: widths differ")
+    _need(R == x.shape[0] if rows is None else (rows.dtype == torch.int32 and rows.numel() >= R), "layernorm_join: rows")
+    with _timed("layernorm_join", 2 * _nbytes(x) + _nbytes(partial, out, weight, bias), 12 * x.numel(), "fp32"):
+        _check(_lib().da_layernorm_join(_ptr(x), _ptr(rows), *args, _ptr(weight), _dt(weight), _ptr(bias), _dt(bias) if bias is not None else 0,
+                                        eps, _ptr(out), _dt(out), R, E, _stream()))
     return out
 
 

@@ -44,7 +44,11 @@ class DenseFeedForward(FeedForward):
         N = h.shape[0]
         mid = ctx.buf("ff_mid", N, self.inner, ctx.dtype)
         ops.linear(h, self.fc_weight, self.fc_bias, mid, act=self.activation)
-        ops.linear(mid, self.proj_weight, self.proj_bias, x, accumulate=ctx.part_accumulate)
+        shares = ops.product_shares(N, self.width, self.inner) if ctx.part_accumulate and ops.shares_ok(mid, self.proj_weight, self.proj_bias) else 1
+        if shares > 1:          # (the same sums as the step issued from C++, whose norms add them in passing)
+            ops.join_rows(x, ops.linear_shares(mid, self.proj_weight, ctx.buf("proj_partial", shares * N, self.width, torch.float32)), self.proj_bias)
+        else:
+            ops.linear(mid, self.proj_weight, self.proj_bias, x, accumulate=ctx.part_accumulate)
 
 
 register_feed_forward("dense", DenseFeedForward)

@@ -197,6 +197,42 @@ def test_gemm_32bit_of_few_rows_and_many_columns_of_a(ops, M, N, K):
         assert torch.equal(ops.linear_f32(a, w, None, torch.empty(M, N, device=DEV), form=form), tiles), form
 
 
+@pytest.mark.parametrize("M,N,K,bf16", [helpers.quick(17, 64, 4096, True), (9, 1028, 4160, True), (16, 1600, 6400, True), (33, 1024, 4096, False),
+                                        (64, 1600, 6400, True), (48, 100, 4608, False), (65, 260, 2048, True), (129, 768, 3072, False),
+                                        (552, 1024, 4096, True), (1025, 1024, 2112, True), (640, 2048, 6400, True)])
+def test_products_shared_out_over_k(ops, M, N, K, bf16):
+    """The shares' sums, added to a stream with a bias, and the norm of the new rows, whole and of repeated rows; ragged last
+    shares, edges of tiles, both forms.  32-bit sums of K products of magnitudes a, w: sqrt(K) roundings of 2^-24 of the sum."""
+    helpers.skip_in_simulation_if(M * N * K > 1e7)
+    n = ops.product_shares(M, N, K)
+    assert n > 1
+    g = torch.Generator().manual_seed(M + K)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    a, w = bf(torch.randn(M, K, generator=g)).to(DEV), bf(torch.randn(N, K, generator=g) * 0.1).to(DEV)
+    bias, gain, add = (torch.randn(N, generator=g).to(dt).to(DEV) for _ in range(3))
+    x = torch.randn(M, N, generator=g).to(DEV)
+    partial = ops.linear_shares(a, w, torch.full((n * M, N), float("nan"), device=DEV))
+    new = x.double() + a.double() @ w.double().t() + add.double()
+    tol = 2.0 ** -22 * K ** 0.5 * (a.float().abs() @ w.float().abs().t()).max().item() / K ** 0.5
+    joined = ops.join_rows(x.clone(), partial, add)
+    assert (joined.double() - new).abs().max() < tol
+    kept, h = x.clone(), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    ops.layernorm_join(kept, partial, add, gain, bias, 1e-5, h)
+    assert torch.equal(kept, joined) and torch.equal(h, ops.layernorm(joined, gain, bias, 1e-5, torch.empty_like(h)))
+    rows = torch.tensor([M - 1, 0, M - 1, M // 2], dtype=torch.int32, device=DEV)
+    few = ops.layernorm_join(x, partial, None, gain, bias, 1e-5, torch.empty(4, N, dtype=torch.bfloat16, device=DEV), rows)
+    plain = ops.join_rows(x.clone(), partial, None)
+    assert torch.equal(few, ops.layernorm(plain, gain, bias, 1e-5, torch.empty_like(few), rows))
+
+
+def test_products_that_are_not_shared_out_are_refused(ops):
+    for M, N, K in ((8, 1600, 6400), (64, 768, 3072), (100, 1024, 1024), (100, 2304, 4096), (100, 1022, 4096), (1500, 1024, 4096), (4096, 1600, 6400)):
+        assert ops.product_shares(M, N, K) == 1
+    a, w = (torch.zeros(s, 1024, dtype=torch.bfloat16, device=DEV) for s in (100, 1024))
+    with pytest.raises(ops.KernelError):
+        ops.linear_shares(a, w, torch.zeros(100, 1024, device=DEV))
+
+
 @pytest.mark.parametrize("M,N,K", [helpers.quick(3, 700, 772), helpers.quick(4, 1030, 132), (2, 250, 6400), (4, 2100, 1284), (1, 13000, 260),
                                    helpers.quick(8, 1100, 388), (5, 2050, 644), (7, 10500, 132), (8, 5000, 3072), (8, 10500, 3076),
                                    helpers.quick(9, 300, 260), (16, 1000, 6400), (33, 3000, 388), (12, 4100, 516), (16, 10240, 1028),

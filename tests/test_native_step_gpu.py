@@ -57,6 +57,22 @@ def test_native_step_at_a_width_with_separate_norms_and_split_decode_attention(t
         assert np.array_equal(native[rid], parts[rid]), rid
 
 
+def test_native_step_with_second_products_shared_out_over_k(tmp_path):
+    """A feed-forward of 4,096 inner columns: steps of 17 to 64 and of more rows leave its second product's sums share by share,
+    and the next layer's norm, the final norm (several wanted rows of a sequence) and a head that takes its norm itself (few
+    wanted rows, a small vocabulary) each have to find them added up."""
+    cfg = dict(architectures=["GPT2LMHeadModel"], model_type="gpt2", n_layer=2, n_embd=256, n_head=4, n_inner=4096, vocab_size=301,
+               n_positions=512, layer_norm_epsilon=1e-5, activation_function="gelu_new", bos_token_id=0, eos_token_id=1)
+    m = helpers.make_model(tmp_path, cfg, seed=22)
+    reqs = [(f"r{i}", m.prompt(n, salt=40 + i)) for i, n in enumerate((150, 40, 64, 70, 9))]
+    for steps in (helpers.trace_whole(*reqs[0]), helpers.trace_whole(*reqs[1]), helpers.trace_mixed(reqs, seed=6),
+                  helpers.trace_portions(*reqs[0], (70, 17, 60, 3))):
+        native, parts = both_ways(m, steps, max(helpers.max_live_tokens(steps), 128))
+        for rid in native:
+            assert np.array_equal(native[rid], parts[rid]), rid
+    helpers.check_against_plain(m, native, [reqs[0]], "bfloat16", "shared out over k")
+
+
 def test_the_plan_is_made_only_for_what_it_describes(models):
     m = models["A"]
     assert helpers.trace_session(m.folder, "float32", 128).runner.native is None
