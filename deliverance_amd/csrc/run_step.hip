@@ -23,6 +23,10 @@ int da_attn_decode(const void* q, int q_ld, const void* cache, const int* block_
 int da_attn_decode_split(const void* q, int q_ld, const void* cache, const int* block_table, int max_blocks,
                          const int* seq_lens, int S, int Hq, int Hkv, int D, int page, float scale, int window, void* out,
                          int out_ld, int n_splits, void* workspace, long workspace_bytes, void* stream);
+int da_attn_both_takes(int n_decode, int n_portions, int max_query_len, int Hq, int D, int page, int splits);
+int da_attn_both(const void* q, int q_ld, const void* cache, const int* block_table, int max_blocks, const int* q_start, const int* seq_lens,
+                 int n_decode, int n_portions, int max_query_len, int Hq, int Hkv, int D, int page, float scale, int window, void* out,
+                 int out_ld, void* stream);
 int da_attn_prefill(const void* q, int q_ld, const void* cache, const int* block_table, int max_blocks, const int* q_start,
                     const int* seq_lens, int seq0, int n_seqs, int max_query_len, int Hq, int Hkv, int D, int page,
                     float scale, int window, void* out, int out_ld, int form, void* stream);
@@ -93,9 +97,13 @@ extern "C" int da_run_step(const DaModel* model, const DaStep* step) {
     DA_TRY(normed_product(st, x, left, nullptr, N, L.norm1, E, L.qkv_w, L.qkv_b, L.qkv_b_dtype, DA_ACT_NONE, st.norm, st.qkv, DA_BF16, qkv_cols,
                           L.write ? L.kv_cache : nullptr, L.write ? st.slot_map[g] : nullptr, L.write ? q_cols : 0,
                           L.write ? kv_cols : 0, L.write ? L.n_kv_heads : 0, L.write ? D : 0, L.write ? m.page : 0));
-    // attention: the one-token sequences first, then the portions
-    if (st.n_decode > 0) {
-      const int splits = da_decode_splits(st.n_decode, L.n_heads, st.max_blocks[g], m.page);
+    // attention: one-token sequences and portions in one launch, or the one and then the other
+    const int splits = st.n_decode > 0 ? da_decode_splits(st.n_decode, L.n_heads, st.max_blocks[g], m.page) : 1;
+    const bool both = da_attn_both_takes(st.n_decode, st.S - st.n_decode, st.max_query_len, L.n_heads, D, m.page, splits);
+    if (both)
+      DA_TRY(da_attn_both(st.qkv, qkv_cols, L.kv_cache, st.block_table[g], st.max_blocks[g], st.q_start, st.seq_lens, st.n_decode,
+                          st.S - st.n_decode, st.max_query_len, L.n_heads, L.n_kv_heads, D, m.page, L.scale, L.window, st.attn_out, q_cols, st.stream));
+    if (!both && st.n_decode > 0) {
       if (splits > 1) {
         DA_REQUIRE(st.decode_partial && st.decode_partial_floats >= (long)st.n_decode * L.n_heads * splits * (D + 2),
                    "run_step: the scratch of decode attention is too small");
@@ -107,7 +115,7 @@ extern "C" int da_run_step(const DaModel* model, const DaStep* step) {
                               L.n_kv_heads, D, m.page, L.scale, L.window, st.attn_out, q_cols, st.stream));
       }
     }
-    if (st.S > st.n_decode)
+    if (!both && st.S > st.n_decode)
       DA_TRY(da_attn_prefill(st.qkv, qkv_cols, L.kv_cache, st.block_table[g], st.max_blocks[g], st.q_start, st.seq_lens, st.n_decode,
                              st.S - st.n_decode, st.max_query_len, L.n_heads, L.n_kv_heads, D, m.page, L.scale, L.window, st.attn_out,
                              q_cols, 0, st.stream));

@@ -34,6 +34,7 @@ HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
 # registers and moves every value out and in again.
 EXTRA_FLAGS = {"attn_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_prefill_rel": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+               "attn_both": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_latent_mfma": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_window": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_f32": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
@@ -41,10 +42,10 @@ EXTRA_FLAGS = {"attn_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 BASE_UNIT = "rowwise"
 # Units whose functions a unit calls.
 NEEDS = {"gemm_mfma": ("gemm_wide",),
-         "run_step": ("dispatch", "gemm_mfma", "gemm_fused", "attn_decode", "attn_prefill")}
-# Units that are another unit's source compiled with a definition in front, and entry points that are not found by
+         "run_step": ("dispatch", "gemm_mfma", "gemm_fused", "attn_decode", "attn_prefill", "attn_both")}
+# Units that are other units' sources compiled with a definition in front, and entry points that are not found by
 # reading their unit's own source.
-INCLUDES = {"attn_decode_rel": "attn_decode", "attn_prefill_rel": "attn_prefill"}
+INCLUDES = {"attn_decode_rel": ("attn_decode",), "attn_prefill_rel": ("attn_prefill",), "attn_both": ("attn_decode", "attn_prefill")}
 _ELSEWHERE = {"da_attn_decode_rel": "attn_decode_rel", "da_attn_prefill_rel": "attn_prefill_rel",
               "da_attn_prefill_rel_max_dist": "attn_prefill_rel", "da_gemm_wide_choice": "gemm_wide"}
 
@@ -125,7 +126,7 @@ def _find_hipcc():
 def _newest_source(unit: str) -> float:
     files = [_source(unit)] + glob.glob(os.path.join(CSRC, "*.h"))
     if unit in INCLUDES:
-        files.append(_source(INCLUDES[unit]))
+        files += [_source(u) for u in INCLUDES[unit]]
     return max(os.path.getmtime(f) for f in files)
 
 

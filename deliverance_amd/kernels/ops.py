@@ -93,6 +93,8 @@ _ARGTYPES = {
     "da_attn_ref": [_VP, _I, _VP, _I, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
     "da_attn_f32": [_VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
     "da_attn_decode": [_VP, _I, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
+    "da_attn_both_takes": [_I, _I, _I, _I, _I, _I, _I],
+    "da_attn_both": [_VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
     "da_attn_decode_split": [_VP, _I, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _I, _VP, ctypes.c_long, _VP],
     "da_attn_prefill": [_VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _I, _VP],
     "da_sample": [_VP, _I, _I, _I, _VP, _VP, _VP],
@@ -1197,6 +1199,25 @@ def attention_prefill(q: torch.Tensor, cache_slot: torch.Tensor, block_table: to
     return out
 
 
+def attention_both(q: torch.Tensor, cache_slot: torch.Tensor, block_table: torch.Tensor, q_start: torch.Tensor, seq_lens: torch.Tensor,
+                   n_decode: int, n_portions: int, max_query_len: int, n_heads: int, scale: float, window: Optional[int],
+                   out: torch.Tensor) -> torch.Tensor:
+    """``attention_decode`` of the first ``n_decode`` sequences and ``attention_prefill`` of the ``n_portions`` behind them in one
+    launch (steps that da_attn_both_takes names)."""
+    _dev(q, cache_slot, block_table, q_start, seq_lens, out)
+    _rows_2d(q, "q"); _rows_2d(out, "out")
+    _need(cache_slot.dim() == 5 and cache_slot.is_contiguous() and cache_slot.dtype == torch.bfloat16 and q.dtype == torch.bfloat16
+          and out.dtype == torch.bfloat16, "attention_both: bfloat16 rows and a contiguous cache slot [pages,2,Hkv,page,D]")
+    _, _, Hkv, page, D = cache_slot.shape
+    S = n_decode + n_portions
+    _need(block_table.dtype == torch.int32 and block_table.is_contiguous() and block_table.shape[0] >= S, "attention_both: block_table must be int32 [S, blocks]")
+    _need(q_start.dtype == torch.int32 and q_start.numel() >= S + 1 and seq_lens.dtype == torch.int32 and seq_lens.numel() >= S, "attention_both: q_start, seq_lens")
+    _need(q.shape[1] == n_heads * D and out.shape[1] >= n_heads * D and out.shape[0] >= q.shape[0], "attention_both: q and out")
+    _check(_lib().da_attn_both(_ptr(q), q.stride(0), _ptr(cache_slot), _ptr(block_table), block_table.shape[1], _ptr(q_start), _ptr(seq_lens),
+                               n_decode, n_portions, max_query_len, n_heads, Hkv, D, page, scale, int(window or 0), _ptr(out), out.stride(0), _stream()))
+    return out
+
+
 def paged_attention(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: int, n_heads: int,
                     scale: float, window: Optional[int], out: torch.Tensor) -> torch.Tensor:
     """Attention of every row of the step over its sequence's pages.  In bfloat16 the one-token
@@ -1225,8 +1246,11 @@ def paged_attention(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: int, 
         return keys * 2 * Hkv * D * el + 2 * rows * n_heads * D * el, 4 * pairs * n_heads * D
 
     if _MODE == "tuned" and q.dtype == torch.bfloat16 and D % 16 == 0 and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0:
+        n_splits = decode_splits(nd, n_heads, bt.shape[1], page) if nd else 1
+        if nd and _lib().da_attn_both_takes(nd, ctx.n_seqs - nd, ctx.max_query_len, n_heads, D, page, n_splits):
+            with _timed("attention_both", *cost(0, ctx.n_seqs)):
+                return attention_both(q, cache_slot, bt, ctx.q_start, ctx.seq_lens, nd, ctx.n_seqs - nd, ctx.max_query_len, n_heads, scale, window, out)
         if nd:
-            n_splits = decode_splits(nd, n_heads, bt.shape[1], page)
             ws = None
             if n_splits > 1:
                 ws = ctx.buf("decode_partial", 1, decode_workspace_floats(nd, n_heads, D, n_splits), torch.float32)

@@ -162,7 +162,7 @@ class CausalSelfAttention(Mixer):
         if dtype != torch.bfloat16:
             return out + (("attn_rel",) if self.extras else ("attn_ref", "attn_f32"))
         if not self.extras:
-            return out + (("attn_decode", "attn_prefill") if D % 16 == 0 else ("attn_ref",))
+            return out + (("attn_decode", "attn_prefill", "attn_both") if D % 16 == 0 else ("attn_ref",))
         scores_only = self.v_head_dim == D and D % 16 == 0 and D <= 128 and self.softcap == 0.0 and not self.keep_first
         if scores_only and self.sink is None and self.out_gate is None and self.chunk is None and self.slopes is None:
             return out + ("attn_decode_rel", "attn_prefill_rel")

@@ -836,6 +836,33 @@ def test_attention_prefill_kernel(ops, Hq, Hkv, D, page, window):
                                   scale, window, out, form=14)
 
 
+@pytest.mark.parametrize("Hq,Hkv,page,window,new", [
+    helpers.quick(2, 1, 16, None, (1, 1, 1, 2)), (16, 16, 16, None, (1,) * 20 + (260, 129, 3)), (5, 5, 8, 100, (1, 1, 128)),
+    (12, 4, 64, None, (1, 33, 64, 65)), helpers.quick(3, 3, 32, 40, (1, 1, 70)), (30, 30, 16, None, (1,) * 9 + (512, 40))])
+def test_attention_of_one_token_sequences_and_portions_in_one_launch(ops, Hq, Hkv, page, window, new):
+    """Few and many pairs, portions of 2 to 512 rows after nothing and after a past; the portions' rows have the bits of the prefill
+    kernel's form of 4 row blocks x 2 key phases."""
+    new = sorted(new, key=lambda n: n != 1)
+    lens = [n + (37 * i * i) % 300 for i, n in enumerate(new)]
+    nd = sum(n == 1 for n in new)
+    case = PagedCase(lens=lens, new=new, Hq=Hq, Hkv=Hkv, D=64, page=page, dtype=torch.bfloat16, seed=Hq + page)
+    assert ops._lib().da_attn_both_takes(nd, len(new) - nd, max(new), Hq, 64, page, 1)
+    out = torch.full_like(case.qcat, float("nan"))
+    ops.attention_both(case.qcat, case.cache, case.bt, case.q_start, case.seq_lens, nd, len(new) - nd, max(new), Hq, 0.09, window, out)
+    assert np.abs(out.double().cpu().numpy() - case.plain(0.09, window)).max() < ATT_TOL[torch.bfloat16]
+    alone = torch.full_like(case.qcat, float("nan"))
+    ops.attention_prefill(case.qcat, case.cache, case.bt, case.q_start, case.seq_lens, nd, len(new) - nd, max(new), Hq, 0.09, window, alone, form=42)
+    assert torch.equal(out[nd:], alone[nd:])
+
+
+def test_when_attention_goes_in_one_launch(ops):
+    takes = ops._lib().da_attn_both_takes
+    assert takes(40, 1, 512, 16, 64, 16, 1) and takes(1, 1, 2, 12, 64, 16, 1)
+    for a in ((0, 1, 512, 16, 64, 16, 1), (4, 0, 1, 16, 64, 16, 1), (4, 1, 512, 16, 48, 16, 1), (4, 1, 512, 16, 64, 16, 2), (4, 8, 1024, 16, 64, 16, 1),
+              (4, 1, 512, 16, 64, 128, 1)):
+        assert not takes(*a), a
+
+
 @pytest.mark.simt_quick
 @pytest.mark.parametrize("form", [41, 42, 22, 14])
 def test_attention_prefill_finds_a_far_key_in_every_phase(ops, form):
