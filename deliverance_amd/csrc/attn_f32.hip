@@ -1,25 +1,27 @@
 // Paged attention in 32-bit on the matrix cores (v_mfma_f32_16x16x4_f32): portions of prompts and one-token sequences alike.
 //
-// One workgroup per (sequence, query head, 16 query rows); 8 wavefronts share out the keys in aligned chunks of 64:
+// One workgroup per (sequence, query head, 16 query rows); 8 wavefronts share out the keys in aligned chunks of 32:
 // wavefront v takes the chunks whose number is v modulo 8, in ascending order, with a running maximum and sum per row,
 // and the wavefronts' partial results are merged in LDS in order.  Every sum's order so depends on a row's own position
 // and the window only, never on how the step was cut or what else is in the batch; a chunk that a row does not see
 // changes nothing in its sums.
-//   scores : S[row, key] = Q . K^T, 4 pieces of 16 keys; a lane's 16-byte piece of a key row is 4 of the inner sum's
+//   scores : S[row, key] = Q . K^T, 2 pieces of 16 keys; a lane's 16-byte piece of a key row is 4 of the inner sum's
 //            terms (an instruction takes the dimensions with d % 4 = j; see gemm_f32.hip for the fragments);
 //   softmax: a lane holds 4 rows of one key column, so a row's maximum and sum are exchanges among 16 lanes;
 //   values : stored dimension-major, so a lane's 16-byte piece is 4 consecutive keys of its dimension, which is the
 //            right operand as it lies in memory; the weights turn from columns into rows through LDS.
 // All key and value loads of a chunk are asked for before any is used (for head sizes up to 64; above, the values once
-// the scores are done).  Bound by two trips to memory and 2 D instructions of 32 cycles a chunk.
-// Beside the plain kernel (attn_ref.hip), 8 heads, us at head size 64 / 128: two prompts of 300 112 -> 16 / 221 -> 29, a prompt of 1,024
-// 589 -> 32 / 1,172 -> 61, 8 sequences of 1,000 keys 189 -> 21 / 379 -> 43.  (Head size 128 keeps 64 bytes a lane in scratch; 112: 1,024
-// rows 46 us.)
+// the scores are done).  Bound by two trips to memory and D instructions of 32 cycles a chunk.  (Chunks of 64 keys leave most wavefronts
+// of a short context without any and the others a chain twice as long; us, 64 / 32 keys a chunk, 12 heads of 64: 4 sequences of 61
+// keys 7.4 / 5.7, of 200 9.2 / 8.0, 64 of 1,000 91 / 82, two prompts of 300 17.6 / 14.8, of 1,024 85 / 78; 8 heads, 8 of 1,000 keys 21.2 / 21.5.)
+// Beside the plain kernel (attn_ref.hip), 8 heads, us at head size 64 / 128: a prompt of 1,024 589 -> 29 /
+// 1,172 -> 50, 8 sequences of 1,000 keys 189 -> 21 / 379 -> 38.
 // Formulas: core/src/main/java/io/teknek/deliverance/generator/CausalSelfAttention.java:481-491,512-527.
 #include "gemm_common.h"
 
 #define AF_WAVES 8
-#define AF_CHUNK 64
+#define AF_CHUNK 32
+#define AF_PIECES (AF_CHUNK / 16)
 #define AF_PLD (AF_CHUNK + 4)        // padded row of weights in LDS, floats
 
 __device__ __forceinline__ floatx4 af_group(const float4& a, const float4& b, floatx4 c) {
@@ -104,13 +106,13 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
   const int first_chunk = lo_min / AF_CHUNK;
   for (int ci = first_chunk + (wave + AF_WAVES - first_chunk % AF_WAVES) % AF_WAVES; ci * AF_CHUNK <= p_max; ci += AF_WAVES) {
     const int c0 = ci * AF_CHUNK;
-    // The pages of the chunk's 4 pieces of 16 keys (a piece lies in one page), the same for the whole wavefront.  A piece
+    // The pages of the chunk's pieces of 16 keys (a piece lies in one page), the same for the whole wavefront.  A piece
     // that no row sees, or whose page was given back, reads page 0 and is dropped.
-    bool seen[4];
-    const float* kp[4];
-    const float* vp[4];
+    bool seen[AF_PIECES];
+    const float* kp[AF_PIECES];
+    const float* vp[AF_PIECES];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < AF_PIECES; ++j) {
       const int k0 = c0 + j * 16;
       const bool in = k0 <= p_max && k0 + 15 >= lo_min;
       const int pg = in ? __builtin_amdgcn_readfirstlane(bt[k0 >> lg]) : -1;
@@ -119,22 +121,22 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
       kp[j] = kbase + off + (k0 & pmask) * D;
       vp[j] = vbase + off + (k0 & pmask);
     }
-    float4 kf[4][D16], vf[4][D16];
+    float4 kf[AF_PIECES][D16], vf[AF_PIECES][D16];
     constexpr bool EARLY_V = D16 <= 4;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < AF_PIECES; ++j)
 #pragma unroll
       for (int g = 0; g < D16; ++g) kf[j][g] = *(const float4*)(kp[j] + col * D + g * 16 + quad * 4);
     if (EARLY_V) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < AF_PIECES; ++j)
 #pragma unroll
         for (int d = 0; d < D16; ++d) vf[j][d] = *(const float4*)(vp[j] + (d * 16 + col) * page + quad * 4);
     }
     __builtin_amdgcn_sched_barrier(0);                          // (the loads stay ahead of the arithmetic)
-    floatx4 sc[4];
+    floatx4 sc[AF_PIECES];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < AF_PIECES; ++j) {
       sc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int g = 0; g < D16; ++g) sc[j] = af_group(qf[g], kf[j][g], sc[j]);
@@ -144,10 +146,10 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
     for (int r = 0; r < 4; ++r) {
       const int i = i0 + quad * 4 + r, p = past + i;
       const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
-      bool ok[4];
+      bool ok[AF_PIECES];
       float top = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < AF_PIECES; ++j) {
         const int key = c0 + j * 16 + col;
         ok[j] = seen[j] && i < T && key <= p && key >= lo;
         sc[j][r] = ok[j] ? sc[j][r] * scale : -INFINITY;        // (a select: an unseen key's row may hold anything)
@@ -158,7 +160,7 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
       const float m_ref = m_new == -INFINITY ? 0.f : m_new;     // (scores of minus infinity alone weigh nothing here: another chunk may hold more)
       float sum = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < AF_PIECES; ++j) {
         const float e = ok[j] ? expf(sc[j][r] - m_ref) : 0.f;
         ps[(quad * 4 + r) * AF_PLD + j * 16 + col] = e;
         sum += e;
@@ -175,12 +177,12 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
       for (int r = 0; r < 4; ++r) o[d][r] *= alpha[r];
     if (!EARLY_V) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < AF_PIECES; ++j)
 #pragma unroll
         for (int d = 0; d < D16; ++d) vf[j][d] = *(const float4*)(vp[j] + (d * 16 + col) * page + quad * 4);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < AF_PIECES; ++j) {
       const float4 w = *(const float4*)&ps[col * AF_PLD + j * 16 + quad * 4];
       // keys past the last seen one were never written and keys in front of a window may be anybody's: zeros in their
       // place (their weights are zero, but zero times an infinity is not)
