@@ -151,15 +151,6 @@ class StepPacker:
         meta.update(q_start=q_start, seq_lens=seq_lens, state_slots=state_slots)
 
 
-def graph_bucket(n_seqs: int) -> int:
-    """How many sequences a recorded decode step of ``n_seqs`` is padded to: the next power of two, and 48.  Products of up to 64
-    rows come in row tiles of 16 and take time by them (355M sizes, 33 requests: 1,231 us a step as 64, 1,194 as 48); up to
-    32 the powers of two hold no idle tile, and above 64 the block tiles have 64 rows and more."""
-    if 32 < n_seqs <= 48:
-        return 48
-    return 1 << (n_seqs - 1).bit_length()
-
-
 class StepRunner:
     def __init__(self, model: CausalLM, cache: DeviceCache, use_graphs: bool = False, max_graph_batch: int = 256,
                  kernels: str = "tuned", native_step: bool = True):
@@ -352,7 +343,9 @@ class StepRunner:
         Only the step's integers change: they are copied into the bucket's own buffer first."""
         from ..kernels import ops
         S = len(entries)
-        bucket = graph_bucket(S)
+        bucket = 1
+        while bucket < S:
+            bucket *= 2
         order = list(range(S))
         offs, meta, n_words = self._layout(entries, order, pad_to=bucket, max_blocks=self.max_blocks_cap,
                                            extra=sample_records)
