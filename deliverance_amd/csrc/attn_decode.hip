@@ -37,7 +37,6 @@
 
 #ifdef DEC_REL
 #define DEC_KERNEL attn_decode_rel_kernel
-#define DEC_BODY attn_decode_rel_body
 #define DEC_MERGE_KERNEL attn_decode_rel_merge_kernel
 #define DEC_REL_PARAMS , const float* __restrict__ rel_bias, int n_dist, const float* __restrict__ slopes, float t_coef, int t_every, int chunk DEC_END_PARAMS
 #define DEC_REL_DECL , const float* rel_bias, int n_dist, const float* slopes, float t_coef, int t_every, int chunk, const float* sink, const bf16_t* gate, int gate_ld
@@ -46,7 +45,6 @@
 #define DEC_END_ARGS , sink, gate, gate_ld
 #else
 #define DEC_KERNEL attn_decode_kernel
-#define DEC_BODY attn_decode_body
 #define DEC_MERGE_KERNEL attn_decode_merge_kernel
 #define DEC_REL_PARAMS
 #define DEC_REL_DECL
@@ -84,10 +82,24 @@ __device__ __forceinline__ float dec_gate(float z) {
 // sequences' lengths, so a recorded graph can hold it.
 //
 // DK: dimensions in steps of 32, rounded up to a power of two (1, 2, 4, 8)
-// pair, share of n_shares: which workgroup this is.
+// Included by attn_both.hip (DA_ATTN_BODIES) the kernel is a function that is told which workgroup it is.  (A function in both
+// files, called by a kernel, compiles to other code: one-token steps of the Virudra 1,101 -> 1,106 us.)
 template <int DK, int DEC_WAVES, bool SPLIT>
+#ifdef DA_ATTN_BODIES
+#define DEC_PAIR dec_pair
+#define DEC_SHARE 0
+#define DEC_SHARES 1
 __device__ __forceinline__ void
-DEC_BODY(int pair, int share, int n_shares, const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
+attn_decode_body(int dec_pair,
+#else
+#define DEC_PAIR blockIdx.x
+#define DEC_SHARE (int)blockIdx.y
+#define DEC_SHARES gridDim.y
+// (registers are held to 128 for head sizes up to 64, so that two workgroups share a compute unit)
+__global__ void __launch_bounds__(DEC_WAVES * DA_WAVE, (DK <= 2 || DEC_WAVES == 16) ? 4 : 2)
+DEC_KERNEL(
+#endif
+           const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
            const int* __restrict__ block_table, int max_blocks,
            const int* __restrict__ seq_lens, int Hq, int Hkv, int D, int page, float scale,
            int window, bf16_t* __restrict__ out, int out_ld, int span, float* __restrict__ partial DEC_REL_PARAMS) {
@@ -97,7 +109,7 @@ DEC_BODY(int pair, int share, int n_shares, const bf16_t* __restrict__ q, int q_
   __shared__ __attribute__((aligned(16))) float part_acc[DEC_WAVES][DMAX];
   __shared__ float part_m[DEC_WAVES], part_l[DEC_WAVES];
 
-  const int s = pair / Hq, h = pair % Hq;
+  const int s = DEC_PAIR / Hq, h = DEC_PAIR % Hq;
   const int hk = h / (Hq / Hkv);
   const int t = threadIdx.x, lane = t % DA_WAVE, wave = __builtin_amdgcn_readfirstlane(t / DA_WAVE);
   const int col = lane % 16, quad = lane / 16;
@@ -118,7 +130,7 @@ DEC_BODY(int pair, int share, int n_shares, const bf16_t* __restrict__ q, int q_
     const int d = 32 * k + 8 * quad;
     qf[k] = *(const uint4*)(q + (size_t)s * q_ld + h * D + (d < D ? d : 0));
   }
-  const int split0 = SPLIT ? share * span : 0;          // the first key of this workgroup's share
+  const int split0 = SPLIT ? DEC_SHARE * span : 0;          // the first key of this workgroup's share
   const int c0_guess = split0 + wave * DA_WAVE;
   int btk0[4], btv0[2];
 #pragma unroll
@@ -369,7 +381,7 @@ DEC_BODY(int pair, int share, int n_shares, const bf16_t* __restrict__ q, int q_
   }
   if (SPLIT) {
     // the share's result before the division, its maximum and its sum of weights
-    float* mine = partial + ((size_t)pair * n_shares + share) * (D + 2);
+    float* mine = partial + ((size_t)DEC_PAIR * DEC_SHARES + blockIdx.y) * (D + 2);
     for (int d = t; d < D; d += DEC_WAVES * DA_WAVE) {
       float o = 0.f;
 #pragma unroll
@@ -400,18 +412,7 @@ DEC_BODY(int pair, int share, int n_shares, const bf16_t* __restrict__ q, int q_
 #endif
 }
 
-#ifndef DA_ATTN_BODIES        // (attn_both.hip takes the body alone)
-template <int DK, int DEC_WAVES, bool SPLIT>
-// (registers are held to 128 for head sizes up to 64, so that two workgroups share a compute unit)
-__global__ void __launch_bounds__(DEC_WAVES * DA_WAVE, (DK <= 2 || DEC_WAVES == 16) ? 4 : 2)
-DEC_KERNEL(const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
-           const int* __restrict__ block_table, int max_blocks,
-           const int* __restrict__ seq_lens, int Hq, int Hkv, int D, int page, float scale,
-           int window, bf16_t* __restrict__ out, int out_ld, int span, float* __restrict__ partial DEC_REL_PARAMS) {
-  DEC_BODY<DK, DEC_WAVES, SPLIT>(blockIdx.x, blockIdx.y, gridDim.y, q, q_ld, cache, block_table, max_blocks, seq_lens, Hq, Hkv, D, page,
-                                 scale, window, out, out_ld, span, partial DEC_REL_ARGS);
-}
-
+#ifndef DA_ATTN_BODIES
 // The partial results of a (sequence, head) pair, merged in ascending order of the shares.
 __global__ void __launch_bounds__(256)
 DEC_MERGE_KERNEL(const float* __restrict__ partial, int n_splits, int Hq, int D,

@@ -40,14 +40,12 @@
 
 #ifdef PF_REL
 #define PF_KERNEL attn_prefill_rel_kernel
-#define PF_BODY attn_prefill_rel_body
 #define PF_REL_MAX_DIST 1024       // entries of the bias row that the workgroup keeps in LDS
 #define PF_REL_PAD 96              // a tile's keys reach at most 59 + 35 distances past either end of the row
 #define PF_REL_PARAMS , const float* __restrict__ rel_bias, int n_dist, float t_coef, int t_every
 #define PF_REL_ARGS , rel_bias, n_dist, t_coef, t_every
 #else
 #define PF_KERNEL attn_prefill_kernel
-#define PF_BODY attn_prefill_body
 #define PF_REL_PARAMS
 #define PF_REL_ARGS
 #endif
@@ -64,10 +62,23 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 // head size / 16; wavefronts (32 query rows each) per workgroup; whether the block table's entries
 // for the workgroup's keys fit its LDS copy (a table entry read from memory in front of a tile's loads
 // makes them wait for it, and for every load still in flight)
-// pair, block of n_blocks: which workgroup this is.
+// Included by attn_both.hip (DA_ATTN_BODIES) the kernel is a function that is told which workgroup it is.
 template <int D16, int RB, int KP, bool BT_LDS>
+#ifdef DA_ATTN_BODIES
+#define PF_PAIR pf_pair
+#define PF_BLOCK pf_block
+#define PF_BLOCKS pf_blocks
 __device__ __forceinline__ void
-PF_BODY(int pair, int block, int n_blocks, const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
+attn_prefill_body(int pf_pair, int pf_block, int pf_blocks,
+#else
+#define PF_PAIR (int)blockIdx.x
+#define PF_BLOCK (int)blockIdx.y
+#define PF_BLOCKS (int)gridDim.y
+// (head sizes up to 64 with four wavefronts: registers held to 256, so that two workgroups share a compute unit)
+__global__ void __launch_bounds__(RB * KP * DA_WAVE, (RB * KP == 4 && D16 <= 4) ? 2 : 1)
+PF_KERNEL(
+#endif
+          const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
           const int* __restrict__ block_table, int max_blocks,
           const int* __restrict__ q_start, const int* __restrict__ seq_lens, int seq0,
           int Hq, int Hkv, int page, float scale, int window,
@@ -103,9 +114,9 @@ PF_BODY(int pair, int block, int n_blocks, const bf16_t* __restrict__ q, int q_l
   // other way round, the long workgroups of the later pairs start when the chip is already full of short ones, and
   // the step ends with a few compute units walking their keys alone: at 2 x 4,096 rows and 12 heads the wavefronts
   // resident over the kernel's time averaged 0.9 a SIMD of 2.)
-  const int s = seq0 + pair / Hq, h = pair % Hq;
+  const int s = seq0 + PF_PAIR / Hq, h = PF_PAIR % Hq;
   const int row0 = q_start[s], T = q_start[s + 1] - row0;
-  const int i0 = (n_blocks - 1 - block) * PF_BQ;
+  const int i0 = (PF_BLOCKS - 1 - PF_BLOCK) * PF_BQ;
   if (i0 >= T) return;
   const int past = seq_lens[s] - T;
   const int hk = h / (Hq / Hkv);
@@ -534,19 +545,7 @@ PF_BODY(int pair, int block, int n_blocks, const bf16_t* __restrict__ q, int q_l
   }
 }
 
-#ifndef DA_ATTN_BODIES        // (attn_both.hip takes the body alone)
-template <int D16, int RB, int KP, bool BT_LDS>
-// (head sizes up to 64 with four wavefronts: registers held to 256, so that two workgroups share a compute unit)
-__global__ void __launch_bounds__(RB * KP * DA_WAVE, (RB * KP == 4 && D16 <= 4) ? 2 : 1)
-PF_KERNEL(const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
-          const int* __restrict__ block_table, int max_blocks,
-          const int* __restrict__ q_start, const int* __restrict__ seq_lens, int seq0,
-          int Hq, int Hkv, int page, float scale, int window,
-          bf16_t* __restrict__ out, int out_ld PF_REL_PARAMS) {
-  PF_BODY<D16, RB, KP, BT_LDS>((int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y, q, q_ld, cache, block_table, max_blocks, q_start, seq_lens, seq0,
-                               Hq, Hkv, page, scale, window, out, out_ld PF_REL_ARGS);
-}
-
+#ifndef DA_ATTN_BODIES
 #ifdef PF_REL
 extern "C" int da_attn_prefill_rel_max_dist() { return PF_REL_MAX_DIST; }
 

@@ -1066,16 +1066,16 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
 // tiles and a long K most compute units have no tile; cut, share by share, they have one, and what the shares' sums cost is
 // that the norm behind reads them (da_layernorm_join; never a norm that is fused into its product: more rows than
 // da_can_fuse_ln takes).  Whole slabs of 64 k, 512 k a share at least, 8 shares at most.
-//  - up to 64 rows (32 columns a workgroup, gemm_skinny32), K from 4,096: us, cold weights, += / shares: 64 rows, N = 1,600, K = 6,400
-//    14.1 / 10.2 (5), 32 rows 11.1 / 8.0, 16 rows 10.3 / 7.9; N = 1,024, K = 4,096 64 rows 7.4 / 6.5 (8), 48 rows 7.5 / 5.9.  Not K = 3,072,
-//    N = 768: 64 rows 4.9 / 5.5;
+//  - up to 64 rows (32 columns a workgroup, gemm_skinny32), K from 4,096, more than 1,024 columns: us, cold weights, += / shares: 64
+//    rows, N = 1,600, K = 6,400 14.1 / 10.2 (5), 32 rows 11.1 / 8.0, 16 rows 10.3 / 7.9.  Not N = 1,024, K = 4,096: 64 rows 7.4 / 6.5, 48 rows
+//    7.5 / 5.9, but with 8 shares for the norm to read a step of 64 rows takes 1,249 us for 1,232; nor N = 768, K = 3,072 (64 rows 4.9 / 5.5);
 //  - more rows: tiles of 128 x 128 where they are at most 85, as many shares as bring them to about 256 (552 rows, N = 1,024,
 //    K = 4,096 20.1 / 12.2 (6)).  K from 2,048.  (K = 1,024: 552 rows 7.5 / 6.5, which the norm's reads take up; so do they
 //    with two shares of more rows: 1,624 rows, K = 4,096 29.7 / 23.9, a step of them 2,834 / 2,841.)
 struct GemmShares { int shares, k_share, shape; };     // shape: DA_WIDE_..., or DA_WIDE_NONE for gemm_skinny32
 static GemmShares gemm_shares(int M, int N, int K) {
   const GemmShares none{1, K, DA_WIDE_NONE};
-  if (M <= 8 || (M <= 16 && N <= 1024) || N % 4 || K % 64 || N > 2048) return none;
+  if (M <= 8 || (M <= 64 && N <= 1024) || N % 4 || K % 64 || N > 2048) return none;
   GemmShares g = none;
   long tiles;
   if (M <= 64) {

@@ -197,8 +197,8 @@ def test_gemm_32bit_of_few_rows_and_many_columns_of_a(ops, M, N, K):
         assert torch.equal(ops.linear_f32(a, w, None, torch.empty(M, N, device=DEV), form=form), tiles), form
 
 
-@pytest.mark.parametrize("M,N,K,bf16", [helpers.quick(17, 64, 4096, True), (9, 1028, 4160, True), (16, 1600, 6400, True), (33, 1024, 4096, False),
-                                        (64, 1600, 6400, True), (48, 100, 4608, False), (65, 260, 2048, True), (129, 768, 3072, False),
+@pytest.mark.parametrize("M,N,K,bf16", [(17, 1056, 4096, True), (9, 1028, 4160, True), (16, 1600, 6400, True), (33, 2048, 4096, False),
+                                        (64, 1600, 6400, True), (48, 1100, 4608, False), helpers.quick(65, 68, 2048, True), (66, 260, 2112, True), (129, 768, 3072, False),
                                         (552, 1024, 4096, True), (1025, 1024, 2112, True), (640, 2048, 6400, True)])
 def test_products_shared_out_over_k(ops, M, N, K, bf16):
     """The shares' sums, added to a stream with a bias, and the norm of the new rows, whole and of repeated rows; ragged last
@@ -226,7 +226,7 @@ def test_products_shared_out_over_k(ops, M, N, K, bf16):
 
 
 def test_products_that_are_not_shared_out_are_refused(ops):
-    for M, N, K in ((8, 1600, 6400), (64, 768, 3072), (100, 1024, 1024), (100, 2304, 4096), (100, 1022, 4096), (1500, 1024, 4096), (4096, 1600, 6400)):
+    for M, N, K in ((8, 1600, 6400), (64, 768, 3072), (64, 1024, 4096), (100, 1024, 1024), (100, 2304, 4096), (100, 1022, 4096), (1500, 1024, 4096), (4096, 1600, 6400)):
         assert ops.product_shares(M, N, K) == 1
     a, w = (torch.zeros(s, 1024, dtype=torch.bfloat16, device=DEV) for s in (100, 1024))
     with pytest.raises(ops.KernelError):

@@ -58,7 +58,7 @@ def test_native_step_at_a_width_with_separate_norms_and_split_decode_attention(t
 
 
 def test_native_step_with_second_products_shared_out_over_k(tmp_path):
-    """A feed-forward of 4,096 inner columns: steps of 17 to 64 and of more rows leave its second product's sums share by share,
+    """A feed-forward of 4,096 inner columns: steps of more than 64 rows leave its second product's sums share by share,
     and the next layer's norm, the final norm (several wanted rows of a sequence) and a head that takes its norm itself (few
     wanted rows, a small vocabulary) each have to find them added up."""
     cfg = dict(architectures=["GPT2LMHeadModel"], model_type="gpt2", n_layer=2, n_embd=256, n_head=4, n_inner=4096, vocab_size=301,
