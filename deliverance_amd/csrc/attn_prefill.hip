@@ -578,7 +578,7 @@ extern "C" int da_attn_prefill(const void* q, int q_ld, const void* cache, const
   hipStream_t st = (hipStream_t)stream;
   // The workgroup's form, row blocks x key phases.  Short portions (after a long past, beside decoded
   // tokens) have few rows to a sequence and head: 1 x 4 up to 32 rows, 2 x 2 up to 64, so that all four
-  // wavefronts work and share out the keys.  Longer ones take 128 rows a workgroup (smaller row blocks
+  // wavefronts work and share out the keys (see below for how many keys).  Longer ones take 128 rows a workgroup (smaller row blocks
   // read the keys more often, and that traffic binds), and 4 x 2, eight wavefronts, while there is no
   // more than one workgroup a compute unit; else 4 x 1.  Measured on MI355X, head size 64, microseconds
   // 4x1 / 4x2 / 2x2 / 1x4: 2 x 1,024 rows, 12 heads 23.3 / 19.3 / 23.4 / 34.6; 2,048 rows 40.0 / 31.8 /
@@ -595,8 +595,20 @@ extern "C" int da_attn_prefill(const void* q, int q_ld, const void* cache, const
   // choice reads the step's shape only.
   // form: 0 leaves the choice to this rule; 41, 42, 22 or 14 fixes it
   const long per128 = (long)da_ceil_div(max_query_len, 128) * Hq * n_seqs;
+  // Up to 64 rows, by the most keys that any sequence has (the block table's width), head size up to 64, us 4x1 / 2x2 / 1x4, 12 heads, 8 and 64
+  // rows: 64 keys 4.5 / 6.0 / 9.3 and 4.9 / 6.5 / 10.0 (one tile: there is nothing to share out, and a round that is not whole
+  // asks for its tiles the slow way); 128 keys 5.9 / 5.0 / 8.9 and 6.2 / 5.4 / 9.6; 256 7.2 / 6.1 / 6.9 and 7.6 / 6.6 / 9.0; 512 11.0 / 8.4 / 8.7 and
+  // 11.4 / 8.9 / 12.3; 1,024 18.8 / 13.0 / 12.3 and 19.2 / 13.6 / 16.0.  So 4 x 1 up to one tile, 1 x 4 for up to 32 rows with
+  // more than 768 keys, else 2 x 2.
+  const long keys = (long)max_blocks * page;
+#ifdef PF_REL
+  const bool one_tile = false, far = true;          // (measured without a bias only)
+#else
+  const bool one_tile = D <= 64 && keys <= PF_BK, far = keys > 768;
+#endif
   const int chosen = form ? form
-                     : (D <= 64 && max_query_len <= 32) ? 14
+                     : (one_tile && max_query_len <= 64) ? 41
+                     : (D <= 64 && max_query_len <= 32 && far) ? 14
                      : (D <= 128 && max_query_len <= 64) ? 22
                      : (D <= 64 && per128 <= PF_PHASED_MAX_WORKGROUPS) ? 42 : 41;
   DA_REQUIRE(chosen == 41 || (chosen == 22 && D <= 128) || ((chosen == 42 || chosen == 14) && D <= 64),

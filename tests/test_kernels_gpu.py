@@ -836,6 +836,16 @@ def test_attention_prefill_kernel(ops, Hq, Hkv, D, page, window):
                                   scale, window, out, form=14)
 
 
+@pytest.mark.parametrize("lens,new", [helpers.quick([64, 37, 1], [64, 37, 1]), ([64, 33], [2, 32]), helpers.quick([65, 20], [20, 20]), ([768, 5], [32, 5]),
+                                      ([769, 64], [32, 32]), ([769, 64], [33, 64])])
+def test_attention_prefill_of_short_portions_by_their_keys(ops, lens, new):
+    """The kernel's own choice for up to 64 rows, at the lines between its forms: one tile of keys, up to and above 768."""
+    case = PagedCase(lens=lens, new=new, Hq=3, Hkv=1, D=64, page=16, dtype=torch.bfloat16, seed=sum(lens))
+    out = torch.full_like(case.qcat, float("nan"))
+    ops.attention_prefill(case.qcat, case.cache, case.bt, case.q_start, case.seq_lens, 0, len(lens), max(new), 3, 0.1, None, out)
+    assert np.abs(out.double().cpu().numpy() - case.plain(0.1, None)).max() < ATT_TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("Hq,Hkv,page,window,new", [
     helpers.quick(2, 1, 16, None, (1, 1, 1, 2)), (16, 16, 16, None, (1,) * 20 + (260, 129, 3)), (5, 5, 8, 100, (1, 1, 128)),
     (12, 4, 64, None, (1, 33, 64, 65)), helpers.quick(3, 3, 32, 40, (1, 1, 70)), (30, 30, 16, None, (1,) * 9 + (512, 40))])
