@@ -46,7 +46,7 @@ class DenseFeedForward(FeedForward):
         ops.linear(h, self.fc_weight, self.fc_bias, mid, act=self.activation)
         shares = ops.product_shares(N, self.width, self.inner) if ctx.part_accumulate and ops.shares_ok(mid, self.proj_weight, self.proj_bias) else 1
         if shares > 1:          # (the same sums as the step issued from C++, whose norms add them in passing)
-            ops.join_rows(x, ops.linear_shares(mid, self.proj_weight, ctx.buf("proj_partial", shares * N, self.width, torch.float32)), self.proj_bias)
+            ops.join_rows(x, ops.linear_shares(mid, self.proj_weight, ctx.flat("proj_partial", shares * N * self.width, torch.float32)), self.proj_bias)
         else:
             ops.linear(mid, self.proj_weight, self.proj_bias, x, accumulate=ctx.part_accumulate)
 

@@ -137,3 +137,45 @@ def test_a_launch_that_fails_leaves_no_reservation_behind(tmp_path):
     assert mgr.live() == ["old"] and mgr.length("old") == 20 and mgr.pending("old") == 0
     assert mgr.pools[0].n_free == free
     mgr.check()
+
+
+def arena_bytes(arena, name):
+    held = [t for key, t in arena._bufs.items() if key[0] == name] + [e[0] for key, e in arena._flats.items() if key[0] == name]
+    return len(held), sum(t.numel() * t.element_size() for t in held)
+
+
+def test_scratch_of_steps_of_many_sizes_is_one_buffer(monkeypatch, tmp_path):
+    """The plan of a step issued from C++ asks for scratch whose size follows the step's: over steps of many sizes, in no
+    order, an engine keeps one buffer of each kind, at most twice the largest need, and a size within the largest one
+    allocates nothing."""
+    import torch
+    from types import SimpleNamespace
+    from deliverance_amd.engine.device_cache import DeviceCache
+    from deliverance_amd.engine.native_step import NativeStep
+    from deliverance_amd.kernels import ops
+    from deliverance_amd.models.causal_lm import load_model
+    from deliverance_amd.parts.base import Arena, StepContext
+    shares = lambda M, N, K: max(1, min(8, 2048 // M)) if M > 8 else 1
+    monkeypatch.setattr(ops, "_lib", lambda: SimpleNamespace(da_run_step=lambda *a: 0))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "product_shares", shares)
+    model = load_model(helpers.make_model(tmp_path, helpers.CONFIG_A, 0).folder, torch.bfloat16, "cpu")
+    cache = DeviceCache(model.cache_needs(), torch.bfloat16, "cpu", 16, 256, n_state_slots=4)
+    step, width = NativeStep(model, cache), model.config.width
+    arena = Arena("cpu")
+    largest = 0
+    for N in [int(n) for n in np.random.default_rng(3).permutation(np.arange(1, 1500, 7))]:
+        ctx = StepContext()
+        ints = torch.zeros(N + 1, dtype=torch.int32)
+        ctx.n_tokens, ctx.n_seqs, ctx.n_decode, ctx.max_query_len = N, 1, 0, N
+        ctx.tokens = ctx.positions = ctx.seq_of_token = ctx.q_start = ctx.seq_lens = ints
+        ctx.block_tables, ctx.slot_maps, ctx._arena = [ints.view(1, -1)], [ints], arena
+        before = arena_bytes(arena, "proj_partial")
+        step.forward(ctx, None, 0)
+        need = 4 * shares(N, width, 0) * N * width if shares(N, width, 0) > 1 else 0
+        if need <= largest:
+            assert arena_bytes(arena, "proj_partial") == before
+        largest = max(largest, need)
+        assert step._step.proj_partial_floats * 4 == need
+    count, held = arena_bytes(arena, "proj_partial")
+    assert count == 1 and largest <= held <= 2 * largest
