@@ -165,7 +165,7 @@ class NativeStep:
                     if splits > 1:
                         floats = max(floats, ops.decode_workspace_floats(ctx.n_decode, heads, d, splits))
                 self._partial_floats[key] = floats
-        st.decode_partial = ctx.buf("decode_partial", 1, floats, torch.float32).data_ptr() if floats else None
+        st.decode_partial = ctx.flat("decode_partial", floats, torch.float32).data_ptr() if floats else None
         st.decode_partial_floats = floats
         floats = self._share_floats.get(N)
         if floats is None:

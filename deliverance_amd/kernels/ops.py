@@ -1253,7 +1253,7 @@ def paged_attention(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: int, 
         if nd:
             ws = None
             if n_splits > 1:
-                ws = ctx.buf("decode_partial", 1, decode_workspace_floats(nd, n_heads, D, n_splits), torch.float32)
+                ws = ctx.flat("decode_partial", decode_workspace_floats(nd, n_heads, D, n_splits), torch.float32)
             with _timed("attention_decode", *cost(0, nd)):
                 attention_decode(q, cache_slot, bt, ctx.seq_lens, nd, n_heads, scale, window, out, n_splits, ws)
         if ctx.n_seqs > nd:
@@ -1417,7 +1417,7 @@ def paged_attention_rel(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: i
         n_splits = decode_splits(nd, n_heads, bt.shape[1], page)
         ws = None
         if n_splits > 1:
-            ws = ctx.buf("decode_partial", 1, decode_workspace_floats(nd, n_heads, D, n_splits), torch.float32)
+            ws = ctx.flat("decode_partial", decode_workspace_floats(nd, n_heads, D, n_splits), torch.float32)
         with _timed("attention_decode", *cost(0, nd)):
             attention_decode_rel(q, cache_slot, bt, ctx.seq_lens, nd, n_heads, scale, window, dist_bias, temp_coef,
                                  temp_every, out, n_splits, ws, chunk=chunk or 0, sink=sink, gate_col=gate_col, slopes=slopes)
@@ -1856,7 +1856,7 @@ def paged_attention_latent(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group
             n_splits = int(_lib().da_attn_latent_splits(nd, n_heads, bt.shape[1], page))
             ws = None
             if n_splits > 1:
-                ws = ctx.buf("latent_partial", 1, latent_partial_floats(nd, 1, n_heads, v_dim, n_splits), torch.float32)
+                ws = ctx.flat("latent_partial", latent_partial_floats(nd, 1, n_heads, v_dim, n_splits), torch.float32)
             with _timed("attention_latent_decode", *cost(0, nd)):
                 go(0, nd, 1, n_splits, ws)
         if ctx.n_seqs > nd:

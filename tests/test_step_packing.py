@@ -144,10 +144,8 @@ def arena_bytes(arena, name):
     return len(held), sum(t.numel() * t.element_size() for t in held)
 
 
-def test_scratch_of_steps_of_many_sizes_is_one_buffer(monkeypatch, tmp_path):
-    """The plan of a step issued from C++ asks for scratch whose size follows the step's: over steps of many sizes, in no
-    order, an engine keeps one buffer of each kind, at most twice the largest need, and a size within the largest one
-    allocates nothing."""
+def native_step(monkeypatch, tmp_path, **rules):
+    """The plan of a step issued from C++, without a library behind it, and a context of a step of N rows on an arena."""
     import torch
     from types import SimpleNamespace
     from deliverance_amd.engine.device_cache import DeviceCache
@@ -155,23 +153,34 @@ def test_scratch_of_steps_of_many_sizes_is_one_buffer(monkeypatch, tmp_path):
     from deliverance_amd.kernels import ops
     from deliverance_amd.models.causal_lm import load_model
     from deliverance_amd.parts.base import Arena, StepContext
-    shares = lambda M, N, K: max(1, min(8, 2048 // M)) if M > 8 else 1
-    monkeypatch.setattr(ops, "_lib", lambda: SimpleNamespace(da_run_step=lambda *a: 0))
+    monkeypatch.setattr(ops, "_lib", lambda: SimpleNamespace(da_run_step=lambda *a: 0, da_attn_both_takes=lambda *a: 0))
     monkeypatch.setattr(ops, "_stream", lambda: 0)
-    monkeypatch.setattr(ops, "product_shares", shares)
+    for name, rule in rules.items():
+        monkeypatch.setattr(ops, name, rule)
     model = load_model(helpers.make_model(tmp_path, helpers.CONFIG_A, 0).folder, torch.bfloat16, "cpu")
     cache = DeviceCache(model.cache_needs(), torch.bfloat16, "cpu", 16, 256, n_state_slots=4)
-    step, width = NativeStep(model, cache), model.config.width
     arena = Arena("cpu")
+
+    def context(N, n_decode, blocks):
+        ctx = StepContext()
+        ctx.n_tokens, ctx.n_seqs, ctx.n_decode, ctx.max_query_len = N, max(1, n_decode), n_decode, 1 if n_decode else N
+        ctx.tokens = ctx.positions = ctx.seq_of_token = ctx.q_start = ctx.seq_lens = torch.zeros(N + 1, dtype=torch.int32)
+        ctx.block_tables, ctx.slot_maps, ctx._arena = [torch.zeros(ctx.n_seqs, blocks, dtype=torch.int32)], [ctx.tokens], arena
+        return ctx
+    return NativeStep(model, cache), arena, context
+
+
+def test_scratch_of_steps_of_many_sizes_is_one_buffer(monkeypatch, tmp_path):
+    """The plan of a step issued from C++ asks for scratch whose size follows the step's: over steps of many sizes, in no
+    order, an engine keeps one buffer of each kind, at most twice the largest need, and a size within the largest one
+    allocates nothing."""
+    shares = lambda M, N, K: max(1, min(8, 2048 // M)) if M > 8 else 1
+    step, arena, context = native_step(monkeypatch, tmp_path, product_shares=shares)
+    width = step.model.config.width
     largest = 0
     for N in [int(n) for n in np.random.default_rng(3).permutation(np.arange(1, 1500, 7))]:
-        ctx = StepContext()
-        ints = torch.zeros(N + 1, dtype=torch.int32)
-        ctx.n_tokens, ctx.n_seqs, ctx.n_decode, ctx.max_query_len = N, 1, 0, N
-        ctx.tokens = ctx.positions = ctx.seq_of_token = ctx.q_start = ctx.seq_lens = ints
-        ctx.block_tables, ctx.slot_maps, ctx._arena = [ints.view(1, -1)], [ints], arena
         before = arena_bytes(arena, "proj_partial")
-        step.forward(ctx, None, 0)
+        step.forward(context(N, 0, 4), None, 0)
         need = 4 * shares(N, width, 0) * N * width if shares(N, width, 0) > 1 else 0
         if need <= largest:
             assert arena_bytes(arena, "proj_partial") == before
@@ -179,3 +188,29 @@ def test_scratch_of_steps_of_many_sizes_is_one_buffer(monkeypatch, tmp_path):
         assert step._step.proj_partial_floats * 4 == need
     count, held = arena_bytes(arena, "proj_partial")
     assert count == 1 and largest <= held <= 2 * largest
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_scratch_of_decode_attention_of_many_sizes_is_one_buffer(monkeypatch, tmp_path, native):
+    """Likewise the partial results of decode attention that shares a pair's keys out, in steps issued either way."""
+    import torch
+    from deliverance_amd.kernels import ops
+    splits = lambda n_seqs, n_heads, blocks, page: max(1, min(blocks // 4, 512 // (n_seqs * n_heads)))
+    step, arena, context = native_step(monkeypatch, tmp_path, decode_splits=splits, product_shares=lambda *a: 1,
+                                       attention_decode=lambda *a, **k: None)
+    at = step.model.blocks[0].mixer
+    cache_slot = step.cache.kv[0]
+    largest = 0
+    for n, blocks in [(int(i) // 8 + 1, int(i) % 8 * 16 + 8) for i in np.random.default_rng(5).permutation(240)]:
+        ctx = context(n, n, blocks)
+        if native:
+            step.forward(ctx, None, 0)
+        else:
+            q = torch.zeros(n, at.n_heads * at.head_dim, dtype=torch.bfloat16)
+            with ops.kernel_mode_scope("tuned"):
+                ops.paged_attention(ctx, q, cache_slot, 0, at.n_heads, 1.0, None, torch.empty_like(q))
+        k = splits(n, at.n_heads, blocks, 16)
+        if k > 1:
+            largest = max(largest, 4 * ops.decode_workspace_floats(n, at.n_heads, at.head_dim, k))
+    count, held = arena_bytes(arena, "decode_partial")
+    assert count == 1 and 0 < largest <= held <= 2 * largest
