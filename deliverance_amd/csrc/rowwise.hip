@@ -256,9 +256,14 @@ __device__ __forceinline__ float4 join_sums(const RowJoin& j, size_t at, int c) 
   return v;
 }
 
+// The rows that a kernel reads; those that it may also write (JOIN: the stream, which is `keep` as well) go without the promise
+// that no other pointer reaches them.
+template <bool JOIN> struct RowSource { typedef const float* __restrict__ type; };
+template <> struct RowSource<true> { typedef const float* type; };
+
 template <int VPL, int W, bool PBF16, bool YBF16, bool JOIN = false>
 __global__ void __launch_bounds__(4 * DA_WAVE)
-layernorm_row_kernel(const float* __restrict__ x, const int* __restrict__ rows,
+layernorm_row_kernel(typename RowSource<JOIN>::type x, const int* __restrict__ rows,
                      const void* __restrict__ w, const void* __restrict__ b,
                      float eps, void* __restrict__ y, int R, int E, RowJoin join) {
   __shared__ float red[2][4];

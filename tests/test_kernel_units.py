@@ -81,3 +81,22 @@ def test_models_name_units_that_exist(tmp_path):
     from deliverance_amd.kernels import ops
     if build.is_built():
         assert all(bool(ops._lib().da_rglru_serve_takes(n)) == ops.rglru_block_fits(n) for n in range(1, 300))
+
+
+def test_a_norm_that_writes_the_stream_promises_nothing_about_it(tmp_path):
+    """The kernels that add shares to the stream read it through one pointer and write it through another: the front end's
+    code must not tell the optimizer that the two never meet (``noalias``); the plain norms, which only read, may."""
+    import re
+    import subprocess
+    from deliverance_amd.kernels import build
+    hipcc = build._find_hipcc()
+    if hipcc is None:
+        pytest.skip("needs hipcc")
+    out = str(tmp_path / "rowwise.ll")
+    subprocess.run([hipcc, "-std=c++17", f"--offload-arch={build.ARCH}", "--cuda-device-only", "-S", "-emit-llvm", "-O1", "-Xclang",
+                    "-disable-llvm-passes", "-w", build._source("rowwise"), "-o", out], check=True)
+    with open(out) as f:
+        found = re.findall(r"define [^\n]*@_Z\d+layernorm_row_kernelILi\d+ELi\d+ELb[01]ELb[01]ELb([01])EE[^(]*\(([^,]*),", f.read())
+    assert {join for join, _ in found} == {"0", "1"}
+    for join, stream in found:
+        assert ("noalias" in stream) == (join == "0"), (join, stream)
