@@ -26,11 +26,29 @@ attn_both_kernel(const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restric
   attn_decode_body<2, 8, false>(id, q, q_ld, cache, block_table, max_blocks, seq_lens, Hq, Hkv, 64, page, scale, window, out, out_ld, 0, nullptr);
 }
 
-// 1 when a step's attention goes to this kernel: both kinds of sequences, heads of 64, contexts whose pairs are not shared out, and
+// 1 for the steps that this kernel takes: both kinds of sequences, heads of 64, contexts whose pairs are not shared out, and
 // portions that leave compute units idle (128-row workgroups no more than compute units).
 extern "C" int da_attn_both_takes(int n_decode, int n_portions, int max_query_len, int Hq, int D, int page, int splits) {
   if (n_decode <= 0 || n_portions <= 0 || D != 64 || splits > 1 || !(page == 8 || page == 16 || page == 32 || page == 64)) return 0;
   return (long)da_ceil_div(max_query_len, 128) * Hq * n_portions <= PF_PHASED_MAX_WORKGROUPS && (long)n_decode * Hq < (1L << 30);
+}
+
+// 1 when a step's attention goes to this kernel.  It holds one workgroup a compute unit where the decode kernel holds two, and its
+// portions have 4 row blocks x 2 key phases whatever their length.  us, the two kernels / this one:
+//  - many pairs of one-token rows, which want that second workgroup: 1,024 pairs of 20 keys beside 15 rows 13.0 / 13.3, of 300 21.6 / 18.6;
+//    1,575 of 50 beside 2 rows 16.6 / 17.0, beside 16 rows 20.9 / 17.4; 1,536 of 20 beside 16 rows of a table of 16 keys 15.4 / 17.2, beside five
+//    times 512 rows 32.0 / 33.8; 2,048 of 50 beside 256 rows 20.7 / 21.6, of 300 32.1 / 32.6; 3,060 and more 10 to 40 % behind up to 300 keys (of
+//    1,000: 119 / 114).  So up to 1,024 pairs, or 1,600 beside 16 rows or more, if the block tables are wider than 256 keys and the
+//    portions' workgroups at most 128;
+//  - portions of up to 64 rows after many keys, which the prefill kernel gives four key phases: 360 pairs of 20 keys beside 16 rows
+//    after 500 keys 16.8 / 13.0, after 1,000 21.3 / 17.2, after 1,900 28.9 / 27.2 (32 rows 28.6 / 28.8), after 4,000 42.4 / 51.4, after
+//    8,000 77 / 96.  So up to 1,920 keys by the block table's width; longer portions have the same form in both.
+extern "C" int da_attn_both_pays(int n_decode, int n_portions, int max_query_len, int Hq, int D, int page, int splits, int max_blocks) {
+  if (!da_attn_both_takes(n_decode, n_portions, max_query_len, Hq, D, page, splits)) return 0;
+  const long pairs = (long)n_decode * Hq;
+  const long keys = (long)max_blocks * page, portions = (long)da_ceil_div(max_query_len, 128) * Hq * n_portions;
+  const bool more = max_query_len >= 16 && keys > 256 && portions <= 128;
+  return pairs <= (more ? 1600 : 1024) && (max_query_len > 64 || keys <= 1920);
 }
 
 // The first n_decode sequences bring one row each (row s is sequence s's), the n_portions behind them the rows q_start says.

@@ -23,7 +23,7 @@ int da_attn_decode(const void* q, int q_ld, const void* cache, const int* block_
 int da_attn_decode_split(const void* q, int q_ld, const void* cache, const int* block_table, int max_blocks,
                          const int* seq_lens, int S, int Hq, int Hkv, int D, int page, float scale, int window, void* out,
                          int out_ld, int n_splits, void* workspace, long workspace_bytes, void* stream);
-int da_attn_both_takes(int n_decode, int n_portions, int max_query_len, int Hq, int D, int page, int splits);
+int da_attn_both_pays(int n_decode, int n_portions, int max_query_len, int Hq, int D, int page, int splits, int max_blocks);
 int da_attn_both(const void* q, int q_ld, const void* cache, const int* block_table, int max_blocks, const int* q_start, const int* seq_lens,
                  int n_decode, int n_portions, int max_query_len, int Hq, int Hkv, int D, int page, float scale, int window, void* out,
                  int out_ld, void* stream);
@@ -99,7 +99,7 @@ extern "C" int da_run_step(const DaModel* model, const DaStep* step) {
                           L.write ? kv_cols : 0, L.write ? L.n_kv_heads : 0, L.write ? D : 0, L.write ? m.page : 0));
     // attention: one-token sequences and portions in one launch, or the one and then the other
     const int splits = st.n_decode > 0 ? da_decode_splits(st.n_decode, L.n_heads, st.max_blocks[g], m.page) : 1;
-    const bool both = da_attn_both_takes(st.n_decode, st.S - st.n_decode, st.max_query_len, L.n_heads, D, m.page, splits);
+    const bool both = da_attn_both_pays(st.n_decode, st.S - st.n_decode, st.max_query_len, L.n_heads, D, m.page, splits, st.max_blocks[g]);
     if (both)
       DA_TRY(da_attn_both(st.qkv, qkv_cols, L.kv_cache, st.block_table[g], st.max_blocks[g], st.q_start, st.seq_lens, st.n_decode,
                           st.S - st.n_decode, st.max_query_len, L.n_heads, L.n_kv_heads, D, m.page, L.scale, L.window, st.attn_out, q_cols, st.stream));

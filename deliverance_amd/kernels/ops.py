@@ -94,6 +94,7 @@ _ARGTYPES = {
     "da_attn_f32": [_VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
     "da_attn_decode": [_VP, _I, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
     "da_attn_both_takes": [_I, _I, _I, _I, _I, _I, _I],
+    "da_attn_both_pays": [_I, _I, _I, _I, _I, _I, _I, _I],
     "da_attn_both": [_VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _VP],
     "da_attn_decode_split": [_VP, _I, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _I, _VP, ctypes.c_long, _VP],
     "da_attn_prefill": [_VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _F, _I, _VP, _I, _I, _VP],
@@ -1247,7 +1248,7 @@ def paged_attention(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: int, 
 
     if _MODE == "tuned" and q.dtype == torch.bfloat16 and D % 16 == 0 and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0:
         n_splits = decode_splits(nd, n_heads, bt.shape[1], page) if nd else 1
-        if nd and _lib().da_attn_both_takes(nd, ctx.n_seqs - nd, ctx.max_query_len, n_heads, D, page, n_splits):
+        if nd and _lib().da_attn_both_pays(nd, ctx.n_seqs - nd, ctx.max_query_len, n_heads, D, page, n_splits, bt.shape[1]):
             with _timed("attention_both", *cost(0, ctx.n_seqs)):
                 return attention_both(q, cache_slot, bt, ctx.q_start, ctx.seq_lens, nd, ctx.n_seqs - nd, ctx.max_query_len, n_heads, scale, window, out)
         if nd:

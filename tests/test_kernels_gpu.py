@@ -873,6 +873,17 @@ def test_when_attention_goes_in_one_launch(ops):
         assert not takes(*a), a
 
 
+def test_when_one_launch_is_ahead_of_two(ops):
+    """The rule's lines: pairs of one-token rows, few rows beside them, keys in front of a short portion; never what the kernel
+    does not take."""
+    pays = ops._lib().da_attn_both_pays
+    for a in ((40, 1, 512, 16, 64, 16, 1, 38), (64, 1, 2, 16, 64, 16, 1, 96), (100, 1, 16, 16, 64, 16, 1, 96), (63, 1, 512, 25, 64, 16, 1, 200), (1, 1, 65, 12, 64, 16, 1, 500), (30, 1, 64, 12, 64, 16, 1, 120)):
+        assert pays(*a), a
+    for a in ((65, 1, 15, 16, 64, 16, 1, 38), (65, 1, 16, 16, 64, 16, 1, 16), (128, 4, 512, 12, 64, 16, 1, 38), (101, 1, 512, 16, 64, 16, 1, 38), (255, 1, 64, 12, 64, 16, 1, 38), (30, 1, 64, 12, 64, 16, 1, 121), (30, 8, 2, 12, 64, 64, 1, 31),
+              (0, 1, 512, 16, 64, 16, 1, 38), (4, 1, 512, 16, 48, 16, 1, 38), (4, 1, 512, 16, 64, 16, 2, 38)):
+        assert not pays(*a), a
+
+
 @pytest.mark.simt_quick
 @pytest.mark.parametrize("form", [41, 42, 22, 14])
 def test_attention_prefill_finds_a_far_key_in_every_phase(ops, form):

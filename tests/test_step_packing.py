@@ -153,7 +153,7 @@ def native_step(monkeypatch, tmp_path, **rules):
     from deliverance_amd.kernels import ops
     from deliverance_amd.models.causal_lm import load_model
     from deliverance_amd.parts.base import Arena, StepContext
-    monkeypatch.setattr(ops, "_lib", lambda: SimpleNamespace(da_run_step=lambda *a: 0, da_attn_both_takes=lambda *a: 0))
+    monkeypatch.setattr(ops, "_lib", lambda: SimpleNamespace(da_run_step=lambda *a: 0, da_attn_both_pays=lambda *a: 0))
     monkeypatch.setattr(ops, "_stream", lambda: 0)
     for name, rule in rules.items():
         monkeypatch.setattr(ops, name, rule)
