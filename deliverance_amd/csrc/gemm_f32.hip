@@ -14,16 +14,16 @@
 //
 //  * gemm_f32_rows: few rows.  A workgroup owns 4, 8 or 16 rows and as many columns as give every compute unit one workgroup (16 at
 //    most); its wavefronts take whole chunks, from memory through their own pieces of LDS into fragments, and the chunks' sums are
-//    added through LDS.  Bound by the bytes of w.  gemm_f32_rows16: straight into fragments, where that is ahead.
+//    added through LDS.  Bound by the bytes of w.
+//  * gemm_f32_rows_direct: few rows, from memory straight into fragments; where that is ahead (f32_rows_staged).
 //  * gemm_f32_tile: block tiles of 64 x 64 or 32 x 32 through two LDS buffers, slabs of 32 k, the next four slabs in flight
 //    in registers.  Bound by the matrix cores (157 TFLOP/s in 32-bit) where the tiles fill the chip several times over:
 //    1,000 x 50,257 x 768 in 687 us, 72 % of that rate; below, by the latency of a slab, which small tiles, several of
 //    them on a compute unit, hide better than large ones (526 x 3,072 x 768: 32 x 32 31 us, 64 x 64 34, 128 x 128 72).
 //
-// Measured on MI355X with cold weights, us (before: 16 rows and 16, 8 or 4 columns a workgroup, fragments straight from memory, a
-// chunk a product): 4 rows, K x N 768 x 768 4.5 -> 3.8, 768 x 2,304 5.3 -> 4.7, 768 x 3,072 5.6 -> 5.2, 3,072 x 768 10.8 -> 6.1,
+// Measured on MI355X with cold weights, us, gemm_f32_rows_direct -> gemm_f32_rows: 4 rows, K x N 768 x 768 4.5 -> 3.8, 768 x 2,304 5.3 -> 4.7, 768 x 3,072 5.6 -> 5.2, 3,072 x 768 10.8 -> 6.1,
 // 768 x 50,257 39.9 -> 32.1; 8 rows, 3,072 x 768 12.0 -> 7.7; 16 rows 13.8 -> 9.6; 64 rows 14.3 -> 11.4; 32 rows, 768 x 3,072 8.7 -> 7.9.
-// Tiles: 526 x 768 x 3,072 38, 526 x 2,304 x 768 27, 526 x 50,257 x 768 440.
+// Tiles: 526 x 768 x 3,072 38, 526 x 2,304 x 768 27, 526 x 50,257 x 768 392.
 #include "gemm_common.h"
 #include <type_traits>
 
@@ -165,24 +165,25 @@ gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restri
 }
 
 // ---------------------------------------------------------------------------------------------
-// Up to 16 rows, and either one chunk or 257 to 640 groups of 16 columns: the same products from fragments that come straight from memory (16 rows x
-// 64 bytes a load), a chunk a wavefront.  The loads are half cache lines, but a product starts with its first fragment, and with two
-// workgroups on most compute units that is ahead: K = 768, N = 8,192 4 rows 7.7 us against 8.8, 8 rows 8.5 against 9.6, 16 rows 9.9
-// against 9.4; N = 12,288 4 rows 12.6 against 11.3, N = 2,304 5.3 against 4.7; K = 64, N = 2,304 2.6 against 3.0.
+// Few rows, fragments straight from memory (16 rows x 64 bytes a load), a chunk a wavefront: 16 rows and 16, 8 or 4 columns a
+// workgroup (the fewer, the fewer the products of 16 x 16 are; a fragment of w then holds its columns several times and the copies'
+// results are dropped).  The loads are half cache lines, but a product starts with its first fragment, nothing waits for LDS, and
+// four to twelve wavefronts that need little of it leave room for other workgroups.  Bound by the latency of its few loads at short
+// k, else by half lines.
 // ---------------------------------------------------------------------------------------------
-template <int NW, int CAP>
+template <int COLS, int NW, int CAP>
 __global__ void __launch_bounds__(NW * 64)
-gemm_f32_rows16_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w, int ldw, Epilogue ep, KvScatter kv,
-                     int M, int N, int K, int n_chunks) {
-  __shared__ float gf_red[CAP * 16 * 17];                      // [n_chunks][16][COLS + 1]
+gemm_f32_rows_direct_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w, int ldw, Epilogue ep, KvScatter kv,
+                            int M, int N, int K, int n_chunks) {
+  __shared__ float gf_red[CAP * 16 * (COLS + 1)];               // [n_chunks][16][COLS + 1]
   const int t = threadIdx.x, lane = t % 64, wave = t / 64;
-  const int n0 = blockIdx.x * 16, r0 = blockIdx.y * 16;
+  const int n0 = blockIdx.x * COLS, r0 = blockIdx.y * 16;
   const int fr = lane % 16, kq = (lane / 16) * 4;
   const float* pa = a + (size_t)(r0 + fr < M ? r0 + fr : r0) * lda;
-  const float* pw = w + (size_t)(n0 + fr < N ? n0 + fr : n0) * ldw;
+  const float* pw = w + (size_t)(n0 + fr % COLS < N ? n0 + fr % COLS : n0) * ldw;
   // what the epilogue needs is asked for first, from places that always exist
-  const int em = r0 + t / 16, en = n0 + t % 16;
-  const bool e_ok = t < 256 && em < M && en < N;
+  const int em = r0 + t / COLS, en = n0 + t % COLS;
+  const bool e_ok = t < 16 * COLS && em < M && en < N;
   const float e_bias_raw = (e_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, en) : 0.f;
   const float e_old = *((e_ok && ep.accumulate) ? (const float*)ep.out + (size_t)em * ep.ldo + en : w);
   const int e_slot = *((e_ok && kv.cache) ? kv.slot_map + em : (const int*)w);
@@ -202,8 +203,10 @@ gemm_f32_rows16_kernel(const float* __restrict__ a, int lda, const float* __rest
       if (CUT && c * GF_CHUNK + g * 16 + kq >= K) av[g] = wv[g] = make_float4(0.f, 0.f, 0.f, 0.f);
       part = gf_group(av[g], wv[g], part);
     }
+    if (COLS == 16 || fr < COLS) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) gf_red[(c * 16 + 4 * (lane / 16) + r) * 17 + fr] = part[r];
+      for (int r = 0; r < 4; ++r) gf_red[(c * 16 + 4 * (lane / 16) + r) * (COLS + 1) + fr] = part[r];
+    }
   };
   const int whole = K / GF_CHUNK;
   for (int c = wave; c < n_chunks; c += NW) {
@@ -212,10 +215,10 @@ gemm_f32_rows16_kernel(const float* __restrict__ a, int lda, const float* __rest
   }
   lds_barrier();
   if (!e_ok) return;
-  const float* mine = gf_red + (t / 16) * 17 + t % 16;
+  const float* mine = gf_red + (t / COLS) * (COLS + 1) + t % COLS;
   float v = mine[0];
 #pragma unroll 4
-  for (int c = 1; c < n_chunks; ++c) v += mine[c * 16 * 17];
+  for (int c = 1; c < n_chunks; ++c) v += mine[c * 16 * (COLS + 1)];
   v = apply_act(v + e_bias_raw, ep.act);
   float* o = (float*)ep.out + (size_t)em * ep.ldo + en;
   *o = ep.accumulate ? e_old + v : v;
@@ -393,16 +396,19 @@ static void launch_f32_rows(hipStream_t s, const float* a, int lda, const float*
   hipLaunchKernelGGL((gemm_f32_rows_kernel<WL, AL, NW, CAP>), dim3(da_ceil_div(N, cols), da_ceil_div(M, 4 * AL)), dim3(NW * 64), 0, s, a, lda,
                      w, ldw, ep, kv, M, N, K, da_ceil_div(K, GF_CHUNK), cols);
 }
-// The wavefronts and the room for partial sums, by K.  More workgroups than compute units: few wavefronts each, so that several
-// workgroups share a compute unit's LDS and one's loads run beside another's products (K = 768, N = 50,257: 4 rows 32 us with 3
-// wavefronts, 45 with 6; 8 rows 38 / 51; 32 rows, N = 3,072 7.9 with 4, 8.8 with 6).
+// The wavefronts and the room for partial sums, by K.  More workgroups than compute units (16 columns each, then): few wavefronts
+// each, so that several workgroups share a compute unit's LDS and one's loads run beside another's products (K = 768, N = 50,257: 4 rows
+// 32 us with 3 wavefronts, 45 with 6; 8 rows 38 / 51; 32 rows, N = 3,072 7.9 with 4, 8.8 with 6).
 template <int WL, int AL>
 static void launch_f32_rows_k(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
                               int M, int N, int K, int cols) {
-  const bool many = (long)da_ceil_div(N, cols) * da_ceil_div(M, 4 * AL) > 256;
-  if (many && AL == 4 && K <= 8 * GF_CHUNK) launch_f32_rows<WL, AL, 4, 8>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
-  else if (many && AL < 4 && K <= 24 * GF_CHUNK) launch_f32_rows<WL, AL, AL == 4 ? 4 : 3, 24>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
-  else if (K <= 6 * GF_CHUNK) launch_f32_rows<WL, AL, 6, 6>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+  if constexpr (WL == 4) {
+    if ((long)da_ceil_div(N, cols) * da_ceil_div(M, 4 * AL) > 256 && K <= (AL == 4 ? 8 : 24) * GF_CHUNK) {
+      launch_f32_rows<WL, AL, AL == 4 ? 4 : 3, AL == 4 ? 8 : 24>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+      return;
+    }
+  }
+  if (K <= 6 * GF_CHUNK) launch_f32_rows<WL, AL, 6, 6>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
   else if (K <= 24 * GF_CHUNK) launch_f32_rows<WL, AL, 8, 24>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
   else launch_f32_rows<WL, AL, AL == 4 ? 6 : 8, GF_ROWS_CAP>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
 }
@@ -415,20 +421,74 @@ static void launch_f32_rows_n(hipStream_t s, const float* a, int lda, const floa
   else launch_f32_rows_k<4, AL>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
 }
 
-enum { GF_AUTO = 0, GF_ROWS, GF_64x64, GF_32x32, GF_LAST = GF_32x32 };
+template <int COLS, int NW, int CAP>
+static void launch_f32_rows_direct_k(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
+                                     int M, int N, int K) {
+  hipLaunchKernelGGL((gemm_f32_rows_direct_kernel<COLS, NW, CAP>), dim3(da_ceil_div(N, COLS), da_ceil_div(M, 16)), dim3(NW * 64), 0, s, a,
+                     lda, w, ldw, ep, kv, M, N, K, da_ceil_div(K, GF_CHUNK));
+}
+template <int COLS>
+static void launch_f32_rows_direct(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
+                                   int M, int N, int K) {
+  if (K <= 4 * GF_CHUNK) launch_f32_rows_direct_k<COLS, 4, 4>(s, a, lda, w, ldw, ep, kv, M, N, K);
+  else if (K <= 8 * GF_CHUNK) launch_f32_rows_direct_k<COLS, 8, 8>(s, a, lda, w, ldw, ep, kv, M, N, K);
+  else if (K <= 24 * GF_CHUNK) launch_f32_rows_direct_k<COLS, 12, 24>(s, a, lda, w, ldw, ep, kv, M, N, K);
+  else launch_f32_rows_direct_k<COLS, 12, GF_ROWS_CAP>(s, a, lda, w, ldw, ep, kv, M, N, K);
+}
+
+enum { GF_AUTO = 0, GF_ROWS, GF_64x64, GF_32x32, GF_ROWS_DIRECT, GF_ROWS_STAGED, GF_LAST = GF_ROWS_STAGED };
 
 // Which kernel a product goes to.  Measured on MI355X with K from 768 to 4,096:
-//  - the kernel for few rows up to 8 rows (768 x 50,257: 4 rows 32 us against 38 in tiles of 32 x 32, 8 rows 38.1 against 38.4, 16
+//  - the kernel for few rows up to 8 rows (768 x 50,257: 4 rows 31 us against 38 in tiles of 32 x 32, 8 rows 38.1 against 38.4, 16
 //    rows 46 against 38) and where its products of 16 x 16 are at most 512 (100 x 768 x 768 6.8 us against 9.8, 64 x 768 x 3,072
 //    11.4 against 27, 32 x 3,072 x 768 7.9 against 10.9; with 528 of them, 170 x 768 x 768, 10.9 against 9.7);
 //  - else tiles of 64 x 64 where there are 700 and more, counting what M and N waste of them (1,000 x 3,072 x 768 47 against
-//    51 us, 526 x 50,257 x 768 384 against 401, but 200 x 50,257 x 768 183 against 167);
+//    51 us, 526 x 50,257 x 768 392 against 400, but 200 x 50,257 x 768 183 against 167);
 //  - else tiles of 32 x 32 (526 x 3,072 x 768, 432 of the larger tiles: 31 against 34 us).
 static int f32_form(int M, int N, int K) {
   if (K <= GF_ROWS_MAX_K && (M <= 8 || (long)da_ceil_div(M, 16) * da_ceil_div(N, 16) <= 512)) return GF_ROWS;
   const long large = (long)da_ceil_div(M, 64) * da_ceil_div(N, 64), small = (long)da_ceil_div(M, 32) * da_ceil_div(N, 32);
   return large >= 700 && large * 40 <= small * 11 ? GF_64x64 : GF_32x32;      // (a small tile's share of the chip costs 10 % more)
 }
+
+// Which of the two kernels for few rows.  The staged one reads whole lines, and below about 208 products of 16 x 16 its columns are
+// divided so that every compute unit has a workgroup; the direct one has the shorter chain, and more workgroups a compute unit.
+// Measured over 7,190 sizes (K 256 to 6,400, N 64 to 50,257, M 1 to 256, cold weights), the rule takes 0.892 of the direct kernel's time in
+// the mean, the better of the two 0.885; what it takes is at most 12 % (0.8 us) behind the direct kernel.  us, direct / staged:
+//  - up to 3 chunks of k: direct (K = 256: 4 x 512 2.8 / 3.4, 8 x 9,216 5.4 / 6.1; K = 384: 8 x 11,264 6.2 / 7.3);
+//  - 25 rows and more: staged (K = 768: 100 x 768 7.7 / 6.6; K = 3,072: 48 x 2,304 26 / 22), but for 33 to 40 rows, whose last 16 are mostly
+//    padding, with 9 to 13 chunks (wavefronts of the staged kernel left over) and up to 400 products (K = 1,152: 33 x 2,048 9.7 / 10.9);
+//  - 17 to 24 rows: staged up to 256 products (K = 3,072: 17 x 1,920 13.6 / 12.1), direct above (17 x 2,304 17.0 / 19.8);
+//  - up to 16 rows and 208 products: staged (4 rows, K = 768 x 768 4.4 / 3.6; K = 4,096 x 1,024 13.3 / 6.6), but direct up to 12 rows with 9 to 13
+//    chunks and more than 128 products (K = 1,152, 4 x 3,072 6.0 / 6.5);
+//  - up to 16 rows and more products: a second round of workgroups begins.  13 to 16 rows: staged from 14 chunks on (K = 5,120, 16 x 4,800
+//    48 / 37; K = 1,152 16 x 6,144 12.1 / 13.4).  Up to 12 rows: staged from 40 chunks on (K = 6,400, 8 x 6,144 46.7 / 42.7), and up to 8 rows with 4
+//    or 14 to 16 chunks and up to 256 products, with 14 to 20 chunks (K = 1,920, 8 x 5,120 17.4 / 14.0), and for vocabularies (K = 768, 4 x 50,257
+//    39 / 31); else direct (K = 768, 4 x 6,144 6.8 / 7.9; K = 1,024, 4 x 4,100 6.8 / 8.6; K = 4,096, 4 x 8,192 29.8 / 33.9).
+static bool f32_rows_staged(int M, int N, int K) {
+  const int chunks = da_ceil_div(K, GF_CHUNK);
+  const long products = (long)da_ceil_div(M, 16) * da_ceil_div(N, 16);
+  const bool left_over = chunks >= 9 && chunks <= 13;
+  if (chunks <= 3) return false;
+  if (M > 24) return !(left_over && M > 32 && M <= 40 && products > 176 && products <= 400);
+  if (M > 16) return products <= 256;
+  if (products <= 208) return M > 12 || !(left_over && products > 128);
+  if (M > 12) return chunks > 13;
+  if (chunks >= 40) return true;
+  if (M > 8) return false;
+  if (products <= 256) return chunks == 4 || (chunks >= 14 && chunks <= 16);
+  if (chunks >= 14) return chunks <= 20 || (chunks <= 24 && N >= 16384);
+  return N >= (chunks >= 9 ? 16384 : 32000) && chunks >= 5;
+}
+
+// The columns a workgroup of the staged kernel: every compute unit a workgroup, and no second round of them for less than 16
+// columns (48 x 1,024, K = 1,600: 13 columns in 79 x 3 workgroups 8.8 us, 12 in 86 x 3 13.0; direct 8.3).
+static int f32_rows_columns(int M, int N) {
+  const int blocks = da_ceil_div(M, M <= 4 ? 4 : (M <= 8 ? 8 : 16)), share = da_ceil_div(N, blocks < 256 ? 256 / blocks : 1);
+  return share > 16 ? 16 : share;
+}
+// 0 where a product of few rows goes to the direct kernel, else the columns a workgroup of the staged one.
+extern "C" int da_gemm_f32_rows_choice(int M, int N, int K) { return f32_rows_staged(M, N, K) ? f32_rows_columns(M, N) : 0; }
 
 // out (+)= act(a @ w.T + bias).  `form` 0: chosen by the sizes; else that kernel (tests and timing), where it takes them.
 extern "C" int da_gemm_f32(const float* a, int lda, const float* w, int ldw, const void* bias, int bias_dtype, int act, int accumulate,
@@ -440,7 +500,7 @@ extern "C" int da_gemm_f32(const float* a, int lda, const float* w, int ldw, con
   DA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm_f32: leading sizes too small (lda=%d ldw=%d ldo=%d)", lda, ldw, ldo);
   DA_REQUIRE(act >= DA_ACT_NONE && act <= DA_ACT_LAST, "gemm_f32: unknown activation %d", act);
   DA_REQUIRE(form >= GF_AUTO && form <= GF_LAST, "gemm_f32: unknown form %d", form);
-  DA_REQUIRE(form != GF_ROWS || K <= GF_ROWS_MAX_K, "gemm_f32: the kernel for few rows takes K up to %d (K=%d)", GF_ROWS_MAX_K, K);
+  DA_REQUIRE(form == GF_AUTO || form == GF_64x64 || form == GF_32x32 || K <= GF_ROWS_MAX_K, "gemm_f32: the kernel for few rows takes K up to %d (K=%d)", GF_ROWS_MAX_K, K);
   if (kv_cache) {
     DA_REQUIRE(!accumulate && slot_map && q_cols >= 0 && kv_cols == Hkv * D && q_cols + 2 * kv_cols == N && page > 0,
                "gemm_f32: the q|k|v columns (%d + 2*%d) must add up to N=%d", q_cols, kv_cols, N);
@@ -450,22 +510,19 @@ extern "C" int da_gemm_f32(const float* a, int lda, const float* w, int ldw, con
   const KvScatter kv{kv_cache, slot_map, q_cols, kv_cols, Hkv, D, page};
   hipStream_t s = (hipStream_t)stream;
   if (form == GF_AUTO) form = f32_form(M, N, K);
+  if (form == GF_ROWS) form = f32_rows_staged(M, N, K) ? GF_ROWS_STAGED : GF_ROWS_DIRECT;
   switch (form) {
-    case GF_ROWS: {
-      const long groups = da_ceil_div(N, 16);
-      if (M <= 16 && (K <= GF_CHUNK || (groups > 256 && groups <= 640 && K <= 24 * GF_CHUNK))) {
-        const dim3 grid(groups);
-        const int n_chunks = da_ceil_div(K, GF_CHUNK);
-        if (K <= 8 * GF_CHUNK) hipLaunchKernelGGL((gemm_f32_rows16_kernel<8, 8>), grid, dim3(512), 0, s, a, lda, w, ldw, ep, kv, M, N, K, n_chunks);
-        else hipLaunchKernelGGL((gemm_f32_rows16_kernel<12, 24>), grid, dim3(768), 0, s, a, lda, w, ldw, ep, kv, M, N, K, n_chunks);
-        break;
-      }
-      const int rows = M <= 4 ? 4 : (M <= 8 ? 8 : 16);
-      // every compute unit a workgroup, 16 columns at most
-      const long share = ((long)N * da_ceil_div(M, rows) + 255) / 256;
-      const int cols = share > 16 ? 16 : (int)share;
-      if (rows == 4) launch_f32_rows_n<1>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
-      else if (rows == 8) launch_f32_rows_n<2>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+    case GF_ROWS_DIRECT: {
+      const long tiles = (long)da_ceil_div(M, 16) * da_ceil_div(N, 16);
+      if (tiles <= 64) launch_f32_rows_direct<4>(s, a, lda, w, ldw, ep, kv, M, N, K);
+      else if (tiles <= 128) launch_f32_rows_direct<8>(s, a, lda, w, ldw, ep, kv, M, N, K);
+      else launch_f32_rows_direct<16>(s, a, lda, w, ldw, ep, kv, M, N, K);
+      break;
+    }
+    case GF_ROWS_STAGED: {
+      const int cols = f32_rows_columns(M, N);
+      if (M <= 4) launch_f32_rows_n<1>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
+      else if (M <= 8) launch_f32_rows_n<2>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
       else launch_f32_rows_n<4>(s, a, lda, w, ldw, ep, kv, M, N, K, cols);
       break;
     }

@@ -80,6 +80,7 @@ _ARGTYPES = {
     "da_layernorm": [_VP, _VP, _VP, _I, _VP, _I, _F, _VP, _I, _I, _I, _VP],
     "da_gemm_ref": [_VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_f32": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _VP],
+    "da_gemm_f32_rows_choice": [_I, _I, _I],
     "da_gemm_bf16": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_few_rows": [_I, _I],
     "da_gemm_bf16_kv_split": [_VP, _I, _VP, _I, _VP, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
@@ -1033,7 +1034,7 @@ def _f32_ok(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
             and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-F32_FORMS = {"auto": 0, "rows": 1, "64x64": 2, "32x32": 3}
+F32_FORMS = {"auto": 0, "rows": 1, "64x64": 2, "32x32": 3, "rows_direct": 4, "rows_staged": 5}
 
 
 def linear_f32(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,

@@ -249,6 +249,35 @@ def test_gemm_32bit_of_few_rows_by_columns(ops, M, N, K):
     assert torch.equal(rows, ops.linear_f32(a, w, None, torch.empty(M, N, device=DEV), form="32x32"))
 
 
+@pytest.mark.parametrize("M,N,K", [helpers.quick(1, 68, 64), helpers.quick(4, 1030, 132), (5, 1400, 388), helpers.quick(17, 260, 516), (8, 9300, 260), (20, 2100, 1284),
+                                   (33, 1100, 1156), (48, 1024, 772), (100, 260, 3076), (3, 2500, 6400), (12, 4100, 644)])
+def test_gemm_32bit_of_few_rows_both_kernels(ops, M, N, K):
+    """The direct and the staged kernel, 4 to 16 columns a workgroup and K in every set of wavefronts: the bits of the tiles."""
+    helpers.skip_in_simulation_if(M * N * K > 1e7)
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w, b, x = (torch.randn(*s, generator=g).to(DEV) for s in ((M, K), (N, K), (N,), (M, N)))
+    tiles = ops.linear_f32(a, w, b, x.clone(), act="gelu_new", accumulate=True, form="32x32")
+    for form in ("rows_direct", "rows_staged"):
+        assert torch.equal(ops.linear_f32(a, w, b, x.clone(), act="gelu_new", accumulate=True, form=form), tiles), form
+    with pytest.raises(ops.KernelError):
+        ops.linear_f32(torch.zeros(2, 6404, device=DEV), torch.zeros(4, 6404, device=DEV), None, torch.empty(2, 4, device=DEV), form="rows_direct")
+
+
+def test_which_kernel_32bit_products_of_few_rows_take(ops):
+    """The rule's lines, and never a second round of workgroups of the staged kernel for less than 16 columns each."""
+    choice = ops._lib().da_gemm_f32_rows_choice
+    for M, N, K in ((4, 512, 256), (8, 50257, 384), (8, 9216, 512), (4, 6144, 768), (16, 6144, 1152), (4, 3072, 1600), (12, 4100, 2048), (17, 2304, 3072), (33, 2048, 1152),
+                    (8, 16384, 1024), (4, 8192, 4096)):
+        assert choice(M, N, K) == 0, (M, N, K)
+    for M, N, K, cols in ((4, 768, 768, 3), (4, 3072, 768, 12), (4, 50257, 768, 16), (8, 1024, 4096, 4), (16, 4800, 5120, 16), (48, 1024, 1600, 13), (100, 256, 768, 8), (1, 64, 512, 1)):
+        assert choice(M, N, K) == cols, (M, N, K)
+    for M in (1, 4, 5, 8, 9, 16, 17, 33, 48, 64, 100, 256):
+        for N in (1, 64, 250, 256, 770, 1024, 2304, 4096, 50257):
+            cols = choice(M, N, 6400)
+            if 0 < cols < 16:
+                assert -(-N // cols) * -(-M // (4 if M <= 4 else 8 if M <= 8 else 16)) <= 256, (M, N)
+
+
 def test_gemm_32bit_writes_keys_and_values(ops):
     g = torch.Generator().manual_seed(7)
     Hq, Hkv, D, page, K = 5, 3, 20, 16, 132
