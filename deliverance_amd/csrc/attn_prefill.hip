@@ -595,16 +595,17 @@ extern "C" int da_attn_prefill(const void* q, int q_ld, const void* cache, const
   // choice reads the step's shape only.
   // form: 0 leaves the choice to this rule; 41, 42, 22 or 14 fixes it
   const long per128 = (long)da_ceil_div(max_query_len, 128) * Hq * n_seqs;
-  // Up to 64 rows, by the most keys that any sequence has (the block table's width), head size up to 64, us 4x1 / 2x2 / 1x4, 12 heads, 8 and 64
+  // Up to 64 rows, by the most keys that any sequence has (the block table's width), head size 64, us 4x1 / 2x2 / 1x4, 12 heads, 8 and 64
   // rows: 64 keys 4.5 / 6.0 / 9.3 and 4.9 / 6.5 / 10.0 (one tile: there is nothing to share out, and a round that is not whole
   // asks for its tiles the slow way); 128 keys 5.9 / 5.0 / 8.9 and 6.2 / 5.4 / 9.6; 256 7.2 / 6.1 / 6.9 and 7.6 / 6.6 / 9.0; 512 11.0 / 8.4 / 8.7 and
   // 11.4 / 8.9 / 12.3; 1,024 18.8 / 13.0 / 12.3 and 19.2 / 13.6 / 16.0.  So 4 x 1 up to one tile, 1 x 4 for up to 32 rows with
-  // more than 768 keys, else 2 x 2.
+  // more than 768 keys, else 2 x 2.  Head sizes up to 32, with half the work a tile or less: 1 x 4 from more than 384 keys on (head size
+  // 32, 2x2 / 1x4: 320 keys 6.8 / 7.6, 448 7.6 / 7.3, 640 7.8 / 8.5, 704 9.2 / 8.4, 1,024 10.1 / 8.5; 16: 448 7.3 / 6.8; 48: as 64).
   const long keys = (long)max_blocks * page;
 #ifdef PF_REL
   const bool one_tile = false, far = true;          // (measured without a bias only)
 #else
-  const bool one_tile = D <= 64 && keys <= PF_BK, far = keys > 768;
+  const bool one_tile = D <= 64 && keys <= PF_BK, far = keys > (D <= 32 ? 384 : 768);
 #endif
   const int chosen = form ? form
                      : (one_tile && max_query_len <= 64) ? 41

@@ -875,6 +875,16 @@ def test_attention_prefill_of_short_portions_by_their_keys(ops, lens, new):
     assert np.abs(out.double().cpu().numpy() - case.plain(0.1, None)).max() < ATT_TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("lens,new", [([384, 9], [32, 9]), ([385, 30], [32, 2]), helpers.quick([400, 40], [3, 20]), ([700, 400], [16, 16])])
+def test_attention_prefill_of_short_portions_of_small_heads(ops, lens, new):
+    """Likewise at head size 32, whose line lies lower: more than 384 keys have the bits of 1 x 4, fewer those of 2 x 2."""
+    case = PagedCase(lens=lens, new=new, Hq=2, Hkv=1, D=32, page=16, dtype=torch.bfloat16, seed=sum(lens))
+    outs = [ops.attention_prefill(case.qcat, case.cache, case.bt, case.q_start, case.seq_lens, 0, len(lens), max(new), 2, 0.1, None,
+                                  torch.full_like(case.qcat, float("nan")), form=f) for f in (0, 14 if max(lens) > 384 else 22)]
+    assert np.abs(outs[0].double().cpu().numpy() - case.plain(0.1, None)).max() < ATT_TOL[torch.bfloat16]
+    assert torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("Hq,Hkv,page,window,new", [
     helpers.quick(2, 1, 16, None, (1, 1, 1, 2)), (16, 16, 16, None, (1,) * 20 + (260, 129, 3)), (5, 5, 8, 100, (1, 1, 128)),
     (12, 4, 64, None, (1, 33, 64, 65)), helpers.quick(3, 3, 32, 40, (1, 1, 70)), (30, 30, 16, None, (1,) * 9 + (512, 40))])
