@@ -1062,10 +1062,10 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
   return 0;
 }
 
-// How many shares the k of a product into the residual stream is cut into (1: none; da_gemm_bf16 adds into the stream).  With few
+// How many shares the k of a product into the residual stream can be cut into (1: none; da_gemm_bf16 adds into the stream).  With few
 // tiles and a long K most compute units have no tile; cut, share by share, they have one, and what the shares' sums cost is
 // that the norm behind reads them (da_layernorm_join; never a norm that is fused into its product: more rows than
-// da_can_fuse_ln takes).  Whole slabs of 64 k, 512 k a share at least, 8 shares at most.
+// da_can_fuse_ln takes).  Whole slabs of 64 k, 8 shares at most; the last share may be shorter than the others, which have 512 k and more.
 //  - up to 64 rows (32 columns a workgroup, gemm_skinny32), K from 4,096, more than 1,024 columns: us, cold weights, += / shares: 64
 //    rows, N = 1,600, K = 6,400 14.1 / 10.2 (5), 32 rows 11.1 / 8.0, 16 rows 10.3 / 7.9.  Not N = 1,024, K = 4,096: 64 rows 7.4 / 6.5, 48 rows
 //    7.5 / 5.9, but with 8 shares for the norm to read a step of 64 rows takes 1,249 us for 1,232; nor N = 768, K = 3,072 (64 rows 4.9 / 5.5);
@@ -1096,6 +1096,27 @@ static GemmShares gemm_shares(int M, int N, int K) {
   return g;
 }
 extern "C" int da_gemm_shares(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? gemm_shares(M, N, K).shares : 1; }
+
+// How many shares a step cuts it into: as many, where a layer with its norm is faster by them.  Measured as whole steps of 12 layers, us
+// a layer gained (all of K = 4 N but where said):
+//  - up to 64 rows: K = 6,400 16 rows 0.0, 24 and 32 -0.6, 33 0.3, 48 and 64 1.6; K = 5,120 16 rows 0.4, 33 -1.2, 48 -0.1, 49 0.6, 64 1.0 (and,
+//    product and norm alone, N = 2,048, K = 4,096 -0.8 to -1.0 from 24 to 64 rows): from 33 rows with K from 6,144, from 49 with K from 5,120;
+//  - more rows: 2 to 18 up to 840 rows (K = 4,096 0.9 at 400, -0.9 to 1.5 from 552 to 700); above, K = 2,048 -0.4 from 1,100 rows, K = 3,072 -0.6
+//    at 900, -2.5 at 1,100, -2.4 at 1,300, K = 4,096 -1.3 at 900, -1.6 at 1,024, but 5.3 at 1,100, K = 5,120 10 and more.  With a shorter K
+//    (product and norm alone): N = 1,024, K = 2,048 0.5 at 400 rows, -0.6 at 552, -3.7 at 1,024; N = 2,048, K = 4,096 1.6 at 256, -1.1 at 400 (64
+//    tiles), 6.9 at 552 (80).
+extern "C" int da_gemm_step_shares(int M, int N, int K) {
+  const int n = da_gemm_shares(M, N, K);
+  if (n == 1) return 1;
+  bool pays;
+  if (M <= 64) pays = (M > 32 && K >= 6144) || (M > 48 && K >= 5120);
+  else {
+    const bool many = M > 840 && ((N >= 512 && K < 4096) || (N >= 1024 && K < 5120 && M <= 1024));
+    const bool short_k = K < 3 * N && M > 384 && (long)da_ceil_div(M, 128) * da_ceil_div(N, 128) <= 64;
+    pays = !many && !short_k;
+  }
+  return pays ? n : 1;
+}
 
 // partial[s] = a @ w.T over share s of k, [M, N] each, 32-bit; as many shares as da_gemm_shares says (more than one).
 extern "C" int da_gemm_bf16_shares(const void* a, int lda, const void* w, int ldw, float* partial, int M, int N, int K, void* stream) {

@@ -84,7 +84,7 @@ typedef struct {
   float* logits;
   float* decode_partial;       // for decode attention that shares a pair's keys out over workgroups
   long decode_partial_floats;
-  float* proj_partial;         // for feed-forwards whose second product is shared out over k (da_gemm_shares)
+  float* proj_partial;         // for feed-forwards whose second product is shared out over k (da_gemm_step_shares)
   long proj_partial_floats;
   void* stream;
 } DaStep;
@@ -94,8 +94,8 @@ int da_run_step(const DaModel* model, const DaStep* step);
 
 // How many shares decode attention gives a (sequence, head) pair's keys (1: none), from the step's shape only.
 int da_decode_splits(int n_seqs, int n_heads, int max_blocks, int page);
-// How many shares the k of a product of M rows, N columns into the stream is cut into (1: none).
-int da_gemm_shares(int M, int N, int K);
+// How many shares a step cuts the k of a product of M rows, N columns into the stream into (1: none).
+int da_gemm_step_shares(int M, int N, int K);
 // Whether the fused norm + product kernel takes a product of `n_rows` rows, inner size K and N columns.
 int da_can_fuse_ln(int n_rows, int K, int N);
 }

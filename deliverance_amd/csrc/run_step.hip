@@ -126,7 +126,7 @@ extern "C" int da_run_step(const DaModel* model, const DaStep* step) {
       DA_REQUIRE(st.ff_mid, "run_step: the feed-forward's scratch buffer is missing");
       DA_TRY(normed_product(st, x, left, nullptr, N, L.norm2, E, L.fc_w, L.fc_b, L.fc_b_dtype, L.act, st.norm, st.ff_mid, DA_BF16, L.inner, nullptr,
                             nullptr, 0, 0, 0, 0, 0));
-      const int shares = (uintptr_t)L.proj_b % 16 == 0 ? da_gemm_shares(N, E, L.inner) : 1;
+      const int shares = (uintptr_t)L.proj_b % 16 == 0 ? da_gemm_step_shares(N, E, L.inner) : 1;
       if (shares > 1) {
         // few tiles, a long K: the shares' sums join the stream in the norm that reads it next
         DA_REQUIRE(st.proj_partial && st.proj_partial_floats >= (long)shares * N * E, "run_step: the scratch of the feed-forward's second product is too small");

@@ -169,7 +169,7 @@ class NativeStep:
         st.decode_partial_floats = floats
         floats = self._share_floats.get(N)
         if floats is None:
-            floats = self._share_floats[N] = max([s * N * cfg.width for s in (ops.product_shares(N, cfg.width, k) for k in self._inners) if s > 1], default=0)
+            floats = self._share_floats[N] = max([s * N * cfg.width for s in (ops.step_shares(N, cfg.width, k) for k in self._inners) if s > 1], default=0)
         st.proj_partial = ctx.flat("proj_partial", floats, torch.float32).data_ptr() if floats else None
         st.proj_partial_floats = floats
         st.stream = ops._stream()

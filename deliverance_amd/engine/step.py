@@ -158,11 +158,9 @@ class StepRunner:
         self.cache = cache
         self.kernels = kernels                       # "tuned" | "reference" (EngineConfig.kernels)
         # the layer loop in one call into the library, where the model's parts allow it (engine/native_step.py)
-        self.native = None
-        if native_step:
-            from .native_step import NativeStep
-            if NativeStep.takes(model, cache, kernels):
-                self.native = NativeStep(model, cache)
+        from .native_step import NativeStep
+        self.joins_shares = NativeStep.takes(model, cache, kernels)
+        self.native = NativeStep(model, cache) if native_step and self.joins_shares else None
         # hook(layer, stage, tensor) for named intermediates of every step; steps then run kernel by
         # kernel, never from a recorded graph
         self.debug_hook = None
@@ -321,6 +319,7 @@ class StepRunner:
         ctx = StepContext()
         ctx.device = self.device
         ctx.dtype = self.model.dtype
+        ctx.joins_shares = self.joins_shares
         ctx.n_tokens, ctx.n_seqs, ctx.n_decode = N, S, meta["n_decode"]
         ctx.tokens, ctx.positions, ctx.seq_of_token = view("tokens"), view("positions"), view("seq_of")
         ctx.token_src = view("token_src")

@@ -103,6 +103,7 @@ _ARGTYPES = {
     "da_decode_splits": [_I, _I, _I, _I],
     "da_can_fuse_ln": [_I, _I, _I],
     "da_gemm_shares": [_I, _I, _I],
+    "da_gemm_step_shares": [_I, _I, _I],
     "da_gemm_bf16_shares": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP],
     "da_layernorm_join": [_VP, _VP, _VP, ctypes.c_long, _I, _VP, _I, _VP, _I, _VP, _I, _F, _VP, _I, _I, _I, _VP],
     "da_join_rows": [_VP, _VP, ctypes.c_long, _I, _VP, _I, _I, _I, _VP],
@@ -894,8 +895,13 @@ def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
 
 
 def product_shares(M: int, N: int, K: int) -> int:
-    """How many shares the k of a bfloat16 product of M rows into the residual stream is cut into (1: none)."""
+    """How many shares the k of a bfloat16 product of M rows into the residual stream can be cut into (1: none)."""
     return int(_lib().da_gemm_shares(int(M), int(N), int(K)))
+
+
+def step_shares(M: int, N: int, K: int) -> int:
+    """How many shares a step cuts it into: as many where that pays, else 1."""
+    return int(_lib().da_gemm_step_shares(int(M), int(N), int(K)))
 
 
 def shares_ok(a: torch.Tensor, w: torch.Tensor, add: Optional[torch.Tensor]) -> bool:

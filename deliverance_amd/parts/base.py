@@ -123,6 +123,9 @@ class StepContext:
         # False while a part runs that was given a buffer of its own to fill (a norm follows it): a part
         # with ``can_store`` then stores its result there instead of adding to what the buffer holds
         self.part_accumulate = True
+        # True when the model's steps are issued from C++ (engine/native_step.py), whose norms add what a product left share by
+        # share: part by part its steps then make the same sums.  Elsewhere the addition would be a kernel of its own.
+        self.joins_shares = False
         # Called as hook(layer, stage, tensor) with copies of named intermediates (layer -1: the
         # embedding), when set: core/src/main/java/io/teknek/deliverance/model/AbstractModel.java:122-128,505-515.
         self.debug_hook: Optional[Callable] = None

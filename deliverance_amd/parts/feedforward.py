@@ -44,7 +44,9 @@ class DenseFeedForward(FeedForward):
         N = h.shape[0]
         mid = ctx.buf("ff_mid", N, self.inner, ctx.dtype)
         ops.linear(h, self.fc_weight, self.fc_bias, mid, act=self.activation)
-        shares = ops.product_shares(N, self.width, self.inner) if ctx.part_accumulate and ops.shares_ok(mid, self.proj_weight, self.proj_bias) else 1
+        shares = 1
+        if ctx.joins_shares and ctx.part_accumulate and ops.shares_ok(mid, self.proj_weight, self.proj_bias):
+            shares = ops.step_shares(N, self.width, self.inner)
         if shares > 1:          # (the same sums as the step issued from C++, whose norms add them in passing)
             ops.join_rows(x, ops.linear_shares(mid, self.proj_weight, ctx.flat("proj_partial", shares * N * self.width, torch.float32)), self.proj_bias)
         else:

@@ -233,6 +233,15 @@ def test_products_that_are_not_shared_out_are_refused(ops):
         ops.linear_shares(a, w, torch.zeros(100, 1024, device=DEV))
 
 
+def test_which_products_a_step_shares_out(ops):
+    """The rule's lines; never more shares than the product can be cut into."""
+    for M, N, K in ((48, 1600, 6400), (33, 1600, 6400), (64, 1280, 5120), (552, 1024, 4096), (840, 768, 3072), (1100, 1024, 4096), (1024, 1280, 5120), (66, 260, 2112), (552, 2048, 4096)):
+        assert ops.step_shares(M, N, K) == ops.product_shares(M, N, K) > 1, (M, N, K)
+    for M, N, K in ((32, 1600, 6400), (48, 1280, 5120), (64, 2048, 4096), (841, 768, 3072), (1300, 512, 2048), (1024, 1024, 4096), (552, 1024, 2048), (400, 2048, 4096)):
+        assert ops.step_shares(M, N, K) == 1 < ops.product_shares(M, N, K), (M, N, K)
+    assert ops.step_shares(64, 1024, 4096) == ops.step_shares(8, 1600, 6400) == ops.step_shares(1500, 1024, 4096) == 1
+
+
 @pytest.mark.parametrize("M,N,K", [helpers.quick(3, 700, 772), helpers.quick(4, 1030, 132), (2, 250, 6400), (4, 2100, 1284), (1, 13000, 260),
                                    helpers.quick(8, 1100, 388), (5, 2050, 644), (7, 10500, 132), (8, 5000, 3072), (8, 10500, 3076),
                                    helpers.quick(9, 300, 260), (16, 1000, 6400), (33, 3000, 388), (12, 4100, 516), (16, 10240, 1028),

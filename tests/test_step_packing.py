@@ -175,7 +175,7 @@ def test_scratch_of_steps_of_many_sizes_is_one_buffer(monkeypatch, tmp_path):
     order, an engine keeps one buffer of each kind, at most twice the largest need, and a size within the largest one
     allocates nothing."""
     shares = lambda M, N, K: max(1, min(8, 2048 // M)) if M > 8 else 1
-    step, arena, context = native_step(monkeypatch, tmp_path, product_shares=shares)
+    step, arena, context = native_step(monkeypatch, tmp_path, step_shares=shares)
     width = step.model.config.width
     largest = 0
     for N in [int(n) for n in np.random.default_rng(3).permutation(np.arange(1, 1500, 7))]:
@@ -196,7 +196,7 @@ def test_scratch_of_decode_attention_of_many_sizes_is_one_buffer(monkeypatch, tm
     import torch
     from deliverance_amd.kernels import ops
     splits = lambda n_seqs, n_heads, blocks, page: max(1, min(blocks // 4, 512 // (n_seqs * n_heads)))
-    step, arena, context = native_step(monkeypatch, tmp_path, decode_splits=splits, product_shares=lambda *a: 1,
+    step, arena, context = native_step(monkeypatch, tmp_path, decode_splits=splits, step_shares=lambda *a: 1,
                                        attention_decode=lambda *a, **k: None)
     at = step.model.blocks[0].mixer
     cache_slot = step.cache.kv[0]
@@ -214,3 +214,28 @@ def test_scratch_of_decode_attention_of_many_sizes_is_one_buffer(monkeypatch, tm
             largest = max(largest, 4 * ops.decode_workspace_floats(n, at.n_heads, at.head_dim, k))
     count, held = arena_bytes(arena, "decode_partial")
     assert count == 1 and 0 < largest <= held <= 2 * largest
+
+
+@pytest.mark.parametrize("joins", [False, True])
+def test_parts_share_products_out_only_where_norms_add_the_shares(monkeypatch, joins):
+    """A feed-forward's second product adds into the stream in one kernel, unless the model's steps are issued from C++, whose
+    norms add the shares in passing: any other model would pay for a kernel of its own."""
+    import torch
+    from types import SimpleNamespace
+    from deliverance_amd.kernels import ops
+    from deliverance_amd.parts.base import Arena, StepContext
+    from deliverance_amd.parts.feedforward import DenseFeedForward
+    calls = []
+    for name in ("linear", "linear_shares", "join_rows"):
+        monkeypatch.setattr(ops, name, lambda *a, _n=name, **k: calls.append(_n))
+    monkeypatch.setattr(ops, "shares_ok", lambda *a: True)
+    monkeypatch.setattr(ops, "step_shares", lambda M, N, K: 4)
+    monkeypatch.setattr(ops, "product_shares", lambda M, N, K: 4, raising=False)
+    ff = DenseFeedForward(SimpleNamespace(width=16, inner=64, activation="gelu_new", bias=False),
+                          {"fc_weight": torch.zeros(64, 16), "proj_weight": torch.zeros(16, 64)}, torch.bfloat16, "cpu")
+    ctx = StepContext()
+    ctx._arena, ctx.dtype = Arena("cpu"), torch.bfloat16
+    if joins:
+        ctx.joins_shares = True
+    ff.forward(ctx, torch.zeros(100, 16, dtype=torch.bfloat16), torch.zeros(100, 16))
+    assert calls == (["linear", "linear_shares", "join_rows"] if joins else ["linear", "linear"])
