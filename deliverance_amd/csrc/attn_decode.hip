@@ -87,14 +87,10 @@ __device__ __forceinline__ float dec_gate(float z) {
 template <int DK, int DEC_WAVES, bool SPLIT>
 #ifdef DA_ATTN_BODIES
 #define DEC_PAIR dec_pair
-#define DEC_SHARE 0
-#define DEC_SHARES 1
 __device__ __forceinline__ void
 attn_decode_body(int dec_pair,
 #else
 #define DEC_PAIR blockIdx.x
-#define DEC_SHARE (int)blockIdx.y
-#define DEC_SHARES gridDim.y
 // (registers are held to 128 for head sizes up to 64, so that two workgroups share a compute unit)
 __global__ void __launch_bounds__(DEC_WAVES * DA_WAVE, (DK <= 2 || DEC_WAVES == 16) ? 4 : 2)
 DEC_KERNEL(
@@ -130,7 +126,7 @@ DEC_KERNEL(
     const int d = 32 * k + 8 * quad;
     qf[k] = *(const uint4*)(q + (size_t)s * q_ld + h * D + (d < D ? d : 0));
   }
-  const int split0 = SPLIT ? DEC_SHARE * span : 0;          // the first key of this workgroup's share
+  const int split0 = SPLIT ? (int)blockIdx.y * span : 0;          // the first key of this workgroup's share
   const int c0_guess = split0 + wave * DA_WAVE;
   int btk0[4], btv0[2];
 #pragma unroll
@@ -381,7 +377,7 @@ DEC_KERNEL(
   }
   if (SPLIT) {
     // the share's result before the division, its maximum and its sum of weights
-    float* mine = partial + ((size_t)DEC_PAIR * DEC_SHARES + blockIdx.y) * (D + 2);
+    float* mine = partial + ((size_t)DEC_PAIR * gridDim.y + blockIdx.y) * (D + 2);
     for (int d = t; d < D; d += DEC_WAVES * DA_WAVE) {
       float o = 0.f;
 #pragma unroll

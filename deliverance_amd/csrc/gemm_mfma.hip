@@ -400,8 +400,7 @@ gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__
 template <int BM, int BN, int WM, int WN, int PF, int ACT, int OUTMODE>
 __global__ void __launch_bounds__(WM * WN * 64)
 gemm_tile_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                 Epilogue ep, KvScatter kv, int M, int N, int K, int tiles_m, int tiles_n, Grouping gr, int k_share) {
-  gemm_take_share(a, w, ep, M, K, k_share);
+                 Epilogue ep, KvScatter kv, int M, int N, int K, int tiles_m, int tiles_n, Grouping gr) {
   // two buffers of a slab of a and of w; the epilogue parks the tile's results in the same memory
   constexpr int SLAB_BYTES = 2 * (BM + BN) * LDS_LD * (int)sizeof(bf16_t);
   constexpr int OUT_BYTES = tile_out_bytes<BM, BN, OUTMODE>() + tile_slot_bytes<BM, OUTMODE>();
@@ -412,28 +411,27 @@ gemm_tile_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict
 
 template <int BM, int BN, int WM, int WN, int PF, int ACT>
 static void launch_tile_act(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
-                            const KvScatter& kv, int M, int N, int K, const Grouping& gr, int k_share) {
+                            const KvScatter& kv, int M, int N, int K, const Grouping& gr) {
   const int tiles_m = da_ceil_div(M, BM), tiles_n = da_ceil_div(N, BN);
-  const dim3 grid(tiles_m * tiles_n, da_ceil_div(K, k_share)), block(WM * WN * 64);
+  const dim3 grid(tiles_m * tiles_n), block(WM * WN * 64);
   if (ep.accumulate)
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 2>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, k_share);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 2>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr);
   else if (ep.out_dtype == DA_F32)
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 1>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, k_share);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 1>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr);
   else
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 0>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, k_share);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 0>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr);
 }
 
 template <int BM, int BN, int WM, int WN, int PF>
 static void launch_tile(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
-                        const KvScatter& kv, int M, int N, int K, const Grouping& gr = Grouping{nullptr, 0, 0}, int k_share = 0) {
-  if (k_share <= 0) k_share = K;
+                        const KvScatter& kv, int M, int N, int K, const Grouping& gr = Grouping{nullptr, 0, 0}) {
   switch (ep.act) {
-    case DA_ACT_GELU_TANH: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_GELU_TANH>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
-    case DA_ACT_GELU_ERF: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_GELU_ERF>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
-    case DA_ACT_RELU: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_RELU>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
-    case DA_ACT_SILU: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_SILU>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
-    case DA_ACT_RELU2: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_RELU2>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
-    default: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_NONE>(s, A, lda, W, ldw, ep, kv, M, N, K, gr, k_share); break;
+    case DA_ACT_GELU_TANH: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_GELU_TANH>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
+    case DA_ACT_GELU_ERF: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_GELU_ERF>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
+    case DA_ACT_RELU: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_RELU>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
+    case DA_ACT_SILU: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_SILU>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
+    case DA_ACT_RELU2: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_RELU2>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
+    default: launch_tile_act<BM, BN, WM, WN, PF, DA_ACT_NONE>(s, A, lda, W, ldw, ep, kv, M, N, K, gr); break;
   }
 }
 
@@ -651,15 +649,14 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
   const int t = threadIdx.x, lane = t % 64, wave = __builtin_amdgcn_readfirstlane(t / 64);
   const int n0 = blockIdx.x * cols;
   const int n_end = n0 + cols < N ? n0 + cols : N;   // behind the workgroup's last column
-  const int r0 = blockIdx.z * AR;                    // the workgroup's first row
   const int lr = lane / 8, lc = (lane % 8) * 8;      // a load: row lr of 8, 16-byte piece lane % 8
   const int fr = lane % 16, fk = (lane / 16) * 8;    // a fragment: row fr of 16, k-group lane / 16
-  // byte offsets of the lane's rows behind the workgroup's first row of a and of w (64 rows at most: 32 bits hold them)
-  const char* const a0 = (const char*)(a + (size_t)r0 * lda);
+  // byte offsets of the lane's rows behind the first row of a and the workgroup's first of w (64 rows at most: 32 bits hold them)
+  const char* const a0 = (const char*)a;
   const char* const w0 = (const char*)(w + (size_t)n0 * ldw);
   uint32_t oa[AL], ow[WL];
 #pragma unroll
-  for (int i = 0; i < AL; ++i) oa[i] = 2u * (uint32_t)((r0 + i * 8 + lr < M ? i * 8 + lr : 0) * lda);
+  for (int i = 0; i < AL; ++i) oa[i] = 2u * (uint32_t)((i * 8 + lr < M ? i * 8 + lr : 0) * lda);
 #pragma unroll
   for (int i = 0; i < WL; ++i) ow[i] = 2u * (uint32_t)((n0 + i * 8 + lr < n_end ? i * 8 + lr : 0) * ldw);
   // what the epilogue needs is asked for first, as raw bits from places that always exist
@@ -670,7 +667,7 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
   const bool bias_bf16 = ep.bias_dtype == DA_BF16;
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
-    const int e = t + j * NW * 64, m = r0 + e / COLS, n = n0 + e % COLS;
+    const int e = t + j * NW * 64, m = e / COLS, n = n0 + e % COLS;
     const bool ok = e < AR * COLS && m < M && n < n_end;
     const void* bsrc = (ok && ep.bias) ? ep.bias : (const void*)w;
     const int bidx = (ok && ep.bias) ? n : 0;
@@ -742,11 +739,11 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
   lds_barrier();
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
-    const int e = t + j * NW * 64, ml = e / COLS, m = r0 + ml, c = e % COLS, n = n0 + c;
+    const int e = t + j * NW * 64, m = e / COLS, c = e % COLS, n = n0 + c;
     if (e < AR * COLS && m < M && n < n_end) {
-      float v = red[0][ml][c];
+      float v = red[0][m][c];
 #pragma unroll
-      for (int v2 = 1; v2 < NW; ++v2) v += red[v2][ml][c];
+      for (int v2 = 1; v2 < NW; ++v2) v += red[v2][m][c];
       const float e_bias = !ep.bias ? 0.f : (bias_bf16 ? __uint_as_float(e_braw[j] << 16) : __uint_as_float(e_braw[j]));
       v = ep.out_dtype == DA_BF16 ? apply_act_bf16(v + e_bias, ep.act) : apply_act(v + e_bias, ep.act);
       const size_t o = (size_t)m * ep.ldo + n;
