@@ -73,6 +73,24 @@ def test_native_step_with_second_products_shared_out_over_k(tmp_path):
     helpers.check_against_plain(m, native, [reqs[0]], "bfloat16", "shared out over k")
 
 
+def test_native_step_with_few_rows_shared_out_over_k(tmp_path):
+    """Forty requests at a width of 1,600: the second product's shares come from the kernel for few rows, with 32 columns a
+    workgroup, and the next layer's norm and the final norm add them, launched one by one and in a recorded step (of 64)."""
+    from test_engine_paths_gpu import decode_trace
+    cfg = dict(architectures=["GPT2LMHeadModel"], model_type="gpt2", n_layer=2, n_embd=1600, n_head=25, vocab_size=301,
+               n_positions=64, layer_norm_epsilon=1e-5, activation_function="gelu_new", bos_token_id=0, eos_token_id=1)
+    from deliverance_amd.kernels import ops
+    assert ops.step_shares(40, 1600, 6400) > 1 and ops.step_shares(64, 1600, 6400) > 1
+    m = helpers.make_model(tmp_path, cfg, seed=23)
+    reqs = [(f"r{i}", m.prompt(7 + i % 9, salt=300 + i)) for i in range(40)]
+    steps = decode_trace(reqs, [3] * 40)
+    for options in ({}, dict(use_graphs=True, sample=True)):
+        native, parts = both_ways(m, steps, 2048, **options)
+        for rid in native:
+            assert np.array_equal(native[rid], parts[rid]), (rid, options)
+        helpers.check_against_plain(m, native, reqs[:2], "bfloat16", "few rows shared out over k")
+
+
 def test_the_plan_is_made_only_for_what_it_describes(models):
     m = models["A"]
     assert helpers.trace_session(m.folder, "float32", 128).runner.native is None
