@@ -22,6 +22,7 @@
 // row 8 * (r / 4) + 4 * (l / 32) + r % 4, column l % 32.  16x16x32: lane l gives row / column
 // l % 16 and k = 8 * (l / 16) .. +7; it receives rows 4 * (l / 16) + r, r in 0..3, column l % 16.
 #include "gemm_common.h"
+#include "gemm_skinny32.h"
 #include <type_traits>
 
 #define BKT 64               // k per slab
@@ -444,7 +445,6 @@ static void launch_tile(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W
 // straight in fragment order, 16 rows x 64 bytes a load, they pass a compute unit's L1 at a third
 // of the rate, and that rate, not the memory's, bounds a workgroup.)
 // ---------------------------------------------------------------------------------------------
-#define SK_LD (64 + 8)       // padded row of a step in LDS, elements (144 bytes)
 // AL: loads of 8 rows that cover the workgroup's rows of a (1: up to 8 rows; else two a row tile);
 // COLS: 16 output columns a workgroup, or 8 (the fragment of w then holds them twice and half of the
 // result is dropped: with few columns twice the workgroups pull on memory).
@@ -587,174 +587,6 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restri
   }
 }
 
-// ---------------------------------------------------------------------------------------------
-// M <= 64 where 16 columns a workgroup would give more workgroups than the chip has compute units (sk_one_a_unit: which
-// sizes).  A compute unit pulls in 70 GB/s at best, whatever the pattern, so the bytes of the busiest
-// one are what a product of few rows takes: with two workgroups of all rows and 16 columns it pulls the rows of a
-// twice.  Here a workgroup owns all rows (row tiles) and `cols` columns, 32 at most, chosen so that every
-// compute unit has one; the rest is as above, except that P steps are in flight in registers at any time: a step's
-// registers take the step P further on as soon as they are parked.  The same sums in the same order as gemm_skinny with 8
-// wavefronts.
-// Measured on MI355X with cold weights, K = 1,600, N = 4,800 / 6,400 (16 columns -> 19 / 25): 16 rows 7.1 / 6.8 -> 6.4 / 6.8 us,
-// 32 rows 10.0 / 10.4 -> 7.8 / 8.4, 48 rows 11.3 / 13.6 -> 8.6 / 9.3, 64 rows 12.4 / 14.6 -> 10.3 / 10.8.
-// ---------------------------------------------------------------------------------------------
-// What one lane of a wavefront leaves in LDS another lane of it reads: LDS serves a wavefront's instructions in order, so
-// it is the compiler alone that must keep them.
-__device__ __forceinline__ void sk_wave_order() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-// (the vector type of the language: arrays of HIP's uint4, a class, that are only copied stay in memory)
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
-// a step's operands, k in elements (a lane past K reads its rows' first piece)
-template <int AL, int WL>
-__device__ __forceinline__ void sk_fetch(u32x4_t (&av)[AL], u32x4_t (&wv)[WL], const char* a0, const char* w0, const uint32_t (&oa)[AL],
-                                         const uint32_t (&ow)[WL], int k, int K) {
-  const uint32_t ko = k < K ? 2u * (uint32_t)k : 0u;
-#pragma unroll
-  for (int u = 0; u < AL; ++u) av[u] = *(const u32x4_t*)(a0 + (oa[u] + ko));
-#pragma unroll
-  for (int u = 0; u < WL; ++u) wv[u] = *(const u32x4_t*)(w0 + (ow[u] + ko));
-}
-// ... into the wavefront's piece of LDS, zeros where the lane lies past K
-template <int AR, int AL, int WL>
-__device__ __forceinline__ void sk_park(const u32x4_t (&av)[AL], const u32x4_t (&wv)[WL], bf16_t* mine, int lr, int lc, bool past) {
-#pragma unroll
-  for (int u = 0; u < AL; ++u) *(u32x4_t*)&mine[(u * 8 + lr) * SK_LD + lc] = av[u];
-#pragma unroll
-  for (int u = 0; u < WL; ++u) *(u32x4_t*)&mine[(AR + u * 8 + lr) * SK_LD + lc] = wv[u];
-  if (past) {
-    const u32x4_t zero = {0, 0, 0, 0};
-#pragma unroll
-    for (int u = 0; u < AL; ++u) *(u32x4_t*)&mine[(u * 8 + lr) * SK_LD + lc] = zero;
-#pragma unroll
-    for (int u = 0; u < WL; ++u) *(u32x4_t*)&mine[(AR + u * 8 + lr) * SK_LD + lc] = zero;
-  }
-}
-// AL: loads of 8 rows that cover the workgroup's rows of a (1: up to 8 rows; else two a row tile).
-template <int AL, int NW, int P>
-__global__ void __launch_bounds__(NW * 64)
-gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                     Epilogue ep, KvScatter kv, int M, int N, int K, int cols, int k_share) {
-  gemm_take_share(a, w, ep, M, K, k_share);
-  constexpr int COLS = 32, MT = (AL + 1) / 2, WL = COLS / 8;    // row tiles of 16; loads of 8 rows that cover w's columns
-  constexpr int CT = (COLS + 15) / 16;               // column tiles of 16
-  constexpr int AR = MT * 16, TR = AR + COLS;        // rows of a; rows of a step: a's, then w's
-  // the wavefronts' partial sums take the place of the parked steps once all products are done
-  constexpr int STAGE_BYTES = NW * TR * SK_LD * 2, RED_BYTES = NW * AR * (COLS + 1) * 4;
-  __shared__ __attribute__((aligned(16))) char smem[STAGE_BYTES > RED_BYTES ? STAGE_BYTES : RED_BYTES];
-  bf16_t (*stage)[TR * SK_LD] = (bf16_t (*)[TR * SK_LD])smem;
-  float (*red)[AR][COLS + 1] = (float (*)[AR][COLS + 1])smem;
-  const int t = threadIdx.x, lane = t % 64, wave = __builtin_amdgcn_readfirstlane(t / 64);
-  const int n0 = blockIdx.x * cols;
-  const int n_end = n0 + cols < N ? n0 + cols : N;   // behind the workgroup's last column
-  const int lr = lane / 8, lc = (lane % 8) * 8;      // a load: row lr of 8, 16-byte piece lane % 8
-  const int fr = lane % 16, fk = (lane / 16) * 8;    // a fragment: row fr of 16, k-group lane / 16
-  // byte offsets of the lane's rows behind the first row of a and the workgroup's first of w (64 rows at most: 32 bits hold them)
-  const char* const a0 = (const char*)a;
-  const char* const w0 = (const char*)(w + (size_t)n0 * ldw);
-  uint32_t oa[AL], ow[WL];
-#pragma unroll
-  for (int i = 0; i < AL; ++i) oa[i] = 2u * (uint32_t)((i * 8 + lr < M ? i * 8 + lr : 0) * lda);
-#pragma unroll
-  for (int i = 0; i < WL; ++i) ow[i] = 2u * (uint32_t)((n0 + i * 8 + lr < n_end ? i * 8 + lr : 0) * ldw);
-  // what the epilogue needs is asked for first, as raw bits from places that always exist
-  constexpr int EPT = (AR * COLS + NW * 64 - 1) / (NW * 64);
-  uint32_t e_braw[EPT];
-  float e_old[EPT];
-  int e_slot[EPT];
-  const bool bias_bf16 = ep.bias_dtype == DA_BF16;
-#pragma unroll
-  for (int j = 0; j < EPT; ++j) {
-    const int e = t + j * NW * 64, m = e / COLS, n = n0 + e % COLS;
-    const bool ok = e < AR * COLS && m < M && n < n_end;
-    const void* bsrc = (ok && ep.bias) ? ep.bias : (const void*)w;
-    const int bidx = (ok && ep.bias) ? n : 0;
-    e_braw[j] = bias_bf16 ? (uint32_t)((const bf16_t*)bsrc)[bidx] : ((const uint32_t*)bsrc)[bidx];
-    e_old[j] = *((ok && ep.accumulate) ? (const float*)ep.out + (size_t)m * ep.ldo + n : (const float*)w);
-    e_slot[j] = *((ok && kv.cache) ? kv.slot_map + m : (const int*)w);
-  }
-  floatx4 acc[MT][CT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) acc[i][c] = floatx4{0.f, 0.f, 0.f, 0.f};
-  bf16_t* mine = stage[wave];
-  // (With AL == 1 the rows 8..15 of the tile are never parked: whatever LDS holds there gives rows of
-  // the result that are never stored.)
-  // The very last step may be the one that K cuts: lanes past K read the row's first piece instead and park zeros.
-  const int steps = (K + 63) / 64;
-  const int count = wave < steps ? (steps - wave + NW - 1) / NW : 0;
-  u32x4_t av0[AL], wv0[WL], av1[AL], wv1[WL], av2[AL], wv2[WL], av3[AL], wv3[WL];
-  const bool cut = K % 64 != 0;
-#define SK_FETCH(j, i) sk_fetch(av##j, wv##j, a0, w0, oa, ow, (wave + (i) * NW) * 64 + lc, K);
-#define SK_PARK(j, i) sk_park<AR>(av##j, wv##j, mine, lr, lc, cut && (wave + (i) * NW) * 64 + lc >= K);
-  auto products = [&]() {
-    sk_wave_order();
-#pragma unroll
-    for (int c = 0; c < 64; c += 32) {
-      bf16x8_t wf[CT];
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-        wf[ct] = __builtin_bit_cast(bf16x8_t, *(const uint4*)&mine[(AR + ct * 16 + fr) * SK_LD + c + fk]);
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const bf16x8_t af = __builtin_bit_cast(bf16x8_t, *(const uint4*)&mine[(i * 16 + fr) * SK_LD + c + fk]);
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) acc[i][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, wf[ct], acc[i][ct], 0, 0, 0);
-      }
-    }
-    sk_wave_order();
-  };
-#define SK_EACH(DO)                                     \
-  {                                                     \
-    DO(0)                                               \
-    if constexpr (P > 1) DO(1)                          \
-    if constexpr (P > 2) DO(2)                          \
-    if constexpr (P > 3) DO(3)                          \
-  }
-#define SK_FIRST(j) if (j < count) SK_FETCH(j, j)
-#define SK_STEADY(j) { SK_PARK(j, i + j) SK_FETCH(j, i + j + P) products(); }
-#define SK_LAST(j) if (i + j < count) { SK_PARK(j, i + j) if (i + j + P < count) SK_FETCH(j, i + j + P) products(); }
-  static_assert(P >= 1 && P <= 4, "steps in flight");
-  SK_EACH(SK_FIRST)
-  int i = 0;
-  for (; i + 2 * P <= count; i += P) SK_EACH(SK_STEADY)
-  for (; i < count; i += P) SK_EACH(SK_LAST)
-#undef SK_EACH
-#undef SK_FETCH
-#undef SK_PARK
-#undef SK_FIRST
-#undef SK_STEADY
-#undef SK_LAST
-  lds_barrier();
-#pragma unroll
-  for (int i2 = 0; i2 < MT; ++i2)
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        red[wave][i2 * 16 + 4 * (lane / 16) + r][ct * 16 + fr] = acc[i2][ct][r];
-  lds_barrier();
-#pragma unroll
-  for (int j = 0; j < EPT; ++j) {
-    const int e = t + j * NW * 64, m = e / COLS, c = e % COLS, n = n0 + c;
-    if (e < AR * COLS && m < M && n < n_end) {
-      float v = red[0][m][c];
-#pragma unroll
-      for (int v2 = 1; v2 < NW; ++v2) v += red[v2][m][c];
-      const float e_bias = !ep.bias ? 0.f : (bias_bf16 ? __uint_as_float(e_braw[j] << 16) : __uint_as_float(e_braw[j]));
-      v = ep.out_dtype == DA_BF16 ? apply_act_bf16(v + e_bias, ep.act) : apply_act(v + e_bias, ep.act);
-      const size_t o = (size_t)m * ep.ldo + n;
-      if (ep.accumulate) ((float*)ep.out)[o] = e_old[j] + v;
-      else if (ep.out_dtype == DA_BF16) ((bf16_t*)ep.out)[o] = f32_to_bf16(v);
-      else ((float*)ep.out)[o] = v;
-      if (kv.cache && n >= kv.q_cols && e_slot[j] >= 0) kv_scatter_store(kv, e_slot[j], n, v);
-    }
-  }
-}
-
 // Whether a product of few rows goes to gemm_skinny32: more than 4,096 columns (fewer give no compute unit two workgroups of
 // 16) and up to 8,192.  More than 16 rows: always (K from 64 to 8,192: 0.55 to 0.98 of the time of 16 columns a
 // workgroup).  Up to 16 rows the rows are few bytes and two workgroups a compute unit hide more latency than one, so it
@@ -786,7 +618,7 @@ static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* 
   if (NW == 8 && sk_one_a_unit(M, N, K, lda, ldw)) {
     const int cols = da_ceil_div(N, 256);            // every compute unit one workgroup
     const dim3 grid(da_ceil_div(N, cols));
-#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, cols, K)
+#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P, false>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, cols, K)
     // (steps in flight: what the registers of a workgroup that is alone on its compute unit allow)
     if (M <= 8) DA_SK32_GO(1, 4);
     else if (mt == 1) DA_SK32_GO(2, 4);
@@ -1056,88 +888,6 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
     else launch_tile<64, 64, 2, 2, 4>(s, A, lda, W, ldw, ep, kv, M, N, K);
   }
   DA_CHECK_LAUNCH("gemm_bf16");
-  return 0;
-}
-
-// How many shares the k of a product into the residual stream can be cut into (1: none; da_gemm_bf16 adds into the stream).  With few
-// tiles and a long K most compute units have no tile; cut, share by share, they have one, and what the shares' sums cost is
-// that the norm behind reads them (da_layernorm_join; never a norm that is fused into its product: more rows than
-// da_can_fuse_ln takes).  Whole slabs of 64 k, 8 shares at most; the last share may be shorter than the others, which have 512 k and more.
-//  - up to 64 rows (32 columns a workgroup, gemm_skinny32), K from 4,096, more than 1,024 columns: us, cold weights, += / shares: 64
-//    rows, N = 1,600, K = 6,400 14.1 / 10.2 (5), 32 rows 11.1 / 8.0, 16 rows 10.3 / 7.9.  Not N = 1,024, K = 4,096: 64 rows 7.4 / 6.5, 48 rows
-//    7.5 / 5.9, but with 8 shares for the norm to read a step of 64 rows takes 1,249 us for 1,232; nor N = 768, K = 3,072 (64 rows 4.9 / 5.5);
-//  - more rows: tiles of 128 x 128 where they are at most 85, as many shares as bring them to about 256 (552 rows, N = 1,024,
-//    K = 4,096 20.1 / 12.2 (6)).  K from 2,048.  (K = 1,024: 552 rows 7.5 / 6.5, which the norm's reads take up; so do they
-//    with two shares of more rows: 1,624 rows, K = 4,096 29.7 / 23.9, a step of them 2,834 / 2,841.)
-struct GemmShares { int shares, k_share, shape; };     // shape: DA_WIDE_..., or DA_WIDE_NONE for gemm_skinny32
-static GemmShares gemm_shares(int M, int N, int K) {
-  const GemmShares none{1, K, DA_WIDE_NONE};
-  if (M <= 8 || (M <= 64 && N <= 1024) || N % 4 || K % 64 || N > 2048) return none;
-  GemmShares g = none;
-  long tiles;
-  if (M <= 64) {
-    if (K < 4096) return none;
-    tiles = da_ceil_div(N, 32);
-  } else {
-    if (K < 2048) return none;
-    tiles = (long)da_ceil_div(M, 128) * da_ceil_div(N, 128);
-    if (tiles > 85) return none;
-    g.shape = DA_WIDE_128x128;
-  }
-  long n = 256 / tiles;
-  if (n > K / 512) n = K / 512;
-  if (n > 8) n = 8;
-  if (n < 2) return none;
-  g.k_share = da_ceil_div(K / 64, n) * 64;
-  g.shares = da_ceil_div(K, g.k_share);
-  return g;
-}
-extern "C" int da_gemm_shares(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? gemm_shares(M, N, K).shares : 1; }
-
-// How many shares a step cuts it into: as many, where a layer with its norm is faster by them.  Measured as whole steps of 12 layers, us
-// a layer gained (all of K = 4 N but where said):
-//  - up to 64 rows: K = 6,400 16 rows 0.0, 24 and 32 -0.6, 33 0.3, 48 and 64 1.6; K = 5,120 16 rows 0.4, 33 -1.2, 48 -0.1, 49 0.6, 64 1.0 (and,
-//    product and norm alone, N = 2,048, K = 4,096 -0.8 to -1.0 from 24 to 64 rows): from 33 rows with K from 6,144, from 49 with K from 5,120;
-//  - more rows: 2 to 18 up to 840 rows (K = 4,096 0.9 at 400, -0.9 to 1.5 from 552 to 700); above, K = 2,048 -0.4 from 1,100 rows, K = 3,072 -0.6
-//    at 900, -2.5 at 1,100, -2.4 at 1,300, K = 4,096 -1.3 at 900, -1.6 at 1,024, but 5.3 at 1,100, K = 5,120 10 and more.  With a shorter K
-//    (product and norm alone): N = 1,024, K = 2,048 0.5 at 400 rows, -0.6 at 552, -3.7 at 1,024; N = 2,048, K = 4,096 1.6 at 256, -1.1 at 400 (64
-//    tiles), 6.9 at 552 (80).
-extern "C" int da_gemm_step_shares(int M, int N, int K) {
-  const int n = da_gemm_shares(M, N, K);
-  if (n == 1) return 1;
-  bool pays;
-  if (M <= 64) pays = (M > 32 && K >= 6144) || (M > 48 && K >= 5120);
-  else {
-    const bool many = M > 840 && ((N >= 512 && K < 4096) || (N >= 1024 && K < 5120 && M <= 1024));
-    const bool short_k = K < 3 * N && M > 384 && (long)da_ceil_div(M, 128) * da_ceil_div(N, 128) <= 64;
-    pays = !many && !short_k;
-  }
-  return pays ? n : 1;
-}
-
-// partial[s] = a @ w.T over share s of k, [M, N] each, 32-bit; as many shares as da_gemm_shares says (more than one).
-extern "C" int da_gemm_bf16_shares(const void* a, int lda, const void* w, int ldw, float* partial, int M, int N, int K, void* stream) {
-  if (gemm_bf16_checks(a, lda, w, ldw, DA_ACT_NONE, 0, DA_F32, N, M, N, K)) return 1;
-  if (M == 0) return 0;
-  const GemmShares g = gemm_shares(M, N, K);
-  DA_REQUIRE(g.shares > 1, "gemm_bf16_shares: a product of %d rows, N=%d, K=%d is not shared out", M, N, K);
-  DA_REQUIRE(partial && (uintptr_t)partial % 16 == 0, "gemm_bf16_shares: the sums' place must be 16-byte aligned");
-  const Epilogue ep{nullptr, 0, DA_ACT_NONE, 0, partial, DA_F32, N};
-  const KvScatter kv{nullptr, nullptr, 0, 0, 0, 0, 0};
-  hipStream_t s = (hipStream_t)stream;
-  const bf16_t *A = (const bf16_t*)a, *W = (const bf16_t*)w;
-  if (g.shape != DA_WIDE_NONE) da_gemm_wide_launch(s, A, lda, W, ldw, ep, kv, M, N, K, g.shape, g.k_share);
-  else {
-    DA_REQUIRE(lda <= (1 << 24) && ldw <= (1 << 24), "gemm_bf16_shares: rows lie too far apart (lda=%d ldw=%d)", lda, ldw);
-    const dim3 grid(da_ceil_div(N, 32), g.shares);
-#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, 32, g.k_share)
-    if (M <= 16) DA_SK32_GO(2, 4);
-    else if (M <= 32) DA_SK32_GO(4, 3);
-    else if (M <= 48) DA_SK32_GO(6, 2);
-    else DA_SK32_GO(8, 2);
-#undef DA_SK32_GO
-  }
-  DA_CHECK_LAUNCH("gemm_bf16_shares");
   return 0;
 }
 

@@ -41,8 +41,8 @@ EXTRA_FLAGS = {"attn_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 # The unit that holds the error message every entry point may leave; every other unit needs it.
 BASE_UNIT = "rowwise"
 # Units whose functions a unit calls.
-NEEDS = {"gemm_mfma": ("gemm_wide",),
-         "run_step": ("dispatch", "gemm_mfma", "gemm_fused", "attn_decode", "attn_prefill", "attn_both")}
+NEEDS = {"gemm_mfma": ("gemm_wide",), "gemm_shares": ("gemm_wide",),
+         "run_step": ("dispatch", "gemm_mfma", "gemm_shares", "gemm_fused", "attn_decode", "attn_prefill", "attn_both")}
 # Units that are other units' sources compiled with a definition in front, and entry points that are not found by
 # reading their unit's own source.
 INCLUDES = {"attn_decode_rel": ("attn_decode",), "attn_prefill_rel": ("attn_prefill",), "attn_both": ("attn_decode", "attn_prefill")}
