@@ -13,7 +13,8 @@
 // All key and value loads of a chunk are asked for before any is used (for head sizes up to 64; above, the values once
 // the scores are done).  Bound by two trips to memory and D instructions of 32 cycles a chunk.  (Chunks of 64 keys leave most wavefronts
 // of a short context without any and the others a chain twice as long; us, 64 / 32 keys a chunk, 12 heads of 64: 4 sequences of 61
-// keys 7.4 / 5.7, of 200 9.2 / 8.0, 64 of 1,000 91 / 82, two prompts of 300 17.6 / 14.8, of 1,024 85 / 78; 8 heads, 8 of 1,000 keys 21.2 / 21.5.)
+// keys 7.4 / 5.7, of 200 9.2 / 8.0, 64 of 1,000 91 / 82, two prompts of 300 17.6 / 14.8, of 1,024 85 / 78; 8 heads, 8 of 1,000 keys 21.2 / 21.5; 6 heads of 32: a sequence of
+// 61 keys 7.0 / 5.6, of 500 9.7 / 9.8, of 2,000 25.0 / 26.3.  One size for all contexts, so that a row's sums have one order.)
 // Beside the plain kernel (attn_ref.hip), 8 heads, us at head size 64 / 128: a prompt of 1,024 589 -> 29 /
 // 1,172 -> 50, 8 sequences of 1,000 keys 189 -> 21 / 379 -> 38.
 // Formulas: core/src/main/java/io/teknek/deliverance/generator/CausalSelfAttention.java:481-491,512-527.
