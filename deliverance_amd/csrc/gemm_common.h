@@ -17,6 +17,13 @@ struct Epilogue {
   int ldo;
 };
 
+// The products of few rows take pointers and sizes first, as single arguments: the first 14 words are in registers when a wavefront
+// starts (build.py: KERNARG_PRELOAD).  A structure among a kernel's arguments never is, so an Epilogue comes in two parts.
+struct EpilogueRest {
+  int bias_dtype, act, accumulate, out_dtype;
+};
+static inline EpilogueRest epilogue_rest(const Epilogue& ep) { return EpilogueRest{ep.bias_dtype, ep.act, ep.accumulate, ep.out_dtype}; }
+
 __device__ __forceinline__ void epilogue_store(const Epilogue& ep, int m, int n, float v, float bias) {
   v = ep.out_dtype == DA_BF16 ? apply_act_bf16(v + bias, ep.act) : apply_act(v + bias, ep.act);
   const size_t o = (size_t)m * ep.ldo + n;
@@ -56,16 +63,25 @@ __device__ __forceinline__ void kv_scatter_bits(const KvScatter& kv, int pg, int
   else cache[cache_k_row(pg, h, row, kv.Hkv, kv.page, kv.D) + d] = bits;
 }
 
-__device__ __forceinline__ void kv_scatter_store(const KvScatter& kv, int slot, int n, float v) {
-  const int pg = slot / kv.page, row = slot % kv.page;
-  if (kv.Dv == 0) {
-    kv_scatter_bits(kv, pg, row, n, f32_to_bf16(v));
-    return;
-  }
-  bf16_t* base = (bf16_t*)kv.cache + (long long)pg * kv.Hkv * kv.page * (kv.D + kv.Dv);
-  const int c = n - kv.q_cols, cv = c - kv.kv_cols;
-  if (cv < 0) base[((long long)(c / kv.D) * kv.page + row) * kv.D + c % kv.D] = f32_to_bf16(v);
-  else if (cv < kv.Hkv * kv.Dv) base[(long long)kv.Hkv * kv.page * kv.D + (long long)cv * kv.page + row] = f32_to_bf16(v);
+// x / d for numbers that are the same for the whole wavefront's divisor (x >= 0): head and page sizes are nearly always powers of two,
+// and the general division is some forty instructions of a chain that everything waits for.
+__device__ __forceinline__ int div_uniform(int x, int d) { return (d & (d - 1)) == 0 ? x >> (31 - __builtin_clz(d)) : x / d; }
+
+// Where column n of a row goes in its page: entry `at` of the page for the page's first row, `step` entries further for each row
+// behind it (0: the column is not kept).  It needs no row, so kernels work it out while their operands are on the way.
+struct KvColumn {
+  long long at;
+  int step;
+};
+__device__ __forceinline__ KvColumn kv_column(const KvScatter& kv, int n) {
+  const int c = n - kv.q_cols, cv = c - kv.kv_cols, Dv = kv.Dv ? kv.Dv : kv.D;
+  if (c < 0) return KvColumn{0, 0};
+  if (cv < 0) return KvColumn{c + (long long)div_uniform(c, kv.D) * (kv.page - 1) * kv.D, kv.D};
+  return KvColumn{((long long)kv.Hkv * kv.D + cv) * kv.page, cv < kv.Hkv * Dv ? 1 : 0};
+}
+__device__ __forceinline__ void kv_column_store(const KvScatter& kv, const KvColumn& col, int slot, float v) {
+  const int pg = div_uniform(slot, kv.page), row = slot - pg * kv.page;
+  ((bf16_t*)kv.cache)[pg * ((long long)kv.Hkv * kv.page * (kv.D + (kv.Dv ? kv.Dv : kv.D))) + col.at + (long long)row * col.step] = f32_to_bf16(v);
 }
 
 // The values of 32 rows of a product whose k and v columns go to the cache.  Values are dimension-major: 4 rows whose places

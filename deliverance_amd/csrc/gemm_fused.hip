@@ -14,6 +14,7 @@
 // Formulas: core/src/main/java/io/teknek/deliverance/generator/LayerNorm.java:127-150,
 // CausalSelfAttention.java:266-291,315-336, MLPBlock.java:250-292.
 #include "gemm_common.h"
+#include <da_read_arg.h>
 
 #define FZ_COLS 16
 #define FZ_VPL 8          // float4 per lane when a row is held in registers: K <= 2048
@@ -179,7 +180,7 @@ gemm_ln_skinny_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epil
     for (int v2 = 1; v2 < NW; ++v2) v += red[v2][em][ec];
     epilogue_store(ep, em, n, v, e_bias[j]);
     if (kv.cache && n >= kv.q_cols && e_slot[j] >= 0)
-      kv_scatter_store(kv, e_slot[j], n, apply_act_bf16(v + e_bias[j], ep.act));
+      kv_column_store(kv, kv_column(kv, n), e_slot[j], apply_act_bf16(v + e_bias[j], ep.act));
   }
 }
 
@@ -200,10 +201,17 @@ gemm_ln_skinny_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epil
 // where there are more than 256: the launch then takes as many columns (CT 2) as give every compute unit one workgroup, or
 // two.  A compute unit pulls in about 70 GB/s at best, so its bytes are
 // what the kernel takes: rows of w, the rows of x, and gain and bias once a wavefront that has a row.
+// The arguments that the loads need are the first 14 words (build.py: KERNARG_PRELOAD; M and cols, 16 and 32 at most, share one);
+// what the epilogue needs is asked for behind the operands, with the place in the cache of the thread's column.
+struct LnRest {
+  float eps, center, gain_offset;
+};
 template <int RV, bool PBF16, bool TWO_ROWS, int CT = 1>
 __global__ void __launch_bounds__(512)
-gemm_ln_rows_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epilogue ep, KvScatter kv,
-                   int M, int N, int K, int cols) {
+gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, const void* __restrict__ gain, const void* __restrict__ shift,
+                    const bf16_t* __restrict__ w, int ldw, int N, int K, int rows_cols, LnRest lr_, Epilogue ep, KvScatter kv) {
+  const int M = rows_cols & 0xff, cols = rows_cols >> 8;
+  const LnPrologue ln{x, rows, gain, 0, shift, 0, lr_.eps, lr_.center, lr_.gain_offset};
   constexpr int NW = 8, KMAX = RV * 256, ALD = KMAX + 8;      // ALD: padded row of a in LDS, elements
   constexpr int SW = (RV * 4 + NW - 1) / NW;                   // steps a wavefront
   constexpr int RPW = TWO_ROWS ? 2 : 1, AR = RPW * NW;         // rows a wavefront normalises; rows in LDS
@@ -251,14 +259,6 @@ gemm_ln_rows_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epilog
     }
     if (TWO_ROWS && row0 + NW < M) load_row(sv[RPW - 1], row0 + NW);
   }
-  // this thread's output element (16 x COLS of them, a thread one at most), with what its epilogue needs
-  static_assert(16 * COLS <= NW * 64, "an output element a thread");
-  const int em = t / COLS, ec = t % COLS, en = n0 + ec;
-  const bool e_ok = em < 16 && em < M && en < n_end;
-  const void* e_bsrc = ep.bias ? ep.bias : (const void*)w;
-  const int e_slot = kv.cache ? kv.slot_map[e_ok ? em : 0] : -1;
-  const int e_bidx = (ep.bias && e_ok) ? en : 0;
-  const uint32_t e_bias_raw = PBF16 ? (uint32_t)((const bf16_t*)e_bsrc)[e_bidx] : ((const uint32_t*)e_bsrc)[e_bidx];
   uint4 wv[SW][WL];
 #pragma unroll
   for (int u = 0; u < SW; ++u) {
@@ -270,6 +270,18 @@ gemm_ln_rows_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epilog
       wv[u][i] = load16(w + (size_t)(n < n_end ? n : n0) * ldw + kk);
     }
   }
+  // this thread's output element (16 x COLS of them, a thread one at most), with what its epilogue needs
+  static_assert(16 * COLS <= NW * 64, "an output element a thread");
+  const int em = t / COLS, ec = t % COLS, en = n0 + ec;
+  const bool e_ok = em < 16 && em < M && en < n_end;
+  const void* e_bsrc = ep.bias ? ep.bias : (const void*)w;
+  const int e_slot = kv.cache ? kv.slot_map[e_ok ? em : 0] : -1;
+  const int e_bidx = (ep.bias && e_ok) ? en : 0;
+  const uint32_t e_bias_raw = PBF16 ? (uint32_t)((const bf16_t*)e_bsrc)[e_bidx] : ((const uint32_t*)e_bsrc)[e_bidx];
+  da_read_arg(ep.act);
+  da_read_arg(ep.out_dtype);
+  KvColumn e_col;
+  if (kv.cache) e_col = kv_column(kv, en);
   __builtin_amdgcn_sched_barrier(0);                 // the loads stay in this order, ahead of the arithmetic
 
   // ---- statistics and the normalised rows
@@ -360,7 +372,7 @@ gemm_ln_rows_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epilog
     for (int v2 = 1; v2 < NW; ++v2) v += red[v2][em][ec];
     const float e_bias = !ep.bias ? 0.f : (PBF16 ? __uint_as_float(e_bias_raw << 16) : __uint_as_float(e_bias_raw));
     epilogue_store(ep, em, en, v, e_bias);
-    if (kv.cache && en >= kv.q_cols && e_slot >= 0) kv_scatter_store(kv, e_slot, en, apply_act_bf16(v + e_bias, ep.act));
+    if (kv.cache && e_col.step && e_slot >= 0) kv_column_store(kv, e_col, e_slot, apply_act_bf16(v + e_bias, ep.act));
   }
 }
 
@@ -412,9 +424,9 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
   do {                                                                                                            \
     const dim3 g2(da_ceil_div(N, cols));                                                                          \
     if (wide)                                                                                                     \
-      hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO, (TWO && RV > 4 ? 1 : 2)>), g2, dim3(512), 0, s, ln, (const bf16_t*)w, ldw, ep, kv, M, N, K, cols); \
+      hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO, (TWO && RV > 4 ? 1 : 2)>), g2, dim3(512), 0, s, x, rows, g, b, (const bf16_t*)w, ldw, N, K, M | cols << 8, LnRest{eps, center, gain_offset}, ep, kv); \
     else                                                                                                          \
-      hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO>), g2, dim3(512), 0, s, ln, (const bf16_t*)w, ldw, ep, kv, M, N, K, cols); \
+      hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO>), g2, dim3(512), 0, s, x, rows, g, b, (const bf16_t*)w, ldw, N, K, M | cols << 8, LnRest{eps, center, gain_offset}, ep, kv); \
   } while (0)
 #define LAUNCH_LDS_P(RV, PB)                                                                                      \
   do {                                                                                                            \

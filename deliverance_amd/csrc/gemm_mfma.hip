@@ -457,8 +457,8 @@ static void launch_tile(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W
 // result is dropped: with few columns twice the workgroups pull on memory).
 template <int AL, int COLS, int NW, int UNROLL>
 __global__ void __launch_bounds__(NW * 64)
-gemm_skinny_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                   Epilogue ep, KvScatter kv, int M, int N, int K) {
+gemm_skinny_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const void* bias, void* out, int lda, int ldw, int ldo,
+                   int M, int N, int K, EpilogueRest er, KvScatter kv) {
   constexpr int MT = (AL + 1) / 2, WL = COLS / 8;    // row tiles of 16; loads of 8 rows that cover w's columns
   constexpr int AR = MT * 16, TR = AR + COLS;        // rows of a; rows of a step: a's, then w's
   static_assert(COLS == 8 || COLS == 16, "8 or 16 columns a workgroup");
@@ -484,22 +484,28 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restri
     const int n = n0 + i * 8 + lr;
     pw[i] = w + (size_t)(n < N ? n : 0) * ldw + lc;
   }
-  // what the epilogue needs is asked for first, as raw bits from places that always exist
+  // What the epilogue needs is asked for behind the last group of operands, as raw bits from places that always exist: its arguments
+  // lie in other lines than the operands' and are still on the way when those are asked for.
   constexpr int EPT = (AR * COLS + NW * 64 - 1) / (NW * 64);
   uint32_t e_braw[EPT];
   float e_old[EPT];
   int e_slot[EPT];
-  const bool bias_bf16 = ep.bias_dtype == DA_BF16;
+  KvColumn e_col[EPT];
+  auto load_epilogue = [&]() {
+    da_read_arg(er.act);
+    da_read_arg(er.out_dtype);
 #pragma unroll
-  for (int j = 0; j < EPT; ++j) {
-    const int e = t + j * NW * 64, m = r0 + e / COLS, n = n0 + e % COLS;
-    const bool ok = e < AR * COLS && m < M && n < N;
-    const void* bsrc = (ok && ep.bias) ? ep.bias : (const void*)w;
-    const int bidx = (ok && ep.bias) ? n : 0;
-    e_braw[j] = bias_bf16 ? (uint32_t)((const bf16_t*)bsrc)[bidx] : ((const uint32_t*)bsrc)[bidx];
-    e_old[j] = *((ok && ep.accumulate) ? (const float*)ep.out + (size_t)m * ep.ldo + n : (const float*)w);
-    e_slot[j] = *((ok && kv.cache) ? kv.slot_map + m : (const int*)w);
-  }
+    for (int j = 0; j < EPT; ++j) {
+      const int e = t + j * NW * 64, m = r0 + e / COLS, n = n0 + e % COLS;
+      const bool ok = e < AR * COLS && m < M && n < N;
+      const void* bsrc = (ok && bias) ? bias : (const void*)w;
+      const int bidx = (ok && bias) ? n : 0;
+      e_braw[j] = er.bias_dtype == DA_BF16 ? (uint32_t)((const bf16_t*)bsrc)[bidx] : ((const uint32_t*)bsrc)[bidx];
+      e_old[j] = *((ok && er.accumulate) ? (const float*)out + (size_t)m * ldo + n : (const float*)w);
+      e_slot[j] = *((ok && kv.cache) ? kv.slot_map + m : (const int*)w);
+      if (kv.cache) e_col[j] = kv_column(kv, n);
+    }
+  };
   floatx4 acc[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -529,6 +535,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restri
 #pragma unroll
       for (int i = 0; i < WL; ++i) wv[u][i] = load16(pw[i] + kk);
     }
+    if (LAST) load_epilogue();
 #pragma unroll
     for (int u = 0; u < G; ++u) {
 #pragma unroll
@@ -567,7 +574,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restri
     case 3: if (UNROLL >= 3) group(std::integral_constant<int, (UNROLL >= 3 ? 3 : 1)>{}, std::true_type{}); break;
     case 2: if (UNROLL >= 2) group(std::integral_constant<int, (UNROLL >= 2 ? 2 : 1)>{}, std::true_type{}); break;
     case 1: group(std::integral_constant<int, 1>{}, std::true_type{}); break;
-    default: break;
+    default: load_epilogue(); break;
   }
   lds_barrier();
 #pragma unroll
@@ -583,13 +590,13 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restri
       float v = red[0][ml][c];
 #pragma unroll
       for (int v2 = 1; v2 < NW; ++v2) v += red[v2][ml][c];
-      const float e_bias = !ep.bias ? 0.f : (bias_bf16 ? __uint_as_float(e_braw[j] << 16) : __uint_as_float(e_braw[j]));
-      v = ep.out_dtype == DA_BF16 ? apply_act_bf16(v + e_bias, ep.act) : apply_act(v + e_bias, ep.act);
-      const size_t o = (size_t)m * ep.ldo + n;
-      if (ep.accumulate) ((float*)ep.out)[o] = e_old[j] + v;
-      else if (ep.out_dtype == DA_BF16) ((bf16_t*)ep.out)[o] = f32_to_bf16(v);
-      else ((float*)ep.out)[o] = v;
-      if (kv.cache && n >= kv.q_cols && e_slot[j] >= 0) kv_scatter_store(kv, e_slot[j], n, v);
+      const float e_bias = !bias ? 0.f : (er.bias_dtype == DA_BF16 ? __uint_as_float(e_braw[j] << 16) : __uint_as_float(e_braw[j]));
+      v = er.out_dtype == DA_BF16 ? apply_act_bf16(v + e_bias, er.act) : apply_act(v + e_bias, er.act);
+      const size_t o = (size_t)m * ldo + n;
+      if (er.accumulate) ((float*)out)[o] = e_old[j] + v;
+      else if (er.out_dtype == DA_BF16) ((bf16_t*)out)[o] = f32_to_bf16(v);
+      else ((float*)out)[o] = v;
+      if (kv.cache && e_col[j].step && e_slot[j] >= 0) kv_column_store(kv, e_col[j], e_slot[j], v);
     }
   }
 }
@@ -615,7 +622,7 @@ static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* 
                          const Epilogue& ep, const KvScatter& kv, int M, int N, int K) {
   const dim3 block(NW * 64);
   int mt = da_ceil_div(M, 16);
-#define DA_SK_GO(AL, COLS, U) hipLaunchKernelGGL((gemm_skinny_kernel<AL, COLS, NW, U>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K)
+#define DA_SK_GO(AL, COLS, U) hipLaunchKernelGGL((gemm_skinny_kernel<AL, COLS, NW, U>), grid, block, 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv)
   if (mt == 1 && NW != 4 && da_ceil_div(N, 16) < 128) {
     // few columns and one row tile: 8 columns a workgroup
     const dim3 grid(da_ceil_div(N, 8));
@@ -625,7 +632,7 @@ static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* 
   if (NW == 8 && sk_one_a_unit(M, N, K, lda, ldw)) {
     const int cols = da_ceil_div(N, 256);            // every compute unit one workgroup
     const dim3 grid(da_ceil_div(N, cols));
-#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P, false>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, cols, K)
+#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P, false>), grid, dim3(512), 0, s, A, W, ep.out, lda, ldw, ep.ldo, M, N, K, cols, K, ep.bias, epilogue_rest(ep), kv)
     // (steps in flight: what the registers of a workgroup that is alone on its compute unit allow)
     if (M <= 8) DA_SK32_GO(1, 4);
     else if (mt == 1) DA_SK32_GO(2, 4);
@@ -667,8 +674,8 @@ static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* 
 // ---------------------------------------------------------------------------------------------
 template <int NG, int NW, int UNROLL>
 __global__ void __launch_bounds__(NW * 64)
-gemm_skinny4_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                    Epilogue ep, KvScatter kv, int M, int N, int K) {
+gemm_skinny4_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const void* bias, void* out, int lda, int ldw, int ldo,
+                    int M, int N, int K, EpilogueRest er, KvScatter kv) {
   constexpr int MG = 1;                        // row groups of 4 (from 5 rows on gemm_skinny is faster)
   constexpr int ROWS = MG * 4, COLS = NG * 4;
   __shared__ __attribute__((aligned(16))) float red[4 * NW][COLS][ROWS];
@@ -688,19 +695,27 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restr
     const int m = g * 4 + q;
     ap[g] = a + (size_t)(m < M ? m : 0) * lda + kb;
   }
-  // what the epilogue needs is asked for first, as raw bits from places that always exist
   // Four threads an output element (the host launches 4 * ROWS * COLS threads at least): each sums
-  // a quarter of the partial sums, the first of them stores.
+  // a quarter of the partial sums, the first of them stores.  What the epilogue needs is asked for behind the last operands, as in
+  // gemm_skinny.
   const int e_id = t / 4, e_q = t % 4;
   const int e_m = e_id / COLS, e_c = e_id % COLS, e_n = n0 + e_c;
   const bool e_ok = e_id < ROWS * COLS && e_m < M && e_n < N;
   const bool e_st = e_ok && e_q == 0;
-  const bool bias_bf16 = ep.bias_dtype == DA_BF16;
-  const void* e_bsrc = (e_st && ep.bias) ? ep.bias : (const void*)w;
-  const int e_bidx = (e_st && ep.bias) ? e_n : 0;
-  const uint32_t e_braw = bias_bf16 ? (uint32_t)((const bf16_t*)e_bsrc)[e_bidx] : ((const uint32_t*)e_bsrc)[e_bidx];
-  const float e_old = *((e_st && ep.accumulate) ? (const float*)ep.out + (size_t)e_m * ep.ldo + e_n : (const float*)w);
-  const int e_slot = *((e_st && kv.cache) ? kv.slot_map + e_m : (const int*)w);
+  uint32_t e_braw;
+  float e_old;
+  int e_slot;
+  KvColumn e_col;
+  auto load_epilogue = [&]() {
+    da_read_arg(er.act);
+    da_read_arg(er.out_dtype);
+    const void* e_bsrc = (e_st && bias) ? bias : (const void*)w;
+    const int e_bidx = (e_st && bias) ? e_n : 0;
+    e_braw = er.bias_dtype == DA_BF16 ? (uint32_t)((const bf16_t*)e_bsrc)[e_bidx] : ((const uint32_t*)e_bsrc)[e_bidx];
+    e_old = *((e_st && er.accumulate) ? (const float*)out + (size_t)e_m * ldo + e_n : (const float*)w);
+    e_slot = *((e_st && kv.cache) ? kv.slot_map + e_m : (const int*)w);
+    if (kv.cache) e_col = kv_column(kv, e_n);
+  };
 
   floatx4 acc[MG][NG];
 #pragma unroll
@@ -731,6 +746,7 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restr
 #pragma unroll
       for (int j = 0; j < NG; ++j) wv[u][j] = load16(wp[j] + kk);
     }
+    if (LAST) load_epilogue();
 #pragma unroll
     for (int u = 0; u < G; ++u) {
       if (LAST && u == G - 1) {
@@ -759,7 +775,7 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restr
     case 3: if (UNROLL >= 3) group(std::integral_constant<int, (UNROLL >= 3 ? 3 : 1)>{}, std::true_type{}); break;
     case 2: if (UNROLL >= 2) group(std::integral_constant<int, (UNROLL >= 2 ? 2 : 1)>{}, std::true_type{}); break;
     case 1: group(std::integral_constant<int, 1>{}, std::true_type{}); break;
-    default: break;
+    default: load_epilogue(); break;
   }
   // sum over the four products of a row of 16 lanes, then one partial a row of lanes goes to LDS
 #pragma unroll
@@ -783,13 +799,13 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restr
     v += dpp_move<0xB1, 0xF>(v, v);
     v += dpp_move<0x4E, 0xF>(v, v);
     if (e_st) {
-      const float e_bias = !ep.bias ? 0.f : (bias_bf16 ? __uint_as_float(e_braw << 16) : __uint_as_float(e_braw));
-      v = ep.out_dtype == DA_BF16 ? apply_act_bf16(v + e_bias, ep.act) : apply_act(v + e_bias, ep.act);
-      const size_t o = (size_t)e_m * ep.ldo + e_n;
-      if (ep.accumulate) ((float*)ep.out)[o] = e_old + v;
-      else if (ep.out_dtype == DA_BF16) ((bf16_t*)ep.out)[o] = f32_to_bf16(v);
-      else ((float*)ep.out)[o] = v;
-      if (kv.cache && e_n >= kv.q_cols && e_slot >= 0) kv_scatter_store(kv, e_slot, e_n, v);
+      const float e_bias = !bias ? 0.f : (er.bias_dtype == DA_BF16 ? __uint_as_float(e_braw << 16) : __uint_as_float(e_braw));
+      v = er.out_dtype == DA_BF16 ? apply_act_bf16(v + e_bias, er.act) : apply_act(v + e_bias, er.act);
+      const size_t o = (size_t)e_m * ldo + e_n;
+      if (er.accumulate) ((float*)out)[o] = e_old + v;
+      else if (er.out_dtype == DA_BF16) ((bf16_t*)out)[o] = f32_to_bf16(v);
+      else ((float*)out)[o] = v;
+      if (kv.cache && e_col.step && e_slot >= 0) kv_column_store(kv, e_col, e_slot, v);
     }
   }
 }
@@ -799,9 +815,9 @@ static int launch_skinny4(int nw, hipStream_t s, const bf16_t* A, int lda, const
                           const Epilogue& ep, const KvScatter& kv, int M, int N, int K) {
   DA_REQUIRE(M <= 4, "gemm_bf16: %d rows for one group of 4", M);
   const dim3 grid(da_ceil_div(N, NG * 4));
-  if (nw == 16) hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 16, 4>), grid, dim3(1024), 0, s, A, lda, W, ldw, ep, kv, M, N, K);
-  else if (nw == 8) hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 8, 4>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K);
-  else hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 4, 4>), grid, dim3(256), 0, s, A, lda, W, ldw, ep, kv, M, N, K);
+  if (nw == 16) hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 16, 4>), grid, dim3(1024), 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv);
+  else if (nw == 8) hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 8, 4>), grid, dim3(512), 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv);
+  else hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 4, 4>), grid, dim3(256), 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv);
   return 0;
 }
 

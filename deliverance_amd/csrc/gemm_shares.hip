@@ -76,7 +76,7 @@ extern "C" int da_gemm_bf16_shares(const void* a, int lda, const void* w, int ld
   else {
     DA_REQUIRE(lda <= (1 << 24) && ldw <= (1 << 24), "gemm_bf16_shares: rows lie too far apart (lda=%d ldw=%d)", lda, ldw);
     const dim3 grid(da_ceil_div(N, 32), g.shares);
-#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P, true>), grid, dim3(512), 0, s, A, lda, W, ldw, ep, kv, M, N, K, 32, g.k_share)
+#define DA_SK32_GO(AL, P) hipLaunchKernelGGL((gemm_skinny32_kernel<AL, 8, P, true>), grid, dim3(512), 0, s, A, W, ep.out, lda, ldw, ep.ldo, M, N, K, 32, g.k_share, ep.bias, epilogue_rest(ep), kv)
     if (M <= 16) DA_SK32_GO(2, 4);
     else if (M <= 32) DA_SK32_GO(4, 3);
     else if (M <= 48) DA_SK32_GO(6, 2);

@@ -1,6 +1,7 @@
 // Products of up to 64 rows, 32 columns a workgroup: a kernel of gemm_mfma.hip and, with k shared out over workgroups, of gemm_shares.hip.
 #pragma once
 #include "gemm_common.h"
+#include <da_read_arg.h>
 
 #define SK_LD (64 + 8)       // padded row of a step in LDS, elements (144 bytes)
 
@@ -53,8 +54,9 @@ __device__ __forceinline__ void sk_park(const u32x4_t (&av)[AL], const u32x4_t (
 // SHARES: k is shared out over blockIdx.y (gemm_take_share).
 template <int AL, int NW, int P, bool SHARES>
 __global__ void __launch_bounds__(NW * 64)
-gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                     Epilogue ep, KvScatter kv, int M, int N, int K, int cols, int k_share) {
+gemm_skinny32_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, void* out, int lda, int ldw, int ldo, int M, int N, int K,
+                     int cols, int k_share, const void* bias, EpilogueRest er, KvScatter kv) {
+  Epilogue ep{bias, er.bias_dtype, er.act, er.accumulate, out, er.out_dtype, ldo};
   if constexpr (SHARES) gemm_take_share(a, w, ep, M, K, k_share);
   constexpr int COLS = 32, MT = (AL + 1) / 2, WL = COLS / 8;    // row tiles of 16; loads of 8 rows that cover w's columns
   constexpr int CT = (COLS + 15) / 16;               // column tiles of 16
@@ -77,22 +79,13 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
   for (int i = 0; i < AL; ++i) oa[i] = 2u * (uint32_t)((i * 8 + lr < M ? i * 8 + lr : 0) * lda);
 #pragma unroll
   for (int i = 0; i < WL; ++i) ow[i] = 2u * (uint32_t)((n0 + i * 8 + lr < n_end ? i * 8 + lr : 0) * ldw);
-  // what the epilogue needs is asked for first, as raw bits from places that always exist
+  // what the epilogue needs is asked for behind the first steps' operands (its arguments are still on the way when those are asked for),
+  // as raw bits from places that always exist
   constexpr int EPT = (AR * COLS + NW * 64 - 1) / (NW * 64);
   uint32_t e_braw[EPT];
   float e_old[EPT];
   int e_slot[EPT];
   const bool bias_bf16 = ep.bias_dtype == DA_BF16;
-#pragma unroll
-  for (int j = 0; j < EPT; ++j) {
-    const int e = t + j * NW * 64, m = e / COLS, n = n0 + e % COLS;
-    const bool ok = e < AR * COLS && m < M && n < n_end;
-    const void* bsrc = (ok && ep.bias) ? ep.bias : (const void*)w;
-    const int bidx = (ok && ep.bias) ? n : 0;
-    e_braw[j] = bias_bf16 ? (uint32_t)((const bf16_t*)bsrc)[bidx] : ((const uint32_t*)bsrc)[bidx];
-    e_old[j] = *((ok && ep.accumulate) ? (const float*)ep.out + (size_t)m * ep.ldo + n : (const float*)w);
-    e_slot[j] = *((ok && kv.cache) ? kv.slot_map + m : (const int*)w);
-  }
   floatx4 acc[MT][CT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -137,6 +130,18 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
 #define SK_LAST(j) if (i + j < count) { SK_PARK(j, i + j) if (i + j + P < count) SK_FETCH(j, i + j + P) products(); }
   static_assert(P >= 1 && P <= 4, "steps in flight");
   SK_EACH(SK_FIRST)
+  da_read_arg(ep.act);
+  da_read_arg(ep.out_dtype);
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    const int e = t + j * NW * 64, m = e / COLS, n = n0 + e % COLS;
+    const bool ok = e < AR * COLS && m < M && n < n_end;
+    const void* bsrc = (ok && ep.bias) ? ep.bias : (const void*)w;
+    const int bidx = (ok && ep.bias) ? n : 0;
+    e_braw[j] = bias_bf16 ? (uint32_t)((const bf16_t*)bsrc)[bidx] : ((const uint32_t*)bsrc)[bidx];
+    e_old[j] = *((ok && ep.accumulate) ? (const float*)ep.out + (size_t)m * ep.ldo + n : (const float*)w);
+    e_slot[j] = *((ok && kv.cache) ? kv.slot_map + m : (const int*)w);
+  }
   int i = 0;
   for (; i + 2 * P <= count; i += P) SK_EACH(SK_STEADY)
   for (; i < count; i += P) SK_EACH(SK_LAST)
@@ -168,7 +173,7 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __rest
       if (ep.accumulate) ((float*)ep.out)[o] = e_old[j] + v;
       else if (ep.out_dtype == DA_BF16) ((bf16_t*)ep.out)[o] = f32_to_bf16(v);
       else ((float*)ep.out)[o] = v;
-      if (kv.cache && n >= kv.q_cols && e_slot[j] >= 0) kv_scatter_store(kv, e_slot[j], n, v);
+      if (kv.cache && n >= kv.q_cols && e_slot[j] >= 0) kv_column_store(kv, kv_column(kv, n), e_slot[j], v);
     }
   }
 }

@@ -38,6 +38,10 @@ EXTRA_FLAGS = {"attn_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_latent_mfma": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_window": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "attn_f32": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# Units whose kernels find their first arguments in registers when a wavefront starts: the hardware reads up to 14 words of them ahead,
+# as long as they are single numbers and pointers (a structure ends them).
+KERNARG_PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
+PRELOADED = ("gemm_mfma", "gemm_fused", "gemm_shares")
 # The unit that holds the error message every entry point may leave; every other unit needs it.
 BASE_UNIT = "rowwise"
 # Units whose functions a unit calls.
@@ -196,7 +200,7 @@ def _build_locked(hipcc: str, out_dir: str, todo: Sequence[str], verbose: bool) 
 
     def compile_one(unit):
         obj = os.path.join(out_dir, unit + ".o")
-        run([hipcc, *HIPCC_FLAGS, *EXTRA_FLAGS.get(unit, []), "-I", CSRC, "-c", _source(unit), "-o", obj], f"hipcc on {unit}.hip")
+        run([hipcc, *HIPCC_FLAGS, *EXTRA_FLAGS.get(unit, []), *(KERNARG_PRELOAD if unit in PRELOADED else []), "-I", CSRC, "-c", _source(unit), "-o", obj], f"hipcc on {unit}.hip")
         tmp = os.path.join(out_dir, f".libda_{unit}.so.{os.getpid()}")
         run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", obj, "-o", tmp], f"linking {unit}")
         os.replace(tmp, os.path.join(out_dir, f"libda_{unit}.so"))
