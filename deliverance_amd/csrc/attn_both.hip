@@ -23,7 +23,7 @@ attn_both_kernel(const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restric
                                        q_start, seq_lens, n_decode, Hq, Hkv, page, scale, window, out, out_ld);
     return;
   }
-  attn_decode_body<2, 8, false>(id, q, q_ld, cache, block_table, max_blocks, seq_lens, Hq, Hkv, 64, page, scale, window, out, out_ld, 0, nullptr);
+  attn_decode_body<2, 8, false>(id / Hq, id % Hq, q, cache, block_table, seq_lens, q_ld, max_blocks, Hq, Hkv, 64, page, scale, window, out, out_ld, 0, nullptr);
 }
 
 // 1 for the steps that this kernel takes: both kinds of sequences, heads of 64, contexts whose pairs are not shared out, and

@@ -32,6 +32,7 @@
 // of which o is multiplied with the logistic function.  The last two act once, after everything has been merged.  The
 // plain build has none of that code.
 #include "gemm_common.h"
+#include <da_read_arg.h>
 
 #define DEC_MAX_D 256
 
@@ -43,6 +44,7 @@
 #define DEC_REL_ARGS , rel_bias, n_dist, slopes, t_coef, t_every, chunk DEC_END_ARGS
 #define DEC_END_PARAMS , const float* __restrict__ sink, const bf16_t* __restrict__ gate, int gate_ld
 #define DEC_END_ARGS , sink, gate, gate_ld
+#define DEC_REL_OF_ROWS(s0) , rel_bias, n_dist, slopes, t_coef, t_every, chunk, sink, gate ? gate + (size_t)(s0) * gate_ld : nullptr, gate_ld
 #else
 #define DEC_KERNEL attn_decode_kernel
 #define DEC_MERGE_KERNEL attn_decode_merge_kernel
@@ -51,6 +53,7 @@
 #define DEC_REL_ARGS
 #define DEC_END_PARAMS
 #define DEC_END_ARGS
+#define DEC_REL_OF_ROWS(s0)
 #endif
 
 // e^x by the hardware's exp2 (two instructions; the library's expf is a dozen, and the merge of 16 wavefronts'
@@ -86,27 +89,26 @@ __device__ __forceinline__ float dec_gate(float z) {
 // files, called by a kernel, compiles to other code: one-token steps of the Virudra 1,101 -> 1,106 us.)
 template <int DK, int DEC_WAVES, bool SPLIT>
 #ifdef DA_ATTN_BODIES
-#define DEC_PAIR dec_pair
 __device__ __forceinline__ void
-attn_decode_body(int dec_pair,
+attn_decode_body(int s, int h,
 #else
-#define DEC_PAIR blockIdx.x
 // (registers are held to 128 for head sizes up to 64, so that two workgroups share a compute unit)
 __global__ void __launch_bounds__(DEC_WAVES * DA_WAVE, (DK <= 2 || DEC_WAVES == 16) ? 4 : 2)
 DEC_KERNEL(
 #endif
-           const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
-           const int* __restrict__ block_table, int max_blocks,
-           const int* __restrict__ seq_lens, int Hq, int Hkv, int D, int page, float scale,
+           const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, const int* __restrict__ block_table,
+           const int* __restrict__ seq_lens, int q_ld, int max_blocks, int Hq, int Hkv, int D, int page, float scale,
            int window, bf16_t* __restrict__ out, int out_ld, int span, float* __restrict__ partial DEC_REL_PARAMS) {
+#ifndef DA_ATTN_BODIES
+  const int h = blockIdx.x, s = blockIdx.y;
+#endif
   constexpr int DV = 2 * DK;                  // pieces of 16 value dimensions
   constexpr int DMAX = 32 * DK;
   __shared__ __attribute__((aligned(16))) bf16_t ps[DEC_WAVES][4][DA_WAVE];     // a chunk's weights in three parts; part 3: zeros
   __shared__ __attribute__((aligned(16))) float part_acc[DEC_WAVES][DMAX];
   __shared__ float part_m[DEC_WAVES], part_l[DEC_WAVES];
 
-  const int s = DEC_PAIR / Hq, h = DEC_PAIR % Hq;
-  const int hk = h / (Hq / Hkv);
+  const int hk = Hq == Hkv ? h : h / (Hq / Hkv);
   const int t = threadIdx.x, lane = t % DA_WAVE, wave = __builtin_amdgcn_readfirstlane(t / DA_WAVE);
   const int col = lane % 16, quad = lane / 16;
   const int* bt = block_table + (size_t)s * max_blocks;
@@ -126,7 +128,7 @@ DEC_KERNEL(
     const int d = 32 * k + 8 * quad;
     qf[k] = *(const uint4*)(q + (size_t)s * q_ld + h * D + (d < D ? d : 0));
   }
-  const int split0 = SPLIT ? (int)blockIdx.y * span : 0;          // the first key of this workgroup's share
+  const int split0 = SPLIT ? (int)blockIdx.z * span : 0;          // the first key of this workgroup's share
   const int c0_guess = split0 + wave * DA_WAVE;
   int btk0[4], btv0[2];
 #pragma unroll
@@ -144,6 +146,17 @@ DEC_KERNEL(
   const int gd = t < D ? t : 0;
   const bf16_t graw = !SPLIT && gate ? gate[(size_t)s * gate_ld + h * D + gd] : (bf16_t)0;
   const float s0 = !SPLIT && sink ? sink[h] : 0.f;
+#endif
+  // the arguments behind the first 14 words, now: each line of them that is first asked for at its use is a wait of its own
+  da_read_arg(scale);
+  da_read_arg(window);
+  da_read_arg(out);
+  da_read_arg(out_ld);
+#ifdef DEC_REL
+  da_read_arg(rel_bias);
+  da_read_arg(slopes);
+  da_read_arg(t_every);
+  da_read_arg(gate_ld);
 #endif
   // the row's position is seq_lens[s] - 1; it sees the keys lo..p (of which this workgroup takes its share)
   const int p_row = seq_lens[s] - 1;
@@ -377,7 +390,7 @@ DEC_KERNEL(
   }
   if (SPLIT) {
     // the share's result before the division, its maximum and its sum of weights
-    float* mine = partial + ((size_t)DEC_PAIR * gridDim.y + blockIdx.y) * (D + 2);
+    float* mine = partial + (((size_t)s * Hq + h) * gridDim.z + blockIdx.z) * (D + 2);
     for (int d = t; d < D; d += DEC_WAVES * DA_WAVE) {
       float o = 0.f;
 #pragma unroll
@@ -459,13 +472,25 @@ static int decode_checks(const void* q, int q_ld, const void* cache, int max_blo
 static int decode_launch(const void* q, int q_ld, const void* cache, const int* block_table, int max_blocks,
                          const int* seq_lens, int S, int Hq, int Hkv, int D, int page, float scale, int window,
                          void* out, int out_ld, int n_splits, int span, float* partial, hipStream_t st DEC_REL_DECL) {
+  // (a head and a sequence a workgroup, found without a division; the second size of a launch ends at 65,535)
+  constexpr int MAX_S = 65535;
+  if (S > MAX_S) {
+    const int part = da_ceil_div(S, da_ceil_div(S, MAX_S));
+    for (int s0 = 0; s0 < S; s0 += part) {
+      const int n = S - s0 < part ? S - s0 : part;
+      decode_launch((const bf16_t*)q + (size_t)s0 * q_ld, q_ld, cache, block_table + (size_t)s0 * max_blocks, max_blocks, seq_lens + s0, n, Hq, Hkv,
+                    D, page, scale, window, (bf16_t*)out + (size_t)s0 * out_ld, out_ld, n_splits, span,
+                    partial ? partial + (size_t)s0 * Hq * n_splits * (D + 2) : nullptr, st DEC_REL_OF_ROWS(s0));
+    }
+    return 0;
+  }
   // 8 wavefronts; 16 where the workgroups are no more than the compute units (a context above 512 is then
   // still one chunk a wavefront, and the larger workgroup's start is paid once per compute unit)
   const bool wide = (long)S * Hq * n_splits <= 256 && D <= 64;         // larger heads need the registers of 8 wavefronts
-  dim3 grid(S * Hq, n_splits);
+  dim3 grid(Hq, S, n_splits);
 #define LAUNCH3(C, W, SP)                                                                                   \
-  hipLaunchKernelGGL((DEC_KERNEL<C, W, SP>), grid, dim3(W * DA_WAVE), 0, st, (const bf16_t*)q, q_ld, \
-                     (const bf16_t*)cache, block_table, max_blocks, seq_lens, Hq, Hkv, D, page, scale, window, \
+  hipLaunchKernelGGL((DEC_KERNEL<C, W, SP>), grid, dim3(W * DA_WAVE), 0, st, (const bf16_t*)q, \
+                     (const bf16_t*)cache, block_table, seq_lens, q_ld, max_blocks, Hq, Hkv, D, page, scale, window, \
                      (bf16_t*)out, out_ld, span, partial DEC_REL_ARGS)
 #define LAUNCH2(C, W) do { if (n_splits > 1) LAUNCH3(C, W, true); else LAUNCH3(C, W, false); } while (0)
 #define LAUNCH(C) do { if (wide) LAUNCH2(C, 16); else LAUNCH2(C, 8); } while (0)

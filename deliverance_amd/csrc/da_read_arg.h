@@ -3,4 +3,5 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-__device__ __forceinline__ void da_read_arg(int v) { asm volatile("" ::"s"(v)); }
+template <typename T>
+__device__ __forceinline__ void da_read_arg(T v) { asm volatile("" ::"s"(v)); }

@@ -39,9 +39,10 @@ __device__ __forceinline__ void rms_store4(void* y, int y_dtype, size_t at, floa
 // and (if h) the new x is normalised with (wb) into h.  !ADD: y = rms(x) with wa.
 template <int VPL, int W, bool ADD>
 __global__ void __launch_bounds__(4 * DA_WAVE)
-rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, const void* __restrict__ wa, int wa_dtype,
-                   float* __restrict__ x, const void* __restrict__ wb, int wb_dtype, float offset, float eps,
-                   void* __restrict__ y, int y_dtype, int R, int E) {
+rmsnorm_row_kernel(const float* __restrict__ src, const int* __restrict__ rows, const void* __restrict__ wa, float* __restrict__ x,
+                   const void* __restrict__ wb, void* __restrict__ y, int E, int dtypes, int R, float offset, float eps) {
+  // (the first 14 words, with the three types in one, are in registers when the wavefront starts: build.py, KERNARG_PRELOAD)
+  const int wa_dtype = dtypes & 0xff, wb_dtype = (dtypes >> 8) & 0xff, y_dtype = dtypes >> 16;
   __shared__ float red[2][4];
   constexpr int STRIDE = 4 * W * DA_WAVE;
   const int t = threadIdx.x, c0 = (W == 4 ? t : t % DA_WAVE) * 4;
@@ -144,8 +145,8 @@ static void rms_launch(const float* src, const int* rows, const void* wa, int wa
   const bool aligned = ((uintptr_t)src % 16 == 0) && ((uintptr_t)y % 16 == 0) && ((uintptr_t)wa % 16 == 0) &&
                        ((uintptr_t)wb % 16 == 0) && ((uintptr_t)x % 16 == 0);
 #define RMS_LAUNCH(V, W)                                                                                             \
-  hipLaunchKernelGGL((rmsnorm_row_kernel<V, W, ADD>), dim3(g.blocks), dim3(g.threads), 0, st, src, rows, wa, wa_dtype, x, \
-                     wb, wb_dtype, offset, eps, y, y_dtype, R, E)
+  hipLaunchKernelGGL((rmsnorm_row_kernel<V, W, ADD>), dim3(g.blocks), dim3(g.threads), 0, st, src, rows, wa, x, wb, y, E, \
+                     wa_dtype | wb_dtype << 8 | y_dtype << 16, R, offset, eps)
   if (E % 4 == 0 && E <= 4096 && aligned) {
     const NormGrid g = norm_grid(R, E, 2048, ADD ? INT_MAX : 4096);
     if (g.waves == 1) {

@@ -265,7 +265,7 @@ template <int VPL, int W, bool PBF16, bool YBF16, bool JOIN = false>
 __global__ void __launch_bounds__(4 * DA_WAVE)
 layernorm_row_kernel(typename RowSource<JOIN>::type x, const int* __restrict__ rows,
                      const void* __restrict__ w, const void* __restrict__ b,
-                     float eps, void* __restrict__ y, int R, int E, RowJoin join) {
+                     void* __restrict__ y, int E, int R, float eps, RowJoin join) {
   __shared__ float red[2][4];
   constexpr int STRIDE = 4 * W * DA_WAVE;
   const int t = threadIdx.x, c0 = (W == 4 ? t : t % DA_WAVE) * 4;
@@ -355,7 +355,7 @@ extern "C" int da_layernorm(const float* x, const int* rows, const void* w, int 
   const bool same = (!b || b_dtype == w_dtype) && (w_dtype == DA_BF16 || w_dtype == DA_F32);   // gain and bias alike
   if (E % 4 == 0 && E <= 2048 && aligned && same) {
     const NormGrid g = norm_grid(R, E, 768, 1024);
-#define LN_LAUNCH(V, W, P, Y) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, Y>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, eps, y, R, E, RowJoin{})
+#define LN_LAUNCH(V, W, P, Y) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, Y>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, y, E, R, eps, RowJoin{})
 #define LN_LAUNCH_Y(V, W, P) do { if (y_dtype == DA_BF16) LN_LAUNCH(V, W, P, true); else LN_LAUNCH(V, W, P, false); } while (0)
 #define LN_LAUNCH_P(V, W) do { if (w_dtype == DA_BF16) LN_LAUNCH_Y(V, W, true); else LN_LAUNCH_Y(V, W, false); } while (0)
     if (g.waves == 1) {
@@ -393,7 +393,7 @@ extern "C" int da_layernorm_join(float* x, const int* rows, const float* partial
   hipStream_t st = (hipStream_t)stream;
   const RowJoin j{partial, stride, n, add, add_dtype, rows ? nullptr : x};
   const NormGrid g = norm_grid(R, E, 768, 1024);
-#define LN_LAUNCH(V, W, P) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, true, true>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, eps, y, R, E, j)
+#define LN_LAUNCH(V, W, P) hipLaunchKernelGGL((layernorm_row_kernel<V, W, P, true, true>), dim3(g.blocks), dim3(g.threads), 0, st, x, rows, w, b, y, E, R, eps, j)
 #define LN_LAUNCH_P(V, W) do { if (w_dtype == DA_BF16) LN_LAUNCH(V, W, true); else LN_LAUNCH(V, W, false); } while (0)
   if (g.waves == 1) {
     if (E <= 256) LN_LAUNCH_P(1, 1);
