@@ -19,6 +19,7 @@
 // 1,172 -> 50, 8 sequences of 1,000 keys 189 -> 21 / 379 -> 38.
 // Formulas: core/src/main/java/io/teknek/deliverance/generator/CausalSelfAttention.java:481-491,512-527.
 #include "gemm_common.h"
+#include <da_read_arg.h>
 
 #define AF_WAVES 8
 #define AF_CHUNK 32
@@ -64,8 +65,8 @@ __device__ __forceinline__ float af_entry(const float* qr, const float* kb, cons
 
 template <int D16>
 __global__ void __launch_bounds__(AF_WAVES * DA_WAVE)
-attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__ cache, const int* __restrict__ block_table,
-                int max_blocks, const int* __restrict__ q_start, const int* __restrict__ seq_lens, int Hq, int Hkv, int page,
+attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ cache, const int* __restrict__ block_table,
+                const int* __restrict__ q_start, const int* __restrict__ seq_lens, int q_ld, int max_blocks, int Hq, int Hkv, int page,
                 float scale, int window, float* __restrict__ out, int out_ld) {
   constexpr int D = D16 * 16;
   constexpr int OLD = D + 4;                                   // padded row of a partial result
@@ -73,18 +74,30 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
   __shared__ __attribute__((aligned(16))) float smem[P_FLOATS > O_FLOATS ? P_FLOATS : O_FLOATS];   // weights, then partial results
   __shared__ float part_m[AF_WAVES][16], part_l[AF_WAVES][16];
 
-  const int s = (int)blockIdx.x / Hq, h = (int)blockIdx.x % Hq, hk = h / (Hq / Hkv);
-  const int row0 = q_start[s], T = q_start[s + 1] - row0;
-  const int i0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * 16;  // (the rows with the most keys are launched first)
-  if (i0 >= T) return;
-  const int past = seq_lens[s] - T;
+  const int s = blockIdx.y, h = blockIdx.x, hk = Hq == Hkv ? h : h / (Hq / Hkv);
   const int t = threadIdx.x, lane = t % DA_WAVE, wave = __builtin_amdgcn_readfirstlane(t / DA_WAVE);
   const int col = lane % 16, quad = lane / 16;
+  const int* bt = block_table + (size_t)s * max_blocks;
+  const int lg = 31 - __builtin_clz(page), pmask = page - 1;   // (a power of two, checked on the host)
+  // Asked for side by side: the sequence's rows and length, and the pages of the chunk that this wavefront starts with where no window
+  // cuts keys off (entries past the sequence's pages are read, the table has max_blocks of them, and never used).
+  const int row0 = q_start[s], row1 = q_start[s + 1], len = seq_lens[s];
+  int guess[AF_PIECES];
+#pragma unroll
+  for (int j = 0; j < AF_PIECES; ++j) {
+    const int i = (wave * AF_CHUNK + j * 16) >> lg;
+    guess[j] = bt[i < max_blocks ? i : max_blocks - 1];
+  }
+  da_read_arg(scale);
+  da_read_arg(out);
+  da_read_arg(out_ld);
+  const int T = row1 - row0;
+  const int i0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * 16;  // (the rows with the most keys are launched first)
+  if (i0 >= T) return;
+  const int past = len - T;
   const int last_row = i0 + 15 < T ? i0 + 15 : T - 1;
   const int p_max = past + last_row;                           // the last key that any of the rows sees (-1: a padding row)
   const int lo_min = (window > 0 && past + i0 - window + 1 > 0) ? past + i0 - window + 1 : 0;
-  const int* bt = block_table + (size_t)s * max_blocks;
-  const int lg = 31 - __builtin_clz(page), pmask = page - 1;   // (a power of two, checked on the host)
   const long long page_elems = 2LL * Hkv * page * D;
   const float* kbase = cache + (long long)hk * page * D;
   const float* vbase = cache + (long long)(Hkv + hk) * page * D;
@@ -116,7 +129,7 @@ attn_f32_kernel(const float* __restrict__ q, int q_ld, const float* __restrict__
     for (int j = 0; j < AF_PIECES; ++j) {
       const int k0 = c0 + j * 16;
       const bool in = k0 <= p_max && k0 + 15 >= lo_min;
-      const int pg = in ? __builtin_amdgcn_readfirstlane(bt[k0 >> lg]) : -1;
+      const int pg = !in ? -1 : (ci == wave ? __builtin_amdgcn_readfirstlane(guess[j]) : __builtin_amdgcn_readfirstlane(bt[k0 >> lg]));
       seen[j] = pg >= 0;
       const long long off = (long long)(pg >= 0 ? pg : 0) * page_elems;
       kp[j] = kbase + off + (k0 & pmask) * D;
@@ -249,16 +262,25 @@ extern "C" int da_attn_f32(const float* q, int q_ld, const float* cache, const i
   DA_REQUIRE((uintptr_t)q % 16 == 0 && (uintptr_t)cache % 16 == 0, "attn_f32: q and the cache must be 16-byte aligned");
   DA_REQUIRE(window >= 0 && max_blocks > 0, "attn_f32: bad window or block table");
   if (n_seqs == 0) return 0;
-  const dim3 grid(n_seqs * Hq, da_ceil_div(max_query_len, 16)), block(AF_WAVES * DA_WAVE);
-#define AF_LAUNCH(X)                                                                                                            \
-  case X: hipLaunchKernelGGL(attn_f32_kernel<X>, grid, block, 0, (hipStream_t)stream, q, q_ld, cache, block_table, max_blocks, \
-                             q_start, seq_lens, Hq, Hkv, page, scale, window, out, out_ld); break
-  switch (D / 16) {
-    AF_LAUNCH(1); AF_LAUNCH(2); AF_LAUNCH(3); AF_LAUNCH(4); AF_LAUNCH(5); AF_LAUNCH(6); AF_LAUNCH(7);
-    default: hipLaunchKernelGGL(attn_f32_kernel<8>, grid, block, 0, (hipStream_t)stream, q, q_ld, cache, block_table, max_blocks,
-                                q_start, seq_lens, Hq, Hkv, page, scale, window, out, out_ld); break;
-  }
+  // (a head and a sequence a workgroup, found without a division; a launch's second size ends at 65,535)
+  for (int s0 = 0; s0 < n_seqs; s0 += 65535) {
+    const int n = n_seqs - s0 < 65535 ? n_seqs - s0 : 65535;
+    const dim3 grid(Hq, n, da_ceil_div(max_query_len, 16)), block(AF_WAVES * DA_WAVE);
+#define AF_LAUNCH(X)                                                                                                                       \
+  hipLaunchKernelGGL(attn_f32_kernel<X>, grid, block, 0, (hipStream_t)stream, q, cache, block_table + (size_t)s0 * max_blocks, q_start + s0, \
+                     seq_lens + s0, q_ld, max_blocks, Hq, Hkv, page, scale, window, out, out_ld)
+    switch (D / 16) {
+      case 1: AF_LAUNCH(1); break;
+      case 2: AF_LAUNCH(2); break;
+      case 3: AF_LAUNCH(3); break;
+      case 4: AF_LAUNCH(4); break;
+      case 5: AF_LAUNCH(5); break;
+      case 6: AF_LAUNCH(6); break;
+      case 7: AF_LAUNCH(7); break;
+      default: AF_LAUNCH(8); break;
+    }
 #undef AF_LAUNCH
+  }
   DA_CHECK_LAUNCH("attn_f32");
   return 0;
 }

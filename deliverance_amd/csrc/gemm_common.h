@@ -79,9 +79,10 @@ __device__ __forceinline__ KvColumn kv_column(const KvScatter& kv, int n) {
   if (cv < 0) return KvColumn{c + (long long)div_uniform(c, kv.D) * (kv.page - 1) * kv.D, kv.D};
   return KvColumn{((long long)kv.Hkv * kv.D + cv) * kv.page, cv < kv.Hkv * Dv ? 1 : 0};
 }
+template <typename T = bf16_t>
 __device__ __forceinline__ void kv_column_store(const KvScatter& kv, const KvColumn& col, int slot, float v) {
   const int pg = div_uniform(slot, kv.page), row = slot - pg * kv.page;
-  ((bf16_t*)kv.cache)[pg * ((long long)kv.Hkv * kv.page * (kv.D + (kv.Dv ? kv.Dv : kv.D))) + col.at + (long long)row * col.step] = f32_to_bf16(v);
+  from_f32((T*)kv.cache + (pg * ((long long)kv.Hkv * kv.page * (kv.D + (kv.Dv ? kv.Dv : kv.D))) + col.at + (long long)row * col.step), v);
 }
 
 // The values of 32 rows of a product whose k and v columns go to the cache.  Values are dimension-major: 4 rows whose places

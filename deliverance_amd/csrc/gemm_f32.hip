@@ -25,6 +25,7 @@
 // 768 x 50,257 39.9 -> 32.1; 8 rows, 3,072 x 768 12.0 -> 7.7; 16 rows 13.8 -> 9.6; 64 rows 14.3 -> 11.4; 32 rows, 768 x 3,072 8.7 -> 7.9.
 // Tiles: 526 x 768 x 3,072 38, 526 x 2,304 x 768 27, 526 x 50,257 x 768 392.
 #include "gemm_common.h"
+#include <da_read_arg.h>
 #include <type_traits>
 
 #define GF_CHUNK 128
@@ -49,15 +50,15 @@ __device__ __forceinline__ void gf_wave_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// the k and v columns of a q|k|v product (column n >= q_cols of the row whose place in the cache is `slot`)
-__device__ __forceinline__ void gf_scatter(const KvScatter& kv, int slot, int n, float v) {
-  const int pg = slot / kv.page, row = slot % kv.page;
-  const int c2 = n - kv.q_cols, is_v = c2 >= kv.kv_cols, cc = is_v ? c2 - kv.kv_cols : c2;
-  const int h = cc / kv.D, d = cc % kv.D;
-  float* cache = (float*)kv.cache;
-  if (is_v) cache[cache_v_base(pg, h, kv.Hkv, kv.page, kv.D) + (long long)d * kv.page + row] = v;
-  else cache[cache_k_row(pg, h, row, kv.Hkv, kv.page, kv.D) + d] = v;
-}
+
+// An output element's bias, old value, place in the cache and the column's offset in a page.
+#define GF_EPILOGUE_LOADS                                                                                                      \
+  da_read_arg(ep.act);                                                                                                         \
+  const float e_bias_raw = (e_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, en) : 0.f;                                   \
+  const float e_old = *((e_ok && ep.accumulate) ? (const float*)ep.out + (size_t)em * ep.ldo + en : w);                        \
+  const int e_slot = *((e_ok && kv.cache) ? kv.slot_map + em : (const int*)w);                                                 \
+  KvColumn e_col;                                                                                                              \
+  if (kv.cache) e_col = kv_column(kv, en);
 
 // ---------------------------------------------------------------------------------------------
 // Few rows: blockIdx.x: `cols` columns (4 WL at most), blockIdx.y: 4 AL rows.  A wavefront takes sets of P chunks, v, v + NW,
@@ -75,8 +76,9 @@ __device__ __forceinline__ int gf_place(int row, int kk) { return row * 32 + (kk
 // CAP: chunks that the partial sums in LDS have room for.
 template <int WL, int AL, int NW, int CAP>
 __global__ void __launch_bounds__(NW * 64)
-gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w, int ldw, Epilogue ep, KvScatter kv,
-                     int M, int N, int K, int n_chunks, int cols) {
+gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w, void* out, int lda, int ldw, int ldo, int M, int N, int K,
+                     int n_chunks, int cols, const void* bias, EpilogueRest er, KvScatter kv) {
+  const Epilogue ep{bias, er.bias_dtype, er.act, er.accumulate, out, DA_F32, ldo};
   constexpr int P = WL == 1 && AL == 1 ? 4 : (WL <= 2 && AL <= 2 ? 2 : 1), S = 16 / P;    // chunks of a product; rows and columns of each
   constexpr int RA = 4 * AL, CW = 4 * WL, LA = RA / 2, LW = CW / 2;     // rows, columns; loads a chunk
   static_assert(RA <= S && CW <= S, "a chunk's rows and columns fit their part of the fragments");
@@ -96,13 +98,6 @@ gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restri
   for (int i = 0; i < LA; ++i) pa[i] = a + (size_t)(r0 + i * 2 + l_row < M ? r0 + i * 2 + l_row : r0) * lda;
 #pragma unroll
   for (int i = 0; i < LW; ++i) pw[i] = w + (size_t)(n0 + i * 2 + l_row < n_end ? n0 + i * 2 + l_row : n0) * ldw;
-  // what the epilogue needs is asked for first, from places that always exist
-  const int em = r0 + t / CW, en = n0 + t % CW;
-  const bool e_ok = t < RA * CW && em < M && en < n_end;
-  const float e_bias_raw = (e_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, en) : 0.f;
-  const float e_old = *((e_ok && ep.accumulate) ? (const float*)ep.out + (size_t)em * ep.ldo + en : w);
-  const int e_slot = *((e_ok && kv.cache) ? kv.slot_map + em : (const int*)w);
-
   struct Set { f32x4_t a[P][LA], w[P][LW]; };
   auto fetch = [&](Set& x, int set) {                                  // (past K: the row's first piece, dropped when it is parked)
 #pragma unroll
@@ -146,6 +141,10 @@ gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restri
   Set x, y;
   int set = wave;
   if (set < n_sets) fetch(x, set);
+  // what the epilogue needs is asked for behind the first operands, from places that always exist
+  const int em = r0 + t / CW, en = n0 + t % CW;
+  const bool e_ok = t < RA * CW && em < M && en < n_end;
+  GF_EPILOGUE_LOADS
   for (; set < n_sets; set += 2 * NW) {
     if (set + NW < n_sets) fetch(y, set + NW);
     products(x, set);
@@ -161,7 +160,7 @@ gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restri
   v = apply_act(v + e_bias_raw, ep.act);
   float* o = (float*)ep.out + (size_t)em * ep.ldo + en;
   *o = ep.accumulate ? e_old + v : v;
-  if (kv.cache && en >= kv.q_cols && e_slot >= 0) gf_scatter(kv, e_slot, en, v);
+  if (kv.cache && e_col.step && e_slot >= 0) kv_column_store<float>(kv, e_col, e_slot, v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -173,20 +172,20 @@ gemm_f32_rows_kernel(const float* __restrict__ a, int lda, const float* __restri
 // ---------------------------------------------------------------------------------------------
 template <int COLS, int NW, int CAP>
 __global__ void __launch_bounds__(NW * 64)
-gemm_f32_rows_direct_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w, int ldw, Epilogue ep, KvScatter kv,
-                            int M, int N, int K, int n_chunks) {
+gemm_f32_rows_direct_kernel(const float* __restrict__ a, const float* __restrict__ w, void* out, int lda, int ldw, int ldo, int M, int N, int K,
+                            int n_chunks, const void* bias, EpilogueRest er, KvScatter kv) {
+  const Epilogue ep{bias, er.bias_dtype, er.act, er.accumulate, out, DA_F32, ldo};
   __shared__ float gf_red[CAP * 16 * (COLS + 1)];               // [n_chunks][16][COLS + 1]
   const int t = threadIdx.x, lane = t % 64, wave = t / 64;
   const int n0 = blockIdx.x * COLS, r0 = blockIdx.y * 16;
   const int fr = lane % 16, kq = (lane / 16) * 4;
   const float* pa = a + (size_t)(r0 + fr < M ? r0 + fr : r0) * lda;
   const float* pw = w + (size_t)(n0 + fr % COLS < N ? n0 + fr % COLS : n0) * ldw;
-  // what the epilogue needs is asked for first, from places that always exist
+  // what the epilogue needs is asked for first, from places that always exist (a wavefront has one chunk, so there is no place behind
+  // its first operands)
   const int em = r0 + t / COLS, en = n0 + t % COLS;
   const bool e_ok = t < 16 * COLS && em < M && en < N;
-  const float e_bias_raw = (e_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, en) : 0.f;
-  const float e_old = *((e_ok && ep.accumulate) ? (const float*)ep.out + (size_t)em * ep.ldo + en : w);
-  const int e_slot = *((e_ok && kv.cache) ? kv.slot_map + em : (const int*)w);
+  GF_EPILOGUE_LOADS
 
   auto chunk = [&](int c, auto cutc) {
     constexpr bool CUT = decltype(cutc)::value;                        // the chunk that K cuts
@@ -222,7 +221,7 @@ gemm_f32_rows_direct_kernel(const float* __restrict__ a, int lda, const float* _
   v = apply_act(v + e_bias_raw, ep.act);
   float* o = (float*)ep.out + (size_t)em * ep.ldo + en;
   *o = ep.accumulate ? e_old + v : v;
-  if (kv.cache && en >= kv.q_cols && e_slot >= 0) gf_scatter(kv, e_slot, en, v);
+  if (kv.cache && e_col.step && e_slot >= 0) kv_column_store<float>(kv, e_col, e_slot, v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -349,6 +348,8 @@ gemm_f32_tile_body(const float* __restrict__ a, int lda, const float* __restrict
     const int n = n0 + wn + j * 16 + fr;
     const bool n_ok = n < N;
     const float bias = (n_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, n) : 0.f;
+    KvColumn col;
+    if (kv.cache) col = kv_column(kv, n);
     float old[TM][4];
     int slot[TM][4];
 #pragma unroll
@@ -368,7 +369,7 @@ gemm_f32_tile_body(const float* __restrict__ a, int lda, const float* __restrict
         if (!n_ok || m >= M) continue;
         const float v = apply_act(acc[i][j][r] + bias, ep.act);
         ((float*)ep.out)[(size_t)m * ep.ldo + n] = ep.accumulate ? old[i][r] + v : v;
-        if (kv.cache && n >= kv.q_cols && slot[i][r] >= 0) gf_scatter(kv, slot[i][r], n, v);
+        if (kv.cache && n >= kv.q_cols && slot[i][r] >= 0) kv_column_store<float>(kv, col, slot[i][r], v);
       }
   }
 }
@@ -393,8 +394,8 @@ static void launch_f32_tile(hipStream_t s, const float* a, int lda, const float*
 template <int WL, int AL, int NW, int CAP>
 static void launch_f32_rows(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
                             int M, int N, int K, int cols) {
-  hipLaunchKernelGGL((gemm_f32_rows_kernel<WL, AL, NW, CAP>), dim3(da_ceil_div(N, cols), da_ceil_div(M, 4 * AL)), dim3(NW * 64), 0, s, a, lda,
-                     w, ldw, ep, kv, M, N, K, da_ceil_div(K, GF_CHUNK), cols);
+  hipLaunchKernelGGL((gemm_f32_rows_kernel<WL, AL, NW, CAP>), dim3(da_ceil_div(N, cols), da_ceil_div(M, 4 * AL)), dim3(NW * 64), 0, s, a, w,
+                     ep.out, lda, ldw, ep.ldo, M, N, K, da_ceil_div(K, GF_CHUNK), cols, ep.bias, epilogue_rest(ep), kv);
 }
 // The wavefronts and the room for partial sums, by K.  More workgroups than compute units (16 columns each, then): few wavefronts
 // each, so that several workgroups share a compute unit's LDS and one's loads run beside another's products (K = 768, N = 50,257: 4 rows
@@ -424,8 +425,8 @@ static void launch_f32_rows_n(hipStream_t s, const float* a, int lda, const floa
 template <int COLS, int NW, int CAP>
 static void launch_f32_rows_direct_k(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
                                      int M, int N, int K) {
-  hipLaunchKernelGGL((gemm_f32_rows_direct_kernel<COLS, NW, CAP>), dim3(da_ceil_div(N, COLS), da_ceil_div(M, 16)), dim3(NW * 64), 0, s, a,
-                     lda, w, ldw, ep, kv, M, N, K, da_ceil_div(K, GF_CHUNK));
+  hipLaunchKernelGGL((gemm_f32_rows_direct_kernel<COLS, NW, CAP>), dim3(da_ceil_div(N, COLS), da_ceil_div(M, 16)), dim3(NW * 64), 0, s, a, w,
+                     ep.out, lda, ldw, ep.ldo, M, N, K, da_ceil_div(K, GF_CHUNK), ep.bias, epilogue_rest(ep), kv);
 }
 template <int COLS>
 static void launch_f32_rows_direct(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
