@@ -604,23 +604,35 @@ extern "C" int da_moe_slot_weights(const int* slot_of_pair, const float* weights
 
 // y[n] (+)= sum_k weight(n, k) * out[slot_of_pair[n * top + k]]; weights: per pair, or one for all.  h (optional): a pair
 // without a slot adds weight * h[n], an expert that hands its input on.  shared (optional): + logistic(gate[n]) * shared[n].
+// (A column a thread, rows over blockIdx.y: a pair's slot and weight are the same for a workgroup, and nothing is divided; by a 64-bit division
+// of one number for both a decode step's 8 rows of 1,024 took 4.8 us in a profiled step, of which a launch alone is 2.5.)
 template <typename T>
-__global__ void moe_combine_kernel(const float* __restrict__ out, int ldo, const int* __restrict__ slot_of_pair,
-                                   const float* __restrict__ weights, float uniform, int top, float* __restrict__ y,
-                                   int ldy, int N, int width, int accumulate, const T* __restrict__ h, int ldh,
-                                   const float* __restrict__ shared, int lds, const float* __restrict__ gate, int ldg) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)N * width) return;
-  const int n = (int)(i / width), c = (int)(i % width);
-  float s = 0.f;
-  for (int k = 0; k < top; ++k) {
-    const int slot = slot_of_pair[n * top + k];
-    if (slot >= 0) s += (weights ? weights[n * top + k] : uniform) * out[(size_t)slot * ldo + c];
-    else if (h) s += (weights ? weights[n * top + k] : uniform) * to_f32(h[(size_t)n * ldh + c]);
+__global__ void __launch_bounds__(256)
+moe_combine_kernel(const float* __restrict__ out, const int* __restrict__ slot_of_pair, const float* __restrict__ weights, float* __restrict__ y,
+                   int ldo, int top, int N, int width, int ldy, float uniform, int accumulate, const T* __restrict__ h, int ldh,
+                   const float* __restrict__ shared, int lds, const float* __restrict__ gate, int ldg) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= width) return;
+  for (int n = blockIdx.y; n < N; n += gridDim.y) {
+    float* dst = y + (size_t)n * ldy + c;
+    const float old = accumulate ? *dst : 0.f;
+    float s = 0.f;
+    for (int k0 = 0; k0 < top; k0 += 4) {            // four pairs' rows side by side, added in their order
+      float v[4], wt[4];
+      bool in[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int pair = n * top + (k0 + k < top ? k0 + k : top - 1), slot = slot_of_pair[pair];
+        in[k] = k0 + k < top && (slot >= 0 || h);
+        wt[k] = weights ? weights[pair] : uniform;
+        v[k] = slot >= 0 ? out[(size_t)slot * ldo + c] : (h ? to_f32(h[(size_t)n * ldh + c]) : 0.f);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) s = in[k] ? fmaf(wt[k], v[k], s) : s;
+    }
+    if (shared) s += shared[(size_t)n * lds + c] / (1.f + expf(-gate[(size_t)n * ldg]));
+    *dst = accumulate ? old + s : s;
   }
-  if (shared) s += shared[(size_t)n * lds + c] / (1.f + expf(-gate[(size_t)n * ldg]));
-  float* dst = y + (size_t)n * ldy + c;
-  *dst = accumulate ? *dst + s : s;
 }
 
 extern "C" int da_moe_combine(const float* out, int ldo, const int* slot_of_pair, const float* weights, float uniform,
@@ -629,13 +641,13 @@ extern "C" int da_moe_combine(const float* out, int ldo, const int* slot_of_pair
   DA_REQUIRE(N >= 0 && width > 0 && top > 0 && ldo >= width && ldy >= width, "moe_combine: bad sizes");
   DA_REQUIRE((!h || ldh >= width) && (!shared || (lds >= width && gate && ldg > 0)), "moe_combine: the input's or the shared result's rows");
   if (N == 0) return 0;
-  const dim3 grid(da_ceil_div((long)N * width, 256));
+  const dim3 grid(da_ceil_div(width, 256), N < 65535 ? N : 65535);
   if (h && h_dtype == DA_BF16)
-    hipLaunchKernelGGL(moe_combine_kernel<bf16_t>, grid, dim3(256), 0, (hipStream_t)stream, out, ldo, slot_of_pair, weights,
-                       uniform, top, y, ldy, N, width, accumulate, (const bf16_t*)h, ldh, shared, lds, gate, ldg);
+    hipLaunchKernelGGL(moe_combine_kernel<bf16_t>, grid, dim3(256), 0, (hipStream_t)stream, out, slot_of_pair, weights, y, ldo, top, N,
+                       width, ldy, uniform, accumulate, (const bf16_t*)h, ldh, shared, lds, gate, ldg);
   else
-    hipLaunchKernelGGL(moe_combine_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, out, ldo, slot_of_pair, weights,
-                       uniform, top, y, ldy, N, width, accumulate, (const float*)h, ldh, shared, lds, gate, ldg);
+    hipLaunchKernelGGL(moe_combine_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, out, slot_of_pair, weights, y, ldo, top, N,
+                       width, ldy, uniform, accumulate, (const float*)h, ldh, shared, lds, gate, ldg);
   DA_CHECK_LAUNCH("moe_combine");
   return 0;
 }
@@ -802,7 +814,8 @@ extern "C" int da_moe_combine_norm(const float* out, int ldo, const int* slot_of
 // streams the expert's weights once, and narrow columns mean many workgroups for that (8 experts of 512 x 768: 256).  The
 // wavefronts' sums meet in LDS and are added in the order of the wavefronts.  GATED: the gate and up rows of the same
 // columns are multiplied side by side and out = act(g) * u leaves in bfloat16; else one product leaves in 32-bit.  A row's
-// sums run in one order whatever else is in the step.  Measured on MI355X against 64 columns a workgroup without shared k
+// sums run in one order whatever else is in the step.  (Whole cache lines a load, a lane's 32 bytes for two products of a step of 64 k: a
+// Virudra's step of 355M sizes 1,038 -> 1,049 us; the two wavefronts that share a line ask for it side by side as it is.)  Measured on MI355X against 64 columns a workgroup without shared k
 // (8 tokens, 2 of 8 experts of 512 x 768): 10.7 -> 5.7 us, down 6.2 -> 5.3.
 #define MM_ROWS 32
 #define MM_COLS 16
@@ -810,9 +823,9 @@ extern "C" int da_moe_combine_norm(const float* out, int ldo, const int* slot_of
 
 template <int MODE, int NW>
 __global__ void __launch_bounds__(NW * DA_WAVE)
-moe_mfma_kernel(const bf16_t* __restrict__ a, int lda, const int* __restrict__ row_of_slot,
-                const int* __restrict__ tile_expert, const bf16_t* __restrict__ w, void* __restrict__ out, int ldo,
-                int K, int F, int act, const float* __restrict__ slot_scale, float limit) {
+moe_mfma_kernel(const bf16_t* __restrict__ a, const int* __restrict__ row_of_slot, const int* __restrict__ tile_expert,
+                const bf16_t* __restrict__ w, int lda, int K, int F, int ldo, int act, float limit, void* __restrict__ out,
+                const float* __restrict__ slot_scale) {
   constexpr bool GATED = MODE == MOE_GATED, GATHER = MODE != MOE_DOWN;
   constexpr int G = GATED ? 2 : 1;
   __shared__ float sums[NW][G][8][DA_WAVE];                 // [wavefront][product][register of the tile][lane]
@@ -925,7 +938,7 @@ extern "C" int da_moe_gated_mfma(const void* a, int lda, const int* row_of_slot,
   DA_REQUIRE(act >= DA_ACT_NONE && act <= DA_ACT_LAST, "moe_gated_mfma: unknown activation %d", act);
   if (moe_mfma_checks(a, lda, w, K, "moe_gated_mfma")) return 1;
   if (T_cap == 0) return 0;
-  MM_LAUNCH(MOE_GATED, F, K, (const bf16_t*)a, lda, row_of_slot, tile_expert, (const bf16_t*)w, mid, ldm, K, F, act, nullptr, limit);
+  MM_LAUNCH(MOE_GATED, F, K, (const bf16_t*)a, row_of_slot, tile_expert, (const bf16_t*)w, lda, K, F, ldm, act, limit, mid, nullptr);
   DA_CHECK_LAUNCH("moe_gated_mfma");
   return 0;
 }
@@ -936,7 +949,7 @@ extern "C" int da_moe_up_mfma(const void* a, int lda, const int* row_of_slot, co
   DA_REQUIRE(act >= DA_ACT_NONE && act <= DA_ACT_LAST, "moe_up_mfma: unknown activation %d", act);
   if (moe_mfma_checks(a, lda, w, K, "moe_up_mfma")) return 1;
   if (T_cap == 0) return 0;
-  MM_LAUNCH(MOE_UP, F, K, (const bf16_t*)a, lda, row_of_slot, tile_expert, (const bf16_t*)w, mid, ldm, K, F, act, slot_scale, 0.f);
+  MM_LAUNCH(MOE_UP, F, K, (const bf16_t*)a, row_of_slot, tile_expert, (const bf16_t*)w, lda, K, F, ldm, act, 0.f, mid, slot_scale);
   DA_CHECK_LAUNCH("moe_up_mfma");
   return 0;
 }
@@ -946,8 +959,8 @@ extern "C" int da_moe_down_mfma(const void* mid, int ldm, const int* row_of_slot
   DA_REQUIRE(T_cap >= 0 && F > 0 && width > 0 && ldm >= F && ldo >= width, "moe_down_mfma: bad sizes");
   if (moe_mfma_checks(mid, ldm, w, F, "moe_down_mfma")) return 1;
   if (T_cap == 0) return 0;
-  MM_LAUNCH(MOE_DOWN, width, F, (const bf16_t*)mid, ldm, row_of_slot, tile_expert, (const bf16_t*)w, out, ldo, F, width, 0,
-            nullptr, 0.f);
+  MM_LAUNCH(MOE_DOWN, width, F, (const bf16_t*)mid, row_of_slot, tile_expert, (const bf16_t*)w, ldm, F, width, ldo, 0,
+            0.f, out, nullptr);
   DA_CHECK_LAUNCH("moe_down_mfma");
   return 0;
 }
