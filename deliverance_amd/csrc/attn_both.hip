@@ -14,13 +14,14 @@
 // spill: the first of the above 24.6, 8 sequences beside 512 rows 18.0, 60 of 1,000 keys 41.6)
 template <bool BT_LDS>
 __global__ void __launch_bounds__(512, 2)
-attn_both_kernel(const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache, const int* __restrict__ block_table, int max_blocks,
-                 const int* __restrict__ q_start, const int* __restrict__ seq_lens, int n_decode, int n_portions, int n_blocks, int Hq, int Hkv,
-                 int page, float scale, int window, bf16_t* __restrict__ out, int out_ld) {
+attn_both_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, const int* __restrict__ block_table,
+                 const int* __restrict__ seq_lens, int n_portions, int n_blocks, int Hq, int q_ld, int max_blocks, int Hkv,
+                 const int* __restrict__ q_start, int n_decode, int page, float scale, int window, bf16_t* __restrict__ out, int out_ld) {
   const int pairs = n_portions * Hq, id = (int)blockIdx.x - pairs * n_blocks;
   if (id < 0) {
-    attn_prefill_body<4, 4, 2, BT_LDS>((int)blockIdx.x % pairs, (int)blockIdx.x / pairs, n_blocks, q, q_ld, cache, block_table, max_blocks,
-                                       q_start, seq_lens, n_decode, Hq, Hkv, page, scale, window, out, out_ld);
+    const int pair = (int)blockIdx.x % pairs;
+    attn_prefill_body<4, 4, 2, BT_LDS>(pair / Hq, pair % Hq, (int)blockIdx.x / pairs, n_blocks, q, cache, block_table, q_start, seq_lens, q_ld,
+                                       max_blocks, Hq, Hkv, n_decode, page, scale, window, out, out_ld);
     return;
   }
   attn_decode_body<2, 8, false>(id / Hq, id % Hq, q, cache, block_table, seq_lens, q_ld, max_blocks, Hq, Hkv, 64, page, scale, window, out, out_ld, 0, nullptr);
@@ -63,8 +64,9 @@ extern "C" int da_attn_both(const void* q, int q_ld, const void* cache, const in
   DA_REQUIRE(window >= 0 && max_blocks > 0 && scale > 0.f, "attn_both: bad window, block table or scale");
   const int n_blocks = da_ceil_div(max_query_len, 128);
   const dim3 grid(n_portions * Hq * n_blocks + n_decode * Hq);
-#define AB_GO(L) hipLaunchKernelGGL((attn_both_kernel<L>), grid, dim3(512), 0, (hipStream_t)stream, (const bf16_t*)q, q_ld, (const bf16_t*)cache, \
-                                    block_table, max_blocks, q_start, seq_lens, n_decode, n_portions, n_blocks, Hq, Hkv, page, scale, window, (bf16_t*)out, out_ld)
+#define AB_GO(L) hipLaunchKernelGGL((attn_both_kernel<L>), grid, dim3(512), 0, (hipStream_t)stream, (const bf16_t*)q, (const bf16_t*)cache, \
+                                    block_table, seq_lens, n_portions, n_blocks, Hq, q_ld, max_blocks, Hkv, q_start, n_decode, page, scale, window, \
+                                    (bf16_t*)out, out_ld)
   if (max_blocks <= PF_BT_MAX_PHASED) AB_GO(true); else AB_GO(false);
 #undef AB_GO
   DA_CHECK_LAUNCH("attn_both");

@@ -36,6 +36,7 @@
 // build has none of that code.
 #include "common.h"
 #include <da_lane_swap.h>
+#include <da_read_arg.h>
 #include <type_traits>
 
 #ifdef PF_REL
@@ -65,24 +66,25 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 // Included by attn_both.hip (DA_ATTN_BODIES) the kernel is a function that is told which workgroup it is.
 template <int D16, int RB, int KP, bool BT_LDS>
 #ifdef DA_ATTN_BODIES
-#define PF_PAIR pf_pair
+#define PF_SEQ pf_seq
 #define PF_BLOCK pf_block
 #define PF_BLOCKS pf_blocks
 __device__ __forceinline__ void
-attn_prefill_body(int pf_pair, int pf_block, int pf_blocks,
+attn_prefill_body(int pf_seq, int h, int pf_block, int pf_blocks,
 #else
-#define PF_PAIR (int)blockIdx.x
-#define PF_BLOCK (int)blockIdx.y
-#define PF_BLOCKS (int)gridDim.y
+#define PF_SEQ (int)blockIdx.y
+#define PF_BLOCK (int)blockIdx.z
+#define PF_BLOCKS (int)gridDim.z
 // (head sizes up to 64 with four wavefronts: registers held to 256, so that two workgroups share a compute unit)
 __global__ void __launch_bounds__(RB * KP * DA_WAVE, (RB * KP == 4 && D16 <= 4) ? 2 : 1)
 PF_KERNEL(
 #endif
-          const bf16_t* __restrict__ q, int q_ld, const bf16_t* __restrict__ cache,
-          const int* __restrict__ block_table, int max_blocks,
-          const int* __restrict__ q_start, const int* __restrict__ seq_lens, int seq0,
-          int Hq, int Hkv, int page, float scale, int window,
-          bf16_t* __restrict__ out, int out_ld PF_REL_PARAMS) {
+          const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, const int* __restrict__ block_table,
+          const int* __restrict__ q_start, const int* __restrict__ seq_lens, int q_ld, int max_blocks, int Hq, int Hkv, int seq0,
+          int page, float scale, int window, bf16_t* __restrict__ out, int out_ld PF_REL_PARAMS) {
+#ifndef DA_ATTN_BODIES
+  const int h = blockIdx.x;
+#endif
   constexpr int D = D16 * 16;
   constexpr int DT = (D + 31) / 32;       // 32-dimension tiles of the output
   constexpr int KLD = D + 8;              // padded length of a key row in LDS
@@ -110,16 +112,20 @@ PF_KERNEL(
 #endif
 
   // The workgroups with the most keys (the last rows) are launched first, those of every (sequence, head) pair
-  // before anybody's second-longest: blockIdx.x, which the dispatcher counts up first, is the pair.  (Counted the
+  // before anybody's second-longest: the head and the sequence are the sizes that the dispatcher counts up first.  (Counted the
   // other way round, the long workgroups of the later pairs start when the chip is already full of short ones, and
   // the step ends with a few compute units walking their keys alone: at 2 x 4,096 rows and 12 heads the wavefronts
   // resident over the kernel's time averaged 0.9 a SIMD of 2.)
-  const int s = seq0 + PF_PAIR / Hq, h = PF_PAIR % Hq;
-  const int row0 = q_start[s], T = q_start[s + 1] - row0;
+  const int s = seq0 + PF_SEQ;
+  const int row0 = q_start[s], row1 = q_start[s + 1], len = seq_lens[s];
+  da_read_arg(scale);
+  da_read_arg(out);
+  da_read_arg(out_ld);
+  const int T = row1 - row0;
   const int i0 = (PF_BLOCKS - 1 - PF_BLOCK) * PF_BQ;
   if (i0 >= T) return;
-  const int past = seq_lens[s] - T;
-  const int hk = h / (Hq / Hkv);
+  const int past = len - T;
+  const int hk = Hq == Hkv ? h : h / (Hq / Hkv);
   const int* bt = block_table + (size_t)s * max_blocks;
   const int t = threadIdx.x, lane = t % DA_WAVE, wave = t / DA_WAVE;
   const int col = lane % 32, hf = lane / 32;
@@ -617,9 +623,9 @@ extern "C" int da_attn_prefill(const void* q, int q_ld, const void* cache, const
   // every key a workgroup can see lies within max_blocks pages
   const bool bt_lds = max_blocks <= (chosen == 41 ? PF_BT_MAX : PF_BT_MAX_PHASED);
 #define LAUNCH2(N, RB, KP, L)                                                                                  \
-  hipLaunchKernelGGL((PF_KERNEL<N, RB, KP, L>), dim3(Hq * n_seqs, da_ceil_div(max_query_len, 32 * RB)), \
-                     dim3(RB * KP * DA_WAVE), 0, st, (const bf16_t*)q, q_ld, (const bf16_t*)cache, block_table, \
-                     max_blocks, q_start, seq_lens, seq0, Hq, Hkv, page, scale, window, (bf16_t*)out, out_ld PF_REL_ARGS)
+  hipLaunchKernelGGL((PF_KERNEL<N, RB, KP, L>), dim3(Hq, n_here, da_ceil_div(max_query_len, 32 * RB)), \
+                     dim3(RB * KP * DA_WAVE), 0, st, (const bf16_t*)q, (const bf16_t*)cache, block_table, q_start, seq_lens, \
+                     q_ld, max_blocks, Hq, Hkv, s0, page, scale, window, (bf16_t*)out, out_ld PF_REL_ARGS)
 #define LAUNCH3(N, RB, KP)                \
   do {                                    \
     if (bt_lds) LAUNCH2(N, RB, KP, true); \
@@ -641,11 +647,15 @@ extern "C" int da_attn_prefill(const void* q, int q_ld, const void* cache, const
   case N:                                   \
     LAUNCH3(N, 4, 1);                       \
     break;
-  switch (D / 16) {
-    LAUNCH_SMALL(1) LAUNCH_SMALL(2) LAUNCH_SMALL(3) LAUNCH_SMALL(4) LAUNCH_MID(5) LAUNCH_MID(6) LAUNCH_MID(7) LAUNCH_MID(8)
+  // (a head, a sequence and a row block a workgroup, found without a division; a launch's second size ends at 65,535)
+  for (int s0 = seq0; s0 < seq0 + n_seqs; s0 += 65535) {
+    const int n_here = seq0 + n_seqs - s0 < 65535 ? seq0 + n_seqs - s0 : 65535;
+    switch (D / 16) {
+      LAUNCH_SMALL(1) LAUNCH_SMALL(2) LAUNCH_SMALL(3) LAUNCH_SMALL(4) LAUNCH_MID(5) LAUNCH_MID(6) LAUNCH_MID(7) LAUNCH_MID(8)
 #ifndef PF_REL
-    LAUNCH(9) LAUNCH(10) LAUNCH(11) LAUNCH(12) LAUNCH(13) LAUNCH(14) LAUNCH(15) LAUNCH(16)
+      LAUNCH(9) LAUNCH(10) LAUNCH(11) LAUNCH(12) LAUNCH(13) LAUNCH(14) LAUNCH(15) LAUNCH(16)
 #endif
+    }
   }
 #undef LAUNCH
 #undef LAUNCH_MID

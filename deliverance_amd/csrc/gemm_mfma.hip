@@ -237,7 +237,7 @@ template <int BM, int BN, int WM, int WN, int PF_SLABS, int ACT, int OUTMODE, bo
 __device__ __forceinline__ void
 gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
                const Epilogue& ep, const KvScatter& kv, int M, int N, int K, int tiles_m, int tiles_n,
-               char* smem, const Grouping& gr) {
+               char* smem, const Grouping& gr, bool grouped) {
   bf16_t (*As)[BM * LDS_LD] = (bf16_t (*)[BM * LDS_LD])smem;
   bf16_t (*Ws)[BN * LDS_LD] = (bf16_t (*)[BN * LDS_LD])(smem + 2 * BM * LDS_LD * sizeof(bf16_t));
   constexpr int THREADS = WM * WN * 64;
@@ -258,7 +258,7 @@ gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__
   }
   const int tm = pid % tiles_m, tn = pid / tiles_m;
   const int m0 = tm * BM, n0 = tn * BN;
-  if (gr.tile_group) {                      // (the same for the whole workgroup, before any barrier)
+  if (grouped) {                            // (the same for the whole workgroup, before any barrier)
     const int g = gr.tile_group[m0 / gr.rows];
     if (g < 0) return;
     w += (size_t)g * gr.stride;
@@ -324,7 +324,10 @@ gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__
   }
   const int fr = lane % 32, fk = (lane / 32) * 8;
   const int nslab = (K + BKT - 1) / BKT;
-  // The bias is asked for now, as raw bits from a place that always exists, and has long arrived when
+#pragma unroll
+  for (int j = 0; j < PF_SLABS; ++j)
+    if (j < nslab) TILE_FETCH(j, j * BKT);
+  // The bias is asked for behind the first slabs, as raw bits from a place that always exists, and has long arrived when
   // the products are done: a load inside the epilogue's conditions would make every store after it
   // wait for the one before.
   const bool bias_bf16 = ep.bias_dtype == DA_BF16;
@@ -344,9 +347,14 @@ gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__
     const int place = *(has ? kv.slot_map + m0 + t : (const int*)w);
     slot = has ? place : -1;
   }
-#pragma unroll
-  for (int j = 0; j < PF_SLABS; ++j)
-    if (j < nslab) TILE_FETCH(j, j * BKT);
+  // (the arguments that only the epilogue uses, too: a line of them asked for there would be waited for there)
+  da_read_arg(ep.out);
+  da_read_arg(ep.ldo);
+  if (OUTMODE == 0) {
+    da_read_arg(kv.q_cols);
+    da_read_arg(kv.Hkv);
+    da_read_arg(kv.page);
+  }
   TILE_STASH(0, 0);
   lds_barrier();
   // One slab: stage j's registers went to LDS before the last barrier and take the slab PF_SLABS
@@ -401,20 +409,17 @@ gemm_tile_body(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__
 
 template <int BM, int BN, int WM, int WN, int PF, int ACT, int OUTMODE>
 __global__ void __launch_bounds__(WM * WN * 64)
-gemm_tile_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                 Epilogue ep, KvScatter kv, int M, int N, int K, int tiles_m, int tiles_n, Grouping gr, int last) {
-  // The argument behind the others is read and dropped.  Its word, 160 bytes behind the first, is asked for with the rest: products of
-  // 64 x 64 tiles take 0.25 us less by it where results are bfloat16 (80 rows, 3,072 x 1,024 7.46 -> 7.23 us, 201 rows, 4,096 x 1,024 8.0 -> 7.8;
-  // the sums into the stream are level), and so does whatever kernel follows: a step of 355M sizes with 201 rows 1,473 -> 1,459.  An argument
-  // that is passed and not read gives nothing, nor do 4 to 32 idle instructions or the other arguments in another order: it is
-  // the line of memory, presumably that where the next launch's arguments begin.
-  if constexpr (OUTMODE == 0) da_read_arg(last);
+gemm_tile_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const void* bias, int lda, int ldw, int M, int N, int K, int tiles_m,
+                 int tiles_n, int flags, void* out, int ldo, KvScatter kv, Grouping gr) {
+  // (the first 14 words are in registers when the wavefront starts; `flags`: the bias's type, and 0x100 where the rows are grouped)
+  const Epilogue ep{bias, flags & 0xff, ACT, OUTMODE == 2, out, OUTMODE == 0 ? DA_BF16 : DA_F32, ldo};
+  const bool grouped = flags & 0x100;
   // two buffers of a slab of a and of w; the epilogue parks the tile's results in the same memory
   constexpr int SLAB_BYTES = 2 * (BM + BN) * LDS_LD * (int)sizeof(bf16_t);
   constexpr int OUT_BYTES = tile_out_bytes<BM, BN, OUTMODE>() + tile_slot_bytes<BM, OUTMODE>();
   __shared__ __attribute__((aligned(16))) char smem[SLAB_BYTES > OUT_BYTES ? SLAB_BYTES : OUT_BYTES];      // shared by the two bodies
-  if (K % BKT == 0) gemm_tile_body<BM, BN, WM, WN, PF, ACT, OUTMODE, false>(a, lda, w, ldw, ep, kv, M, N, K, tiles_m, tiles_n, smem, gr);
-  else gemm_tile_body<BM, BN, WM, WN, PF, ACT, OUTMODE, true>(a, lda, w, ldw, ep, kv, M, N, K, tiles_m, tiles_n, smem, gr);
+  if (K % BKT == 0) gemm_tile_body<BM, BN, WM, WN, PF, ACT, OUTMODE, false>(a, lda, w, ldw, ep, kv, M, N, K, tiles_m, tiles_n, smem, gr, grouped);
+  else gemm_tile_body<BM, BN, WM, WN, PF, ACT, OUTMODE, true>(a, lda, w, ldw, ep, kv, M, N, K, tiles_m, tiles_n, smem, gr, grouped);
 }
 
 template <int BM, int BN, int WM, int WN, int PF, int ACT>
@@ -422,12 +427,13 @@ static void launch_tile_act(hipStream_t s, const bf16_t* A, int lda, const bf16_
                             const KvScatter& kv, int M, int N, int K, const Grouping& gr) {
   const int tiles_m = da_ceil_div(M, BM), tiles_n = da_ceil_div(N, BN);
   const dim3 grid(tiles_m * tiles_n), block(WM * WN * 64);
+  const int flags = ep.bias_dtype | (gr.tile_group ? 0x100 : 0);
   if (ep.accumulate)
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 2>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, K);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 2>), grid, block, 0, s, A, W, ep.bias, lda, ldw, M, N, K, tiles_m, tiles_n, flags, ep.out, ep.ldo, kv, gr);
   else if (ep.out_dtype == DA_F32)
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 1>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, K);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 1>), grid, block, 0, s, A, W, ep.bias, lda, ldw, M, N, K, tiles_m, tiles_n, flags, ep.out, ep.ldo, kv, gr);
   else
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 0>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, gr, K);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, PF, ACT, 0>), grid, block, 0, s, A, W, ep.bias, lda, ldw, M, N, K, tiles_m, tiles_n, flags, ep.out, ep.ldo, kv, gr);
 }
 
 template <int BM, int BN, int WM, int WN, int PF>

@@ -26,6 +26,7 @@
 // values in 8-byte runs where 4 rows' places are consecutive: kv_all_runs).
 #include "gemm_common.h"
 #include <da_lds_dma.h>
+#include <da_read_arg.h>
 #include <type_traits>
 
 #define WD_BK 64
@@ -222,8 +223,10 @@ wide_epilogue(floatx16 (&acc)[TM][TN], const float (&bias)[TN], char* region, co
 // 128 x 128 with 2 x 2 wavefronts of 64 x 64 (7 to 10 % behind the eight wavefronts at a short K).
 template <int BM, int BN, int WM, int WN, int ACT, int OUTMODE>
 __global__ void __launch_bounds__(WM * WN * 64)
-gemm_wide_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict__ w, int ldw,
-                 Epilogue ep, KvScatter kv, int M, int N, int K, int tiles_m, int tiles_n, int k_share) {
+gemm_wide_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const void* bias_p, int lda, int ldw, int M, int N, int K,
+                 int tiles_m, int tiles_n, int k_share, int bias_dtype, void* out, int ldo, KvScatter kv) {
+  // (the first 14 words are in registers when the wavefront starts)
+  Epilogue ep{bias_p, bias_dtype, ACT, OUTMODE == 2, out, OUTMODE == 0 ? DA_BF16 : DA_F32, ldo};
   gemm_take_share(a, w, ep, M, K, k_share);
   // Two stages of a slab of a, three of a slab of w.  The rows of a were written by the kernel before and
   // come from a cache; w comes from memory for the first time and needs the longer way ahead.
@@ -305,23 +308,6 @@ gemm_wide_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  // The bias is asked for now, as raw bits from a place that always exists; it has long arrived when
-  // the products are done.  No other ordinary load stands between here and the end of the slabs, so
-  // that the copies' count of outstanding loads is exact.
-  const bool bias_bf16 = ep.bias_dtype == DA_BF16;
-  uint32_t braw[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn + j * 32 + fr;
-    const bool has = ep.bias && n < N;
-    const void* bsrc = has ? ep.bias : (const void*)w;
-    const int idx = has ? n : 0;
-    braw[j] = bias_bf16 ? (uint32_t)((const bf16_t*)bsrc)[idx] : ((const uint32_t*)bsrc)[idx];
-  }
-  float bias[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) bias[j] = !ep.bias ? 0.f : (bias_bf16 ? __uint_as_float(braw[j] << 16) : __uint_as_float(braw[j]));
-
   // Order of the copies: a(0) w(0) | a(1) w(1) | w(2) | then, after the barrier that ends slab s, a(s + 2)
   // and w(s + 3) into the stages that slab s left.  Copies land in the order they were asked for, so
   // "slab s + 1 is there" is "at most the four youngest copies, w(s + 2), are still under way".
@@ -340,6 +326,27 @@ gemm_wide_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict
   if (nslab > 2) {
 #pragma unroll
     for (int i = 0; i < CW; ++i) WD_COPY_W(i, 2);
+  }
+  // The bias is asked for behind the first slabs, as raw bits from a place that always exists (the waits below count copies: with the
+  // bias's loads among the youngest they wait for a copy or two more than they need, once), with the arguments that only the epilogue
+  // uses.  No other ordinary load stands between here and the end of the slabs.
+  const bool bias_bf16 = ep.bias_dtype == DA_BF16;
+  uint32_t braw[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wn + j * 32 + fr;
+    const bool has = ep.bias && n < N;
+    const void* bsrc = has ? ep.bias : (const void*)w;
+    const int idx = has ? n : 0;
+    braw[j] = bias_bf16 ? (uint32_t)((const bf16_t*)bsrc)[idx] : ((const uint32_t*)bsrc)[idx];
+  }
+  da_read_arg(ep.out);
+  da_read_arg(ep.ldo);
+  if (OUTMODE == 0) {
+    da_read_arg(kv.cache);
+    da_read_arg(kv.q_cols);
+    da_read_arg(kv.Hkv);
+    da_read_arg(kv.page);
   }
   static_assert(CA + 2 * CW <= 15, "the count of copies under way fits its field");
   if (nslab > 2) DA_WAIT_VMCNT(CA + 2 * CW); else if (nslab > 1) DA_WAIT_VMCNT(CA + CW); else DA_WAIT_VMCNT(0);
@@ -411,6 +418,9 @@ gemm_wide_kernel(const bf16_t* __restrict__ a, int lda, const bf16_t* __restrict
 #undef WD_MFMA
 #undef WD_MFMA1
 #undef WD_FENCE
+  float bias[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) bias[j] = !ep.bias ? 0.f : (bias_bf16 ? __uint_as_float(braw[j] << 16) : __uint_as_float(braw[j]));
   // (the last barrier of the loop: nobody reads the stages any more)
   wide_epilogue<TM, TN, ACT, OUTMODE>(acc, bias, smem + wave * WD_REGION_BYTES, (const void*)w, ep, kv, M, N, m0 + wm, n0 + wn, lane);
 }
@@ -421,11 +431,11 @@ static void launch_wide_act(hipStream_t s, const bf16_t* A, int lda, const bf16_
   const int tiles_m = da_ceil_div(M, BM), tiles_n = da_ceil_div(N, BN);
   const dim3 grid(tiles_m * tiles_n, da_ceil_div(K, k_share)), block(WM * WN * 64);
   if (ep.accumulate)
-    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, DA_ACT_NONE, 2>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, k_share);
+    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, DA_ACT_NONE, 2>), grid, block, 0, s, A, W, ep.bias, lda, ldw, M, N, K, tiles_m, tiles_n, k_share, ep.bias_dtype, ep.out, ep.ldo, kv);
   else if (ep.out_dtype == DA_F32)
-    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, DA_ACT_NONE, 1>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, k_share);
+    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, DA_ACT_NONE, 1>), grid, block, 0, s, A, W, ep.bias, lda, ldw, M, N, K, tiles_m, tiles_n, k_share, ep.bias_dtype, ep.out, ep.ldo, kv);
   else
-    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, ACT, 0>), grid, block, 0, s, A, lda, W, ldw, ep, kv, M, N, K, tiles_m, tiles_n, k_share);
+    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WM, WN, ACT, 0>), grid, block, 0, s, A, W, ep.bias, lda, ldw, M, N, K, tiles_m, tiles_n, k_share, ep.bias_dtype, ep.out, ep.ldo, kv);
 }
 
 template <int BM, int BN, int WM, int WN>

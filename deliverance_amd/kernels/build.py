@@ -41,8 +41,8 @@ EXTRA_FLAGS = {"attn_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 # Units whose kernels find their first arguments in registers when a wavefront starts: the hardware reads up to 14 words of them ahead,
 # as long as they are single numbers and pointers (a structure ends them).
 KERNARG_PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
-PRELOADED = ("gemm_mfma", "gemm_fused", "gemm_shares", "attn_decode", "attn_decode_rel", "rowwise", "norm_rms", "gemm_f32",
-             "attn_f32", "moe", "elementwise")
+PRELOADED = ("gemm_mfma", "gemm_wide", "gemm_fused", "gemm_shares", "attn_decode", "attn_decode_rel", "rowwise", "norm_rms", "gemm_f32",
+             "attn_f32", "moe", "elementwise", "attn_prefill", "attn_prefill_rel", "attn_both")
 # The unit that holds the error message every entry point may leave; every other unit needs it.
 BASE_UNIT = "rowwise"
 # Units whose functions a unit calls.
