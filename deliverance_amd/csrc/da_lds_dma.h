@@ -16,3 +16,5 @@ __device__ __forceinline__ void lds_dma16(const void* g, void* lds_wave_base) {
 
 // (lgkmcnt and expcnt are left alone: all ones in their fields)
 #define DA_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(0x0F70 | (n))
+// (up to 63: the count has two fields)
+#define DA_WAIT_VMCNT6(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | ((n) >> 4 << 14))

@@ -425,6 +425,240 @@ gemm_wide_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, con
   wide_epilogue<TM, TN, ACT, OUTMODE>(acc, bias, smem + wave * WD_REGION_BYTES, (const void*)w, ep, kv, M, N, m0 + wm, n0 + wn, lane);
 }
 
+// Which tile a workgroup takes.  Workgroups that follow each other in launch order land on different dies (8, each with an L2 of its
+// own), and what a die reads of a and w it reads from behind its L2 once: with 2^lg_m blocks of tiles by rows and 8 / 2^lg_m by
+// columns, a die a block, as few rows and columns as the shape allows.  Where the blocks' sizes differ so much that a die would have a
+// round of tiles more (DIE_RUNS), runs of tiles, rows first, as gemm_wide_kernel has them.  False: no tile for this workgroup.
+// (1,624 rows, N = 1,024, K = 4,096 and 1,024 in a step, the mean of the two in a profiled run: runs 20.7 us, blocks 20.1.)
+#define DIE_RUNS 4
+__device__ __forceinline__ bool die_tile(int id, int tiles_m, int tiles_n, int lg_m, int& tile_m, int& tile_n) {
+  const int die = id % 8, local = id / 8;
+  if (lg_m == DIE_RUNS) {
+    const int n = tiles_m * tiles_n, per = n / 8, rem = n % 8, pid = die * per + (die < rem ? die : rem) + local;
+    tile_n = pid / tiles_m;
+    tile_m = pid - tile_n * tiles_m;
+    return local < per + (die < rem ? 1 : 0);
+  }
+  const int xm = die & ((1 << lg_m) - 1), xn = die >> lg_m, lg_n = 3 - lg_m;
+  const int m_lo = (xm * tiles_m) >> lg_m, m_n = (((xm + 1) * tiles_m) >> lg_m) - m_lo;
+  const int n_lo = (xn * tiles_n) >> lg_n, n_n = (((xn + 1) * tiles_n) >> lg_n) - n_lo;
+  if (local >= m_n * n_n) return false;
+  const int q = local / m_n;
+  tile_m = m_lo + local - q * m_n;
+  tile_n = n_lo + q;
+  return true;
+}
+struct DieCut { int lg_m, workgroups; };
+static DieCut die_cut(int tiles_m, int tiles_n, int bm, int bn) {
+  const long tiles = (long)tiles_m * tiles_n;
+  const int rounds = da_ceil_div(da_ceil_div(tiles, 8), 32);          // of 32 compute units a die
+  DieCut best{DIE_RUNS, (int)tiles};
+  long least = 0;
+  for (int lg = 0; lg <= 3; ++lg) {
+    const int m = da_ceil_div(tiles_m, 1 << lg), n = da_ceil_div(tiles_n, 8 >> lg);
+    if (da_ceil_div((long)m * n, 32) > rounds) continue;
+    const long rows = (long)m * bm + (long)n * bn;
+    if (best.lg_m == DIE_RUNS || rows < least) { best = DieCut{lg, 8 * m * n}; least = rows; }
+  }
+  return best;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Products into the residual stream that leave a tile or less to a compute unit: k shared out inside the workgroup.
+//
+// A compute unit pulls 62 to 68 GB/s out of L2 whatever is in flight (tiles of 128 x 128 and 128 x 64, one a compute unit, one to five
+// slabs ahead, copies alone: 2,048 rows, N = 1,600, K = 6,400 52 us; 1,624 rows, N = 1,024, K = 4,096 24 us), so the tile is given and
+// what is left is to keep that stream going.  The tiles of gemm_mfma.hip at these sizes wait for LDS instead: their wavefronts of 32 x 64
+// (32 x 32) read 96 KB (64) of fragments for a slab of 32 (24) KB.  Here a wavefront has 64 x 64 of the tile and KG wavefronts share a
+// position, each with every KG-th k-step: 64 KB (32) a slab, and eight wavefronts to hide each other's waits all the same.  Operands go
+// straight into LDS, S slabs ahead (all of LDS: a workgroup a compute unit); a wavefront's fragments of the next slab are read between
+// this slab's products; one barrier a slab, after which the stage it stands for is free.  The wavefronts of a position leave their sums
+// in LDS, and the first of them add them up in order of k-steps, 32 rows each: an element is KG sums, each in ascending k, added one to the other.
+// us alone, cold weights, gemm_mfma.hip's tiles -> this: 2,048 rows, N = 1,600, K = 6,400 64.7 -> 60.4 (695 TFLOP/s), 1,624 rows, N = 1,024,
+// K = 4,096 27.9 -> 24.3 (560); error against 64 bits 4.9e-7 -> 3.4e-7 and 3.8e-7 -> 1.8e-7.
+// ---------------------------------------------------------------------------------------------
+template <int BM, int BN, int KG, int S>
+__global__ void __launch_bounds__(512)
+gemm_deep_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const void* bias_p, int lda, int ldw, int M, int N, int K,
+                 int tiles, int lg_m, int ldo, int bias_dtype, float* out) {
+  constexpr int NW = 8, WM = BM / 64, WN = BN / 64, TM = 2, TN = 2, KS = 4 / KG;      // k-steps of a slab a wavefront
+  static_assert(WM * WN * KG == NW && KS >= 1 && KG >= 2, "eight wavefronts");
+  constexpr int A_BYTES = BM * WD_ROW_BYTES, STAGE = A_BYTES + BN * WD_ROW_BYTES;
+  constexpr int CA = BM / 8 / NW, CW = BN / 8 / NW, C = CA + CW;                      // copies a wavefront and slab
+  static_assert(C * (S - 1) <= 63, "the count of copies under way fits its field");
+  constexpr int SUM_BYTES = WM * WN * TM * TN * (KG - 1) * 4096;
+  static_assert(SUM_BYTES + TM * WM * WN * WD_REGION_BYTES <= S * STAGE, "the wavefronts' sums and the epilogue's regions fit the stages");
+  __shared__ __attribute__((aligned(1024))) char smem[S * STAGE];
+
+  int tile_m, tile_n;
+  if (!die_tile(blockIdx.x, tiles & 0xffff, tiles >> 16, lg_m, tile_m, tile_n)) return;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int t = threadIdx.x, lane = t % 64, wave = __builtin_amdgcn_readfirstlane(t / 64);
+  const int kg = wave / (WM * WN), pos = wave % (WM * WN), wm = (pos % WM) * 64, wn = (pos / WM) * 64;
+  const int fr = lane % 32, fk = lane / 32;
+
+  const bf16_t* src[C];
+  int dst[C];
+  {
+    const int rl = lane / 8, piece = (lane % 8) ^ ((4 * (wave & 1) + (rl >> 1)) & 7);   // (rows lie in LDS as in gemm_wide_kernel)
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const int b = (i < CA ? i : i - CA) * NW + wave, r = (i < CA ? m0 : n0) + b * 8 + rl;
+      src[i] = (i < CA ? a + (size_t)(r < M ? r : M - 1) * lda : w + (size_t)(r < N ? r : N - 1) * ldw) + piece * 8;
+      dst[i] = (i < CA ? 0 : A_BYTES) + b * 1024;
+    }
+  }
+  int a_off[TM], w_off[TN], k_off[KS];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) a_off[i] = (wm + i * 32 + fr) * WD_ROW_BYTES;
+#pragma unroll
+  for (int j = 0; j < TN; ++j) w_off[j] = A_BYTES + (wn + j * 32 + fr) * WD_ROW_BYTES;
+#pragma unroll
+  for (int i = 0; i < KS; ++i) k_off[i] = ((2 * (kg + i * KG) + fk) ^ ((fr >> 1) & 7)) * 16;
+
+  auto copy = [&](int stage) {
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      lds_dma16(src[i], smem + stage * STAGE + dst[i]);
+      src[i] += WD_BK;
+    }
+  };
+  struct Frags { bf16x8_t a[KS][TM], w[KS][TN]; };
+  auto read1 = [&](Frags& f, int stage, int q) {                     // fragment q of a slab's KS (TM + TN)
+    const char* const p = smem + stage * STAGE;
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+#pragma unroll
+      for (int x = 0; x < TM; ++x)
+        if (q == i * (TM + TN) + x) f.a[i][x] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(p + k_off[i] + a_off[x]));
+#pragma unroll
+      for (int x = 0; x < TN; ++x)
+        if (q == i * (TM + TN) + TM + x) f.w[i][x] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(p + k_off[i] + w_off[x]));
+    }
+  };
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  const int nslab = K / WD_BK;                                        // S at least (checked on the host)
+#pragma unroll
+  for (int i = 0; i < S; ++i) copy(i);
+  const bool bias_bf16 = bias_dtype == DA_BF16;
+  uint32_t braw[TN];                                                  // (behind the first copies: as in gemm_wide_kernel)
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wn + j * 32 + fr;
+    const bool has = bias_p && n < N;
+    const void* bsrc = has ? bias_p : (const void*)w;
+    braw[j] = bias_bf16 ? (uint32_t)((const bf16_t*)bsrc)[has ? n : 0] : ((const uint32_t*)bsrc)[has ? n : 0];
+  }
+  da_read_arg(out);
+  DA_WAIT_VMCNT6(C * (S - 1));
+  __builtin_amdgcn_s_barrier();
+  Frags f0, f1;
+#pragma unroll
+  for (int q = 0; q < KS * (TM + TN); ++q) read1(f0, 0, q);
+  int stage = 0;                                                      // slab s's
+  // Slab s: its fragments are in `now` when the barrier is passed, slab s + 1 is in LDS, and stage s % S is free.  LEFT: slabs behind s + 1
+  // that may still be under way; COPY: slab s + S exists; NEXT: slab s + 1 does.
+  auto slab = [&](Frags& now, Frags& next, auto left_c, auto copy_c, auto next_c) {
+    constexpr int LEFT = decltype(left_c)::value;
+    constexpr bool COPY = decltype(copy_c)::value, NEXT = decltype(next_c)::value;
+    const int after = stage + 1 == S ? 0 : stage + 1;
+    if (NEXT) {
+      DA_WAIT_VMCNT6(C * LEFT);
+      __builtin_amdgcn_s_waitcnt(0xC07F);                            // lgkmcnt(0): slab s's fragments have arrived
+      __builtin_amdgcn_s_barrier();
+      if (COPY) copy(stage);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int NQ = KS * TM * TN;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      constexpr int TT = TM * TN;
+      const int i = q / TT, x = q % TT / TN, y = q % TN;
+      acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.a[i][x], now.w[i][y], acc[x][y], 0, 0, 0);
+      if (NEXT && q < KS * (TM + TN)) read1(next, after, q);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    static_assert(NQ >= KS * (TM + TN), "a read behind each product");
+    stage = after;
+  };
+  {
+    const std::true_type yes{};
+    const std::false_type no{};
+    const std::integral_constant<int, S - 2> steady{};
+    int s = 0;
+    for (; s + 1 < nslab - S; s += 2) {
+      slab(f0, f1, steady, yes, yes);
+      slab(f1, f0, steady, yes, yes);
+    }
+    // the last S slabs, whose copies are all asked for
+    auto tail = [&](Frags& x, Frags& y) {
+      slab(x, y, std::integral_constant<int, S - 2>{}, no, yes);
+      if constexpr (S >= 3) slab(y, x, std::integral_constant<int, S - 3>{}, no, yes);
+      if constexpr (S >= 4) slab(x, y, std::integral_constant<int, S >= 4 ? S - 4 : 0>{}, no, yes);
+      if constexpr (S >= 5) slab(y, x, std::integral_constant<int, S >= 5 ? S - 5 : 0>{}, no, yes);
+      if constexpr (S >= 6) slab(x, y, std::integral_constant<int, S >= 6 ? S - 6 : 0>{}, no, yes);
+      static_assert(S >= 5 && S <= 6, "the tail is written out for five and six stages");
+      if constexpr (S == 5) slab(x, y, std::integral_constant<int, 0>{}, no, no);
+      else slab(y, x, std::integral_constant<int, 0>{}, no, no);
+    };
+    if (s < nslab - S) {
+      slab(f0, f1, steady, yes, yes);
+      tail(f1, f0);
+    } else tail(f0, f1);
+  }
+  float bias[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) bias[j] = !bias_p ? 0.f : (bias_bf16 ? __uint_as_float(braw[j] << 16) : __uint_as_float(braw[j]));
+  // the sums of a position's wavefronts meet: wavefront kg < TM owns the rows 32 kg .. of it; a wavefront leaves in LDS what it does not own
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();                                       // (nobody reads the stages any more)
+  float* const sums = (float*)smem;
+  auto place = [&](int x, int g, int y) { return sums + ((((x * (KG - 1) + (g > x ? g - 1 : g)) * WM * WN + pos) * TN + y) * 16) * 64 + lane; };
+#pragma unroll
+  for (int x = 0; x < TM; ++x)
+    if (kg != x) {
+#pragma unroll
+      for (int y = 0; y < TN; ++y)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) place(x, kg, y)[r * 64] = acc[x][y][r];
+    }
+  lds_barrier();
+  if (kg >= TM) return;
+  floatx16 sum[1][TN];
+  auto add = [&](auto xc) {
+    constexpr int x = decltype(xc)::value;
+#pragma unroll
+    for (int y = 0; y < TN; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float v = x == 0 ? acc[x][y][r] : place(x, 0, y)[r * 64];
+#pragma unroll
+        for (int g = 1; g < KG; ++g) v += g == x ? acc[x][y][r] : place(x, g, y)[r * 64];
+        sum[0][y][r] = v;
+      }
+  };
+  if (kg == 0) add(std::integral_constant<int, 0>{});
+  else add(std::integral_constant<int, 1>{});
+  const Epilogue ep{bias_p, bias_dtype, DA_ACT_NONE, 1, out, DA_F32, ldo};
+  const KvScatter kv{nullptr, nullptr, 0, 0, 0, 0, 0};
+  wide_epilogue<1, TN, DA_ACT_NONE, 2>(sum, bias, smem + SUM_BYTES + wave * WD_REGION_BYTES, (const void*)w, ep, kv, M, N, m0 + wm + 32 * kg, n0 + wn, lane);
+}
+
+template <int BM, int BN, int KG, int S>
+static void launch_deep(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep, int M, int N, int K) {
+  const int tiles_m = da_ceil_div(M, BM), tiles_n = da_ceil_div(N, BN);
+  const DieCut cut = die_cut(tiles_m, tiles_n, BM, BN);
+  hipLaunchKernelGGL((gemm_deep_kernel<BM, BN, KG, S>), dim3(cut.workgroups), dim3(512), 0, s, A, W, ep.bias, lda, ldw, M, N, K,
+                     tiles_m | tiles_n << 16, cut.lg_m, ep.ldo, ep.bias_dtype, (float*)ep.out);
+}
+
 template <int BM, int BN, int WM, int WN, int ACT>
 static void launch_wide_act(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
                             const KvScatter& kv, int M, int N, int K, int k_share) {
@@ -482,9 +716,29 @@ int da_gemm_wide_choice(int M, int N, int K) {
   return DA_WIDE_NONE;
 }
 
+// Which of the deep tiles a product into the stream takes, if any: those that are one a compute unit at most, where the tiles that the
+// other forms have are more than that, or wait for LDS.  Measured on MI355X with cold weights, K from 1,024 to 8,192, us, other forms / deep:
+//  - 128 x 64 where there are up to 256 of them and tiles of 64 x 64 would be more: 1,624 rows, N = 1,024, K = 4,096 27.9 / 24.3, K = 1,024
+//    11.1 / 11.1; 1,300 rows, K = 4,096 29.6 / 22.8; 900 rows, N = K = 2,048 19.5 / 16.3; 2,048 rows, N = 768, K = 3,072 21.8 / 21.8.  Where tiles of
+//    64 x 64 are one a compute unit themselves they stay (1,024 rows, N = 1,024, K = 4,096, 256 of them: 20.2 / 22.0);
+//  - 128 x 128 where there are up to 256 of them and of 128 x 64 more, K from 3,072: 2,048 rows, N = 1,600, K = 6,400 64.7 / 60.4, 1,624 rows
+//    73.1 / 56.9; 2,048 rows, N = 1,536, K = 3,072 33.8 / 33.8; 1,300 rows, N = 2,048, K = 8,192 93.9 / 60.5.  (K = 2,048: 4,096 rows, N = 1,024 26.1 / 27.1;
+//    two rounds of them: 4,096 rows, N = 2,048, K = 4,096 84.6 / 102.5.)
+extern "C" int da_gemm_deep_choice(int M, int N, int K) {
+  if (K % WD_BK || K < DA_DEEP_MIN_K) return DA_WIDE_NONE;
+  const long t64 = (long)da_ceil_div(M, 64) * da_ceil_div(N, 64), t12864 = (long)da_ceil_div(M, 128) * da_ceil_div(N, 64);
+  if (t12864 <= 256) return t64 > 256 ? DA_DEEP_128x64 : DA_WIDE_NONE;
+  return K >= 3072 && (long)da_ceil_div(M, 128) * da_ceil_div(N, 128) <= 256 ? DA_DEEP_128x128 : DA_WIDE_NONE;
+}
+
 void da_gemm_wide_launch(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,
                          const KvScatter& kv, int M, int N, int K, int shape, int k_share) {
   if (k_share <= 0) k_share = K;
+  if (shape == DA_DEEP_128x128 || shape == DA_DEEP_128x64) {          // (up to 32,767 tiles each way: checked where a shape is asked for)
+    if (shape == DA_DEEP_128x128) launch_deep<128, 128, 2, 5>(s, A, lda, W, ldw, ep, M, N, K);
+    else launch_deep<128, 64, 4, 6>(s, A, lda, W, ldw, ep, M, N, K);
+    return;
+  }
   if (shape == DA_WIDE_128x128) launch_wide<128, 128, 4, 2>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share);
   else if (shape == DA_WIDE_256x128) launch_wide<256, 128, 4, 2>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share);
   else launch_wide<256, 256, 2, 4>(s, A, lda, W, ldw, ep, kv, M, N, K, k_share);
@@ -496,7 +750,9 @@ extern "C" int da_gemm_bf16_wide(const void* a, int lda, const void* w, int ldw,
                                  int act, int accumulate, void* out, int out_dtype, int ldo, int M, int N, int K,
                                  void* kv_cache, const int* slot_map, int q_cols, int kv_cols, int Hkv, int D, int page,
                                  int shape, void* stream) {
-  DA_REQUIRE(shape >= DA_WIDE_256x256 && shape <= DA_WIDE_128x128, "gemm_bf16_wide: unknown tile shape %d", shape);
+  DA_REQUIRE(shape >= DA_WIDE_256x256 && shape <= DA_DEEP_128x64, "gemm_bf16_wide: unknown tile shape %d", shape);
+  DA_REQUIRE(shape <= DA_WIDE_128x128 || (accumulate && !kv_cache && K >= DA_DEEP_MIN_K), "gemm_bf16_wide: this shape adds into the stream, K from %d on", DA_DEEP_MIN_K);
+  DA_REQUIRE(shape <= DA_WIDE_128x128 || (da_ceil_div(M, 128) < 32768 && da_ceil_div(N, 64) < 32768), "gemm_bf16_wide: too many tiles for this shape");
   DA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_bf16_wide: bad sizes M=%d N=%d K=%d", M, N, K);
   DA_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K && ldo >= N, "gemm_bf16_wide: leading sizes (lda=%d ldw=%d ldo=%d)", lda, ldw, ldo);
   DA_REQUIRE(((uintptr_t)a % 16 == 0) && ((uintptr_t)w % 16 == 0), "gemm_bf16_wide: operands must be 16-byte aligned");

@@ -52,7 +52,7 @@ NEEDS = {"gemm_mfma": ("gemm_wide",), "gemm_shares": ("gemm_wide",),
 # reading their unit's own source.
 INCLUDES = {"attn_decode_rel": ("attn_decode",), "attn_prefill_rel": ("attn_prefill",), "attn_both": ("attn_decode", "attn_prefill")}
 _ELSEWHERE = {"da_attn_decode_rel": "attn_decode_rel", "da_attn_prefill_rel": "attn_prefill_rel",
-              "da_attn_prefill_rel_max_dist": "attn_prefill_rel", "da_gemm_wide_choice": "gemm_wide"}
+              "da_attn_prefill_rel_max_dist": "attn_prefill_rel", "da_gemm_wide_choice": "gemm_wide", "da_gemm_deep_choice": "gemm_wide"}
 
 _lib = None
 

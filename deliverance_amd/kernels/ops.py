@@ -845,7 +845,7 @@ def _kv_args(kv_cache, slot_map, q_cols, n_rows, N, out, name):
     return _ptr(kv_cache), _ptr(slot_map), q_cols, Hkv * D, Hkv, D, page
 
 
-WIDE_TILE_SHAPES = {"wide": 0, "wide_256x128": 1, "wide_128x128": 2}
+WIDE_TILE_SHAPES = {"wide": 0, "wide_256x128": 1, "wide_128x128": 2, "deep_128x128": 3, "deep_128x64": 4}
 
 
 def _wide_tiles(M, N, K, act, accumulate, out) -> bool:
@@ -862,7 +862,8 @@ def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
     ``kv_cache`` the columns from ``q_cols`` on (k | v) also go to the cache rows ``slot_map``.
     ``form``: "auto" lets the library choose by shape; "wide", "wide_256x128" and "wide_128x128" ask for the
     tiles of 256 x 256, 256 x 128 and 128 x 128 whose operands go from memory straight into LDS, whatever
-    the product's sizes (K a multiple of 64; tests and timing)."""
+    the product's sizes (K a multiple of 64; tests and timing); "deep_128x128" and "deep_128x64" for those that share k out
+    over the wavefronts of a workgroup (into a 32-bit stream, K from 1,024 on)."""
     _dev(a, w, bias, out)
     _rows_2d(a, "a"); _rows_2d(w, "w"); _rows_2d(out, "out")
     M, K = a.shape

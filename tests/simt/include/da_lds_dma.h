@@ -9,4 +9,5 @@ static inline void lds_dma16(const void* g, void* lds_wave_base) {
 }
 
 #define DA_WAIT_VMCNT(n) ((void)0)
+#define DA_WAIT_VMCNT6(n) ((void)0)
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)

@@ -447,6 +447,34 @@ def test_gemm_wide_tiles(ops, M, N, K, form):
         ops.linear_mfma(a[:, :K - 8].contiguous(), w[:, :K - 8].contiguous(), b, o1, form=form)
 
 
+@pytest.mark.parametrize("form", ["deep_128x128", "deep_128x64"])
+@pytest.mark.parametrize("M,N,K", [helpers.quick(130, 70, 1024), (128, 128, 1088), (257, 200, 1152), (640, 1600, 6400), (1624, 1024, 4096)])
+def test_gemm_deep_tiles(ops, M, N, K, form):
+    """The tiles that add into the stream with k shared out over the wavefronts of a workgroup (two and four a position), five and six
+    slabs ahead: an odd and an even number of slabs, edges in M and N.  A sum of K products of bfloat16 in 32-bit, in 16 or more
+    partial sums of a product's own k, is off by less than K / 16 roundings of 2^-24 of the sum of absolute values."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = bf(torch.randn(M, K, generator=g) * 0.5).to(DEV)
+    w = bf(torch.randn(N, K, generator=g) * 0.2).to(DEV)
+    x = torch.randn(M, N, generator=g).to(DEV)
+    bound = (a.abs().float() @ w.abs().float().t()) * (K / 16 * 2.0 ** -24) + 1e-5
+    ref = x.double().cpu() + a.double().cpu() @ w.double().cpu().t()
+    for bias in (None, bf(torch.randn(N, generator=g)).to(DEV), torch.randn(N, generator=g).to(DEV)):
+        wide = torch.zeros(M, N + 12, device=DEV)
+        out = wide[:, 4:N + 4] if N % 4 == 0 else wide[:, 3:N + 3]
+        out.copy_(x)
+        ops.linear_mfma(a, w, bias, out, None, True, form=form)
+        want = ref if bias is None else ref + bias.double().cpu()
+        assert ((out.double().cpu() - want).abs() <= bound.double().cpu()).all()
+        assert not wide[:, N + 4:].any() and not wide[:, :3].any()
+        if (M, form) == (1624, "deep_128x64"):       # the library's own choice there
+            auto = x.clone()
+            ops.linear_mfma(a, w, bias, auto, None, True)
+            assert torch.equal(auto, out)
+    with pytest.raises(ops.KernelError, match="adds into the stream"):
+        ops.linear_mfma(a, w, None, torch.empty(M, N, device=DEV), form=form)
+
+
 @pytest.mark.parametrize("form", ["wide", "wide_256x128", "wide_128x128"])
 @pytest.mark.parametrize("M", [helpers.quick(300), 1000])
 def test_gemm_wide_tiles_write_keys_and_values(ops, M, form):
