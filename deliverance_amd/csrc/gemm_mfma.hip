@@ -461,10 +461,13 @@ static void launch_tile(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W
 // AL: loads of 8 rows that cover the workgroup's rows of a (1: up to 8 rows; else two a row tile);
 // COLS: 16 output columns a workgroup, or 8 (the fragment of w then holds them twice and half of the
 // result is dropped: with few columns twice the workgroups pull on memory).
-template <int AL, int COLS, int NW, int UNROLL>
+// GATED: w is [2 N, K], gate rows and then up rows; a workgroup's 16 columns are 8 gate columns and the same 8 up columns, and what leaves
+// is gated_mid of their 32-bit sums in bfloat16 (da_gemm_bf16_gated; `gate_limit` is its).
+template <int AL, int COLS, int NW, int UNROLL, bool GATED = false>
 __global__ void __launch_bounds__(NW * 64)
 gemm_skinny_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const void* bias, void* out, int lda, int ldw, int ldo,
-                   int M, int N, int K, EpilogueRest er, KvScatter kv) {
+                   int M, int N, int K, EpilogueRest er, KvScatter kv, float gate_limit) {
+  static_assert(!GATED || COLS == 16, "eight columns of each");
   constexpr int MT = (AL + 1) / 2, WL = COLS / 8;    // row tiles of 16; loads of 8 rows that cover w's columns
   constexpr int AR = MT * 16, TR = AR + COLS;        // rows of a; rows of a step: a's, then w's
   static_assert(COLS == 8 || COLS == 16, "8 or 16 columns a workgroup");
@@ -474,7 +477,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, c
   bf16_t (*stage)[TR * SK_LD] = (bf16_t (*)[TR * SK_LD])smem;
   float (*red)[AR][COLS + 1] = (float (*)[AR][COLS + 1])smem;
   const int t = threadIdx.x, lane = t % 64, wave = t / 64;
-  const int n0 = blockIdx.x * COLS;
+  const int n0 = blockIdx.x * (GATED ? 8 : COLS);
   const int r0 = blockIdx.y * AR;                    // the workgroup's first row
   const int lr = lane / 8, lc = (lane % 8) * 8;      // a load: row lr of 8, 16-byte piece lane % 8
   const int fr = lane % 16, fk = (lane / 16) * 8;    // a fragment: row fr of 16, k-group lane / 16
@@ -487,18 +490,23 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, c
   }
 #pragma unroll
   for (int i = 0; i < WL; ++i) {
-    const int n = n0 + i * 8 + lr;
-    pw[i] = w + (size_t)(n < N ? n : 0) * ldw + lc;
+    const int n = n0 + (GATED ? 0 : i * 8) + lr;
+    pw[i] = w + (size_t)((n < N ? n : 0) + (GATED ? i * N : 0)) * ldw + lc;
   }
   // What the epilogue needs is asked for behind the last group of operands, as raw bits from places that always exist: its arguments
   // lie in other lines than the operands' and are still on the way when those are asked for.
-  constexpr int EPT = (AR * COLS + NW * 64 - 1) / (NW * 64);
+  constexpr int OC = GATED ? 8 : COLS;               // columns that leave
+  constexpr int EPT = (AR * OC + NW * 64 - 1) / (NW * 64);
   uint32_t e_braw[EPT];
   float e_old[EPT];
   int e_slot[EPT];
   KvColumn e_col[EPT];
   auto load_epilogue = [&]() {
     da_read_arg(er.act);
+    if constexpr (GATED) {
+      da_read_arg(gate_limit);
+      return;
+    }
     da_read_arg(er.out_dtype);
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
@@ -591,11 +599,18 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, c
   lds_barrier();
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
-    const int e = t + j * NW * 64, ml = e / COLS, m = r0 + ml, c = e % COLS, n = n0 + c;
-    if (e < AR * COLS && m < M && n < N) {
+    const int e = t + j * NW * 64, ml = e / OC, m = r0 + ml, c = e % OC, n = n0 + c;
+    if (e < AR * OC && m < M && n < N) {
       float v = red[0][ml][c];
 #pragma unroll
       for (int v2 = 1; v2 < NW; ++v2) v += red[v2][ml][c];
+      if constexpr (GATED) {
+        float u = red[0][ml][8 + c];
+#pragma unroll
+        for (int v2 = 1; v2 < NW; ++v2) u += red[v2][ml][8 + c];
+        ((bf16_t*)out)[(size_t)m * ldo + n] = f32_to_bf16(gated_mid<true>(v, u, er.act, gate_limit));
+        continue;
+      }
       const float e_bias = !bias ? 0.f : (er.bias_dtype == DA_BF16 ? __uint_as_float(e_braw[j] << 16) : __uint_as_float(e_braw[j]));
       v = er.out_dtype == DA_BF16 ? apply_act_bf16(v + e_bias, er.act) : apply_act(v + e_bias, er.act);
       const size_t o = (size_t)m * ldo + n;
@@ -623,14 +638,20 @@ static bool sk_one_a_unit(int M, int N, int K, int lda, int ldw) {
   return (M > 4 && K >= 1280 && cols <= 20) || (K >= 3072 && cols <= 22 + K / 2048);
 }
 
+// The wavefronts that split K of a product of few rows, by K and N alone, so that a row's sums keep their order:
+// 4 where the workgroups are many (a vocabulary: several then share a compute unit), else 8, or 12 for a long K where no compute
+// unit has two workgroups (between 4,097 and 8,192 columns, K from 2,048 on, up to 16 rows 8 take 0.84 to 0.96 of 12's time).
+static int sk_wavefronts(int N, int K) { return da_ceil_div(N, 16) > 1024 ? 4 : (K >= 2048 && (N <= 16 * 256 || N > 32 * 256) ? 12 : 8); }
+// few columns and one row tile: 8 columns a workgroup
+static bool sk_eight_columns(int M, int N, int nw) { return M <= 16 && nw != 4 && da_ceil_div(N, 16) < 128; }
+
 template <int NW>
 static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw,
                          const Epilogue& ep, const KvScatter& kv, int M, int N, int K) {
   const dim3 block(NW * 64);
   int mt = da_ceil_div(M, 16);
-#define DA_SK_GO(AL, COLS, U) hipLaunchKernelGGL((gemm_skinny_kernel<AL, COLS, NW, U>), grid, block, 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv)
-  if (mt == 1 && NW != 4 && da_ceil_div(N, 16) < 128) {
-    // few columns and one row tile: 8 columns a workgroup
+#define DA_SK_GO(AL, COLS, U) hipLaunchKernelGGL((gemm_skinny_kernel<AL, COLS, NW, U>), grid, block, 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv, 0.f)
+  if (sk_eight_columns(M, N, NW)) {
     const dim3 grid(da_ceil_div(N, 8));
     if (M <= 8) DA_SK_GO(1, 8, 4); else DA_SK_GO(2, 8, 4);
     return 0;
@@ -847,6 +868,42 @@ static int gemm_bf16_checks(const void* a, int lda, const void* w, int ldw, int 
 static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, const Epilogue& ep, const KvScatter& kv, int M, int N,
                             int K, void* stream);
 
+// 1 where the gate and up products of few rows and their activation are one kernel: where the product of both matrices' columns would go to
+// gemm_skinny with 16 columns a workgroup and all rows in it.  One rounding to bfloat16 and one launch fewer; us, the product and the
+// activation's kernel / this, cold weights: 8 rows, K = 1,024, 2 x 2,752 columns 6.7 / 4.5; K = 768, 2 x 2,048 columns 1 row 5.2 / 3.4, 64 rows
+// 7.5 / 4.5; K = 3,072, 2 x 8,192 columns 8 rows 19.9 / 17.3.
+extern "C" int da_gemm_gated_takes(int M, int inner, int K) {
+  const long N = 2L * inner;
+  if (M < 1 || inner < 1 || K < 8 || K % 8 || N > 16 * 1024 || !da_gemm_few_rows(M, (int)N) || (M <= 4 && N <= 2048)) return 0;
+  if (sk_eight_columns(M, (int)N, sk_wavefronts((int)N, K)) || (sk_wavefronts((int)N, K) == 8 && sk_one_a_unit(M, (int)N, K, K, K))) return 0;
+  return M <= 16 || da_ceil_div(N, 16) >= 256;
+}
+// mid = act(a @ gate.T) * (a @ up.T), w the gate rows and then the up rows: [2 inner, K].
+extern "C" int da_gemm_bf16_gated(const void* a, int lda, const void* w, int ldw, void* mid, int ldm, int M, int inner, int K, int act, float limit,
+                                  void* stream) {
+  if (gemm_bf16_checks(a, lda, w, ldw, act, 0, DA_BF16, ldm, M, inner, K)) return 1;
+  DA_REQUIRE(act != DA_ACT_GLU_CAPPED || limit > 0.f, "gemm_bf16_gated: the capped form needs a positive limit");
+  if (M == 0) return 0;
+  DA_REQUIRE(da_gemm_gated_takes(M, inner, K), "gemm_bf16_gated: %d rows, 2 x %d columns, K=%d are not taken", M, inner, K);
+  const dim3 grid(da_ceil_div(inner, 8));
+  const int nw = sk_wavefronts(2 * inner, K);
+#define DA_SKG_GO(AL, NW, U) hipLaunchKernelGGL((gemm_skinny_kernel<AL, 16, NW, U, true>), grid, dim3(NW * 64), 0, (hipStream_t)stream, (const bf16_t*)a, \
+                                                (const bf16_t*)w, nullptr, mid, lda, ldw, ldm, M, inner, K, EpilogueRest{0, act, 0, DA_BF16}, KvScatter{}, limit)
+#define DA_SKG_ROWS(NW)                          \
+  do {                                           \
+    if (M <= 8) DA_SKG_GO(1, NW, 4);             \
+    else if (M <= 16) DA_SKG_GO(2, NW, 4);       \
+    else if (M <= 32) DA_SKG_GO(4, NW, 3);       \
+    else if (M <= 48) DA_SKG_GO(6, NW, 2);       \
+    else DA_SKG_GO(8, NW, 2);                    \
+  } while (0)
+  if (nw == 12) DA_SKG_ROWS(12); else DA_SKG_ROWS(8);
+#undef DA_SKG_ROWS
+#undef DA_SKG_GO
+  DA_CHECK_LAUNCH("gemm_bf16_gated");
+  return 0;
+}
+
 extern "C" int da_gemm_bf16(const void* a, int lda, const void* w, int ldw, const void* bias, int bias_dtype,
                             int act, int accumulate, void* out, int out_dtype, int ldo, int M, int N, int K,
                             void* kv_cache, const int* slot_map, int q_cols, int kv_cols, int Hkv, int D, int page,
@@ -889,10 +946,7 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
     if (N <= 1024 ? launch_skinny4<1>(nw, s, A, lda, W, ldw, ep, kv, M, N, K)
                   : launch_skinny4<2>(nw, s, A, lda, W, ldw, ep, kv, M, N, K)) return 1;
   } else if (da_gemm_few_rows(M, N)) {
-    // The number of wavefronts that split K depends on K and N alone, so a row's sums keep their order:
-    // 4 where the workgroups are many (a vocabulary: several then share a compute unit), else 8, or 12 for a long K where no compute
-    // unit has two workgroups (between 4,097 and 8,192 columns, K from 2,048 on, up to 16 rows 8 take 0.84 to 0.96 of 12's time).
-    const int nw = da_ceil_div(N, 16) > 1024 ? 4 : (K >= 2048 && (N <= 16 * 256 || N > 32 * 256) ? 12 : 8);
+    const int nw = sk_wavefronts(N, K);
     if (nw == 4 ? launch_skinny<4>(s, A, lda, W, ldw, ep, kv, M, N, K)
                 : (nw == 8 ? launch_skinny<8>(s, A, lda, W, ldw, ep, kv, M, N, K)
                            : launch_skinny<12>(s, A, lda, W, ldw, ep, kv, M, N, K))) return 1;

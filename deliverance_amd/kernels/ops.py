@@ -83,6 +83,8 @@ _ARGTYPES = {
     "da_gemm_f32_rows_choice": [_I, _I, _I],
     "da_gemm_bf16": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_few_rows": [_I, _I],
+    "da_gemm_gated_takes": [_I, _I, _I],
+    "da_gemm_bf16_gated": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _VP],
     "da_gemm_bf16_kv_split": [_VP, _I, _VP, _I, _VP, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_bf16_wide": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _VP],
     "da_gemm_wide_choice": [_I, _I, _I],
@@ -1462,9 +1464,28 @@ def paged_attention_rel(ctx, q: torch.Tensor, cache_slot: torch.Tensor, group: i
                                  sink=sink, gate_col=gate_col, chunk=chunk or 0, slopes=slopes)
 
 
+def linear_gated(a: torch.Tensor, w: torch.Tensor, mid: torch.Tensor, act: str, limit: float = 0.0) -> torch.Tensor:
+    """mid = act(a @ gate.T) * (a @ up.T) of few rows in one kernel, w the gate rows and then the up rows, all bfloat16; the two
+    products meet as 32-bit sums (where ``da_gemm_gated_takes``)."""
+    _dev(a, w, mid)
+    _rows_2d(a, "a"); _rows_2d(w, "w"); _rows_2d(mid, "mid")
+    M, K = a.shape
+    inner = mid.shape[1]
+    _need(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and mid.dtype == torch.bfloat16, "linear_gated: a, w and mid must be bfloat16")
+    _need(w.shape[0] == 2 * inner and w.shape[1] == K and mid.shape[0] == M, "linear_gated: shapes differ")
+    if not (act in ACTIVATIONS):
+        raise KernelError(f"linear_gated: unknown activation {act!r}")
+    with _timed("product_skinny", _nbytes(a, w, mid), 4 * M * inner * K):
+        _check(_lib().da_gemm_bf16_gated(_ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(mid), mid.stride(0), M, inner, K, ACTIVATIONS[act],
+                                         float(limit), _stream()))
+    return mid
+
+
 def gated_linear(ctx, h: torch.Tensor, gate_up: torch.Tensor, mid: torch.Tensor, act: str, limit: float = 0.0) -> torch.Tensor:
     """mid = act(h @ gate.T) * (h @ up.T) with gate | up as one matrix [2 inner, width]."""
     N, inner = mid.shape
+    if _MODE == "tuned" and mid.dtype == torch.bfloat16 and _mfma_ok(h, gate_up) and _lib().da_gemm_gated_takes(N, inner, h.shape[1]):
+        return linear_gated(h, gate_up, mid, act, limit)
     gu = ctx.buf("ff_gate_up", N, 2 * inner, h.dtype)
     linear(h, gate_up, None, gu)
     return gated_act(gu, mid, act, limit)

@@ -447,6 +447,37 @@ def test_gemm_wide_tiles(ops, M, N, K, form):
         ops.linear_mfma(a[:, :K - 8].contiguous(), w[:, :K - 8].contiguous(), b, o1, form=form)
 
 
+@pytest.mark.parametrize("M", [1, 5, helpers.quick(9), 16, 33, 64])
+@pytest.mark.parametrize("inner,K", [helpers.quick(1030, 72), (2048, 768), (2752, 1024), (1100, 2056), (5000, 2048)])
+def test_gated_products_of_few_rows(ops, M, inner, K):
+    """The gate and up products with their activation in one kernel, against 64 bits: a rounding to bfloat16 of the result and the
+    hardware's exp2 and reciprocal in between; the last workgroup's columns cut, rows that are not whole tiles, both numbers of
+    wavefronts.  What it does not take goes to the two kernels."""
+    g = torch.Generator().manual_seed(M + inner + K)
+    a = bf(torch.randn(M, K, generator=g) * 0.5).to(DEV)
+    w = bf(torch.randn(2 * inner, K, generator=g) * (1.0 / K ** 0.5)).to(DEV)
+    takes = bool(ops._lib().da_gemm_gated_takes(M, inner, K))
+    if inner in (2048, 2752) and M in (9, 16):
+        assert takes
+    wide = torch.zeros(M, inner + 8, dtype=torch.bfloat16, device=DEV)
+    for act, limit in (("silu", 0.0), ("gelu_new", 0.0), ("glu_capped", 1.5)):
+        mid = wide[:, :inner]
+        if not takes:
+            with pytest.raises(ops.KernelError, match="not taken"):
+                ops.linear_gated(a, w, mid, act, limit)
+            return
+        ops.linear_gated(a, w, mid, act, limit)
+        z = a.double().cpu() @ w.double().cpu().t()
+        gate, up = z[:, :inner], z[:, inner:]
+        if act == "glu_capped":
+            gate, up = gate.clamp(max=limit), up.clamp(-limit, limit)
+            ref = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+        else:
+            ref = (F.silu(gate) if act == "silu" else F.gelu(gate, approximate="tanh")) * up
+        assert ((mid.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all(), act
+        assert not wide[:, inner:].any()
+
+
 @pytest.mark.parametrize("form", ["deep_128x128", "deep_128x64"])
 @pytest.mark.parametrize("M,N,K", [helpers.quick(130, 70, 1024), (128, 128, 1088), (257, 200, 1152), (640, 1600, 6400), (1624, 1024, 4096)])
 def test_gemm_deep_tiles(ops, M, N, K, form):
