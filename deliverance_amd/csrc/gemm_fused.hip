@@ -217,11 +217,13 @@ gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, c
   constexpr int RPW = TWO_ROWS ? 2 : 1, AR = RPW * NW;         // rows a wavefront normalises; rows in LDS
   __shared__ __attribute__((aligned(16))) bf16_t a_lds[AR][ALD];
   constexpr int COLS = CT * 16, WL = COLS / 8;                 // columns at most; loads of 8 rows that cover w's
-  // the wavefronts' sums take the place of the parked steps once all products are done
+  // The wavefronts' sums lie behind the parked steps, where two workgroups still share a compute unit; else they take their place once all
+  // products are done, behind a barrier more.
   constexpr int STAGE_BYTES = NW * COLS * FL_LD * 2, RED_BYTES = NW * 16 * (COLS + 1) * 4;
-  __shared__ __attribute__((aligned(16))) char stage_red[STAGE_BYTES > RED_BYTES ? STAGE_BYTES : RED_BYTES];
+  constexpr bool APART = AR * ALD * 2 + STAGE_BYTES + RED_BYTES <= 80 * 1024;
+  __shared__ __attribute__((aligned(16))) char stage_red[APART ? STAGE_BYTES + RED_BYTES : (STAGE_BYTES > RED_BYTES ? STAGE_BYTES : RED_BYTES)];
   bf16_t (*stage)[COLS * FL_LD] = (bf16_t (*)[COLS * FL_LD])stage_red;
-  float (*red)[16][COLS + 1] = (float (*)[16][COLS + 1])stage_red;
+  float (*red)[16][COLS + 1] = (float (*)[16][COLS + 1])(stage_red + (APART ? STAGE_BYTES : 0));
   const int t = threadIdx.x, lane = t % 64, wave = t / 64;
   const int n0 = blockIdx.x * cols;                  // the workgroup's columns: n0 .. n_end - 1
   const int n_end = n0 + cols < N ? n0 + cols : N;
@@ -330,18 +332,23 @@ gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, c
       *(uint2*)&a_lds[m][c] = pk;
     }
   }
+  // ---- products: a step of w is parked (the first one in front of the barrier: most wavefronts have no row and wait there), then both
+  // operands' fragments come out of LDS
+  bf16_t* mine = stage[wave];
+#pragma unroll
+  for (int i = 0; i < WL; ++i) *(uint4*)&mine[(i * 8 + lr) * FL_LD + lc] = wv[0][i];
   lds_barrier();
 
-  // ---- products: a step of w is parked, then both operands' fragments come out of LDS
-  bf16_t* mine = stage[wave];
   floatx4 acc[CT];
 #pragma unroll
   for (int c = 0; c < CT; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < SW; ++u) {
     const int k0 = (wave + u * NW) * 64;               // < KMAX: the rows of a are zero from K on
+    if (u > 0) {
 #pragma unroll
-    for (int i = 0; i < WL; ++i) *(uint4*)&mine[(i * 8 + lr) * FL_LD + lc] = wv[u][i];
+      for (int i = 0; i < WL; ++i) *(uint4*)&mine[(i * 8 + lr) * FL_LD + lc] = wv[u][i];
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -360,7 +367,7 @@ gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, c
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   }
-  lds_barrier();                                       // every wavefront is done with its parked steps
+  if (!APART) lds_barrier();                           // every wavefront is done with its parked steps
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct)
 #pragma unroll

@@ -471,11 +471,13 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, c
   constexpr int MT = (AL + 1) / 2, WL = COLS / 8;    // row tiles of 16; loads of 8 rows that cover w's columns
   constexpr int AR = MT * 16, TR = AR + COLS;        // rows of a; rows of a step: a's, then w's
   static_assert(COLS == 8 || COLS == 16, "8 or 16 columns a workgroup");
-  // the wavefronts' partial sums take the place of the parked steps once all products are done
+  // The wavefronts' partial sums lie behind the parked steps, where that leaves room for the workgroups that registers allow; else they
+  // take their place once all products are done, behind a barrier more.
   constexpr int STAGE_BYTES = NW * TR * SK_LD * 2, RED_BYTES = NW * AR * (COLS + 1) * 4;
-  __shared__ __attribute__((aligned(16))) char smem[STAGE_BYTES > RED_BYTES ? STAGE_BYTES : RED_BYTES];
+  constexpr bool APART = STAGE_BYTES + RED_BYTES <= (NW == 4 ? 32 : 80) * 1024;
+  __shared__ __attribute__((aligned(16))) char smem[APART ? STAGE_BYTES + RED_BYTES : (STAGE_BYTES > RED_BYTES ? STAGE_BYTES : RED_BYTES)];
   bf16_t (*stage)[TR * SK_LD] = (bf16_t (*)[TR * SK_LD])smem;
-  float (*red)[AR][COLS + 1] = (float (*)[AR][COLS + 1])smem;
+  float (*red)[AR][COLS + 1] = (float (*)[AR][COLS + 1])(smem + (APART ? STAGE_BYTES : 0));
   const int t = threadIdx.x, lane = t % 64, wave = t / 64;
   const int n0 = blockIdx.x * (GATED ? 8 : COLS);
   const int r0 = blockIdx.y * AR;                    // the workgroup's first row
@@ -590,7 +592,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, c
     case 1: group(std::integral_constant<int, 1>{}, std::true_type{}); break;
     default: load_epilogue(); break;
   }
-  lds_barrier();
+  if (!APART) lds_barrier();
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
