@@ -378,6 +378,9 @@ DEC_KERNEL(
   if (lane == 0) { part_m[wave] = m; part_l[wave] = l; }
   __syncthreads();
   // merge the wavefronts' partial softmaxes in a fixed order
+#ifdef DEC_REL
+  if (wave * DA_WAVE >= D) return;       // (a dimension a thread: without one, the sink's and the sum's exponentials are in the others' way)
+#endif
   float mm = part_m[0];
 #pragma unroll
   for (int w2 = 1; w2 < DEC_WAVES; ++w2) mm = fmaxf(mm, part_m[w2]);
