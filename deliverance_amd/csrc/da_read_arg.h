@@ -1,5 +1,5 @@
-// Reads a kernel argument and drops it: the compiler asks for its word with the other arguments.  Why a kernel would want that stands
-// where it does (gemm_mfma.hip).
+// Reads a kernel argument and drops it: its word is asked for here and not where it is used, which may be a
+// round trip later (an argument's line of memory is seldom in a cache when its kernel starts).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -972,7 +972,7 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
     const long tiles128 = (long)da_ceil_div(M, 128) * da_ceil_div(N, 128);
     const long tiles12864 = (long)da_ceil_div(M, 128) * da_ceil_div(N, 64);
     // (up to 256 tiles a workgroup has its compute unit to itself: four slabs in flight instead of two, with the
-    // registers that a second workgroup would have needed: GPT-2 1.5B's proj and out-proj, 3.6 % of its prefill)
+    // registers that a second workgroup would have needed; into the stream, with whole slabs of K, the deep tiles are in front)
     if (tiles128 >= 192 && tiles128 <= 256) launch_tile<128, 128, 4, 2, 4>(s, A, lda, W, ldw, ep, kv, M, N, K);
     else if (tiles128 >= 192) launch_tile<128, 128, 4, 2, 2>(s, A, lda, W, ldw, ep, kv, M, N, K);
     else if (tiles12864 >= 192) launch_tile<128, 64, 4, 2, 4>(s, A, lda, W, ldw, ep, kv, M, N, K);

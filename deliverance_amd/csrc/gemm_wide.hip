@@ -706,6 +706,7 @@ bool da_gemm_wide_takes(int act, int accumulate, int out_dtype, int K) {
 //    10.6 against 13.5 us; 512 rows, N = 4,800 16.7 against 22.3; 2,048 rows, N = K = 1,600, += 21.1 against
 //    23.3; 4,096 rows, N = 1,024, K = 4,096 48.6 against 56.4); beyond, the four slabs in flight of
 //    gemm_mfma.hip's tiles win (2,048 rows, N = 1,600, K = 6,400: 65 against 79 us).
+// Into the stream the deep tiles are asked first (da_gemm_deep_choice).
 int da_gemm_wide_choice(int M, int N, int K) {
   const long tiles = (long)da_ceil_div(M, 256) * da_ceil_div(N, 256);
   const long rounds = (tiles + 255) / 256;
