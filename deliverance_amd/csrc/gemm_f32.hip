@@ -295,6 +295,26 @@ gemm_f32_tile_body(const float* __restrict__ a, int lda, const float* __restrict
 #pragma unroll
   for (int j = 0; j < PF; ++j)
     if (j < nslab) GF_FETCH(j, j * GF_BK);
+  // What the epilogue needs, from places that always exist: behind the first slabs where there is a register for it (32 x 32: 5 of them; asked
+  // for behind the products it was a round trip at the end of each tile), else before anything is stored.
+  constexpr bool EARLY = TM * TN == 1;
+  float bias[TN], old[TN][TM][4];
+  auto ask = [&](int j) {
+    const int n = n0 + wn + j * 16 + fr;
+    const bool n_ok = n < N;
+    bias[j] = (n_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, n) : 0.f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + wm + i * 16 + 4 * (lane / 16) + r;
+        old[j][i][r] = *(n_ok && m < M && ep.accumulate ? (const float*)ep.out + (size_t)m * ep.ldo + n : w);
+      }
+  };
+  if (EARLY) {
+    da_read_arg(ep.act);
+    ask(0);
+  }
   GF_STASH(0, 0);
   lds_barrier();
   // Slab s: its registers (stage s % PF) went to LDS buffer s & 1 before the last barrier and take the slab PF further
@@ -342,33 +362,30 @@ gemm_f32_tile_body(const float* __restrict__ a, int lda, const float* __restrict
 #undef GF_JOIN
 
   // A lane holds column l % 16 and rows 4 * (l / 16) + r of each 16 x 16 piece: 64 consecutive bytes a row and store.
-  // What += adds to is asked for before anything is stored, from places that always exist.
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int n = n0 + wn + j * 16 + fr;
-    const bool n_ok = n < N;
-    const float bias = (n_ok && ep.bias) ? load_param(ep.bias, ep.bias_dtype, n) : 0.f;
+    if (!EARLY) ask(j);
     KvColumn col;
-    if (kv.cache) col = kv_column(kv, n);
-    float old[TM][4];
-    int slot[TM][4];
+    int slot[TM][4];                         // (the places in the cache only now: 32 x 32 would hold one workgroup fewer a compute unit)
+    if (kv.cache) {
+      col = kv_column(kv, n);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + wm + i * 16 + 4 * (lane / 16) + r;
+          slot[i][r] = *(n < N && m < M ? kv.slot_map + m : (const int*)w);
+        }
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + wm + i * 16 + 4 * (lane / 16) + r;
-        const bool ok = n_ok && m < M;
-        old[i][r] = ep.accumulate ? *(ok ? (const float*)ep.out + (size_t)m * ep.ldo + n : w) : 0.f;
-        slot[i][r] = kv.cache ? *(ok ? kv.slot_map + m : (const int*)w) : -1;
-      }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm + i * 16 + 4 * (lane / 16) + r;
-        if (!n_ok || m >= M) continue;
-        const float v = apply_act(acc[i][j][r] + bias, ep.act);
-        ((float*)ep.out)[(size_t)m * ep.ldo + n] = ep.accumulate ? old[i][r] + v : v;
+        if (n >= N || m >= M) continue;
+        const float v = apply_act(acc[i][j][r] + bias[j], ep.act);
+        ((float*)ep.out)[(size_t)m * ep.ldo + n] = ep.accumulate ? old[j][i][r] + v : v;
         if (kv.cache && n >= kv.q_cols && slot[i][r] >= 0) kv_column_store<float>(kv, col, slot[i][r], v);
       }
   }
@@ -376,8 +393,9 @@ gemm_f32_tile_body(const float* __restrict__ a, int lda, const float* __restrict
 
 template <int BM, int BN>
 __global__ void __launch_bounds__(256)
-gemm_f32_tile_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w, int ldw, Epilogue ep, KvScatter kv,
-                     int M, int N, int K, int tiles_m, int tiles_n) {
+gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w, void* out, int lda, int ldw, int ldo, int M, int N, int K, int tiles_m,
+                     int tiles_n, const void* bias, EpilogueRest er, KvScatter kv) {
+  const Epilogue ep{bias, er.bias_dtype, er.act, er.accumulate, out, DA_F32, ldo};
   __shared__ __attribute__((aligned(16))) float smem[2 * (BM + BN) * GF_LD];
   if (K % GF_BK == 0) gemm_f32_tile_body<BM, BN, false>(a, lda, w, ldw, ep, kv, M, N, K, tiles_m, tiles_n, smem);
   else gemm_f32_tile_body<BM, BN, true>(a, lda, w, ldw, ep, kv, M, N, K, tiles_m, tiles_n, smem);
@@ -387,8 +405,8 @@ template <int BM, int BN>
 static void launch_f32_tile(hipStream_t s, const float* a, int lda, const float* w, int ldw, const Epilogue& ep, const KvScatter& kv,
                             int M, int N, int K) {
   const int tiles_m = da_ceil_div(M, BM), tiles_n = da_ceil_div(N, BN);
-  hipLaunchKernelGGL((gemm_f32_tile_kernel<BM, BN>), dim3(tiles_m * tiles_n), dim3(256), 0, s, a, lda, w, ldw, ep, kv, M, N, K, tiles_m,
-                     tiles_n);
+  hipLaunchKernelGGL((gemm_f32_tile_kernel<BM, BN>), dim3(tiles_m * tiles_n), dim3(256), 0, s, a, w, ep.out, lda, ldw, ep.ldo, M, N, K,
+                     tiles_m, tiles_n, ep.bias, epilogue_rest(ep), kv);
 }
 
 template <int WL, int AL, int NW, int CAP>
