@@ -296,7 +296,7 @@ gemm_f32_tile_body(const float* __restrict__ a, int lda, const float* __restrict
   for (int j = 0; j < PF; ++j)
     if (j < nslab) GF_FETCH(j, j * GF_BK);
   // What the epilogue needs, from places that always exist: behind the first slabs where there is a register for it (32 x 32: 5 of them; asked
-  // for behind the products it was a round trip at the end of each tile), else before anything is stored.
+  // for behind the products it was a round trip at the end of each tile: 526 x 3,072 x 768 38.9 -> 35.1 us, 526 x 768 x 768 14.3 -> 13.3), else before anything is stored.
   constexpr bool EARLY = TM * TN == 1;
   float bias[TN], old[TN][TM][4];
   auto ask = [&](int j) {
