@@ -1290,3 +1290,35 @@ def test_fused_norm_product_writes_keys_and_values(ops, M, K):
     ops.linear_ln(x, None, M, gw, gb, 1e-5, w, bias, out, kv_cache=c1, slot_map=slots, q_cols=Hq * D)
     ops.kv_write(out, Hq * D, (Hq + Hkv) * D, c2, slots, Hkv, D)      # the separate kernel on the same rows
     assert torch.equal(c1, c2) and c1.abs().sum() > 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_attention_of_more_sequences_than_a_launch_has_rows(ops, dtype):
+    """65,600 sequences of one and two keys: a launch's second size ends at 65,535, so the last ones go in another."""
+    helpers.skip_in_simulation_if(True)
+    g = torch.Generator().manual_seed(3)
+    S, Hq, D, page = 65600, 2, 16, 16
+    cache = torch.randn(3, 2, Hq, page * D, generator=g).to(dtype).to(DEV)
+    q = torch.randn(S, Hq * D, generator=g).to(dtype).to(DEV)
+    table = torch.randint(0, 3, (S, 1), generator=g, dtype=torch.int32).to(DEV)
+    lens = torch.randint(1, 3, (S,), generator=g, dtype=torch.int32).to(DEV)
+    out = torch.zeros(S, Hq * D, dtype=dtype, device=DEV)
+    lib, stream = ops._lib(), ops._stream()
+    if dtype == torch.bfloat16:
+        rc = lib.da_attn_decode(q.data_ptr(), Hq * D, cache.data_ptr(), table.data_ptr(), 1, lens.data_ptr(), S, Hq, Hq, D, page, 0.25, 0,
+                                out.data_ptr(), Hq * D, stream)
+    else:
+        starts = torch.arange(S + 1, dtype=torch.int32, device=DEV)
+        rc = lib.da_attn_f32(q.data_ptr(), Hq * D, cache.data_ptr(), table.data_ptr(), 1, starts.data_ptr(), lens.data_ptr(), S, 1, Hq, Hq, D, page,
+                             0.25, 0, out.data_ptr(), Hq * D, stream)
+    assert rc == 0
+    rows = torch.tensor([0, 1, 32799, 32800, 65534, 65535, 65536, S - 1])
+    pages = cache.double().cpu()[table.cpu()[rows, 0].long()]
+    k = pages[:, 0].reshape(-1, Hq, page, D)[:, :, :2]
+    v = pages[:, 1].reshape(-1, Hq, D, page)[..., :2]
+    score = torch.einsum("shd,shkd->shk", q.double().cpu()[rows].reshape(-1, Hq, D), k) * 0.25
+    score[lens.cpu()[rows] == 1, :, 1] = -float("inf")
+    want = torch.einsum("shk,shdk->shd", score.softmax(-1), v).reshape(-1, Hq * D)
+    tol = 2.0 ** -8 * want.abs() + 1e-4 if dtype == torch.bfloat16 else torch.full_like(want, 1e-5)
+    assert ((out.double().cpu()[rows] - want).abs() <= tol).all()
+    assert bool((out != 0).any(dim=1).all())
