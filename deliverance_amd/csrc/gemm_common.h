@@ -68,7 +68,7 @@ __device__ __forceinline__ void kv_scatter_bits(const KvScatter& kv, int pg, int
 __device__ __forceinline__ int div_uniform(int x, int d) { return (d & (d - 1)) == 0 ? x >> (31 - __builtin_clz(d)) : x / d; }
 
 // Where column n of a row goes in its page: entry `at` of the page for the page's first row, `step` entries further for each row
-// behind it (0: the column is not kept).  It needs no row, so kernels work it out while their operands are on the way.
+// behind it (0: the column is not kept, `at` is no place).  It needs no row, so kernels work it out while their operands are on the way.
 struct KvColumn {
   long long at;
   int step;
@@ -79,8 +79,10 @@ __device__ __forceinline__ KvColumn kv_column(const KvScatter& kv, int n) {
   if (cv < 0) return KvColumn{c + (long long)div_uniform(c, kv.D) * (kv.page - 1) * kv.D, kv.D};
   return KvColumn{((long long)kv.Hkv * kv.D + cv) * kv.page, cv < kv.Hkv * Dv ? 1 : 0};
 }
+// (a column that is not kept is left out here, and not by each caller: its `at` may lie behind the page)
 template <typename T = bf16_t>
 __device__ __forceinline__ void kv_column_store(const KvScatter& kv, const KvColumn& col, int slot, float v) {
+  if (col.step == 0 || slot < 0) return;
   const int pg = div_uniform(slot, kv.page), row = slot - pg * kv.page;
   from_f32((T*)kv.cache + (pg * ((long long)kv.Hkv * kv.page * (kv.D + (kv.Dv ? kv.Dv : kv.D))) + col.at + (long long)row * col.step), v);
 }

@@ -160,7 +160,7 @@ gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w, v
   v = apply_act(v + e_bias_raw, ep.act);
   float* o = (float*)ep.out + (size_t)em * ep.ldo + en;
   *o = ep.accumulate ? e_old + v : v;
-  if (kv.cache && e_col.step && e_slot >= 0) kv_column_store<float>(kv, e_col, e_slot, v);
+  if (kv.cache) kv_column_store<float>(kv, e_col, e_slot, v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -221,7 +221,7 @@ gemm_f32_rows_direct_kernel(const float* __restrict__ a, const float* __restrict
   v = apply_act(v + e_bias_raw, ep.act);
   float* o = (float*)ep.out + (size_t)em * ep.ldo + en;
   *o = ep.accumulate ? e_old + v : v;
-  if (kv.cache && e_col.step && e_slot >= 0) kv_column_store<float>(kv, e_col, e_slot, v);
+  if (kv.cache) kv_column_store<float>(kv, e_col, e_slot, v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -386,7 +386,7 @@ gemm_f32_tile_body(const float* __restrict__ a, int lda, const float* __restrict
         if (n >= N || m >= M) continue;
         const float v = apply_act(acc[i][j][r] + bias[j], ep.act);
         ((float*)ep.out)[(size_t)m * ep.ldo + n] = ep.accumulate ? old[j][i][r] + v : v;
-        if (kv.cache && n >= kv.q_cols && slot[i][r] >= 0) kv_column_store<float>(kv, col, slot[i][r], v);
+        if (kv.cache) kv_column_store<float>(kv, col, slot[i][r], v);
       }
   }
 }

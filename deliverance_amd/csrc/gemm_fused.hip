@@ -179,8 +179,7 @@ gemm_ln_skinny_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epil
 #pragma unroll
     for (int v2 = 1; v2 < NW; ++v2) v += red[v2][em][ec];
     epilogue_store(ep, em, n, v, e_bias[j]);
-    if (kv.cache && n >= kv.q_cols && e_slot[j] >= 0)
-      kv_column_store(kv, kv_column(kv, n), e_slot[j], apply_act_bf16(v + e_bias[j], ep.act));
+    if (kv.cache) kv_column_store(kv, kv_column(kv, n), e_slot[j], apply_act_bf16(v + e_bias[j], ep.act));
   }
 }
 
@@ -379,7 +378,7 @@ gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, c
     for (int v2 = 1; v2 < NW; ++v2) v += red[v2][em][ec];
     const float e_bias = !ep.bias ? 0.f : (PBF16 ? __uint_as_float(e_bias_raw << 16) : __uint_as_float(e_bias_raw));
     epilogue_store(ep, em, en, v, e_bias);
-    if (kv.cache && e_col.step && e_slot >= 0) kv_column_store(kv, e_col, e_slot, apply_act_bf16(v + e_bias, ep.act));
+    if (kv.cache) kv_column_store(kv, e_col, e_slot, apply_act_bf16(v + e_bias, ep.act));
   }
 }
 

@@ -619,7 +619,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, c
       if (er.accumulate) ((float*)out)[o] = e_old[j] + v;
       else if (er.out_dtype == DA_BF16) ((bf16_t*)out)[o] = f32_to_bf16(v);
       else ((float*)out)[o] = v;
-      if (kv.cache && e_col[j].step && e_slot[j] >= 0) kv_column_store(kv, e_col[j], e_slot[j], v);
+      if (kv.cache) kv_column_store(kv, e_col[j], e_slot[j], v);
     }
   }
 }
@@ -834,7 +834,7 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, 
       if (er.accumulate) ((float*)out)[o] = e_old + v;
       else if (er.out_dtype == DA_BF16) ((bf16_t*)out)[o] = f32_to_bf16(v);
       else ((float*)out)[o] = v;
-      if (kv.cache && e_col.step && e_slot >= 0) kv_column_store(kv, e_col, e_slot, v);
+      if (kv.cache) kv_column_store(kv, e_col, e_slot, v);
     }
   }
 }

@@ -173,7 +173,7 @@ gemm_skinny32_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
       if (ep.accumulate) ((float*)ep.out)[o] = e_old[j] + v;
       else if (ep.out_dtype == DA_BF16) ((bf16_t*)ep.out)[o] = f32_to_bf16(v);
       else ((float*)ep.out)[o] = v;
-      if (kv.cache && n >= kv.q_cols && e_slot[j] >= 0) kv_column_store(kv, kv_column(kv, n), e_slot[j], v);
+      if (kv.cache && n >= kv.q_cols) kv_column_store(kv, kv_column(kv, n), e_slot[j], v);
     }
   }
 }

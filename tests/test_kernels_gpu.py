@@ -1272,6 +1272,34 @@ def test_product_writes_keys_and_values(ops, M):
         assert torch.equal(c1, c2) and c1.abs().sum() > 0
 
 
+@pytest.mark.parametrize("M,K,Dv,N", [helpers.quick(17, 72, 16, 4160), helpers.quick(5, 1288, 24, 4160), (5, 1288, 16, 5120), (17, 72, 24, 8192),
+                                      (33, 136, 16, 4801), (64, 72, 24, 8192), (64, 136, 16, 4100), (3, 72, 24, 4160), (9, 72, 16, 1000), (40, 72, 24, 900)])
+def test_split_product_keeps_no_column_behind_the_values(ops, M, K, Dv, N):
+    """q | k | v | rest: keys and values of the rows with a place are in it, bit for bit the product's columns, and every other
+    entry of the cache is what it was; one workgroup a compute unit (4,097 to 8,192 columns) and the other forms for few rows."""
+    g = torch.Generator().manual_seed(M + N)
+    Hkv, D, page, P, rest = 2, 16, 16, 6, 100
+    q_cols = N - rest - Hkv * (D + Dv)
+    a, w, bias = (bf(torch.randn(*shape, generator=g)).to(DEV) for shape in ((M, K), (N, K), (N,)))
+    slots = torch.randperm((P - 1) * page, generator=g)[:M].to(torch.int32)
+    slots[M // 2] = -1
+    slots[0] = (P - 2) * page + 3 if not bool((slots == (P - 2) * page + 3).any()) else slots[0]
+    cache = bf(torch.randn(P, Hkv * page * (D + Dv), generator=g)).to(DEV)
+    want = cache.cpu().clone()
+    out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    ops.linear_kv_split(a, w, bias, out, cache, slots.to(DEV), q_cols, Hkv, D, Dv, page)
+    ref = a.double().cpu() @ w.double().cpu().t() + bias.double().cpu()
+    assert (out.double().cpu() - ref).abs().max() <= 2.0 ** -8 * ref.abs().max() + 1e-3
+    for m, slot in enumerate(slots.tolist()):
+        if slot < 0:
+            continue
+        pg, row = divmod(slot, page)
+        kv = out[m, q_cols:].cpu()
+        want[pg, :Hkv * page * D].view(Hkv, page, D)[:, row] = kv[:Hkv * D].view(Hkv, D)
+        want[pg, Hkv * page * D:].view(Hkv, Dv, page)[:, :, row] = kv[Hkv * D:Hkv * (D + Dv)].view(Hkv, Dv)
+    assert torch.equal(cache.cpu(), want)
+
+
 @pytest.mark.simt_quick
 @pytest.mark.parametrize("M,K", [(9, 96), (7, 1312)])
 def test_fused_norm_product_writes_keys_and_values(ops, M, K):
