@@ -956,13 +956,14 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
     // Smaller tiles where larger ones would leave compute units idle (measured on GPT-2's shapes).
     // Every configuration sums a row's products in the same order (64-wide slabs, 16 at a time), so
     // the choice does not change a result; but for the deep tiles, whose wavefronts share k out.
-    const int deep = accumulate ? da_gemm_deep_choice(M, N, K) : DA_WIDE_NONE;
+    const bool direct = da_gemm_wide_takes(act, accumulate, out_dtype, K);       // (into the stream: without an activation)
+    const int deep = direct && accumulate ? da_gemm_deep_choice(M, N, K) : DA_WIDE_NONE;
     if (deep != DA_WIDE_NONE) {
       da_gemm_wide_launch(s, A, lda, W, ldw, ep, kv, M, N, K, deep);
       DA_CHECK_LAUNCH("gemm_bf16");
       return 0;
     }
-    const int wide = da_gemm_wide_takes(act, accumulate, out_dtype, K) ? da_gemm_wide_choice(M, N, K) : DA_WIDE_NONE;
+    const int wide = direct ? da_gemm_wide_choice(M, N, K) : DA_WIDE_NONE;
     if (wide != DA_WIDE_NONE) {
       // operands straight into LDS where such tiles fill the chip: the same sums in the same order, less LDS traffic
       da_gemm_wide_launch(s, A, lda, W, ldw, ep, kv, M, N, K, wide);

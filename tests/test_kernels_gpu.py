@@ -478,6 +478,17 @@ def test_gated_products_of_few_rows(ops, M, inner, K):
         assert not wide[:, inner:].any()
 
 
+@pytest.mark.parametrize("M,N,K", [helpers.quick(65, 8256, 1024), (1300, 1536, 3072)])
+def test_products_into_the_stream_keep_their_activation(ops, M, N, K):
+    """Sizes that go to each of the two tiles that share k out inside a workgroup, which have no activation: with one the product is
+    another kernel's, without one theirs."""
+    helpers.skip_in_simulation_if(M * N * K > 1e9)
+    g = torch.Generator().manual_seed(M + N)
+    for act in ("gelu_new", None):
+        out, ref = _gemm_case(ops, ops.linear, M, N, K, torch.bfloat16, act, True, True, torch.float32, g)
+        assert (out - ref).abs().max() < 1e-4 * max(1.0, ref.abs().max().item()), act
+
+
 @pytest.mark.parametrize("form", ["deep_128x128", "deep_128x64"])
 @pytest.mark.parametrize("M,N,K", [helpers.quick(130, 70, 1024), (128, 128, 1088), (257, 200, 1152), (640, 1600, 6400), (1624, 1024, 4096)])
 def test_gemm_deep_tiles(ops, M, N, K, form):
