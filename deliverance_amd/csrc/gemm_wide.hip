@@ -718,18 +718,25 @@ int da_gemm_wide_choice(int M, int N, int K) {
 }
 
 // Which of the deep tiles a product into the stream takes, if any: those that are one a compute unit at most, where the tiles that the
-// other forms have are more than that, or wait for LDS.  Measured on MI355X with cold weights, K from 1,024 to 8,192, us, other forms / deep:
-//  - 128 x 64 where there are up to 256 of them and tiles of 64 x 64 would be more: 1,624 rows, N = 1,024, K = 4,096 27.9 / 24.3, K = 1,024
-//    11.1 / 11.1; 1,300 rows, K = 4,096 29.6 / 22.8; 900 rows, N = K = 2,048 19.5 / 16.3; 2,048 rows, N = 768, K = 3,072 21.8 / 21.8.  Where tiles of
-//    64 x 64 are one a compute unit themselves they stay (1,024 rows, N = 1,024, K = 4,096, 256 of them: 20.2 / 22.0);
-//  - 128 x 128 where there are up to 256 of them and of 128 x 64 more, K from 3,072: 2,048 rows, N = 1,600, K = 6,400 64.7 / 60.4, 1,624 rows
-//    73.1 / 56.9; 2,048 rows, N = 1,536, K = 3,072 33.8 / 33.8; 1,300 rows, N = 2,048, K = 8,192 93.9 / 60.5.  (K = 2,048: 4,096 rows, N = 1,024 26.1 / 27.1;
-//    two rounds of them: 4,096 rows, N = 2,048, K = 4,096 84.6 / 102.5.)
+// other forms have are more than that, or wait for LDS.  Measured on MI355X with cold weights, recorded side by side, about 320 sizes with N from 512 to 8,192 and
+// K from 1,024 to 8,192, us, other forms / deep:
+//  - 128 x 64 where there are up to 256 of them and tiles of 64 x 64 would be more: 1,624 rows, N = 1,024, K = 4,096 27.0 / 22.5, K = 1,024
+//    10.9 / 10.4; 1,300 rows, K = 4,096 29.2 / 21.7; 900 rows, N = K = 2,048 16.9 / 16.0; 2,048 rows, N = 768, K = 3,072 22.1 / 18.9.  Where tiles of
+//    64 x 64 are one a compute unit themselves they stay (1,024 rows, N = 1,024, K = 4,096, 256 of them: 20.2 / 22.0).  So do the other forms in two places
+//    where they are level: K = 1,024 with 192 tiles and more of 2,048 columns and more (700 rows, N = 2,048 9.9 / 10.0, 715 rows, N = 2,560 10.7 / 10.9, 354 rows,
+//    N = 5,120 11.0 / 10.9; with 1,535 rows, N = 1,216 11.4 / 11.0, with K = 1,152, 593 rows, N = 2,560 11.3 / 10.3), and more than 16 tiles by rows whose
+//    blocks do not fit the dies (a die then reads nearly all rows: die_tile; 2,600 rows, N = 768, K = 1,024 12.2 / 12.6, K = 3,072 25.0 / 25.0, 2,107 rows, N = 896, K = 1,088
+//    12.4 / 12.2, 3,442 rows, N = 576, K = 1,024 13.7 / 14.5; with 13 tiles by rows, 1,549 rows, N = 1,152, K = 2,048 17.0 / 15.7);
+//  - 128 x 128 where there are up to 256 of them and of 128 x 64 more, K from 3,072: 2,048 rows, N = 1,600, K = 6,400 63.6 / 60.7, 1,624 rows
+//    74.4 / 56.2; 4,096 rows, N = 1,024, K = 4,096 47.4 / 41.0 (gemm_wide_kernel's 128 x 128); 2,048 rows, N = 1,536, K = 3,072 33.3 / 32.8; 1,300 rows, N = 2,048, K = 8,192
+//    91.8 / 60.4.  (K = 2,048: 4,096 rows, N = 1,024 26.1 / 27.1; two rounds of them: 4,096 rows, N = 2,048, K = 4,096 84.6 / 102.5.)
 extern "C" int da_gemm_deep_choice(int M, int N, int K) {
   if (K % WD_BK || K < DA_DEEP_MIN_K) return DA_WIDE_NONE;
-  const long t64 = (long)da_ceil_div(M, 64) * da_ceil_div(N, 64), t12864 = (long)da_ceil_div(M, 128) * da_ceil_div(N, 64);
-  if (t12864 <= 256) return t64 > 256 ? DA_DEEP_128x64 : DA_WIDE_NONE;
-  return K >= 3072 && (long)da_ceil_div(M, 128) * da_ceil_div(N, 128) <= 256 ? DA_DEEP_128x128 : DA_WIDE_NONE;
+  const int rows128 = da_ceil_div(M, 128), cols64 = da_ceil_div(N, 64);
+  const long t64 = (long)da_ceil_div(M, 64) * cols64, t12864 = (long)rows128 * cols64;
+  if (t12864 > 256) return K >= 3072 && (long)rows128 * da_ceil_div(N, 128) <= 256 ? DA_DEEP_128x128 : DA_WIDE_NONE;
+  if (t64 <= 256 || (K <= 1024 && t12864 >= 192 && N >= 2048)) return DA_WIDE_NONE;
+  return rows128 > 16 && die_cut(rows128, cols64, 128, 64).lg_m == DIE_RUNS ? DA_WIDE_NONE : DA_DEEP_128x64;
 }
 
 void da_gemm_wide_launch(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep,

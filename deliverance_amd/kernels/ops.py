@@ -88,6 +88,7 @@ _ARGTYPES = {
     "da_gemm_bf16_kv_split": [_VP, _I, _VP, _I, _VP, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_bf16_wide": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _VP],
     "da_gemm_wide_choice": [_I, _I, _I],
+    "da_gemm_deep_choice": [_I, _I, _I],
     "da_gemm_bf16_ln": [_VP, _VP, _VP, _I, _VP, _I, _F, _VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP,
                         _I, _I, _I, _I, _I, _VP],
     "da_gemm_bf16_rms": [_VP, _VP, _VP, _I, _F, _F, _VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP,

@@ -478,6 +478,16 @@ def test_gated_products_of_few_rows(ops, M, inner, K):
         assert not wide[:, inner:].any()
 
 
+@pytest.mark.simt_quick
+def test_which_products_into_the_stream_share_k_out_inside_a_workgroup(ops):
+    """The tiles of 128 x 64 (4) and 128 x 128 (3) where they were measured ahead, and not (-1) where others are level or ahead."""
+    choice = ops._lib().da_gemm_deep_choice
+    for M, N, K, want in ((1624, 1024, 1024, 4), (1624, 1024, 4096, 4), (2048, 768, 3072, 4), (593, 2560, 1152, 4), (1549, 1152, 2048, 4), (1535, 1216, 1024, 4),
+                          (2048, 1600, 6400, 3), (4096, 1024, 4096, 3), (1300, 1536, 3072, 3), (354, 5120, 1024, -1), (700, 2048, 1024, -1), (2600, 768, 1024, -1),
+                          (2600, 768, 3072, -1), (3104, 640, 1280, -1), (1024, 1024, 4096, -1), (4096, 1024, 2048, -1), (4096, 2048, 4096, -1), (1624, 1024, 4104, -1)):
+        assert choice(M, N, K) == want, (M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [helpers.quick(65, 8256, 1024), (1300, 1536, 3072)])
 def test_products_into_the_stream_keep_their_activation(ops, M, N, K):
     """Sizes that go to each of the two tiles that share k out inside a workgroup, which have no activation: with one the product is
