@@ -851,11 +851,15 @@ def _kv_args(kv_cache, slot_map, q_cols, n_rows, N, out, name):
 WIDE_TILE_SHAPES = {"wide": 0, "wide_256x128": 1, "wide_128x128": 2, "deep_128x128": 3, "deep_128x64": 4}
 
 
-def _wide_tiles(M, N, K, act, accumulate, out) -> bool:
-    """Whether the library gives this product to its tiles whose operands go straight into LDS (the
-    profiler's name for it only; the choice itself is the library's: csrc/gemm_wide.hip)."""
-    takes = K % 64 == 0 and (ACTIVATIONS[act] == 0 or (not accumulate and out.dtype == torch.bfloat16))
-    return takes and _lib().da_gemm_wide_choice(M, N, K) >= 0
+def _tile_name(M, N, K, act, accumulate, out) -> str:
+    """Which of its block tiles the library gives this product (the profiler's name for it only; the choice itself is
+    the library's: csrc/gemm_mfma.hip, csrc/gemm_wide.hip)."""
+    if K % 64 == 0 and (ACTIVATIONS[act] == 0 or (not accumulate and out.dtype == torch.bfloat16)):
+        if accumulate and _lib().da_gemm_deep_choice(M, N, K) >= 0:
+            return "product_deep"
+        if _lib().da_gemm_wide_choice(M, N, K) >= 0:
+            return "product_wide"
+    return "product_tile"
 
 
 def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
@@ -884,7 +888,7 @@ def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
     kvp = _kv_args(kv_cache, slot_map, q_cols, M, N, out, "linear_mfma")
     timing = _NO_TIMING
     if KernelProfiler.enabled:           # (the cost model is worked out only when someone reads it)
-        name = "product_skinny" if (M <= 32 or (M <= 64 and N <= 8192)) else ("product_wide" if _wide_tiles(M, N, K, act, accumulate, out) else "product_tile")
+        name = "product_skinny" if (M <= 32 or (M <= 64 and N <= 8192)) else _tile_name(M, N, K, act, accumulate, out)
         timing = _timed(name, _product_bytes(a, w, bias, out, accumulate), 2 * M * N * K)
     if form != "auto" and form not in WIDE_TILE_SHAPES:
         raise KernelError(f"linear_mfma: unknown form {form!r}")

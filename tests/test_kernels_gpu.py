@@ -488,6 +488,18 @@ def test_which_products_into_the_stream_share_k_out_inside_a_workgroup(ops):
         assert choice(M, N, K) == want, (M, N, K)
 
 
+@pytest.mark.simt_quick
+def test_profiler_names_the_tiles_of_a_product(ops):
+    """One name each for the products into the stream that share k out inside a workgroup, the other tiles with operands straight into LDS and
+    the rest; an activation keeps a product out of the first."""
+    f32, bf16 = torch.empty(0), torch.empty(0, dtype=torch.bfloat16)
+    for M, N, K, act, acc, out, want in ((1624, 1024, 4096, None, True, f32, "deep"), (2048, 1600, 6400, None, True, f32, "deep"),
+                                         (1300, 1536, 3072, "gelu_new", True, f32, "tile"), (2048, 4800, 1600, None, False, bf16, "wide"),
+                                         (4096, 1024, 4096, None, False, f32, "wide"), (2048, 6400, 1600, "gelu_new", False, bf16, "wide"),
+                                         (2048, 6400, 1600, "gelu_new", False, f32, "tile"), (2048, 4800, 1608, None, False, bf16, "tile"), (300, 96, 200, None, True, f32, "tile")):
+        assert ops._tile_name(M, N, K, act, acc, out) == "product_" + want, (M, N, K, act, acc)
+
+
 @pytest.mark.parametrize("M,N,K", [helpers.quick(65, 8256, 1024), (1300, 1536, 3072)])
 def test_products_into_the_stream_keep_their_activation(ops, M, N, K):
     """Sizes that go to each of the two tiles that share k out inside a workgroup, which have no activation: with one the product is
