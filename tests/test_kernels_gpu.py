@@ -447,7 +447,7 @@ def test_gemm_wide_tiles(ops, M, N, K, form):
         ops.linear_mfma(a[:, :K - 8].contiguous(), w[:, :K - 8].contiguous(), b, o1, form=form)
 
 
-@pytest.mark.parametrize("M", [1, 5, helpers.quick(9), 16, 33, 64])
+@pytest.mark.parametrize("M", [1, 5, helpers.quick(9), 16, 17, 32, 33, 48, 49, 64])
 @pytest.mark.parametrize("inner,K", [helpers.quick(1030, 72), (2048, 768), (2752, 1024), (1100, 2056), (5000, 2048)])
 def test_gated_products_of_few_rows(ops, M, inner, K):
     """The gate and up products with their activation in one kernel, against 64 bits: a rounding to bfloat16 of the result and the
@@ -457,8 +457,8 @@ def test_gated_products_of_few_rows(ops, M, inner, K):
     a = bf(torch.randn(M, K, generator=g) * 0.5).to(DEV)
     w = bf(torch.randn(2 * inner, K, generator=g) * (1.0 / K ** 0.5)).to(DEV)
     takes = bool(ops._lib().da_gemm_gated_takes(M, inner, K))
-    if inner in (2048, 2752) and M in (9, 16):
-        assert takes
+    # (above 16 rows: with a workgroup for every compute unit, and no more columns than few rows may have)
+    assert takes == (M <= 16 or inner == 2048 or (inner == 5000 and M <= 32))
     wide = torch.zeros(M, inner + 8, dtype=torch.bfloat16, device=DEV)
     for act, limit in (("silu", 0.0), ("gelu_new", 0.0), ("glu_capped", 1.5)):
         mid = wide[:, :inner]
@@ -1353,33 +1353,49 @@ def test_fused_norm_product_writes_keys_and_values(ops, M, K):
     assert torch.equal(c1, c2) and c1.abs().sum() > 0
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_attention_of_more_sequences_than_a_launch_has_rows(ops, dtype):
-    """65,600 sequences of one and two keys: a launch's second size ends at 65,535, so the last ones go in another."""
+@pytest.mark.parametrize("form", ["decode", "split", "gated", "split gated", "prefill", "32-bit"])
+def test_attention_of_more_sequences_than_a_launch_has_rows(ops, form):
+    """65,600 sequences of one token with 1, 2, 66 or 67 keys: a launch's second size ends at 65,535, so the last ones go in another,
+    with their rows of q, table, gate, result and of the shares' sums."""
     helpers.skip_in_simulation_if(True)
     g = torch.Generator().manual_seed(3)
-    S, Hq, D, page = 65600, 2, 16, 16
-    cache = torch.randn(3, 2, Hq, page * D, generator=g).to(dtype).to(DEV)
+    dtype = torch.float32 if form == "32-bit" else torch.bfloat16
+    S, Hq, D, page, P, B = 65600, 2, 16, 16, 9, 8
+    cache = torch.randn(P, 2, Hq, page * D, generator=g).to(dtype).to(DEV)
     q = torch.randn(S, Hq * D, generator=g).to(dtype).to(DEV)
-    table = torch.randint(0, 3, (S, 1), generator=g, dtype=torch.int32).to(DEV)
-    lens = torch.randint(1, 3, (S,), generator=g, dtype=torch.int32).to(DEV)
+    gate = torch.randn(S, Hq * D, generator=g).to(dtype).to(DEV)
+    table = torch.randint(0, P, (S, B), generator=g, dtype=torch.int32).to(DEV)
+    lens = torch.tensor([1, 2, 66, 67], dtype=torch.int32)[torch.randint(0, 4, (S,), generator=g)].to(DEV)
+    starts = torch.arange(S + 1, dtype=torch.int32, device=DEV)
     out = torch.zeros(S, Hq * D, dtype=dtype, device=DEV)
+    n = 2 if "split" in form else 1
+    shares = torch.empty(S * Hq * n * (D + 2), device=DEV)
     lib, stream = ops._lib(), ops._stream()
-    if dtype == torch.bfloat16:
-        rc = lib.da_attn_decode(q.data_ptr(), Hq * D, cache.data_ptr(), table.data_ptr(), 1, lens.data_ptr(), S, Hq, Hq, D, page, 0.25, 0,
-                                out.data_ptr(), Hq * D, stream)
+    rows = (q.data_ptr(), Hq * D, cache.data_ptr(), table.data_ptr(), B)
+    sizes, result = (Hq, Hq, D, page, 0.25, 0), (out.data_ptr(), Hq * D)
+    if form == "decode":
+        rc = lib.da_attn_decode(*rows, lens.data_ptr(), S, *sizes, *result, stream)
+    elif form == "split":
+        rc = lib.da_attn_decode_split(*rows, lens.data_ptr(), S, *sizes, *result, n, shares.data_ptr(), shares.numel() * 4, stream)
+    elif "gated" in form:
+        rc = lib.da_attn_decode_rel(*rows, lens.data_ptr(), S, *sizes, None, 0, None, 0.0, 0, 0, None, gate.data_ptr(), Hq * D, *result, n,
+                                    shares.data_ptr(), shares.numel() * 4, stream)
+    elif form == "prefill":
+        rc = lib.da_attn_prefill(*rows, starts.data_ptr(), lens.data_ptr(), 0, S, 1, *sizes, *result, 0, stream)
     else:
-        starts = torch.arange(S + 1, dtype=torch.int32, device=DEV)
-        rc = lib.da_attn_f32(q.data_ptr(), Hq * D, cache.data_ptr(), table.data_ptr(), 1, starts.data_ptr(), lens.data_ptr(), S, 1, Hq, Hq, D, page,
-                             0.25, 0, out.data_ptr(), Hq * D, stream)
+        rc = lib.da_attn_f32(*rows, starts.data_ptr(), lens.data_ptr(), S, 1, *sizes, *result, stream)
     assert rc == 0
-    rows = torch.tensor([0, 1, 32799, 32800, 65534, 65535, 65536, S - 1])
-    pages = cache.double().cpu()[table.cpu()[rows, 0].long()]
-    k = pages[:, 0].reshape(-1, Hq, page, D)[:, :, :2]
-    v = pages[:, 1].reshape(-1, Hq, D, page)[..., :2]
-    score = torch.einsum("shd,shkd->shk", q.double().cpu()[rows].reshape(-1, Hq, D), k) * 0.25
-    score[lens.cpu()[rows] == 1, :, 1] = -float("inf")
-    want = torch.einsum("shk,shdk->shd", score.softmax(-1), v).reshape(-1, Hq * D)
+    at = torch.tensor([0, 1, 32799, 32800, 65534, 65535, 65536, S - 1])
+    pages = cache.double().cpu()[table.cpu()[at].long()]                                # [8, B, 2, Hq, page * D]
+    k = pages[:, :, 0].reshape(-1, B, Hq, page, D).transpose(1, 2).reshape(-1, Hq, B * page, D)
+    v = pages[:, :, 1].reshape(-1, B, Hq, D, page).permute(0, 2, 1, 4, 3).reshape(-1, Hq, B * page, D)
+    score = (q.double().cpu()[at].reshape(-1, Hq, 1, D) * k).sum(-1) * 0.25
+    score = score.masked_fill(torch.arange(B * page)[None, None] >= lens.cpu()[at].long()[:, None, None], -float("inf"))
+    want = (score.softmax(-1)[..., None] * v).sum(2).reshape(-1, Hq * D)
+    if "gated" in form:
+        want = want * torch.sigmoid(gate.double().cpu()[at])
     tol = 2.0 ** -8 * want.abs() + 1e-4 if dtype == torch.bfloat16 else torch.full_like(want, 1e-5)
-    assert ((out.double().cpu()[rows] - want).abs() <= tol).all()
+    if form == "prefill":
+        tol = tol + 2.0 ** -8 * v.abs().max()                                           # (its weights are bfloat16)
+    assert ((out.double().cpu()[at] - want).abs() <= tol).all()
     assert bool((out != 0).any(dim=1).all())
