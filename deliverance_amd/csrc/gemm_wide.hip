@@ -12,12 +12,13 @@
 // without passing registers (da_lds_dma.h), into one of two stages for a (one slab ahead of the
 // products) and one of three for w (two slabs ahead: weights come from memory, not from a cache); one
 // barrier a slab.  Rows lie unpadded in LDS (a copy writes 1,024 consecutive bytes: 8 rows); the
-// 16-byte pieces of row r are stored at position piece ^ (r % 8), which the copy does by choosing what
+// 16-byte pieces of row r are stored at position piece ^ (r / 2 % 8), which the copy does by choosing what
 // each lane fetches, so that the fragment reads of 16 consecutive rows spread over all banks.
 // Fragments are read one k-step ahead of the products that use them.
 //
-// An output element sums over k in ascending steps of 16 like the other tile forms: the result has the
-// same bits.  K must be a multiple of 64 (other sizes go to gemm_mfma.hip's kernels).
+// An output element of gemm_wide_kernel sums over k in ascending steps of 16 like the forms of gemm_mfma.hip's
+// tiles: the result has the same bits.  (gemm_deep_kernel, further down, shares k out inside a workgroup: two or
+// four such sums, added.)  K must be a multiple of 64 (other sizes go to gemm_mfma.hip's kernels).
 //
 // The epilogue is per wavefront: 32 rows x 64 columns at a time are parked in the wavefront's own piece
 // of LDS (bias and activation applied, rounded to the output's type), and leave in 16-byte pieces, whole
@@ -706,7 +707,8 @@ bool da_gemm_wide_takes(int act, int accumulate, int out_dtype, int K) {
 //    10.6 against 13.5 us; 512 rows, N = 4,800 16.7 against 22.3; 2,048 rows, N = K = 1,600, += 21.1 against
 //    23.3; 4,096 rows, N = 1,024, K = 4,096 48.6 against 56.4); beyond, the four slabs in flight of
 //    gemm_mfma.hip's tiles win (2,048 rows, N = 1,600, K = 6,400: 65 against 79 us).
-// Into the stream the deep tiles are asked first (da_gemm_deep_choice).
+// Into the stream the deep tiles are asked first (da_gemm_deep_choice): of what adds, the third line decides for K below 3,072
+// and between 3,072 and 4,096 for stores alone.
 int da_gemm_wide_choice(int M, int N, int K) {
   const long tiles = (long)da_ceil_div(M, 256) * da_ceil_div(N, 256);
   const long rounds = (tiles + 255) / 256;
