@@ -475,8 +475,8 @@ static DieCut die_cut(int tiles_m, int tiles_n, int bm, int bn) {
 // straight into LDS, S slabs ahead (all of LDS: a workgroup a compute unit); a wavefront's fragments of the next slab are read between
 // this slab's products; one barrier a slab, after which the stage it stands for is free.  The wavefronts of a position leave their sums
 // in LDS, and the first of them add them up in order of k-steps, 32 rows each: an element is KG sums, each in ascending k, added one to the other.
-// us alone, cold weights, gemm_mfma.hip's tiles -> this: 2,048 rows, N = 1,600, K = 6,400 64.7 -> 60.4 (695 TFLOP/s), 1,624 rows, N = 1,024,
-// K = 4,096 27.9 -> 24.3 (560); error against 64 bits 4.9e-7 -> 3.4e-7 and 3.8e-7 -> 1.8e-7.
+// us, recorded one behind the other, cold weights, gemm_mfma.hip's tiles -> this: 2,048 rows, N = 1,600, K = 6,400 63.6 -> 60.7 (691 TFLOP/s), 1,624 rows,
+// N = 1,024, K = 4,096 27.0 -> 22.5 (605); error against 64 bits 4.9e-7 -> 3.4e-7 and 3.8e-7 -> 1.8e-7.
 // ---------------------------------------------------------------------------------------------
 template <int BM, int BN, int KG, int S>
 __global__ void __launch_bounds__(512)

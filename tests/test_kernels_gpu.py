@@ -409,7 +409,8 @@ def test_gemm_tiles_alone_on_their_compute_units(ops, M, N, K):
     """The library's own choice where 128 x 128 tiles would be 140 to 512: a K that a slab cuts and a long K with
     192 to 256 tiles (operands through registers, four slabs in flight: GPT-2 1.5B's proj), whole slabs (operands
     straight into LDS: 128 x 128 tiles for 208 and 216 tiles, GPT-2 1.5B's out-proj among them, and for 260
-    tiles with a K above 2,048; 256 x 128 for 288 tiles, GPT-2 124M's q|k|v; 128 x 128 for 192 tiles and a K of 3,072)."""
+    tiles with a K above 2,048; 256 x 128 for 288 tiles, GPT-2 124M's q|k|v; 128 x 128 for 192 tiles and a K of 3,072).  What adds into
+    the stream goes to the tiles that share k out inside a workgroup instead where K is 3,072 and more and 256 tiles hold it."""
     helpers.skip_in_simulation_if(True)
     g = torch.Generator().manual_seed(M + N + K)
     for act, acc, bias, od in ((None, False, True, torch.bfloat16), ("gelu_new", False, True, torch.bfloat16),
