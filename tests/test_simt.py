@@ -4,8 +4,8 @@ an operand ends the child process with a message that names the kernel, the work
 and the operand.  The children run the GPU test files themselves (the same cases, with CPU tensors),
 so what the GPU tests cover for results, these runs cover for addresses.
 
-Set DELIVERANCE_SIMT_FULL=1 to run everything the simulated kernels can run (a quarter of an hour
-on 8 cores); the default is a selection that takes about a minute.
+Set DELIVERANCE_SIMT_FULL=1 to run everything the simulated kernels can run (much longer; one child
+alone with its marks takes a minute or two); the default selection takes about ten minutes on 8 cores.
 """
 import os
 import subprocess
