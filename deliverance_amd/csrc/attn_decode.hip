@@ -8,11 +8,15 @@
 // step of few requests waits for, and a chunk takes 16 instructions of 16 cycles here where it took about 700
 // of the vector unit (one head of 64, 512 keys: 6.0 -> 5.7 us a launch in a recorded chain, of which 1.6 are
 // the launch and about 2 the 130 KB that one compute unit pulls in; 64 sequences of 25 heads: 42.5 -> 40.7 us, 5.15 TB/s).
-//   scores : S[key, *] = K . q, 4 pieces of 16 keys (a lane holds row l % 16 and 8 dimensions, 16 bytes of the key
-//            row as it lies in the page; q is the same in all 16 columns).  Products of bfloat16 are exact and
-//            their sums 32-bit; the scale comes after.
-//   softmax: every lane of a quarter-wavefront holds the same 4 keys of each piece; it keeps the piece l % 4.
-//            Running maximum and sum per wavefront
+//   scores : 4 pieces of 16 keys, 16 bytes of a key's row a lane.  Four lanes that follow each other read 64 consecutive
+//            bytes: a compute unit takes four lanes' addresses at once where they lie in one line, one at a time else (130 KB
+//            alone: 2.5 against 4.8 us; a recorded step of 33 requests of the 355M's sizes 1,190 -> 1,153 us).  So row 4 a + b of the left operand holds, in k-group g, dimensions
+//            8 b .. 8 b + 7 (of 32) of key g of the rows' group a, and column 4 g + b of the right operand is q's dimensions 8 b ..
+//            in k-group g and zero elsewhere: the result's row 4 a + b, column 4 g + b is that key's share from these
+//            dimensions, and four neighbouring lanes add up its four shares.  (Zero times an infinite key of the
+//            same rows is no number: a chunk where one appears has its scores once more, a key a row.)  Products of
+//            bfloat16 are exact and their sums 32-bit; the scale comes after.
+//   softmax: four neighbouring lanes hold the same 4 keys that follow each other.  Running maximum and sum per wavefront
 //            (the recurrence of native/src/main/resources/decode_paged_attention_f32.wgsl:31-65).
 //   values : O[d, part] += V^T[d, key] . P[key, part]; values are stored dimension-major, so the left operand is
 //            16 bytes as they lie in the page.  The 32-bit weights lose nothing: column 0 takes a weight rounded to
@@ -111,6 +115,8 @@ DEC_KERNEL(
   const int hk = Hq == Hkv ? h : h / (Hq / Hkv);
   const int t = threadIdx.x, lane = t % DA_WAVE, wave = __builtin_amdgcn_readfirstlane(t / DA_WAVE);
   const int col = lane % 16, quad = lane / 16;
+  const int kd = 8 * (col % 4);               // the dimensions (of 32) that the lane loads of a key
+  const int ka = 16 * (col / 4) + 4 * quad;   // the first of the 4 keys of a chunk that it loads
   const int* bt = block_table + (size_t)s * max_blocks;
   // addressing by shifts: the page size is a power of two (checked on the host)
   const int lg = 31 - __builtin_clz(page), pmask = page - 1;
@@ -125,16 +131,15 @@ DEC_KERNEL(
   uint4 qf[DK];
 #pragma unroll
   for (int k = 0; k < DK; ++k) {
-    const int d = 32 * k + 8 * quad;
+    const int d = 32 * k + kd;
     qf[k] = *(const uint4*)(q + (size_t)s * q_ld + h * D + (d < D ? d : 0));
   }
   const int split0 = SPLIT ? (int)blockIdx.z * span : 0;          // the first key of this workgroup's share
   const int c0_guess = split0 + wave * DA_WAVE;
-  int btk0[4], btv0[2];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int pg = (c0_guess + 16 * j + col) >> lg;
-    btk0[j] = bt[pg < max_blocks ? pg : max_blocks - 1];
+  int btk0, btv0[2];                          // (pages hold whole groups of 4 keys)
+  {
+    const int pg = (c0_guess + ka) >> lg;
+    btk0 = bt[pg < max_blocks ? pg : max_blocks - 1];
   }
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
@@ -177,7 +182,7 @@ DEC_KERNEL(
 #endif
 #pragma unroll
   for (int k = 0; k < DK; ++k)
-    if (32 * k + 8 * quad >= D) qf[k] = make_uint4(0, 0, 0, 0);
+    if (32 * k + kd >= D || quad != col / 4) qf[k] = make_uint4(0, 0, 0, 0);
 
   floatx4 acc[DV];
 #pragma unroll
@@ -188,20 +193,15 @@ DEC_KERNEL(
     const int first = c0 > lo ? c0 : lo;                 // valid keys of the chunk: first..last
     const int last = c0 + DA_WAVE - 1 < p ? c0 + DA_WAVE - 1 : p;
     // the pages of the chunk's keys and value groups: those asked for at the start, or read now
-    int btk[4], btv[2], bt_safe;
+    int btk, btv[2], bt_safe;
     if (c0 == c0_guess && first == c0) {                 // the same for the whole wavefront
-#pragma unroll
-      for (int j = 0; j < 4; ++j) btk[j] = btk0[j];
+      btk = btk0;
       btv[0] = btv0[0];
       btv[1] = btv0[1];
-      bt_safe = __builtin_amdgcn_readfirstlane(btk0[0]); // lane 0 holds the page of key c0
+      bt_safe = __builtin_amdgcn_readfirstlane(btk0);    // lane 0 holds the page of key c0
     } else {
       bt_safe = bt[first >> lg];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int key = c0 + 16 * j + col;
-        btk[j] = bt[((key >= first && key <= last) ? key : first) >> lg];
-      }
+      btk = bt[((c0 + ka + 3 >= first && c0 + ka <= last) ? c0 + ka : first) >> lg];
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
         const int g0 = c0 + 32 * g + 8 * quad;
@@ -220,20 +220,20 @@ DEC_KERNEL(
     auto load_k = [&](int j0) {
 #pragma unroll
       for (int j = 0; j < KJ; ++j) {
-        const int key = c0 + 16 * (j0 + j) + col;
+        const int key = c0 + ka + j0 + j;
         const bool valid = key >= first && key <= last;
-        const char* kp = kbase + (uint64_t)(uint32_t)(valid ? btk[j0 + j] : bt_safe) * page_bytes +
-                         (uint32_t)(2 * (((valid ? key : first) & pmask) * D + (DK > 1 || 8 * quad < D ? 8 * quad : 0)));
+        const char* kp = kbase + (uint64_t)(uint32_t)(valid ? btk : bt_safe) * page_bytes +
+                         (uint32_t)(2 * (((valid ? key : first) & pmask) * D + (DK > 1 || kd < D ? kd : 0)));
 #pragma unroll
         for (int k = 0; k < DK; ++k)         // (D > 16 DK: only the upper half of the steps can lie past D; there the first step is read)
-          kf[j][k] = *(const uint4*)(kp + (2 * k + 1 < DK || 32 * k + 8 * quad < D ? 64 * k : 0));
+          kf[j][k] = *(const uint4*)(kp + (2 * k + 1 < DK || 32 * k + kd < D ? 64 * k : 0));
       }
     };
     // Zeros in place of what lanes past D read: q is zero there, but zero times an infinite key is no number.
     auto clear_k = [&]() {
 #pragma unroll
       for (int k = DK / 2; k < DK; ++k) {
-        const uint32_t keep = 32 * k + 8 * quad < D ? 0xffffffffu : 0u;
+        const uint32_t keep = 32 * k + kd < D ? 0xffffffffu : 0u;
 #pragma unroll
         for (int j = 0; j < KJ; ++j) {
           kf[j][k].x &= keep;
@@ -273,7 +273,7 @@ DEC_KERNEL(
     float brel[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int dist = p_row - (c0 + 16 * (col % 4) + 4 * quad + r);
+      const int dist = p_row - (c0 + 16 * quad + 4 * (col / 4) + r);
       brel[r] = slopes ? -slope * (float)dist : 0.f;
       if (brow) brel[r] += brow[dist < 0 ? 0 : (dist < n_dist ? dist : n_dist - 1)];
     }
@@ -288,17 +288,47 @@ DEC_KERNEL(
       load_k(EARLY_V ? 0 : 2);
       scores(EARLY_V ? 0 : 2);
     }
-    // this lane's 4 keys: rows 4 * quad + r of piece col % 4
-    const int key0 = c0 + 16 * (col % 4) + 4 * quad;
+    // this lane's 4 keys: piece r's row group `quad`, k-group col / 4; of their shares register col % 4
+    const int key0 = c0 + 16 * quad + 4 * (col / 4);
     float sv[4], e[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float s01 = col & 1 ? sc[1][r] : sc[0][r], s23 = col & 1 ? sc[3][r] : sc[2][r];
-      sv[r] = (col & 2 ? s23 : s01) * qscale;
+    auto finish = [&](int r) {
+      sv[r] *= qscale;
 #ifdef DEC_REL
       sv[r] += brel[r];
 #endif
       sv[r] = key0 + r >= first && key0 + r <= last ? sv[r] : -INFINITY;
+    };
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float s01 = col & 1 ? sc[r][1] : sc[r][0], s23 = col & 1 ? sc[r][3] : sc[r][2];
+      sv[r] = group_sum<4>(col & 2 ? s23 : s01);
+      finish(r);
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(sv[0] != sv[0] || sv[1] != sv[1] || sv[2] != sv[2] || sv[3] != sv[3]) != 0, 0)) {
+      // the chunk's scores once more, a key a row of the left operand and q in all columns: product j holds this lane's keys if j = col / 4
+#pragma unroll 1
+      for (int j = 0; j < 4; ++j) {
+        const int key = c0 + 16 * (col / 4) + 4 * j + col % 4, seen = key >= first && key <= last ? key : first;
+        const char* kp = kbase + (uint64_t)(uint32_t)bt[seen >> lg] * page_bytes + (uint32_t)(2 * (seen & pmask) * D);
+        floatx4 one = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int k = 0; k < DK; ++k) {
+          const int d = 32 * k + 8 * quad;
+          uint4 kx = make_uint4(0, 0, 0, 0), qx = kx;
+          if (d < D) {
+            kx = *(const uint4*)(kp + 2 * d);
+            qx = *(const uint4*)(q + (size_t)s * q_ld + h * D + d);
+          }
+          one = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kx), __builtin_bit_cast(bf16x8_t, qx), one, 0, 0, 0);
+        }
+        if (j == col / 4) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            sv[r] = one[r];
+            finish(r);
+          }
+        }
+      }
     }
     const float m_new = fmaxf(m, wave_max(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]))));
     const float alpha = dec_exp(m - m_new);              // (a chunk that is walked has a seen key: m_new is finite)
@@ -307,8 +337,8 @@ DEC_KERNEL(
     l = l * alpha + 0.25f * wave_sum((e[0] + e[1]) + (e[2] + e[3]));      // (four lanes hold each key)
     m = m_new;
     {
-      // lane group col / 4 = 0, 1, 2 parks the first, second, third part of its 4 weights, group 3 zeros
-      const int part = col / 4;
+      // of four neighbouring lanes the first parks the first part of their 4 weights, the others the second, the third, zeros
+      const int part = col % 4;
       uint32_t w2[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -319,7 +349,7 @@ DEC_KERNEL(
         const uint32_t p2 = pack2_bf16(a1 - __uint_as_float(p1 << 16), b1 - __uint_as_float(p1 & 0xffff0000u));
         w2[i] = part == 0 ? p0 : (part == 1 ? p1 : (part == 2 ? p2 : 0u));
       }
-      *(uint2*)&ps[wave][part][16 * (col % 4) + 4 * quad] = make_uint2(w2[0], w2[1]);
+      *(uint2*)&ps[wave][part][16 * quad + 4 * (col / 4)] = make_uint2(w2[0], w2[1]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");   // LDS only: the value loads stay in flight
     __builtin_amdgcn_wave_barrier();

@@ -854,6 +854,39 @@ def test_attention_decode_with_infinite_keys_and_values(ops, D):
 
 
 @pytest.mark.simt_quick
+@pytest.mark.parametrize("rel", [False, True])
+@pytest.mark.parametrize("D,page,window", [(64, 16, None), (64, 8, 75), (128, 64, 75), (32, 32, None)])
+def test_attention_decode_scores_of_an_infinite_keys_neighbours(ops, D, page, window, rel):
+    """The scores of four keys that follow each other by fours are sums over all of their dimensions with zeros in the place of the
+    others' (attn_decode.hip): a key of minus infinity takes its own weight and nobody else's, in each of the four places, in whole
+    chunks and in the one that a window or the length cuts; also with a bias by distance."""
+    inf, n = float("inf"), 150
+    g = torch.Generator().manual_seed(D + page)
+    q, k, v = (bf(torch.randn(m, D, generator=g)) for m in (1, n, n))
+    q = q.abs() + 0.25
+    hit = torch.tensor([0, 5, 10, 15, 64 + 3, 64 + 17, 64 + 42, 128 + 20, n - 1])
+    k[hit, (hit * 7) % D] = -inf
+    pages = -(-n // page)
+    cache = torch.full((pages, 2, 1, page, D), float("nan"), dtype=torch.bfloat16)
+    for j in range(n):
+        cache[j // page, 0, 0, j % page] = k[j]
+        cache[j // page, 1].view(D, page)[:, j % page] = v[j]
+    out = torch.empty(1, D, dtype=torch.bfloat16, device=DEV)
+    args = (q.to(DEV), cache.to(DEV), torch.arange(pages, dtype=torch.int32, device=DEV).view(1, pages),
+            torch.tensor([n], dtype=torch.int32, device=DEV), 1, 1, 0.2, window)
+    lo = n - window if window else 0
+    s = (k[lo:].double() @ q[0].double()) * 0.2
+    if rel:
+        bias = torch.randn(1, 40, generator=g)
+        s = s + bias[0, torch.arange(n - 1 - lo, -1, -1).clamp(max=39)].double()
+        ops.attention_decode_rel(*args, bias.to(DEV), 0.0, 0, out)
+    else:
+        ops.attention_decode(*args, out)
+    want = torch.softmax(s, 0) @ v[lo:].double()
+    assert bool(torch.isfinite(want).all()) and (out[0].double().cpu() - want).abs().max() < ATT_TOL[torch.bfloat16]
+
+
+@pytest.mark.simt_quick
 @pytest.mark.parametrize("D", [16, 64, 80, 144])
 def test_attention_decode_keeps_the_weights_32_bits(ops, D):
     """Pairs of keys whose weights differ by 2^-12 and whose values, 65,536 and its negative, nearly cancel: the result is what
