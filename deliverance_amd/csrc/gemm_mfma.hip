@@ -11,8 +11,8 @@
 //  * gemm_skinny: for M <= 64 (decode); gemm_skinny32 where they would be more workgroups than compute units (sk_one_a_unit).  A workgroup owns 16 output columns; its wavefronts (4 to 12)
 //    split K, pull their part of a and w from memory in whole cache lines, pass it through LDS into
 //    MFMA 16x16x32 fragments and add their sums through LDS in a fixed order.  Bound by the bytes of w.
-//  * gemm_skinny4: for M <= 4 and up to 2,048 columns.  MFMA 4x4x4, whose operand layout lets a row
-//    of w be read in whole cache lines straight into registers; 4 or 8 columns a workgroup.
+//  * gemm_skinny4: for M <= 4 (8 with a long K) and up to 2,048 columns.  MFMA 16x16x32 with four pieces of k side by side, so that
+//    four rows of w are read in whole cache lines straight into registers; 4 or 8 columns a workgroup.
 //
 // In each, an output element sums over k in an order that depends on K only, never on M or on
 // the row's place in the batch.
@@ -692,45 +692,37 @@ static int launch_skinny(hipStream_t s, const bf16_t* A, int lda, const bf16_t* 
 }
 
 // ---------------------------------------------------------------------------------------------
-// M <= 4 and up to 2,048 columns (a decode step of a few requests).  MFMA 4x4x4: 16 independent 4x4
-// products of depth 4 a wavefront.  Lane l gives row (a) /
-// column (b) l % 4 of product l / 4 and 4 consecutive k; it receives column l % 4 of that product,
-// rows 0..3.  The 16 products of a step take 16 consecutive pieces of k of 8 elements (two
-// instructions each), so a lane loads 16 bytes and the 16 lanes of one row of w read 256 consecutive
-// bytes: whole cache lines without a detour through LDS.  A workgroup owns 4 * NG columns; wavefront v of NW takes
-// the steps v, v+NW, ... of 128 elements of k; the products of a wavefront are summed over its 16
-// lanes-groups at the end (two lane rotations, then LDS) in a fixed order.
+// M <= 4, or 8 with a long K, and up to 2,048 columns (a decode step of a few requests).  MFMA 16x16x32 with pieces of k side by side: row 4 n + b
+// of the left operand holds in k-group g the 8 elements from 8 (4 g + b) of a step of 128, of row n of 4 of w; column 4 m + b of
+// the right operand the same of row m of 4 of a.  The result's entry (4 n + b, 4 m + b) is what the pieces b give, and four
+// neighbouring lanes add up the four; the entries of unlike pieces are not looked at.  So four lanes that follow each other read 64
+// consecutive bytes, which a compute unit takes at once; with a row a lane it takes them one at a time.  A workgroup owns
+// 4 * NG columns; wavefront v of NW takes the steps v, v+NW, ...; the wavefronts' sums are added through LDS in a fixed order.
 // ---------------------------------------------------------------------------------------------
-template <int NG, int NW, int UNROLL>
+template <int MG, int NG, int NW, int UNROLL>
 __global__ void __launch_bounds__(NW * 64)
 gemm_skinny4_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, const void* bias, void* out, int lda, int ldw, int ldo,
                     int M, int N, int K, EpilogueRest er, KvScatter kv) {
-  constexpr int MG = 1;                        // row groups of 4 (from 5 rows on gemm_skinny is faster)
-  constexpr int ROWS = MG * 4, COLS = NG * 4;
-  __shared__ __attribute__((aligned(16))) float red[4 * NW][COLS][ROWS];
-  static_assert(NW * 64 >= 4 * ROWS * COLS, "four threads an output element");
+  constexpr int ROWS = 4 * MG, COLS = NG * 4;
+  __shared__ float red[NW][ROWS][COLS];
   const int t = threadIdx.x, lane = t % 64, wave = t / 64;
   const int n0 = blockIdx.x * COLS;
-  const int q = lane % 4, kb = (lane / 4) * 8;
+  const int r4 = lane / 4 % 4, kb = (4 * (lane / 16) + lane % 4) * 8;
   const bf16_t* wp[NG];
-  const bf16_t* ap[MG];
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
-    const int n = n0 + g * 4 + q;
+    const int n = n0 + g * 4 + r4;
     wp[g] = w + (size_t)(n < N ? n : 0) * ldw + kb;
   }
+  const bf16_t* ap[MG];
 #pragma unroll
-  for (int g = 0; g < MG; ++g) {
-    const int m = g * 4 + q;
-    ap[g] = a + (size_t)(m < M ? m : 0) * lda + kb;
-  }
-  // Four threads an output element (the host launches 4 * ROWS * COLS threads at least): each sums
-  // a quarter of the partial sums, the first of them stores.  What the epilogue needs is asked for behind the last operands, as in
-  // gemm_skinny.
+  for (int i = 0; i < MG; ++i) ap[i] = a + (size_t)(4 * i + r4 < M ? 4 * i + r4 : 0) * lda + kb;
+  // Four threads an output element: each sums a quarter of the wavefronts' sums, the first of them stores.  What the epilogue needs is
+  // asked for behind the last operands, as in gemm_skinny.
+  static_assert(NW % 4 == 0 && NW * 64 >= 4 * ROWS * COLS, "four threads an output element");
   const int e_id = t / 4, e_q = t % 4;
   const int e_m = e_id / COLS, e_c = e_id % COLS, e_n = n0 + e_c;
-  const bool e_ok = e_id < ROWS * COLS && e_m < M && e_n < N;
-  const bool e_st = e_ok && e_q == 0;
+  const bool e_st = e_m < M && e_m < ROWS && e_n < N && e_q == 0;
   uint32_t e_braw;
   float e_old;
   int e_slot;
@@ -754,7 +746,7 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, 
   // The wavefront's steps go in groups of UNROLL and one last group of what is left: a group is
   // nothing but its loads, all in flight at once, and then its products.  The last step of the last
   // group may be the one that K cuts: lanes past K read the row's first piece instead and give
-  // zeros for a (a multiple of 8 elements is in or out as a whole).
+  // zeros for both (a multiple of 8 elements is in or out as a whole).
   const int steps = (K + 127) / 128;
   int count = wave < steps ? (steps - wave + NW - 1) / NW : 0;
   int k0 = wave * 128;
@@ -776,24 +768,20 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, 
       for (int j = 0; j < NG; ++j) wv[u][j] = load16(wp[j] + kk);
     }
     if (LAST) load_epilogue();
+    __builtin_amdgcn_sched_barrier(0);       // (else loads are pushed down among the products to save registers)
 #pragma unroll
     for (int u = 0; u < G; ++u) {
-      if (LAST && u == G - 1) {
+      if (LAST && u == G - 1 && !kin) {
 #pragma unroll
-        for (int i = 0; i < MG; ++i)
-          if (!kin) av[u][i] = make_uint4(0, 0, 0, 0);
+        for (int i = 0; i < MG; ++i) av[u][i] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NG; ++j) wv[u][j] = make_uint4(0, 0, 0, 0);
       }
 #pragma unroll
       for (int i = 0; i < MG; ++i)
 #pragma unroll
-        for (int j = 0; j < NG; ++j) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(
-              __builtin_bit_cast(bf16x4s_t, make_uint2(av[u][i].x, av[u][i].y)),
-              __builtin_bit_cast(bf16x4s_t, make_uint2(wv[u][j].x, wv[u][j].y)), acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(
-              __builtin_bit_cast(bf16x4s_t, make_uint2(av[u][i].z, av[u][i].w)),
-              __builtin_bit_cast(bf16x4s_t, make_uint2(wv[u][j].z, wv[u][j].w)), acc[i][j], 0, 0, 0);
-        }
+        for (int j = 0; j < NG; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wv[u][j]), __builtin_bit_cast(bf16x8_t, av[u][i]), acc[i][j], 0, 0, 0);
     }
     k0 += G * NW * 128;
     count -= G;
@@ -806,27 +794,22 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, 
     case 1: group(std::integral_constant<int, 1>{}, std::true_type{}); break;
     default: load_epilogue(); break;
   }
-  // sum over the four products of a row of 16 lanes, then one partial a row of lanes goes to LDS
+  // a lane has column 4 m + b and the rows 4 n .. 4 n + 3, n its quarter of the wavefront: of these, row 4 n + b
 #pragma unroll
   for (int i = 0; i < MG; ++i)
 #pragma unroll
     for (int j = 0; j < NG; ++j) {
-      floatx4 v = acc[i][j];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        v[r] += dpp_move<0x124, 0xF>(v[r], v[r]);      // row_ror:4
-        v[r] += dpp_move<0x128, 0xF>(v[r], v[r]);      // row_ror:8
-      }
-      if (lane % 16 < 4) *(floatx4*)&red[wave * 4 + lane / 16][j * 4 + q][i * 4] = v;
+      const float d01 = lane & 1 ? acc[i][j][1] : acc[i][j][0], d23 = lane & 1 ? acc[i][j][3] : acc[i][j][2];
+      const float v = group_sum<4>(lane & 2 ? d23 : d01);
+      if (lane % 4 == 0) red[wave][4 * i + r4][j * 4 + lane / 16] = v;
     }
   lds_barrier();
-  if (e_id < ROWS * COLS) {               // whole quads
-    // thread e_q of the four takes the partial sums e_q, e_q + 4, ...: one of each wavefront
+  if (e_m < ROWS) {                       // whole quads
+    // thread e_q of the four takes the wavefronts e_q, e_q + 4, ...
     float v = 0.f;
 #pragma unroll
-    for (int i = 0; i < NW; ++i) v += red[e_q + 4 * i][e_c][e_m];
-    v += dpp_move<0xB1, 0xF>(v, v);
-    v += dpp_move<0x4E, 0xF>(v, v);
+    for (int i = 0; i < NW / 4; ++i) v += red[e_q + 4 * i][e_m][e_c];
+    v = group_sum<4>(v);
     if (e_st) {
       const float e_bias = !bias ? 0.f : (er.bias_dtype == DA_BF16 ? __uint_as_float(e_braw << 16) : __uint_as_float(e_braw));
       v = er.out_dtype == DA_BF16 ? apply_act_bf16(v + e_bias, er.act) : apply_act(v + e_bias, er.act);
@@ -839,15 +822,27 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, 
   }
 }
 
-template <int NG>
-static int launch_skinny4(int nw, hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw,
-                          const Epilogue& ep, const KvScatter& kv, int M, int N, int K) {
-  DA_REQUIRE(M <= 4, "gemm_bf16: %d rows for one group of 4", M);
-  const dim3 grid(da_ceil_div(N, NG * 4));
-  if (nw == 16) hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 16, 4>), grid, dim3(1024), 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv);
-  else if (nw == 8) hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 8, 4>), grid, dim3(512), 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv);
-  else hipLaunchKernelGGL((gemm_skinny4_kernel<NG, 4, 4>), grid, dim3(256), 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv);
-  return 0;
+// The wavefronts by K alone, so a row's sums keep their order; columns a workgroup so that the operands of a are no more than those of w
+// where that pays.  us, cold weights, recorded one behind the other, 4x4x4 with a row a lane (up to 4 rows) or gemm_skinny (8 rows) -> this:
+//   1 row   1,600 x 6,400 6.3 -> 5.7, 768 x 3,072 3.8 -> 3.2, 1,600 x 1,600 3.7 -> 3.4, 768 x 768 2.7 -> 2.6
+//   4 rows  1,600 x 6,400 7.3 -> 6.1, 768 x 3,072 4.3 -> 3.5, 1,600 x 1,600 4.0 -> 3.6, 2,048 x 8,192 9.4 -> 7.8
+//   8 rows  1,600 x 6,400 7.4 -> 7.1, 768 x 3,072 4.5 -> 4.0, 1,024 x 4,096 5.5 -> 4.4; 1,600 x 1,600 3.8 -> 3.9 (so from K = 2,048 on)
+// The weights alone, read and dropped, take 5.2, 2.5 and 2.6 us (1,600 x 6,400, 768 x 3,072, 1,600 x 1,600).
+#define SK4_ROWS 4
+#define SK4_LONG_ROWS 8
+#define SK4_LONG_K 2048
+#define SK4_COLS 2048
+static bool sk4_takes(int M, int N, int K) { return N <= SK4_COLS && (M <= SK4_ROWS || (M <= SK4_LONG_ROWS && K >= SK4_LONG_K)); }
+static void launch_skinny4(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep, const KvScatter& kv, int M,
+                           int N, int K) {
+#define DA_SK4_GO(MG, NG, NW, U) hipLaunchKernelGGL((gemm_skinny4_kernel<MG, NG, NW, U>), dim3(da_ceil_div(N, 4 * NG)), dim3(NW * 64), 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv)
+  if (M > SK4_ROWS) {                                     // (K from SK4_LONG_K on)
+    if (N <= 1024) DA_SK4_GO(2, 1, 8, 4);
+    else DA_SK4_GO(2, 2, 8, 3);
+  } else if (K < 1024) DA_SK4_GO(1, 1, 4, 4);
+  else if (N <= 1024 || K < 4096) DA_SK4_GO(1, 1, 8, 4);
+  else DA_SK4_GO(1, 2, 8, 4);
+#undef DA_SK4_GO
 }
 
 // 1 when a product of so many rows and columns goes to the kernels for few rows
@@ -876,7 +871,7 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
 // 7.5 / 4.5; K = 3,072, 2 x 8,192 columns 8 rows 19.9 / 17.3.
 extern "C" int da_gemm_gated_takes(int M, int inner, int K) {
   const long N = 2L * inner;
-  if (M < 1 || inner < 1 || K < 8 || K % 8 || N > 16 * 1024 || !da_gemm_few_rows(M, (int)N) || (M <= 4 && N <= 2048)) return 0;
+  if (M < 1 || inner < 1 || K < 8 || K % 8 || N > 16 * 1024 || !da_gemm_few_rows(M, (int)N) || (M <= SK4_ROWS && N <= SK4_COLS)) return 0;
   if (sk_eight_columns(M, (int)N, sk_wavefronts((int)N, K)) || (sk_wavefronts((int)N, K) == 8 && sk_one_a_unit(M, (int)N, K, K, K))) return 0;
   return M <= 16 || da_ceil_div(N, 16) >= 256;
 }
@@ -942,11 +937,8 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
   hipStream_t s = (hipStream_t)stream;
   const bf16_t* A = (const bf16_t*)a;
   const bf16_t* W = (const bf16_t*)w;
-  if (M <= 4 && N <= 2048) {
-    // Measured: up to 4 rows and 2,048 columns the 4x4x4 form is ahead, by 20 to 25 % with K from 2,048 on.
-    const int nw = K >= 2048 ? 16 : (K >= 1024 ? 8 : 4);   // by K alone, so a row's sums keep their order
-    if (N <= 1024 ? launch_skinny4<1>(nw, s, A, lda, W, ldw, ep, kv, M, N, K)
-                  : launch_skinny4<2>(nw, s, A, lda, W, ldw, ep, kv, M, N, K)) return 1;
+  if (sk4_takes(M, N, K)) {
+    launch_skinny4(s, A, lda, W, ldw, ep, kv, M, N, K);
   } else if (da_gemm_few_rows(M, N)) {
     const int nw = sk_wavefronts(N, K);
     if (nw == 4 ? launch_skinny<4>(s, A, lda, W, ldw, ep, kv, M, N, K)

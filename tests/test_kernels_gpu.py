@@ -332,7 +332,7 @@ def test_product_32bit_keeps_keys_and_values_of_any_call(ops, extra, accumulate)
                                  helpers.quick(50, 24, mark="simt_b"), helpers.quick(300, 2056, mark="simt_b"), (1030, 1160),
                                  (4200, 200), helpers.quick(4096, 8, mark="simt_b")])
 def test_gemm_matrix_cores(ops, M, N, K):
-    """Every kernel form behind ``linear_mfma`` (up to 4 rows and 2,048 columns: 4x4x4 products, 4 to 16
+    """Every kernel form behind ``linear_mfma`` (up to 4 rows and 2,048 columns: 16x16x32 products of four pieces of k, 4 or 8
     wavefronts; up to 64 rows: 16x16x32 products fed through LDS, 1 to 4 row tiles, 8 or 12 wavefronts;
     else block tiles of 64x64, 128x64 and 128x128, chosen by the number of tiles: 1,100 and 2,048 rows
     reach the larger ones), each with a last step that K cuts or a K below one slab."""
@@ -369,6 +369,25 @@ def test_gemm_one_workgroup_a_compute_unit(ops, M, N, K):
         ops.linear_mfma(a[:M], w, None, out, kv_cache=c1, slot_map=slots, q_cols=N - 2 * Hkv * D)
         ops.kv_write(out, N - 2 * Hkv * D, N - Hkv * D, c2, slots, Hkv, D)
         assert torch.equal(c1, c2) and bool(c1.any())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1027, 4104), (4, 2048, 8200), helpers.quick(2, 1030, 1032), (3, 50, 1016), (5, 1024, 2048),
+                                   helpers.quick(8, 129, 2056), (7, 2048, 6408), (6, 1029, 3080)])
+def test_gemm_four_pieces_of_k_side_by_side(ops, M, N, K):
+    """Up to 4 rows, or 8 with K from 2,048 on, and up to 2,048 columns: one or two groups of 4 rows and of 4 columns, several rounds of steps,
+    a last one that K cuts; a row has the same bits beside any other rows of these kernels, and one that is not finite leaves the others alone."""
+    g = torch.Generator().manual_seed(M + N)
+    for act, acc, bias, od in ((None, False, True, torch.bfloat16), ("gelu_new", False, False, torch.bfloat16), (None, True, True, torch.float32)):
+        out, ref = _gemm_case(ops, ops.linear_mfma, M, N, K, torch.bfloat16, act, acc, bias, od, g)
+        tol = (1e-2 if od == torch.bfloat16 else 1e-4) * max(1.0, ref.abs().max().item())
+        assert (out - ref).abs().max() < tol, (act, acc, bias, od)
+    a, w = bf(torch.randn(8, K, generator=g)).to(DEV), bf(torch.randn(N, K, generator=g) * 0.1).to(DEV)
+    rows = lambda lo, hi: ops.linear_mfma(a[lo:hi], w, None, torch.empty(hi - lo, N, device=DEV))
+    most = 8 if K >= 2048 else 4
+    whole = rows(0, most)
+    assert torch.equal(rows(most - M, most), whole[most - M:]) and torch.equal(rows(1, 2)[0], whole[1])
+    a[0, K - 1], a[2, 5] = float("inf"), float("nan")
+    assert torch.equal(rows(0, most)[1], whole[1]) and torch.equal(rows(0, most)[3:], whole[3:])
 
 
 def test_gemm_few_rows_that_lie_far_apart(ops):
@@ -622,7 +641,7 @@ def test_gemm_into_rows_longer_than_the_result(ops, M):
 @pytest.mark.simt_quick
 def test_gemm_rows_do_not_depend_on_the_batch(ops):
     """A row's result is the same, bit for bit, whatever other rows share the call, as long as the call
-    takes the same kernel form (block tiles; 16x16x32 products up to 64 rows; 4x4x4 products up to 4
+    takes the same kernel form (block tiles; 16x16x32 products up to 64 rows; of four pieces of k up to 4
     rows and 2,048 columns); between forms it differs by the rounding of 32-bit sums at most."""
     g = torch.Generator().manual_seed(3)
     K, N = 768, 300
@@ -639,7 +658,7 @@ def test_gemm_rows_do_not_depend_on_the_batch(ops):
     small = rows(0, 64)
     assert torch.equal(rows(3, 23)[7], small[10])                   # 16x16x32: 20 rows, 64 rows
     assert torch.equal(rows(4, 12)[6], small[10])                   # ... 8 rows
-    assert torch.equal(rows(10, 11)[0], rows(8, 12)[2])             # 4x4x4: 1 row, 4 rows
+    assert torch.equal(rows(10, 11)[0], rows(8, 12)[2])             # four pieces of k: 1 row, 4 rows
     assert torch.equal(rows(10, 13)[0], rows(10, 11)[0])            # ... 3 rows
     exact = a[10].double() @ w.double().t()
     scale = exact.abs().max().item()
