@@ -1,4 +1,4 @@
-// The maximum of a value over the two halves of a wavefront (lane l and lane l ^ 32), in every lane.
+// The maximum of a value over the two halves of a wavefront (lane l and lane l ^ 32), in every lane, and the sum over its four quarters.
 //
 // gfx950 has an instruction that swaps the upper 32 lanes of one register with the lower 32 lanes of
 // another (v_permlane32_swap_b32): given the value twice, one register then holds the lower half's values
@@ -13,4 +13,16 @@ __device__ __forceinline__ float half_max(float x) {
   // (two idle cycles in front, as a lane-crossing read of a register that the vector unit has just written wants)
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
   return fmaxf(lo, hi);
+}
+
+// x(l) + x(l ^ 16) + x(l ^ 32) + x(l ^ 48), the quarters of a half first.  (v_permlane16_swap_b32 swaps the odd quarters of one register with
+// the even ones of the other.)
+__device__ __forceinline__ float quarter_sum(float x) {
+  float lo = x, hi = x;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
+  x = lo + hi;
+  lo = x;
+  hi = x;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
+  return lo + hi;
 }

@@ -15,6 +15,7 @@
 // CausalSelfAttention.java:266-291,315-336, MLPBlock.java:250-292.
 #include "gemm_common.h"
 #include <da_read_arg.h>
+#include <da_lane_swap.h>
 
 #define FZ_COLS 16
 #define FZ_VPL 8          // float4 per lane when a row is held in registers: K <= 2048
@@ -183,17 +184,205 @@ gemm_ln_skinny_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epil
   }
 }
 
+struct LnRest {
+  float eps, center, gain_offset;
+};
+
 // ---------------------------------------------------------------------------------------------
-// One row tile (M <= 16), K <= 2048, parameters of one dtype: every load in whole cache lines.
+// M <= 8, K <= 2048, parameters of one dtype.  MFMA 16x16x32 with pieces of k side by side (gemm_skinny4 in gemm_mfma.hip): a lane holds 8
+// consecutive k of row r4 of 4 of w and of 4 rows of x, four neighbouring lanes 64 consecutive bytes, and what it holds of x is what it
+// normalises: nothing passes through LDS but a wavefront's mean and squares of each row.  Wavefront v of NW has the steps v and, SW of them, v + NW of 128
+// elements of k.  A row's statistics join its wavefronts' means and squares around them (M2 = sum of M2_v + n_v (mean_v - mean)^2).
+// Bound by what a wavefront computes for each row (so as few wavefronts as hold k in two steps each: K = 768, 3,072 columns, one row 3.5 us with 6
+// of them, 2.9 with 3) and by the bytes of w.  A workgroup owns `cols` columns, 4 * NG at most: as many as give every compute unit one workgroup, or
+// two.  us, cold weights, one behind the other, the kernel below with a row a wavefront -> this:
+//   1 row  K = 768, N = 2,304 3.2 -> 2.8, 3,072 3.6 -> 2.9; K = 1,024, N = 3,072 3.9 -> 3.3; K = 1,600, N = 4,800 6.7 -> 5.7, 6,400 7.4 -> 6.8
+//   8 rows K = 768, N = 2,304 3.9 -> 3.7, 3,072 4.1 -> 3.7; K = 1,024, N = 3,072 4.6 -> 4.1; K = 1,600, N = 4,800 8.5 -> 7.0, 6,400 9.3 -> 8.4
+// (w alone, read and dropped: 2.5 at K = 768, 4.5 to 5 and 5.2 at 1,600.)
+// ---------------------------------------------------------------------------------------------
+template <int MG, int NG, int NW, int SW, bool PBF16>
+__global__ void __launch_bounds__(NW * 64)
+gemm_ln_quads_kernel(const float* __restrict__ x, const int* __restrict__ rows, const void* __restrict__ gain, const void* __restrict__ shift,
+                     const bf16_t* __restrict__ w, int ldw, int N, int K, int rows_cols, LnRest lr_, Epilogue ep, KvScatter kv) {
+  const int M = rows_cols & 0xff, cols = rows_cols >> 8;
+  constexpr int ROWS = 4 * MG, COLS = 4 * NG;
+  __shared__ float2 stats[NW][ROWS];
+  __shared__ float red[NW][ROWS][COLS + 1];
+  const int t = threadIdx.x, lane = t % 64, wave = __builtin_amdgcn_readfirstlane(t / 64);
+  const int n0 = blockIdx.x * cols;
+  const int n_end = n0 + cols < N ? n0 + cols : N;
+  const int r4 = lane / 4 % 4, kb = (4 * (lane / 16) + lane % 4) * 8;
+  // ---- all loads first, in the order of their use (lanes past K read their rows' first piece, lanes past M or the last column the first row)
+  constexpr int PH = PBF16 ? 1 : 2;                  // 16-byte pieces of a lane's 8 gains
+  float4 xv[SW][MG][2];
+  uint4 gq[SW][PH], bq[SW][PH], wv[SW][NG];
+  const float* xr[MG];
+#pragma unroll
+  for (int i = 0; i < MG; ++i) {
+    const int m = 4 * i + r4 < M ? 4 * i + r4 : 0;
+    xr[i] = x + (size_t)(rows ? rows[m] : m) * K;
+  }
+#pragma unroll
+  for (int u = 0; u < SW; ++u) {
+    const int k = (wave + u * NW) * 128 + kb, ks = k < K ? k : 0;
+#pragma unroll
+    for (int i = 0; i < MG; ++i) {
+      xv[u][i][0] = *(const float4*)(xr[i] + ks);
+      xv[u][i][1] = *(const float4*)(xr[i] + ks + 4);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < SW; ++u) {
+    const int k = (wave + u * NW) * 128 + kb, ks = k < K ? k : 0;
+    const void* sh = shift ? shift : gain;
+#pragma unroll
+    for (int h = 0; h < PH; ++h) {
+      gq[u][h] = *(const uint4*)((const char*)gain + (size_t)(ks + 4 * h) * (PBF16 ? 2 : 4));
+      bq[u][h] = *(const uint4*)((const char*)sh + (size_t)(ks + 4 * h) * (PBF16 ? 2 : 4));
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < SW; ++u) {
+    const int k = (wave + u * NW) * 128 + kb, ks = k < K ? k : 0;
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      const int n = n0 + 4 * j + r4;
+      wv[u][j] = load16(w + (size_t)(n < n_end ? n : n0) * ldw + ks);
+    }
+  }
+  // this thread's output element, with what its epilogue needs
+  static_assert(ROWS * COLS <= NW * 64, "an output element a thread");
+  const int em = t / COLS, ec = t % COLS, en = n0 + ec;
+  const bool e_ok = em < M && en < n_end;                             // (M is ROWS at most)
+  const void* e_bsrc = ep.bias ? ep.bias : (const void*)w;
+  const int e_slot = kv.cache ? kv.slot_map[e_ok ? em : 0] : -1;
+  const int e_bidx = (ep.bias && e_ok) ? en : 0;
+  const uint32_t e_bias_raw = PBF16 ? (uint32_t)((const bf16_t*)e_bsrc)[e_bidx] : ((const uint32_t*)e_bsrc)[e_bidx];
+  da_read_arg(ep.act);
+  da_read_arg(ep.out_dtype);
+  KvColumn e_col;
+  if (kv.cache) e_col = kv_column(kv, en);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- statistics: a wavefront's own mean and squares around it, joined in the order of the wavefronts
+  auto count = [&](int v) {                            // elements of a row that wavefront v holds
+
+    int n = K - v * 128;
+    n = n < 0 ? 0 : (n < 128 ? n : 128);
+#pragma unroll
+    for (int u = 1; u < SW; ++u) {
+      int n2 = K - (v + u * NW) * 128;
+      n += n2 < 0 ? 0 : (n2 < 128 ? n2 : 128);
+    }
+    return n;
+  };
+  const int mine = count(wave);
+  const float inv_mine = mine > 0 ? lr_.center / (float)mine : 0.f;
+#pragma unroll
+  for (int i = 0; i < MG; ++i) {
+    float s = 0.f;
+#pragma unroll
+    for (int u = 0; u < SW; ++u) {
+      const float in = (wave + u * NW) * 128 + kb < K ? 1.f : 0.f;
+      const float4 p = xv[u][i][0], q = xv[u][i][1];
+      s += in * (((p.x + p.y) + (p.z + p.w)) + ((q.x + q.y) + (q.z + q.w)));
+    }
+    const float mean = quarter_sum(group_sum<4>(s)) * inv_mine;
+    float m2 = 0.f;
+#pragma unroll
+    for (int u = 0; u < SW; ++u) {
+      const float in = (wave + u * NW) * 128 + kb < K ? 1.f : 0.f;
+      const float4 p = xv[u][i][0], q = xv[u][i][1];
+      const float d[8] = {p.x - mean, p.y - mean, p.z - mean, p.w - mean, q.x - mean, q.y - mean, q.z - mean, q.w - mean};
+      m2 += in * (((d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3])) + ((d[4] * d[4] + d[5] * d[5]) + (d[6] * d[6] + d[7] * d[7])));
+    }
+    m2 = quarter_sum(group_sum<4>(m2));
+    if (lane < 16 && lane % 4 == 0) stats[wave][4 * i + r4] = make_float2(mean, m2);
+  }
+  lds_barrier();
+  // ---- the normalised rows, straight into fragments, and the products
+  floatx4 acc[MG][NG];
+  const float inv_k = 1.0f / (float)K;
+#pragma unroll
+  for (int i = 0; i < MG; ++i) {
+    float2 st[NW];
+#pragma unroll
+    for (int v = 0; v < NW; ++v) st[v] = stats[v][4 * i + r4];
+    float mean = 0.f;
+#pragma unroll
+    for (int v = 0; v < NW; ++v) mean += (float)count(v) * st[v].x;
+    mean *= inv_k;
+    float m2 = 0.f;
+#pragma unroll
+    for (int v = 0; v < NW; ++v) {
+      const float d = st[v].x - mean;
+      m2 += st[v].y + (float)count(v) * d * d;
+    }
+    const float rstd = 1.0f / sqrtf(m2 * inv_k + lr_.eps);
+#pragma unroll
+    for (int j = 0; j < NG; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < SW; ++u) {
+      const bool in = (wave + u * NW) * 128 + kb < K;
+      const float4 p = xv[u][i][0], q = xv[u][i][1];
+      const float xs[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+      float g8[8], b8[8];
+      if (PBF16) {
+        const uint32_t gw[4] = {gq[u][0].x, gq[u][0].y, gq[u][0].z, gq[u][0].w}, bw[4] = {bq[u][0].x, bq[u][0].y, bq[u][0].z, bq[u][0].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          g8[2 * e] = __uint_as_float(gw[e] << 16); g8[2 * e + 1] = __uint_as_float(gw[e] & 0xffff0000u);
+          b8[2 * e] = __uint_as_float(bw[e] << 16); b8[2 * e + 1] = __uint_as_float(bw[e] & 0xffff0000u);
+        }
+      } else {
+        const uint4 g0 = gq[u][0], g1 = gq[u][PH - 1], b0 = bq[u][0], b1 = bq[u][PH - 1];
+        const uint32_t gw[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w}, bw[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { g8[e] = __uint_as_float(gw[e]); b8[e] = __uint_as_float(bw[e]); }
+      }
+      uint32_t pk[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float y0 = (xs[2 * e] - mean) * rstd * (g8[2 * e] + lr_.gain_offset), y1 = (xs[2 * e + 1] - mean) * rstd * (g8[2 * e + 1] + lr_.gain_offset);
+        if (shift) { y0 += b8[2 * e]; y1 += b8[2 * e + 1]; }
+        pk[e] = in ? pack2_bf16(y0, y1) : 0u;
+      }
+      const uint4 av = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+#pragma unroll
+      for (int j = 0; j < NG; ++j) {
+        const uint4 wz = in ? wv[u][j] : make_uint4(0, 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wz), __builtin_bit_cast(bf16x8_t, av), acc[i][j], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MG; ++i)
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      const float d01 = lane & 1 ? acc[i][j][1] : acc[i][j][0], d23 = lane & 1 ? acc[i][j][3] : acc[i][j][2];
+      const float v = group_sum<4>(lane & 2 ? d23 : d01);
+      if (lane % 4 == 0) red[wave][4 * i + r4][j * 4 + lane / 16] = v;
+    }
+  lds_barrier();
+  
+  if (e_ok) {
+    float v = red[0][em][ec];
+#pragma unroll
+    for (int v2 = 1; v2 < NW; ++v2) v += red[v2][em][ec];
+    const float e_bias = !ep.bias ? 0.f : (PBF16 ? __uint_as_float(e_bias_raw << 16) : __uint_as_float(e_bias_raw));
+    epilogue_store(ep, em, en, v, e_bias);
+    if (kv.cache) kv_column_store(kv, e_col, e_slot, apply_act_bf16(v + e_bias, ep.act));
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// 9 to 16 rows, K <= 2048, parameters of one dtype: every load in whole cache lines.
 // Wavefront v of 8 reads rows v and v + 8 whole (RV float4 a lane), with the gain and bias at the
 // same places, computes their statistics, and writes the normalised rows as bfloat16 into LDS,
 // zeros past K.  The steps of w (64 elements of k, 8 rows x 128 bytes a load; wavefront v takes the
 // steps v, v + 8, ...) are asked for before anything else is computed and parked in the wavefront's
 // own piece of LDS; the fragments of both operands are read from LDS.  Steps past K read step 0 and
 // meet zeros.  The sum over k runs in the order of the steps, whatever M is.
-// TWO_ROWS false: M <= 8, a wavefront has one row and LDS holds 8 (the fragment's rows 8..15 read
-// rows 0..7 again and are never stored): half the LDS, so that with a wide K two workgroups still
-// share a compute unit and N / 16 workgroups run side by side.
 // ---------------------------------------------------------------------------------------------
 #define FL_LD (64 + 8)       // padded row of a parked step of w, elements
 // A workgroup owns `cols` columns, 16 * CT at most.  16 of them leave some compute units with more workgroups than others
@@ -202,10 +391,7 @@ gemm_ln_skinny_kernel(LnPrologue ln, const bf16_t* __restrict__ w, int ldw, Epil
 // what the kernel takes: rows of w, the rows of x, and gain and bias once a wavefront that has a row.
 // The arguments that the loads need are the first 14 words (build.py: KERNARG_PRELOAD; M and cols, 16 and 32 at most, share one);
 // what the epilogue needs is asked for behind the operands, with the place in the cache of the thread's column.
-struct LnRest {
-  float eps, center, gain_offset;
-};
-template <int RV, bool PBF16, bool TWO_ROWS, int CT = 1>
+template <int RV, bool PBF16, int CT>
 __global__ void __launch_bounds__(512)
 gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, const void* __restrict__ gain, const void* __restrict__ shift,
                     const bf16_t* __restrict__ w, int ldw, int N, int K, int rows_cols, LnRest lr_, Epilogue ep, KvScatter kv) {
@@ -213,7 +399,7 @@ gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, c
   const LnPrologue ln{x, rows, gain, 0, shift, 0, lr_.eps, lr_.center, lr_.gain_offset};
   constexpr int NW = 8, KMAX = RV * 256, ALD = KMAX + 8;      // ALD: padded row of a in LDS, elements
   constexpr int SW = (RV * 4 + NW - 1) / NW;                   // steps a wavefront
-  constexpr int RPW = TWO_ROWS ? 2 : 1, AR = RPW * NW;         // rows a wavefront normalises; rows in LDS
+  constexpr int RPW = 2, AR = RPW * NW;                         // rows a wavefront normalises; rows in LDS
   __shared__ __attribute__((aligned(16))) bf16_t a_lds[AR][ALD];
   constexpr int COLS = CT * 16, WL = COLS / 8;                 // columns at most; loads of 8 rows that cover w's
   // The wavefronts' sums lie behind the parked steps, where two workgroups still share a compute unit; else they take their place once all
@@ -258,7 +444,7 @@ gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, c
         bq[i] = *(const uint4*)((const float*)(ln.b ? ln.b : ln.g) + cs);
       }
     }
-    if (TWO_ROWS && row0 + NW < M) load_row(sv[RPW - 1], row0 + NW);
+    if (row0 + NW < M) load_row(sv[RPW - 1], row0 + NW);
   }
   uint4 wv[SW][WL];
 #pragma unroll
@@ -411,42 +597,55 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
   dim3 grid(da_ceil_div(N, FZ_COLS));
   const int mt = da_ceil_div(M, 16);
   hipStream_t s = (hipStream_t)stream;
-  // the kernel with whole-line loads takes one row tile, K up to 2048, and parameters of one dtype
-  // Columns a workgroup: 16 up to 4,096 columns and for a vocabulary; up to 8,192 as many as give every compute unit one
-  // workgroup; up to 16,384 as many as give every one two, where two fit side by side (registers: K up to 1,536).  With more than
-  // 8 rows only up to K = 1,024 (LDS; no step sends wider ones here).  Measured on MI355X with cold weights, 16 columns a workgroup -> this, us:
-  //   K = 1,600, N = 4,800 (19 columns) one row 6.9 -> 6.6, 8 rows 9.6 -> 8.2; N = 6,400 (25) 7.4 -> 7.3, 10.2 -> 9.5
-  //   K =   768, N = 8,320 (17, two a unit) one row 5.5 -> 5.4, 16 rows 10.0 -> 8.6; N = 12,800 (25) 6.4 -> 6.2, 12.2 -> 9.2
-  //   K = 1,536, N = 8,200 (17) one row 7.9 -> 7.6, 8 rows 10.4 -> 10.0; N = 12,800 10.8 -> 9.4, 14.3 -> 11.9; N = 16,384 (32) 11.5 -> 10.9,
-  //              15.0 -> 13.4 (two groups of 16 columns, one after the other: 8 rows 10.4, 13.3 and 14.3)
-  //   K = 1,600, N = 12,800, where only one of 25 fits: one row 11.6 -> 12.4 (so 16 stay; 8 rows: da_can_fuse_ln)
-  const bool one_a_unit = N > 16 * 256 && N <= 32 * 256 && (M <= 8 || K <= 1024);
-  const bool two_a_unit = N > 32 * 256 && N <= 64 * 256 && K <= (M <= 8 ? 1536 : 1024);
-  const bool wide = one_a_unit || two_a_unit;
-  const int cols = one_a_unit ? da_ceil_div(N, 256) : (two_a_unit ? da_ceil_div(N, 512) : FZ_COLS);
+  // These kernels take one row tile, K up to 2048, and parameters of one dtype.
+  // Columns a workgroup, up to 8 rows: every compute unit a workgroup up to 8,192 columns, two up to 16,384 (32 columns at most, and 16
+  // for a vocabulary), whole groups of 4 where that is no matter.  9 to 16 rows: 16 up to 4,096 columns and for a vocabulary; up to 8,192 as many as
+  // give every compute unit one workgroup; up to 16,384 as many as give every one two, both only up to K = 1,024 (LDS; no step sends wider
+  // ones here).  16 columns a workgroup -> this, 16 rows, K = 768, us: N = 8,320 (17, two a unit) 10.0 -> 8.6; N = 12,800 (25) 12.2 -> 9.2.
+  const int units = N <= 32 * 256 ? 256 : 512;
+  const bool wide = N > 16 * 256 && N <= 64 * 256 && K <= 1024;
+  const int share = N <= 64 * 256 ? da_ceil_div(N, units) : FZ_COLS;
+  const int cols = M <= 8 ? (share <= 16 ? da_ceil_div(share, 4) * 4 : share) : (wide ? share : FZ_COLS);
   const int pdt = g_dtype;
   const bool same = (!b || b_dtype == pdt) && (!bias || bias_dtype == pdt) && (pdt == DA_BF16 || pdt == DA_F32);
-#define LAUNCH_LDS_R(RV, PB, TWO)                                                                                  \
+#define LAUNCH_LN(KERNEL, THREADS)                                                                                 \
+  hipLaunchKernelGGL(KERNEL, dim3(da_ceil_div(N, cols)), dim3(THREADS), 0, s, x, rows, g, b, (const bf16_t*)w, ldw, N, K, M | cols << 8, LnRest{eps, center, gain_offset}, ep, kv)
+#define LAUNCH_Q(MG, NG, NW, SW)                                                                                   \
   do {                                                                                                            \
-    const dim3 g2(da_ceil_div(N, cols));                                                                          \
-    if (wide)                                                                                                     \
-      hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO, (TWO && RV > 4 ? 1 : 2)>), g2, dim3(512), 0, s, x, rows, g, b, (const bf16_t*)w, ldw, N, K, M | cols << 8, LnRest{eps, center, gain_offset}, ep, kv); \
-    else                                                                                                          \
-      hipLaunchKernelGGL((gemm_ln_rows_kernel<RV, PB, TWO>), g2, dim3(512), 0, s, x, rows, g, b, (const bf16_t*)w, ldw, N, K, M | cols << 8, LnRest{eps, center, gain_offset}, ep, kv); \
+    if (pdt == DA_BF16) LAUNCH_LN((gemm_ln_quads_kernel<MG, NG, NW, SW, true>), NW * 64);                          \
+    else LAUNCH_LN((gemm_ln_quads_kernel<MG, NG, NW, SW, false>), NW * 64);                                        \
   } while (0)
-#define LAUNCH_LDS_P(RV, PB)                                                                                      \
+#define LAUNCH_Q_K(MG, NG)                                                                                         \
   do {                                                                                                            \
-    if (M <= 8) LAUNCH_LDS_R(RV, PB, false);                                                                      \
-    else LAUNCH_LDS_R(RV, PB, true);                                                                              \
+    if (K <= 512) LAUNCH_Q(MG, NG, 4, 1);                                                                          \
+    else if (K <= 1024) LAUNCH_Q(MG, NG, 4, 2);                                                                    \
+    else if (K <= 1536) LAUNCH_Q(MG, NG, 6, 2);                                                                    \
+    else LAUNCH_Q(MG, NG, 8, 2);                                                                                   \
+  } while (0)
+#define LAUNCH_Q_N(MG)                                                                                             \
+  do {                                                                                                            \
+    switch ((cols + 3) / 4) {                                                                                     \
+      case 1: LAUNCH_Q_K(MG, 1); break;                                                                            \
+      case 2: LAUNCH_Q_K(MG, 2); break;                                                                            \
+      case 3: LAUNCH_Q_K(MG, 3); break;                                                                            \
+      case 4: LAUNCH_Q_K(MG, 4); break;                                                                            \
+      case 5: LAUNCH_Q_K(MG, 5); break;                                                                            \
+      case 6: LAUNCH_Q_K(MG, 6); break;                                                                            \
+      case 7: LAUNCH_Q_K(MG, 7); break;                                                                            \
+      default: LAUNCH_Q_K(MG, 8); break;                                                                           \
+    }                                                                                                             \
   } while (0)
 #define LAUNCH_LDS(RV)                                                                                            \
   do {                                                                                                            \
-    if (pdt == DA_BF16)                                                                                           \
-      LAUNCH_LDS_P(RV, true);                                                                                     \
-    else                                                                                                          \
-      LAUNCH_LDS_P(RV, false);                                                                                    \
+    constexpr int CT = RV > 4 ? 1 : 2;                                                                            \
+    if (pdt == DA_BF16 && wide) LAUNCH_LN((gemm_ln_rows_kernel<RV, true, CT>), 512);                               \
+    else if (pdt == DA_BF16) LAUNCH_LN((gemm_ln_rows_kernel<RV, true, 1>), 512);                                   \
+    else if (wide) LAUNCH_LN((gemm_ln_rows_kernel<RV, false, CT>), 512);                                           \
+    else LAUNCH_LN((gemm_ln_rows_kernel<RV, false, 1>), 512);                                                      \
   } while (0)
-  if (mt == 1 && same && K <= 2048) {
+  if (same && M <= 4 && K <= 2048) LAUNCH_Q_N(1);
+  else if (same && M <= 8 && K <= 2048) LAUNCH_Q_N(2);
+  else if (mt == 1 && same && K <= 2048) {
     if (K <= 256) LAUNCH_LDS(1);
     else if (K <= 512) LAUNCH_LDS(2);
     else if (K <= 768) LAUNCH_LDS(3);

@@ -422,6 +422,37 @@ def test_fused_norm_product_one_workgroup_a_compute_unit(ops, M, N, K):
         assert (out.double() - ref).abs().max() < 2e-2 * max(1.0, ref.abs().max().item())
 
 
+@pytest.mark.parametrize("dt", [helpers.quick(torch.bfloat16, mark="simt_a"), torch.float32])
+@pytest.mark.parametrize("N,K", [helpers.quick(50, 120, mark="simt_b"), (2304, 512), (1021, 520), (4100, 1024), (4801, 1032), (8190, 1536), (8200, 1544),
+                                 helpers.quick(12, 2048, mark="simt_b"), (6401, 1600)])
+def test_norm_and_product_of_up_to_8_rows(ops, N, K, dt):
+    """A wavefront holds one step of 128 k or two, 4 to 8 of them; 4 to 32 columns a workgroup, columns that end inside a group of 4; one group
+    of 4 rows or two; rows in any order.  Rows whose mean is a hundred times their spread (statistics joined from the wavefronts' own means keep it);
+    a row has the same bits beside any others, and one that is not finite leaves the others alone."""
+    g = torch.Generator().manual_seed(N + K)
+    R = 11
+    x = (torch.randn(R, K, generator=g) * 3 + torch.arange(R).view(R, 1) * 30.0).to(DEV)
+    gw, gb, bias = (torch.randn(n, generator=g).to(dt).to(DEV) for n in (K, K, N))
+    w = bf(torch.randn(N, K, generator=g) * 0.1).to(DEV)
+    for M in (1, 4, 5, 8):
+        rows = torch.randperm(R, generator=g)[:M].to(torch.int32).to(DEV)
+        out = ops.linear_ln(x, rows, M, gw, gb, 1e-5, w, bias, torch.empty(M, N, device=DEV))
+        a = F.layer_norm(x[rows.long()].double(), (K,), gw.double(), gb.double(), 1e-5).to(torch.bfloat16).double()
+        ref = a @ w.double().t() + bias.double()
+        # (the norm's 32-bit rounding may move an entry of a to the next bfloat16: 2^-8 of one product among K)
+        assert (out.double() - ref).abs().max() < 2e-2 * max(1.0, ref.abs().max().item()), M
+        rms = ops.linear_rms(x, rows, M, gw, 1.0, 1e-5, w, bias, torch.empty(M, N, device=DEV, dtype=torch.bfloat16), act="gelu_new")
+        xd = x[rows.long()].double()
+        a = (xd / (xd.square().mean(1, keepdim=True) + 1e-5).sqrt() * (1.0 + gw.double())).to(torch.bfloat16).double()
+        ref = F.gelu(a @ w.double().t() + bias.double(), approximate="tanh")
+        assert (rms.double() - ref).abs().max() < 2e-2 * max(1.0, ref.abs().max().item()), M
+    whole = ops.linear_ln(x, None, 8, gw, gb, 1e-5, w, bias, torch.empty(8, N, device=DEV))
+    few = lambda lo, hi: ops.linear_ln(x[lo:hi].contiguous(), None, hi - lo, gw, gb, 1e-5, w, bias, torch.empty(hi - lo, N, device=DEV))
+    assert torch.equal(few(2, 3)[0], whole[2]) and torch.equal(few(1, 5), whole[1:5]) and torch.equal(few(3, 8), whole[3:])
+    x[0, K - 1] = float("inf")
+    assert torch.equal(few(0, 8)[1:], whole[1:])
+
+
 @pytest.mark.parametrize("M,N,K", [(1600, 2000, 200), (1555, 1999, 320), (2048, 1600, 1600), (1536, 2304, 768), (2048, 2304, 768),
                                    (4096, 768, 3072), (2500, 1600, 2112), (2048, 1600, 6400)])
 def test_gemm_tiles_alone_on_their_compute_units(ops, M, N, K):
