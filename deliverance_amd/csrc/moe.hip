@@ -18,6 +18,7 @@
 // sums over k run in the same order for every row.  Expert weights are stacked: gate | up as
 // [n_experts][2 F][K] (gate rows first), down as [n_experts][width][F].
 #include "gemm_common.h"
+#include <type_traits>
 
 #define MOE_MAX_EXPERTS 1024
 
@@ -809,17 +810,25 @@ extern "C" int da_moe_combine_norm(const float* out, int ldo, const int* slot_of
 
 // ---- the grouped products on the matrix cores (bfloat16) ---------------------------------------------------
 // A workgroup owns a tile of 32 slots x 16 columns of one expert, and its wavefronts share out k: wavefront v takes the
-// k-steps of 32 number v, v + NW, ... with MFMA 16x16x32, operands from memory into the lanes' fragments (a lane's 16 bytes
-// are 8 consecutive k of one row), MM_UNROLL steps asked for at once.  With few rows an expert, as in decoding, the kernel
-// streams the expert's weights once, and narrow columns mean many workgroups for that (8 experts of 512 x 768: 256).  The
+// steps of 64 number v, v + NW, ... with MFMA 16x16x32.  With few rows an expert, as in decoding, the kernel
+// streams the expert's weights once, and narrow columns mean many workgroups for that (8 experts of 512 x 768: 256).  Operands come
+// in whole cache lines, 8 rows x 128 bytes a load, of the rows of a only those that hold a pair; the wavefront parks a step in its own
+// piece of LDS and reads the fragments from there, as gemm_skinny does.  (Straight into fragments neighbouring lanes lie in 16 rows, which
+// a compute unit takes one lane at a time.)  The
 // wavefronts' sums meet in LDS and are added in the order of the wavefronts.  GATED: the gate and up rows of the same
 // columns are multiplied side by side and out = act(g) * u leaves in bfloat16; else one product leaves in 32-bit.  A row's
-// sums run in one order whatever else is in the step.  (Whole cache lines a load, a lane's 32 bytes for two products of a step of 64 k: a
-// Virudra's step of 355M sizes 1,038 -> 1,049 us; the two wavefronts that share a line ask for it side by side as it is.)  Measured on MI355X against 64 columns a workgroup without shared k
-// (8 tokens, 2 of 8 experts of 512 x 768): 10.7 -> 5.7 us, down 6.2 -> 5.3.
+// sums run in one order whatever else is in the step.  us, cold weights, recorded one behind the other,
+// fragments straight from memory -> this, first / second product, 8 experts, top 2: 1,376 x 1,024, 1 token 4.7 / 4.3 -> 4.4 / 3.6, 5 tokens 9.9 / 7.1 -> 8.9 / 5.9,
+// 64 tokens 12.8 / 9.4 -> 12.0 / 7.2, 250 tokens 28.1 / 18.7 -> 23.8 / 12.2; 64 experts, top 8, 256 x 512, 30 tokens 13.0 / 17.3 -> 8.0 / 5.4.  (GATED with 16 gate columns
+// a workgroup, which leaves a compute unit two workgroups for four: a Virudra's step 957 us against 942.)
 #define MM_ROWS 32
 #define MM_COLS 16
-#define MM_UNROLL 4
+#define MM_LD (64 + 8)       // padded row of a parked step, elements
+// (the vector type of the language: arrays of HIP's uint4, a class, that are only copied stay in memory)
+typedef __attribute__((ext_vector_type(4))) uint32_t mm_u32x4;
+
+template <int MODE>
+constexpr int mm_cols() { return MODE == MOE_GATED ? MM_COLS / 2 : MM_COLS; }
 
 template <int MODE, int NW>
 __global__ void __launch_bounds__(NW * DA_WAVE)
@@ -827,17 +836,22 @@ moe_mfma_kernel(const bf16_t* __restrict__ a, const int* __restrict__ row_of_slo
                 const bf16_t* __restrict__ w, int lda, int K, int F, int ldo, int act, float limit, void* __restrict__ out,
                 const float* __restrict__ slot_scale) {
   constexpr bool GATED = MODE == MOE_GATED, GATHER = MODE != MOE_DOWN;
-  constexpr int G = GATED ? 2 : 1;
-  __shared__ float sums[NW][G][8][DA_WAVE];                 // [wavefront][product][register of the tile][lane]
-  const int t = threadIdx.x, lane = t % DA_WAVE, wave = t / DA_WAVE;
-  const int fr = lane % 16, fk = (lane / 16) * 8;
-  const int m0 = blockIdx.y * MM_ROWS, n0 = blockIdx.x * MM_COLS;
+  constexpr int OC = mm_cols<MODE>();                                          // columns that leave
+  constexpr int STAGE_BYTES = NW * (16 + MM_COLS) * MM_LD * 2, SUM_BYTES = NW * 8 * DA_WAVE * 4;
+  __shared__ __attribute__((aligned(16))) char smem[STAGE_BYTES > SUM_BYTES ? STAGE_BYTES : SUM_BYTES];
+  bf16_t (*stage)[(16 + MM_COLS) * MM_LD] = (bf16_t (*)[(16 + MM_COLS) * MM_LD])smem;      // 16 rows of a, then the columns' rows of w
+  float (*sums)[8][DA_WAVE] = (float (*)[8][DA_WAVE])smem;                     // [wavefront][register of the tile][lane]
+  const int t = threadIdx.x, lane = t % DA_WAVE, wave = __builtin_amdgcn_readfirstlane(t / DA_WAVE);
+  const int fr = lane % 16, fk = (lane / 16) * 8;    // a fragment: row fr of 16, k-group lane / 16
+  const int lr = lane / 8, lc = (lane % 8) * 8;      // a load: row lr of 8, 16-byte piece lane % 8
+  const int m0 = blockIdx.y * MM_ROWS, n0 = blockIdx.x * OC;
   // every load of the routing at once: the expert, the rows of a, the rows that this thread will store
   constexpr int PER = (8 + NW - 1) / NW;
   const int e = tile_expert[blockIdx.y];
-  int srow[2], used[PER];
+  const int place = row_of_slot[m0 + lane % MM_ROWS];
+  int srow[4], used[PER];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) srow[i] = row_of_slot[m0 + i * 16 + fr];
+  for (int i = 0; i < 4; ++i) srow[i] = row_of_slot[m0 + i * 8 + lr];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int x = (wave + j * NW) % 8;
@@ -846,66 +860,91 @@ moe_mfma_kernel(const bf16_t* __restrict__ a, const int* __restrict__ row_of_slo
   if (e < 0) return;
   // the rows of a: gathered by slot for the first product (a padding slot reads row 0 and is never stored),
   // the slot's own row for the second; an expert's slots are filled from the front
-  const bool two = __builtin_amdgcn_readfirstlane(srow[1]) >= 0;      // (lane 0's: slot m0 + 16; the same for the workgroup)
-  const bf16_t* ap[2];
+  const int filled = __popcll(__builtin_amdgcn_ballot_w64(place >= 0) & 0xffffffffull);
+  const bf16_t* pa[4];
+  const bf16_t* pw[2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = GATHER ? (srow[i] >= 0 ? srow[i] : 0) : m0 + i * 16 + fr;
-    ap[i] = a + (size_t)r * lda + fk;
+  for (int i = 0; i < 4; ++i) {
+    const int r = GATHER ? (srow[i] >= 0 ? srow[i] : 0) : m0 + i * 8 + lr;
+    pa[i] = a + (size_t)r * lda + lc;
   }
-  const int wcol = n0 + fr < F ? n0 + fr : 0;
-  const bf16_t* wg = w + ((size_t)e * G * F + wcol) * K + fk;
-  const bf16_t* wu = wg + (size_t)F * K;
-  floatx4 acc[2][G];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {                        // GATED: the gate rows of the columns, then their up rows
+    const int c = n0 + (GATED ? 0 : i * 8) + lr;
+    pw[i] = w + ((size_t)e * (GATED ? 2 : 1) * F + (GATED ? (size_t)i * F : 0) + (c < F ? c : 0)) * K + lc;
+  }
+  floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+  bf16_t* const mine = stage[wave];
+  // AL: loads of 8 rows that cover the filled slots; UNROLL: steps asked for at once
+  auto walk = [&](auto alc, auto unrollc) {
+    constexpr int AL = decltype(alc)::value, UNROLL = decltype(unrollc)::value, TILES = (AL + 1) / 2;
+#pragma unroll 1
+    for (int k0 = wave * 64; k0 < K; k0 += 64 * NW * UNROLL) {
+      mm_u32x4 av[UNROLL][AL], wv[UNROLL][2];
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        const int k = k0 + u * 64 * NW, ks = k + lc < K ? k : -lc;             // past K: the row's first piece; zeros are parked
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wv[u][i] = *(const mm_u32x4*)(pw[i] + ks);
+#pragma unroll
+        for (int i = 0; i < AL; ++i) av[u][i] = *(const mm_u32x4*)(pa[i] + ks);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        if (u > 0 && k0 + u * 64 * NW >= K) continue;                           // (the same for the whole wavefront)
+        const bool kin = k0 + u * 64 * NW + lc < K;
+        const mm_u32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *(mm_u32x4*)&mine[(16 + i * 8 + lr) * MM_LD + lc] = kin ? wv[u][i] : zero;
+#pragma unroll
+        for (int h = 0; h < TILES; ++h) {
+#pragma unroll
+          for (int i = 2 * h; i < (AL < 2 * h + 2 ? AL : 2 * h + 2); ++i) *(mm_u32x4*)&mine[(i % 2 * 8 + lr) * MM_LD + lc] = kin ? av[u][i] : zero;
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+          for (int c = 0; c < 64; c += 32) {
+            // (rows that were not parked hold anything: what they give is never stored)
+            const bf16x8_t af = __builtin_bit_cast(bf16x8_t, *(const uint4*)&mine[fr * MM_LD + c + fk]);
+            const bf16x8_t wf = __builtin_bit_cast(bf16x8_t, *(const uint4*)&mine[(16 + fr) * MM_LD + c + fk]);
+            acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, wf, acc[h], 0, 0, 0);
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        }
+      }
+    }
+  };
+  const std::integral_constant<int, 2> two{};
+  const std::integral_constant<int, 3> three{};
+  const bool up_to_two = K <= 64 * NW * 2;              // (steps that do not exist would be asked for all the same)
+  if (filled <= 8) {
+    if (up_to_two) walk(std::integral_constant<int, 1>{}, two); else walk(std::integral_constant<int, 1>{}, three);
+  } else if (filled <= 16) {
+    if (up_to_two) walk(two, two); else walk(two, three);
+  } else walk(std::integral_constant<int, 4>{}, two);
+  lds_barrier();                                       // the sums take the parked steps' place
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int g = 0; g < G; ++g) acc[i][g] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const uint4 zero = make_uint4(0, 0, 0, 0);
-  for (int k0 = wave * 32; k0 < K; k0 += 32 * NW * MM_UNROLL) {
-    uint4 av[MM_UNROLL][2], wv[MM_UNROLL][G];
-#pragma unroll
-    for (int u = 0; u < MM_UNROLL; ++u) {
-      const int k = k0 + u * 32 * NW;
-      const int ks = (k + fk < K) ? k : -fk;                // past K: the row's first chunk, met by zeros in a
-      wv[u][0] = load16(wg + ks);
-      if (GATED) wv[u][G - 1] = load16(wu + ks);
-      av[u][0] = load16(ap[0] + ks);
-      av[u][1] = two ? load16(ap[1] + ks) : zero;
-    }
-#pragma unroll
-    for (int u = 0; u < MM_UNROLL; ++u) {
-      const bool kin = k0 + u * 32 * NW + fk < K;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        if (i == 1 && !two) continue;
-        const uint4 x = kin ? av[u][i] : zero;
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-          acc[i][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x),
-                                                              __builtin_bit_cast(bf16x8_t, wv[u][g]), acc[i][g], 0, 0, 0);
-      }
-    }
-  }
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sums[wave][g][i * 4 + r][lane] = acc[i][g][r];
+    for (int r = 0; r < 4; ++r) sums[wave][i * 4 + r][lane] = acc[i][r];
   lds_barrier();
-  // acc[i][.][r] of a lane is row 16 i + 4 (lane / 16) + r of the tile, column n0 + lane % 16
+  // acc[i][r] of a lane is row 16 i + 4 (lane / 16) + r of the tile, column n0 + lane % 16 (GATED: lane % 8, up from lane 8 of 16 on)
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int x = wave + j * NW;
     const int row = x / 4 * 16 + 4 * (lane / 16) + x % 4;
-    if (x >= 8 || used[j] < 0 || n0 + fr >= F) continue;
+    if (x >= 8 || used[j] < 0 || fr >= OC || n0 + fr >= F) continue;
+    constexpr int G = GATED ? 2 : 1;
     float v[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      v[g] = sums[0][g][x][lane];
+      v[g] = sums[0][x][lane + 8 * g];
 #pragma unroll
-      for (int k = 1; k < NW; ++k) v[g] += sums[k][g][x][lane];
+      for (int k = 1; k < NW; ++k) v[g] += sums[k][x][lane + 8 * g];
     }
     const size_t o = (size_t)(m0 + row) * ldo + n0 + fr;
     const float sc = (GATHER && slot_scale) ? slot_scale[m0 + row] : 1.0f;
@@ -918,7 +957,7 @@ moe_mfma_kernel(const bf16_t* __restrict__ a, const int* __restrict__ row_of_slo
 // eight wavefronts where k has steps for them, else four
 #define MM_LAUNCH(MODE, cols, K, ...)                                                                                        \
   do {                                                                                                                       \
-    const dim3 grid_(da_ceil_div(cols, MM_COLS), T_cap);                                                                     \
+    const dim3 grid_(da_ceil_div(cols, mm_cols<MODE>()), T_cap);                                                                     \
     if ((K) > 128) hipLaunchKernelGGL((moe_mfma_kernel<MODE, 8>), grid_, dim3(8 * DA_WAVE), 0, (hipStream_t)stream, __VA_ARGS__); \
     else hipLaunchKernelGGL((moe_mfma_kernel<MODE, 4>), grid_, dim3(4 * DA_WAVE), 0, (hipStream_t)stream, __VA_ARGS__);      \
   } while (0)

@@ -1483,3 +1483,63 @@ def test_attention_of_more_sequences_than_a_launch_has_rows(ops, form):
         tol = tol + 2.0 ** -8 * v.abs().max()                                           # (its weights are bfloat16)
     assert ((out.double().cpu()[at] - want).abs() <= tol).all()
     assert bool((out != 0).any(dim=1).all())
+
+
+@pytest.mark.parametrize("K,F", [helpers.quick(72, 24), (128, 40), (136, 20), (1024, 344), (1376, 72), (1544, 36)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_grouped_products_of_experts_with_few_rows(ops, K, F, gated):
+    """Tiles of 32 slots whose filled slots are 1 to 32 (both sides of 8, 16, and whole loads of 8 rows), an expert with two tiles, a tile of nobody;
+    columns that end inside a workgroup, a K that a step cuts, two and three steps a wavefront; slots without a pair are not written.  First
+    products gathered by slot with a weight a slot (one matrix) or gate and up (two), the second on the slots' own rows.  Bounds: 2^-8 of the
+    largest entry for the bfloat16 results, 1e-5 of it for the 32-bit sums."""
+    g = torch.Generator().manual_seed(K + F)
+    counts, tile = [1, 8, 9, 16, 17, 24, 25, 32 + 5], 32
+    E, N = len(counts), 41
+    rows, experts = [], []
+    for e, c in enumerate(counts):
+        for t0 in range(0, c, tile):
+            n = min(tile, c - t0)
+            rows += [int(x) for x in torch.randint(0, N, (n,), generator=g)] + [-1] * (tile - n)
+            experts.append(e)
+    rows, experts = rows + [-1] * tile, experts + [-1]
+    T = len(experts)
+    row_of_slot, tile_expert = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in (rows, experts))
+    G = 2 if gated else 1
+    h = bf(torch.randn(N, K, generator=g)).to(DEV)
+    up = bf(torch.randn(E, G * F, K, generator=g) * 0.1).to(DEV)
+    scale = torch.rand(T * tile, generator=g).to(DEV) + 0.5
+    mid = torch.full((T * tile, F), 7.0, dtype=torch.bfloat16, device=DEV)
+    lib, ptr = ops._lib(), ops._ptr
+    if gated:
+        ops._check(lib.da_moe_gated_mfma(ptr(h), K, ptr(row_of_slot), ptr(tile_expert), ptr(up), ptr(mid), F, T, K, F, ops.ACTIVATIONS["silu"],
+                                         0.0, ops._stream()))
+    else:
+        ops._check(lib.da_moe_up_mfma(ptr(h), K, ptr(row_of_slot), ptr(tile_expert), ptr(up), ptr(scale), ptr(mid), F, T, K, F,
+                                      ops.ACTIVATIONS["relu"], ops._stream()))
+    used = row_of_slot >= 0
+    expert_of = tile_expert.long().repeat_interleave(tile)
+    hd, ud = h.double(), up.double()
+    for e in range(E):
+        at = (used & (expert_of == e)).nonzero()[:, 0]
+        first = hd[row_of_slot[at].long()] @ ud[e].t()
+        want = F_silu(first[:, :F]) * first[:, F:] if gated else F_relu(first * scale[at].double()[:, None])
+        assert (mid[at].double() - want).abs().max() < 2.0 ** -8 * max(1.0, want.abs().max().item()), (e, counts[e])
+    assert bool((mid[~used] == 7.0).all())
+    if F % 8:
+        return                                       # (rows of the second product's operands are whole pieces of 16 bytes)
+    down = bf(torch.randn(E, K, F, generator=g) * 0.1).to(DEV)
+    out = torch.full((T * tile, K), 7.0, device=DEV)
+    ops._check(lib.da_moe_down_mfma(ptr(mid), F, ptr(row_of_slot), ptr(tile_expert), ptr(down), ptr(out), K, T, F, K, ops._stream()))
+    for e in range(E):
+        at = (used & (expert_of == e)).nonzero()[:, 0]
+        want = mid[at].double() @ down[e].double().t()
+        assert (out[at].double() - want).abs().max() < 1e-5 * max(1.0, want.abs().max().item()), (e, counts[e])
+    assert bool((out[~used] == 7.0).all())
+
+
+def F_silu(x):
+    return x / (1.0 + torch.exp(-x))
+
+
+def F_relu(x):
+    return x.clamp(min=0.0)
