@@ -10,6 +10,16 @@
 //   softmax: a lane holds 4 rows of one key column, so a row's maximum and sum are exchanges among 16 lanes;
 //   values : stored dimension-major, so a lane's 16-byte piece is 4 consecutive keys of its dimension, which is the
 //            right operand as it lies in memory; the weights turn from columns into rows through LDS.
+// A compute unit takes four lanes' addresses at once where they lie in one line and one at a time else, and a fragment's neighbouring lanes
+// are 16 different rows.  Head sizes above 64, whose values are asked for behind the scores, so load 64 consecutive bytes of a row by four
+// neighbouring lanes (lane 4 c + q what lane c + 16 q multiplies), and a load's 64 pieces pass through 1 KB of LDS into their places, the
+// same bits.  us, a row a lane / this, head size 128: 8 heads, 8 sequences of 1,000 keys in pages of 64 45.3 / 31.9, a prompt of 1,024
+// 55.7 / 40.8; 12 heads, pages of 16, 4 prompts of 64 9.6 / 9.4, of 600 119 / 103, 16 sequences of 200 keys 11.9 / 11.3.  (Up to 64, where all loads are asked
+// for at once, the way through LDS takes 0.3 us and gives it back only on a full chip: 4 sequences of 61 keys 5.4 / 5.7.)
+// Up to a head size of 64 registers are held to 128, so that two workgroups share a compute unit; head size 64, us, one / two: 12 heads, 32 sequences of
+// 30 keys 8.7 / 5.6, 64 of 600 43.7 / 39.3, two prompts of 1,024 73.7 / 58.5; 16 heads, prompts of 300 and 180 19.1 / 15.3, one of 600 24.5 / 21.1.  Not
+// for prompts of up to 512 workgroups (ALONE: LDS that leaves no room for a second one), where two long ones meet on a compute unit while others have none: 8 heads, 600 14.7 / 16.2, 16 heads, 300
+// 11.2 / 12.7, 12 heads, 300 and 180 13.1 / 14.4, 600 19.5 / 19.9.
 // All key and value loads of a chunk are asked for before any is used (for head sizes up to 64; above, the values once
 // the scores are done).  Bound by two trips to memory and D instructions of 32 cycles a chunk.  (Chunks of 64 keys leave most wavefronts
 // of a short context without any and the others a chain twice as long; us, 64 / 32 keys a chunk, 12 heads of 64: 4 sequences of 61
@@ -39,6 +49,30 @@ __device__ __forceinline__ float af_max16(float v) {          // the maximum ove
   return fmaxf(v, dpp_move<0x140, 0xF>(v, v));
 }
 
+// Lane 4 c + q of N loads holds the piece of lane c + 16 q: through the wavefront's own part of LDS into their places, up to AF_TURN loads
+// at a time.  (A row's pieces are turned by the row's group of four, so that the reads of 16 rows spread over the banks.  LDS serves a
+// wavefront's instructions in order: it is the compiler alone that must keep them.)
+#define AF_TURN 4
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+template <int N>
+__device__ __forceinline__ void af_turn(float4 (&x)[N], f32x4_t* xs, int lane) {
+  const int to = (lane & ~3) | ((lane & 3) ^ (lane / 16));
+  const int from = 4 * (lane % 16) + ((lane / 16) ^ (lane % 16 / 4));
+#pragma unroll
+  for (int b = 0; b < N; b += AF_TURN) {
+#pragma unroll
+    for (int i = b; i < b + AF_TURN && i < N; ++i) xs[(i - b) * DA_WAVE + to] = __builtin_bit_cast(f32x4_t, x[i]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int i = b; i < b + AF_TURN && i < N; ++i) x[i] = __builtin_bit_cast(float4, xs[(i - b) * DA_WAVE + from]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
 // What the products cannot give: an entry whose weighted sum is not finite (the 16 rows of a tile share their keys, and a
 // weight of zero times another row's infinite value is no number), or whose row has no weight at all (ll is 0: it sees no
 // key, or only scores of minus infinity).  Key by key in ascending order, a value whose weight is zero is not looked at.
@@ -63,20 +97,24 @@ __device__ __forceinline__ float af_entry(const float* qr, const float* kb, cons
   return ll == 0.f ? (any ? NAN : 0.f) : sum / ll;
 }
 
-template <int D16>
-__global__ void __launch_bounds__(AF_WAVES * DA_WAVE)
+template <int D16, bool ALONE = false>
+__global__ void __launch_bounds__(AF_WAVES * DA_WAVE, D16 <= 4 ? 4 : 2)
 attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ cache, const int* __restrict__ block_table,
                 const int* __restrict__ q_start, const int* __restrict__ seq_lens, int q_ld, int max_blocks, int Hq, int Hkv, int page,
                 float scale, int window, float* __restrict__ out, int out_ld) {
   constexpr int D = D16 * 16;
+  constexpr bool TURN = D16 > 4;
   constexpr int OLD = D + 4;                                   // padded row of a partial result
-  constexpr int P_FLOATS = AF_WAVES * 16 * AF_PLD, O_FLOATS = AF_WAVES * 16 * OLD;
-  __shared__ __attribute__((aligned(16))) float smem[P_FLOATS > O_FLOATS ? P_FLOATS : O_FLOATS];   // weights, then partial results
+  constexpr int X_FLOATS = !TURN ? 0 : (D16 < AF_TURN ? D16 : AF_TURN) * DA_WAVE * 4, P_FLOATS = AF_WAVES * (16 * AF_PLD + X_FLOATS), O_FLOATS = AF_WAVES * 16 * OLD;
+  constexpr int USED = P_FLOATS > O_FLOATS ? P_FLOATS : O_FLOATS, MORE_THAN_HALF = 81 * 1024 / 4;      // (of a compute unit's 160 KB)
+  __shared__ __attribute__((aligned(16))) float smem[ALONE ? MORE_THAN_HALF : USED];   // weights and pieces on their way to their lanes, then partial results
   __shared__ float part_m[AF_WAVES][16], part_l[AF_WAVES][16];
 
   const int s = blockIdx.y, h = blockIdx.x, hk = Hq == Hkv ? h : h / (Hq / Hkv);
   const int t = threadIdx.x, lane = t % DA_WAVE, wave = __builtin_amdgcn_readfirstlane(t / DA_WAVE);
   const int col = lane % 16, quad = lane / 16;
+  const int l_row = TURN ? lane / 4 : col, l_at = 4 * (TURN ? lane % 4 : quad);             // the row (of 16) and the first entry (of 16) that the lane loads
+  const uint32_t k_at = 4u * (uint32_t)(l_row * D + l_at), v_at = 4u * (uint32_t)(l_row * page + l_at);      // bytes into a piece's keys and values
   const int* bt = block_table + (size_t)s * max_blocks;
   const int lg = 31 - __builtin_clz(page), pmask = page - 1;   // (a power of two, checked on the host)
   // Asked for side by side: the sequence's rows and length, and the pages of the chunk that this wavefront starts with where no window
@@ -103,9 +141,10 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ cache, co
   const float* vbase = cache + (long long)(Hkv + hk) * page * D;
 
   float4 qf[D16];
+  bool q_placed = !TURN || last_row == i0;                              // (one row: the same piece for all lanes of a quarter, read as it is used)
   {
-    const int qi = i0 + col < T ? i0 + col : T - 1;
-    const float* qr = q + (size_t)(row0 + qi) * q_ld + h * D + quad * 4;
+    const int qi = i0 + l_row < T ? i0 + l_row : T - 1;
+    const float* qr = q + (size_t)(row0 + qi) * q_ld + h * D + (q_placed ? quad * 4 : l_at);
 #pragma unroll
     for (int g = 0; g < D16; ++g) qf[g] = *(const float4*)(qr + g * 16);
   }
@@ -116,6 +155,7 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ cache, co
 #pragma unroll
   for (int r = 0; r < 4; ++r) { m[r] = -INFINITY; l[r] = 0.f; }
   float* const ps = smem + wave * 16 * AF_PLD;
+  f32x4_t* const xs = (f32x4_t*)(smem + AF_WAVES * 16 * AF_PLD + wave * X_FLOATS);
 
   const int first_chunk = lo_min / AF_CHUNK;
   for (int ci = first_chunk + (wave + AF_WAVES - first_chunk % AF_WAVES) % AF_WAVES; ci * AF_CHUNK <= p_max; ci += AF_WAVES) {
@@ -140,17 +180,22 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ cache, co
 #pragma unroll
     for (int j = 0; j < AF_PIECES; ++j)
 #pragma unroll
-      for (int g = 0; g < D16; ++g) kf[j][g] = *(const float4*)(kp[j] + col * D + g * 16 + quad * 4);
+      for (int g = 0; g < D16; ++g) kf[j][g] = *(const float4*)((const char*)(kp[j] + g * 16) + k_at);
     if (EARLY_V) {
 #pragma unroll
       for (int j = 0; j < AF_PIECES; ++j)
 #pragma unroll
-        for (int d = 0; d < D16; ++d) vf[j][d] = *(const float4*)(vp[j] + (d * 16 + col) * page + quad * 4);
+        for (int d = 0; d < D16; ++d) vf[j][d] = *(const float4*)((const char*)(vp[j] + d * 16 * page) + v_at);
     }
     __builtin_amdgcn_sched_barrier(0);                          // (the loads stay ahead of the arithmetic)
+    if (TURN && !q_placed) {                                            // (not in front of the loop, where the keys would be asked for behind it)
+      af_turn(qf, xs, lane);
+      q_placed = true;
+    }
     floatx4 sc[AF_PIECES];
 #pragma unroll
     for (int j = 0; j < AF_PIECES; ++j) {
+      if (TURN) af_turn(kf[j], xs, lane);
       sc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int g = 0; g < D16; ++g) sc[j] = af_group(qf[g], kf[j][g], sc[j]);
@@ -193,11 +238,12 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ cache, co
 #pragma unroll
       for (int j = 0; j < AF_PIECES; ++j)
 #pragma unroll
-        for (int d = 0; d < D16; ++d) vf[j][d] = *(const float4*)(vp[j] + (d * 16 + col) * page + quad * 4);
+        for (int d = 0; d < D16; ++d) vf[j][d] = *(const float4*)((const char*)(vp[j] + d * 16 * page) + v_at);
     }
 #pragma unroll
     for (int j = 0; j < AF_PIECES; ++j) {
       const float4 w = *(const float4*)&ps[col * AF_PLD + j * 16 + quad * 4];
+      if (TURN) af_turn(vf[j], xs, lane);
       // keys past the last seen one were never written and keys in front of a window may be anybody's: zeros in their
       // place (their weights are zero, but zero times an infinity is not)
       const int k0 = c0 + j * 16 + quad * 4;
@@ -265,15 +311,17 @@ extern "C" int da_attn_f32(const float* q, int q_ld, const float* cache, const i
   // (a head and a sequence a workgroup, found without a division; a launch's second size ends at 65,535)
   for (int s0 = 0; s0 < n_seqs; s0 += 65535) {
     const int n = n_seqs - s0 < 65535 ? n_seqs - s0 : 65535;
+    const long workgroups = (long)Hq * n * da_ceil_div(max_query_len, 16);
+    const bool two = workgroups > 512 || (max_query_len <= 16 && workgroups > 256);
     const dim3 grid(Hq, n, da_ceil_div(max_query_len, 16)), block(AF_WAVES * DA_WAVE);
-#define AF_LAUNCH(X)                                                                                                                       \
-  hipLaunchKernelGGL(attn_f32_kernel<X>, grid, block, 0, (hipStream_t)stream, q, cache, block_table + (size_t)s0 * max_blocks, q_start + s0, \
+#define AF_LAUNCH(...)                                                                                                                     \
+  hipLaunchKernelGGL((attn_f32_kernel<__VA_ARGS__>), grid, block, 0, (hipStream_t)stream, q, cache, block_table + (size_t)s0 * max_blocks, q_start + s0, \
                      seq_lens + s0, q_ld, max_blocks, Hq, Hkv, page, scale, window, out, out_ld)
     switch (D / 16) {
       case 1: AF_LAUNCH(1); break;
       case 2: AF_LAUNCH(2); break;
       case 3: AF_LAUNCH(3); break;
-      case 4: AF_LAUNCH(4); break;
+      case 4: if (two) AF_LAUNCH(4); else AF_LAUNCH(4, true); break;
       case 5: AF_LAUNCH(5); break;
       case 6: AF_LAUNCH(6); break;
       case 7: AF_LAUNCH(7); break;
