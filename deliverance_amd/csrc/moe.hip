@@ -860,7 +860,7 @@ moe_mfma_kernel(const bf16_t* __restrict__ a, const int* __restrict__ row_of_slo
   if (e < 0) return;
   // the rows of a: gathered by slot for the first product (a padding slot reads row 0 and is never stored),
   // the slot's own row for the second; an expert's slots are filled from the front
-  const int filled = __popcll(__builtin_amdgcn_ballot_w64(place >= 0) & 0xffffffffull);
+  const int filled = __builtin_popcountll(__builtin_amdgcn_ballot_w64(place >= 0) & 0xffffffffull);
   const bf16_t* pa[4];
   const bf16_t* pw[2];
 #pragma unroll
