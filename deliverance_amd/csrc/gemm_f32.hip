@@ -15,6 +15,7 @@
 //  * gemm_f32_rows: few rows.  A workgroup owns 4, 8 or 16 rows and as many columns as give every compute unit one workgroup (16 at
 //    most); its wavefronts take whole chunks, from memory through their own pieces of LDS into fragments, and the chunks' sums are
 //    added through LDS.  Bound by the bytes of w.
+//  * gemm_f32_ln_rows: the same with a LayerNorm in front (da_gemm_f32_ln).
 //  * gemm_f32_rows_direct: few rows, from memory straight into fragments; where that is ahead (f32_rows_staged).
 //  * gemm_f32_tile: block tiles of 64 x 64 or 32 x 32 through two LDS buffers, slabs of 32 k, the next four slabs in flight
 //    in registers.  Bound by the matrix cores (157 TFLOP/s in 32-bit) where the tiles fill the chip several times over:
@@ -25,6 +26,7 @@
 // 768 x 50,257 39.9 -> 32.1; 8 rows, 3,072 x 768 12.0 -> 7.7; 16 rows 13.8 -> 9.6; 64 rows 14.3 -> 11.4; 32 rows, 768 x 3,072 8.7 -> 7.9.
 // Tiles: 526 x 768 x 3,072 38, 526 x 2,304 x 768 27, 526 x 50,257 x 768 392.
 #include "gemm_common.h"
+#include "norm_common.h"
 #include <da_read_arg.h>
 #include <type_traits>
 
@@ -74,11 +76,20 @@ __device__ __forceinline__ void gf_wave_order() {
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 __device__ __forceinline__ int gf_place(int row, int kk) { return row * 32 + (kk ^ (row & 15)); }
 // CAP: chunks that the partial sums in LDS have room for.
-template <int WL, int AL, int NW, int CAP>
-__global__ void __launch_bounds__(NW * 64)
-gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w, void* out, int lda, int ldw, int ldo, int M, int N, int K,
-                     int n_chunks, int cols, const void* bias, EpilogueRest er, KvScatter kv) {
-  const Epilogue ep{bias, er.bias_dtype, er.act, er.accumulate, out, DA_F32, ldo};
+//
+// LN: a's rows are normalised first (LayerNorm of the stream's rows, up to GF_LN_MAX_K columns: a set a wavefront at most, so that
+// all of a is in registers).  The sums of layernorm_row_kernel's order (norm_common.h): a piece of 256 columns is two chunks, its
+// sum over the lanes (l0 + l1) + (l2 + l3) of 16 lanes each, so the product's operands have the bits that the two kernels give.
+#define GF_LN_MAX_K 1024
+struct GfNorm {
+  const float* g;
+  const float* b;
+  float eps;
+};
+template <int WL, int AL, int NW, int CAP, bool LN>
+__device__ __forceinline__ void
+gemm_f32_rows_body(const float* __restrict__ a, const float* __restrict__ w, int lda, int ldw, int M, int N, int K, int n_chunks, int cols,
+                   const Epilogue& ep, const KvScatter& kv, const GfNorm& norm) {
   constexpr int P = WL == 1 && AL == 1 ? 4 : (WL <= 2 && AL <= 2 ? 2 : 1), S = 16 / P;    // chunks of a product; rows and columns of each
   constexpr int RA = 4 * AL, CW = 4 * WL, LA = RA / 2, LW = CW / 2;     // rows, columns; loads a chunk
   static_assert(RA <= S && CW <= S, "a chunk's rows and columns fit their part of the fragments");
@@ -99,12 +110,30 @@ gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w, v
 #pragma unroll
   for (int i = 0; i < LW; ++i) pw[i] = w + (size_t)(n0 + i * 2 + l_row < n_end ? n0 + i * 2 + l_row : n0) * ldw;
   struct Set { f32x4_t a[P][LA], w[P][LW]; };
+  f32x4_t gain[LN ? P : 1], add[LN ? P : 1];
   auto fetch = [&](Set& x, int set) {                                  // (past K: the row's first piece, dropped when it is parked)
+    if constexpr (LN) {                                                // in the order of their use
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int k = (set * P + p) * GF_CHUNK + l_kk * 4, ks = k < K ? k : 0;
+#pragma unroll
+        for (int i = 0; i < LA; ++i) x.a[p][i] = *(const f32x4_t*)(pa[i] + ks);
+      }
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int k = (set * P + p) * GF_CHUNK + l_kk * 4, ks = k < K ? k : 0;
+        gain[p] = *(const f32x4_t*)(norm.g + ks);
+        add[p] = *(const f32x4_t*)((norm.b ? norm.b : norm.g) + ks);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int k = (set * P + p) * GF_CHUNK + l_kk * 4, ks = k < K ? k : 0;
+      if constexpr (!LN) {
 #pragma unroll
-      for (int i = 0; i < LA; ++i) x.a[p][i] = *(const f32x4_t*)(pa[i] + ks);
+        for (int i = 0; i < LA; ++i) x.a[p][i] = *(const f32x4_t*)(pa[i] + ks);
+      }
 #pragma unroll
       for (int i = 0; i < LW; ++i) x.w[p][i] = *(const f32x4_t*)(pw[i] + ks);
     }
@@ -145,6 +174,58 @@ gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w, v
   const int em = r0 + t / CW, en = n0 + t % CW;
   const bool e_ok = t < RA * CW && em < M && en < n_end;
   GF_EPILOGUE_LOADS
+  if constexpr (LN) {
+    // a row's 16 sums over 16 lanes (two a chunk), of the entries and then of the squares around the mean
+    __builtin_amdgcn_sched_barrier(0);
+    __shared__ __attribute__((aligned(16))) float gf_stat[2][RA][16];
+    const bool on = set < n_sets;
+    if (t < RA * 16 && t % 16 >= 2 * P * n_sets) gf_stat[0][t / 16][t % 16] = gf_stat[1][t / 16][t % 16] = 0.f;      // chunks that no wavefront has
+    auto row_total = [&](int which, int row) {
+      const f32x4_t* q = (const f32x4_t*)gf_stat[which][row];
+      float s4[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s4[j] = (q[j][0] + q[j][1]) + (q[j][2] + q[j][3]);
+      return (s4[0] + s4[1]) + (s4[2] + s4[3]);
+    };
+    auto leave = [&](int which, int p, int i, float sum) {
+      sum = group_sum<16>(sum);
+      if (lane % 16 == 0) gf_stat[which][i * 2 + l_row][2 * (set * P + p) + l_kk / 16] = sum;
+    };
+    if (on) {
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int i = 0; i < LA; ++i) {
+          const f32x4_t& v = x.a[p][i];
+          leave(0, p, i, (set * P + p) * GF_CHUNK + l_kk * 4 < K ? (v[0] + v[1]) + (v[2] + v[3]) : 0.f);
+        }
+    }
+    lds_barrier();
+    if (on) {
+#pragma unroll
+      for (int i = 0; i < LA; ++i) {
+        const float mean = row_total(0, i * 2 + l_row) / (float)K;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          f32x4_t& v = x.a[p][i];
+          v -= mean;
+          leave(1, p, i, (set * P + p) * GF_CHUNK + l_kk * 4 < K ? norm_squares(make_float4(v[0], v[1], v[2], v[3])) : 0.f);
+        }
+      }
+    }
+    lds_barrier();
+    if (on) {
+#pragma unroll
+      for (int i = 0; i < LA; ++i) {
+        const float inv = 1.0f / sqrtf(row_total(1, i * 2 + l_row) / (float)K + norm.eps);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x.a[p][i][e] = norm_scaled(x.a[p][i][e], inv, gain[p][e], norm.b ? add[p][e] : 0.f);
+      }
+      products(x, set);
+    }
+  } else
   for (; set < n_sets; set += 2 * NW) {
     if (set + NW < n_sets) fetch(y, set + NW);
     products(x, set);
@@ -161,6 +242,21 @@ gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w, v
   float* o = (float*)ep.out + (size_t)em * ep.ldo + en;
   *o = ep.accumulate ? e_old + v : v;
   if (kv.cache) kv_column_store<float>(kv, e_col, e_slot, v);
+}
+
+template <int WL, int AL, int NW, int CAP>
+__global__ void __launch_bounds__(NW * 64)
+gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w, void* out, int lda, int ldw, int ldo, int M, int N, int K,
+                     int n_chunks, int cols, const void* bias, EpilogueRest er, KvScatter kv) {
+  const Epilogue ep{bias, er.bias_dtype, er.act, er.accumulate, out, DA_F32, ldo};
+  gemm_f32_rows_body<WL, AL, NW, CAP, false>(a, w, lda, ldw, M, N, K, n_chunks, cols, ep, kv, GfNorm{});
+}
+template <int WL, int AL, int NW>
+__global__ void __launch_bounds__(NW * 64)
+gemm_f32_ln_rows_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ g, const float* __restrict__ b, int ldw,
+                        int M, int N, int K, int cols, float eps, void* out, int ldo, const void* bias, EpilogueRest er, KvScatter kv) {
+  const Epilogue ep{bias, er.bias_dtype, er.act, er.accumulate, out, DA_F32, ldo};
+  gemm_f32_rows_body<WL, AL, NW, GF_LN_MAX_K / GF_CHUNK, true>(x, w, K, ldw, M, N, K, (K + GF_CHUNK - 1) / GF_CHUNK, cols, ep, kv, GfNorm{g, b, eps});
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -508,6 +604,57 @@ static int f32_rows_columns(int M, int N) {
 }
 // 0 where a product of few rows goes to the direct kernel, else the columns a workgroup of the staged one.
 extern "C" int da_gemm_f32_rows_choice(int M, int N, int K) { return f32_rows_staged(M, N, K) ? f32_rows_columns(M, N) : 0; }
+
+// Whether a LayerNorm and the product behind it are one kernel: up to 8 rows and GF_LN_MAX_K columns of the stream (the sizes whose norm alone
+// is layernorm_row_kernel<1, 4>) where that is ahead.  Every workgroup normalises all rows, so the rows count; a launch less is worth 1.6 us.
+// us, cold weights, the two kernels / this, 4 and 8 rows:
+//   K = 768:   N = 64 5.6 / 5.0, 5.6 / 5.7; 1,100 5.8 / 4.9, 6.1 / 6.0; 2,304 6.7 / 5.7, 6.8 / 6.7; 3,072 7.0 / 5.9, 7.1 / 6.7; 4,096 7.7 / 6.3, 7.8 / 7.3
+//   K = 1,024: N = 768 5.9 / 5.3, 6.2 / 6.3; 3,072 7.4 / 6.4, 7.6 / 7.4; 3,600 7.9 / 6.8, 8.0 / 7.9; 4,096 7.8 / 7.4, 8.0 / 8.5
+//   K = 256:   N = 500 5.3 / 4.9, 5.6 / 5.4; 3,072 6.0 / 4.1, 6.0 / 5.0;  K = 64: N = 500 4.7 / 4.8, 4.7 / 5.3; 2,000 4.7 / 4.2, 4.7 / 5.1; 3,100 5.0 / 3.9, 5.0 / 4.8
+// (1 row: 6.2 / 5.6 at K = 768, N = 2,304, 4.2 / 4.8 at K = 64, N = 500.)  More than 4,096 columns are a second round of workgroups.
+extern "C" int da_gemm_f32_ln_takes(int M, int N, int K) {
+  if (M < 1 || M > 8 || K < 1 || K > GF_LN_MAX_K || K % 4 || N < 1 || N > 4096) return 0;
+  if (M <= 4) return K >= 128 || N > 1024;
+  return K >= 128 && N > 1024 && (K <= 896 || N <= 3600);
+}
+
+template <int AL, int NW>
+static void launch_f32_ln_rows(hipStream_t s, const float* x, const float* w, const float* g, const float* b, float eps, int ldw, const Epilogue& ep,
+                               const KvScatter& kv, int M, int N, int K) {
+  const int cols = f32_rows_columns(M, N);
+#define GF_LN_GO(WL)                                                                                                                          \
+  hipLaunchKernelGGL((gemm_f32_ln_rows_kernel<WL, AL, NW>), dim3(da_ceil_div(N, cols)), dim3(NW * 64), 0, s, x, w, g, b, ldw, M, N, K, cols, eps, \
+                     ep.out, ep.ldo, ep.bias, epilogue_rest(ep), kv)
+  if (cols <= 4) GF_LN_GO(1);
+  else if (cols <= 8) GF_LN_GO(2);
+  else if (cols <= 12) GF_LN_GO(3);
+  else GF_LN_GO(4);
+#undef GF_LN_GO
+}
+// out = act(LayerNorm(x) @ w.T + bias): x's rows K apart, gain and bias of the norm 32-bit (b may be null).
+extern "C" int da_gemm_f32_ln(const float* x, const float* g, const float* b, float eps, const float* w, int ldw, const void* bias, int bias_dtype,
+                              int act, float* out, int ldo, int M, int N, int K, float* kv_cache, const int* slot_map, int q_cols, int kv_cols,
+                              int Hkv, int D, int page, void* stream) {
+  DA_REQUIRE(M >= 0 && N > 0 && K > 0 && eps > 0.f, "gemm_f32_ln: bad sizes M=%d N=%d K=%d eps=%g", M, N, K, eps);
+  DA_REQUIRE(ldw % 4 == 0 && ldw >= K && ldo >= N, "gemm_f32_ln: row lengths (ldw=%d ldo=%d)", ldw, ldo);
+  DA_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)g % 16 == 0 && (uintptr_t)b % 16 == 0,
+             "gemm_f32_ln: operands, gain and bias must be 16-byte aligned");
+  DA_REQUIRE(act >= DA_ACT_NONE && act <= DA_ACT_LAST, "gemm_f32_ln: unknown activation %d", act);
+  if (kv_cache) {
+    DA_REQUIRE(slot_map && q_cols >= 0 && kv_cols == Hkv * D && q_cols + 2 * kv_cols == N && page > 0,
+               "gemm_f32_ln: the q|k|v columns (%d + 2*%d) must add up to N=%d", q_cols, kv_cols, N);
+  }
+  if (M == 0) return 0;
+  DA_REQUIRE(da_gemm_f32_ln_takes(M, N, K), "gemm_f32_ln: %d rows, %d columns, K=%d are not taken", M, N, K);
+  const Epilogue ep{bias, bias_dtype, act, 0, out, DA_F32, ldo};
+  const KvScatter kv{kv_cache, slot_map, q_cols, kv_cols, Hkv, D, page};
+  hipStream_t s = (hipStream_t)stream;
+  const bool six = K <= 6 * GF_CHUNK;                      // (a set a wavefront)
+  if (M <= 4) { if (six) launch_f32_ln_rows<1, 6>(s, x, w, g, b, eps, ldw, ep, kv, M, N, K); else launch_f32_ln_rows<1, 8>(s, x, w, g, b, eps, ldw, ep, kv, M, N, K); }
+  else { if (six) launch_f32_ln_rows<2, 6>(s, x, w, g, b, eps, ldw, ep, kv, M, N, K); else launch_f32_ln_rows<2, 8>(s, x, w, g, b, eps, ldw, ep, kv, M, N, K); }
+  DA_CHECK_LAUNCH("gemm_f32_ln");
+  return 0;
+}
 
 // out (+)= act(a @ w.T + bias).  `form` 0: chosen by the sizes; else that kernel (tests and timing), where it takes them.
 extern "C" int da_gemm_f32(const float* a, int lda, const float* w, int ldw, const void* bias, int bias_dtype, int act, int accumulate,

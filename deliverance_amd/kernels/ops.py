@@ -81,6 +81,8 @@ _ARGTYPES = {
     "da_gemm_ref": [_VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_f32": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _VP],
     "da_gemm_f32_rows_choice": [_I, _I, _I],
+    "da_gemm_f32_ln_takes": [_I, _I, _I],
+    "da_gemm_f32_ln": [_VP, _VP, _VP, _F, _VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_bf16": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_few_rows": [_I, _I],
     "da_gemm_gated_takes": [_I, _I, _I],
@@ -1091,6 +1093,42 @@ def linear_f32(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], o
 # portion: keys go over in 16-byte pieces, values in 8-byte ones; behind a prompt of odd length 0.3 to 4 us
 # more), the write kernel after the product 3.7 to
 # 9.2 us; with places in any order the two are level at 2,048 rows and the epilogue is ahead below.
+
+
+def can_fuse_ln_f32(n_rows: int, x: torch.Tensor, norm_weight: torch.Tensor, norm_bias: Optional[torch.Tensor], w: torch.Tensor) -> bool:
+    """Whether ``linear_ln_f32`` takes this step: few rows, 32-bit weights, a width the kernel holds."""
+    return (_MODE == "tuned" and w.dtype == x.dtype == norm_weight.dtype == torch.float32 and (norm_bias is None or norm_bias.dtype == torch.float32)
+            and w.stride(0) % 4 == 0 and all(t is None or t.data_ptr() % 16 == 0 for t in (x, norm_weight, norm_bias, w))
+            and bool(_lib().da_gemm_f32_ln_takes(int(n_rows), int(w.shape[0]), int(w.shape[1]))))
+
+
+def linear_ln_f32(x: torch.Tensor, norm_weight: torch.Tensor, norm_bias: Optional[torch.Tensor], eps: float, w: torch.Tensor,
+                  bias: Optional[torch.Tensor], out: torch.Tensor, act: Optional[str] = None, kv_cache: Optional[torch.Tensor] = None,
+                  slot_map: Optional[torch.Tensor] = None, q_cols: int = 0) -> torch.Tensor:
+    """out = act(LayerNorm(x) @ w.T + bias) in 32-bit in one kernel, for what ``can_fuse_ln_f32`` takes: the bits of ``layernorm``
+    and ``linear_f32``.  With ``kv_cache`` the columns from ``q_cols`` on (k | v) also go to the cache rows ``slot_map``."""
+    _dev(x, norm_weight, norm_bias, w, bias, out, kv_cache, slot_map)
+    _rows_2d(w, "w"); _rows_2d(out, "out")
+    M, K = x.shape
+    N = w.shape[0]
+    _need(x.is_contiguous() and x.dtype == w.dtype == out.dtype == norm_weight.dtype == torch.float32 and
+          (norm_bias is None or norm_bias.dtype == torch.float32), "linear_ln_f32: everything must be float32, x contiguous")
+    _need(w.shape[1] == K and norm_weight.numel() == K and (norm_bias is None or norm_bias.numel() == K), "linear_ln_f32: widths differ")
+    _need(out.shape[0] == M and out.shape[1] == N and (bias is None or bias.numel() == N), "linear_ln_f32: out or bias do not fit")
+    if not (act in ACTIVATIONS):
+        raise KernelError(f"linear_ln_f32: unknown activation {act!r}")
+    kvp = (None, None, 0, 0, 0, 0, 0)
+    if kv_cache is not None:
+        _need(kv_cache.dim() == 5 and kv_cache.is_contiguous() and kv_cache.dtype == torch.float32,
+              "linear_ln_f32: cache slot must be contiguous float32 [pages,2,Hkv,page,D]")
+        _, _, Hkv, page, D = kv_cache.shape
+        _need(slot_map is not None and slot_map.dtype == torch.int32 and slot_map.numel() >= M, "linear_ln_f32: slot_map must be int32 [rows]")
+        _need(q_cols + 2 * Hkv * D == N, "linear_ln_f32: q|k|v columns do not add up to N")
+        kvp = (_ptr(kv_cache), _ptr(slot_map), q_cols, Hkv * D, Hkv, D, page)
+    with _timed("norm_product_f32", _product_bytes(x, w, bias, out, False) + _nbytes(norm_weight, norm_bias), 2 * M * N * K, "fp32"):
+        _check(_lib().da_gemm_f32_ln(_ptr(x), _ptr(norm_weight), _ptr(norm_bias), eps, _ptr(w), w.stride(0), _ptr(bias),
+                                     _dt(bias) if bias is not None else 0, ACTIVATIONS[act], _ptr(out), out.stride(0), M, N, K, *kvp, _stream()))
+    return out
 
 
 def linear(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,

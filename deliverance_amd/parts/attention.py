@@ -184,6 +184,13 @@ class CausalSelfAttention(Mixer):
         N = x.shape[0]
         ln = norm.fusable_params()
         rms = getattr(norm, "rms_params", lambda: None)() if ln is None else None
+        if ln is not None and self._epilogue_write() and ops.can_fuse_ln_f32(N, x, ln[0], ln[1], self.qkv_weight):
+            qkv = ctx.buf("qkv", N, self.qkv_cols, ctx.dtype)
+            slot, group = ctx.cache.kv[call.cache], ctx.group_of(call.cache)
+            ops.linear_ln_f32(x, *ln, self.qkv_weight, self.qkv_bias, qkv, kv_cache=slot if call.write else None,
+                              slot_map=ctx.slot_maps[group] if call.write else None, q_cols=self.q_cols)
+            self._attend(ctx, qkv, x if into is None else into, slot, group, call)
+            return True
         if (ln is None and rms is None) or not ops.can_fuse_ln(N, x, self.qkv_weight):
             return False
         slot = ctx.cache.kv[call.cache]

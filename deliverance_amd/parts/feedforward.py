@@ -32,11 +32,17 @@ class DenseFeedForward(FeedForward):
         """Small steps: LayerNorm, fc, bias and activation in one kernel."""
         N = x.shape[0]
         ln = norm.fusable_params()
-        if ln is None or not ops.can_fuse_ln(N, x, self.fc_weight):
+        if ln is None:
             return False
         gain, bias, eps = ln
+        in32 = ops.can_fuse_ln_f32(N, x, gain, bias, self.fc_weight)
+        if not in32 and not ops.can_fuse_ln(N, x, self.fc_weight):
+            return False
         mid = ctx.buf("ff_mid", N, self.inner, ctx.dtype)
-        ops.linear_ln(x, None, N, gain, bias, eps, self.fc_weight, self.fc_bias, mid, act=self.activation)
+        if in32:
+            ops.linear_ln_f32(x, gain, bias, eps, self.fc_weight, self.fc_bias, mid, act=self.activation)
+        else:
+            ops.linear_ln(x, None, N, gain, bias, eps, self.fc_weight, self.fc_bias, mid, act=self.activation)
         ops.linear(mid, self.proj_weight, self.proj_bias, x, accumulate=True)
         return True
 

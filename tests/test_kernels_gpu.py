@@ -306,6 +306,49 @@ def test_gemm_32bit_writes_keys_and_values(ops):
         assert torch.equal(c1, c2) and c1.abs().sum() > 0
 
 
+@pytest.mark.parametrize("K", [helpers.quick(128), 132, 640, 768, 772, 1000, 1024])
+@pytest.mark.parametrize("M,N", [helpers.quick(1, 300), (4, 192), (3, 1500), (4, 2304), (8, 2304), (5, 1056), (2, 4096), (8, 3075)])
+def test_layer_norm_and_product_32bit_in_one_kernel(ops, M, N, K):
+    """The bits of the norm's kernel and the product's, at every width of a workgroup, k that cuts a chunk and wavefronts without one; with
+    and without the norm's bias, a bias and an activation, and the cache write where N is q | k | v."""
+    helpers.skip_in_simulation_if(M * N * K > 300_000)
+    g = torch.Generator().manual_seed(N + K)
+    x = (torch.randn(M, K, generator=g) * 3 + 1).to(DEV)
+    gain, add = (torch.randn(K, generator=g) + 1).to(DEV), torch.randn(K, generator=g).to(DEV)
+    w, bias = torch.randn(N, K, generator=g).to(DEV), torch.randn(N, generator=g).to(DEV)
+    assert ops.can_fuse_ln_f32(M, x, gain, add, w)
+    D, page = 16, 16
+    heads = N // (3 * D)
+    cached = N % (3 * D) == 0
+    slots = torch.tensor([5, -1, 16, 31, 0, 33, 47, 20][:M], dtype=torch.int32, device=DEV)
+    for b, act, lb in ((bias, "gelu_new", add), (None, None, None)):
+        kv = [dict(kv_cache=torch.zeros(3, 2, heads, page, D, device=DEV), slot_map=slots, q_cols=heads * D) if cached else {} for _ in range(2)]
+        normed = ops.layernorm(x, gain, lb, 1e-5, torch.empty(M, K, device=DEV), None)
+        two = ops.linear_f32(normed, w, b, torch.full((M, N), 7.0, device=DEV), act, **kv[0])
+        one = ops.linear_ln_f32(x, gain, lb, 1e-5, w, b, torch.full((M, N), 8.0, device=DEV), act, **kv[1])
+        assert torch.equal(one, two)
+        if cached:
+            assert torch.equal(kv[0]["kv_cache"], kv[1]["kv_cache"])
+    xd = x.double()
+    c = xd - xd.mean(1, keepdim=True)
+    want = (c / torch.sqrt((c * c).mean(1, keepdim=True) + 1e-5) * gain.double()) @ w.double().t()
+    # (sqrt(K) roundings of 6e-8 of numbers of order one, K of them: far below this)
+    assert float((one.double() - want).norm() / want.norm()) < 2e-6
+
+
+def test_which_steps_32bit_norm_and_product_take(ops):
+    x = torch.zeros(9, 1028, device=DEV)
+    gain = torch.zeros(1028, device=DEV)
+    takes = lambda M, N, K: ops.can_fuse_ln_f32(M, x[:M, :K].contiguous(), gain[:K], None, torch.zeros(N, K, device=DEV))
+    assert takes(4, 1, 128) and takes(1, 1025, 4) and takes(8, 1025, 128) and takes(8, 4096, 896) and takes(8, 3600, 1024)
+    assert not takes(9, 2304, 768) and not takes(4, 4097, 768) and not takes(4, 2304, 1028) and not takes(4, 1024, 124)
+    assert not takes(5, 1024, 768) and not takes(8, 3601, 900) and not takes(5, 2000, 124)
+    w = torch.zeros(8, 256, device=DEV)
+    assert not ops.can_fuse_ln_f32(1, x[:1, :256].contiguous(), gain[1:257], None, w)          # a gain that is not aligned
+    with pytest.raises(ops.KernelError):
+        ops.linear_ln_f32(torch.zeros(9, 256, device=DEV), gain[:256], None, 1e-5, w, None, torch.empty(9, 8, device=DEV))
+
+
 @pytest.mark.simt_quick
 @pytest.mark.parametrize("extra,accumulate", [(0, False), (0, True), (12, False), (12, True)])
 def test_product_32bit_keeps_keys_and_values_of_any_call(ops, extra, accumulate):
