@@ -66,12 +66,14 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 // Included by attn_both.hip (DA_ATTN_BODIES) the kernel is a function that is told which workgroup it is.
 template <int D16, int RB, int KP, bool BT_LDS>
 #ifdef DA_ATTN_BODIES
+#define PF_Q_LATE false
 #define PF_SEQ pf_seq
 #define PF_BLOCK pf_block
 #define PF_BLOCKS pf_blocks
 __device__ __forceinline__ void
 attn_prefill_body(int pf_seq, int h, int pf_block, int pf_blocks,
 #else
+#define PF_Q_LATE true
 #define PF_SEQ (int)blockIdx.y
 #define PF_BLOCK (int)blockIdx.z
 #define PF_BLOCKS (int)gridDim.z
@@ -137,13 +139,18 @@ PF_KERNEL(
   const bool q_ok = qi < T;
   const int pq = past + qi;
   const int q_lo = (window > 0 && pq - window + 1 > 0) ? pq - window + 1 : 0;
+  // Asked for behind the first tile's keys and values: a row a lane is the slow way through a compute unit's address unit (64 cycles a load), and in
+  // front of the block table's entries everything would wait for it.  Steps, in front / behind: 355M, 3 prompts of up to 701 2,797 / 2,763 us, 1.5B, 2 x
+  // 1,024 10,408 / 10,323, 37 tokens level; not beside one-token sequences in one launch (PF_Q_LATE; 355M, 512 beside 40, 1.4 % ahead of the build before
+  // with them in front, 0.6 % with them behind), nor only where the steady state runs (355M 0.3 % for 1.2).  (A column past the portion holds the last
+  // row's query; its results are never stored.)
   bf16x8_t qf[D16];
+  auto load_q = [&]() {
+    const bf16_t* qr = q + (size_t)(row0 + (q_ok ? qi : T - 1)) * q_ld + h * D + hf * 8;
 #pragma unroll
-  for (int kd = 0; kd < D16; ++kd) {
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (q_ok) v = *(const uint4*)(q + (size_t)(row0 + qi) * q_ld + h * D + kd * 16 + hf * 8);
-    qf[kd] = __builtin_bit_cast(bf16x8_t, v);
-  }
+    for (int kd = 0; kd < D16; ++kd) qf[kd] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(qr + kd * 16));
+  };
+  if (!PF_Q_LATE) load_q();
   // the wavefront's rows span positions w_first .. w_last
   const int w_first = past + i0 + wrow;
   const int w_last_row = (i0 + wrow + 31 < T - 1) ? i0 + wrow + 31 : T - 1;
@@ -460,6 +467,7 @@ PF_KERNEL(
   // loop below, which takes any tile, does all of them.
   if (b_lo == kt0 && kt0 + 4 * PF_BK - 1 <= b_last) {
     fetch_fast(rk0, rv0, kt0);
+    if (PF_Q_LATE) load_q();
     fetch_fast(rk1, rv1, kt0 + PF_BK);
     for (; kt + 4 * PF_BK - 1 <= b_last; kt += 2 * PF_BK) {
       stash(rk0, rv0, 0);
@@ -473,6 +481,7 @@ PF_KERNEL(
     }
   } else {
     fetch(rk0, rv0, kt0);
+    if (PF_Q_LATE) load_q();
     if (kt0 + PF_BK <= b_last) fetch(rk1, rv1, kt0 + PF_BK);
   }
   for (int parity = 0; kt <= b_last; kt += PF_BK, parity ^= 1) {
@@ -493,6 +502,7 @@ PF_KERNEL(
     // round: the tiles are parked before anyone reads them and read before they are replaced.
     if (b_lo == kt0 && kt0 + KP * PF_BK - 1 <= b_last) fetch_fast(rk0, rv0, kt0);     // (a first round that is whole: no clamping)
     else fetch(rk0, rv0, kt0);
+    if (PF_Q_LATE) load_q();
     for (int kt = kt0; kt <= b_last; kt += KP * PF_BK) {
       stash(rk0, rv0, 0);
       lds_barrier();
