@@ -15,7 +15,10 @@
 //            in k-group g and zero elsewhere: the result's row 4 a + b, column 4 g + b is that key's share from these
 //            dimensions, and four neighbouring lanes add up its four shares.  (Zero times an infinite key of the
 //            same rows is no number: a chunk where one appears has its scores once more, a key a row.)  Products of
-//            bfloat16 are exact and their sums 32-bit; the scale comes after.
+//            bfloat16 are exact and their sums 32-bit; the scale comes after.  us, a key a row / this, pages of 16: head size 64, 1 sequence of 12 heads
+//            and 512 keys 5.4 / 4.5, 64 of 25 heads 35.3 / 35.1; with a bias, 640 keys, 5 of 16 heads 8.3 / 7.1, 64 of 16 31.7 / 31.4; head size 32, 64
+//            sequences of 16 heads and 512 keys 13.8 / 13.8; 80, 32 of 600 21.8 / 22.0; 128, 4 of 600 10.0 / 7.6; 256, 32 of 8 heads 32.2 / 32.5, with a
+//            bias 38.2 / 34.4; behind at 48 (64 of 600 22.7 / 23.1) and 16 (8 of 8 heads 4.1 / 4.3; 64 of 16 10.6 / 10.3).
 //   softmax: four neighbouring lanes hold the same 4 keys that follow each other.  Running maximum and sum per wavefront
 //            (the recurrence of native/src/main/resources/decode_paged_attention_f32.wgsl:31-65).
 //   values : O[d, part] += V^T[d, key] . P[key, part]; values are stored dimension-major, so the left operand is
@@ -36,6 +39,7 @@
 // of which o is multiplied with the logistic function.  The last two act once, after everything has been merged.  The
 // plain build has none of that code.
 #include "gemm_common.h"
+#include <da_anew.h>
 #include <da_read_arg.h>
 
 #define DEC_MAX_D 256
@@ -75,6 +79,10 @@ __device__ __forceinline__ float dec_inverse(float mm, float ll, bool with_sink,
     ll = ll * shrink + dec_exp(s0 - m_all);
   }
   return ll > 0.f ? shrink / ll : 0.f;
+}
+// a number that is the same in all lanes, in a scalar register
+__device__ __forceinline__ float dec_of_all(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
 }
 __device__ __forceinline__ float dec_gate(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
@@ -175,8 +183,8 @@ DEC_KERNEL(
   const int lo = SPLIT ? (lo_row > split0 ? lo_row : split0) : lo_row;
 #ifdef DEC_REL
   const float* brow = rel_bias ? rel_bias + (size_t)h * n_dist : nullptr;
-  const float slope = slopes ? slopes[h] : 0.f;
-  const float qscale = t_every > 0 ? scale * (1.0f + t_coef * logf((float)((p_row + 1) / t_every + 1))) : scale;
+  const float slope = dec_of_all(slopes ? slopes[h] : 0.f);
+  const float qscale = dec_of_all(t_every > 0 ? scale * (1.0f + t_coef * logf((float)((p_row + 1) / t_every + 1))) : scale);
 #else
   const float qscale = scale;
 #endif
@@ -192,6 +200,7 @@ DEC_KERNEL(
   for (int c0 = (lo / DA_WAVE) * DA_WAVE + wave * DA_WAVE; c0 <= p; c0 += DEC_WAVES * DA_WAVE) {
     const int first = c0 > lo ? c0 : lo;                 // valid keys of the chunk: first..last
     const int last = c0 + DA_WAVE - 1 < p ? c0 + DA_WAVE - 1 : p;
+    auto is_seen = [&](int key) { return (uint32_t)(key - first) <= (uint32_t)(last - first); };      // (one comparison: two of them become a branch)
     // the pages of the chunk's keys and value groups: those asked for at the start, or read now
     int btk, btv[2], bt_safe;
     if (c0 == c0_guess && first == c0) {                 // the same for the whole wavefront
@@ -221,12 +230,12 @@ DEC_KERNEL(
 #pragma unroll
       for (int j = 0; j < KJ; ++j) {
         const int key = c0 + ka + j0 + j;
-        const bool valid = key >= first && key <= last;
+        const bool valid = is_seen(key);
         const char* kp = kbase + (uint64_t)(uint32_t)(valid ? btk : bt_safe) * page_bytes +
-                         (uint32_t)(2 * (((valid ? key : first) & pmask) * D + (DK > 1 || kd < D ? kd : 0)));
+                         (uint32_t)(2 * (((valid ? key : first) & pmask) * D + (DK > 1 || kd < D ? kd : D - 8)));
 #pragma unroll
-        for (int k = 0; k < DK; ++k)         // (D > 16 DK: only the upper half of the steps can lie past D; there the first step is read)
-          kf[j][k] = *(const uint4*)(kp + (2 * k + 1 < DK || 32 * k + kd < D ? 64 * k : 0));
+        for (int k = 0; k < DK; ++k)         // (D > 16 DK: only the upper half of the steps can lie past D; there the row's last piece is read, in its neighbours' line)
+          kf[j][k] = *(const uint4*)(kp + (DK == 1 || 2 * k + 1 < DK || 32 * k + kd < D ? 64 * k : 2 * (D - 8 - kd)));
       }
     };
     // Zeros in place of what lanes past D read: q is zero there, but zero times an infinite key is no number.
@@ -288,32 +297,38 @@ DEC_KERNEL(
       load_k(EARLY_V ? 0 : 2);
       scores(EARLY_V ? 0 : 2);
     }
-    // this lane's 4 keys: piece r's row group `quad`, k-group col / 4; of their shares register col % 4
-    const int key0 = c0 + 16 * quad + 4 * (col / 4);
+    // What a lane works out from its number from here on is worked out here.  Held in registers across the loads, where keys, values and results
+    // fill them, it takes a compute unit's third workgroup at head sizes up to 32 (92 registers for 77; 64 sequences of 16 heads and 512 keys 14.7 us for
+    // 13.8) and spills at 64 with a bias (34.1 for 31.4) and above 128 (36.7 for 32.5).
+    const uint32_t ln = da_anew((uint32_t)lane), ln16 = ln % 16, ln_quad = ln / 16, part = ln % 4;
+    // this lane's 4 keys: piece r's row group ln_quad, k-group ln16 / 4; lane b of four neighbouring ones has their share b in register b
+    const int key0 = c0 + (int)(16 * ln_quad + ln16 / 4 * 4);
     float sv[4], e[4];
     auto finish = [&](int r) {
       sv[r] *= qscale;
 #ifdef DEC_REL
       sv[r] += brel[r];
 #endif
-      sv[r] = key0 + r >= first && key0 + r <= last ? sv[r] : -INFINITY;
+      sv[r] = is_seen(key0 + r) ? sv[r] : -INFINITY;
     };
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float s01 = col & 1 ? sc[r][1] : sc[r][0], s23 = col & 1 ? sc[r][3] : sc[r][2];
-      sv[r] = group_sum<4>(col & 2 ? s23 : s01);
+      // (every lane takes the four shares from their lanes: a lane that picked its own would do so by comparisons with each place)
+      const float s01 = dpp_move<0x00, 0xF>(sc[r][0], sc[r][0]) + dpp_move<0x55, 0xF>(sc[r][1], sc[r][1]);
+      const float s23 = dpp_move<0xAA, 0xF>(sc[r][2], sc[r][2]) + dpp_move<0xFF, 0xF>(sc[r][3], sc[r][3]);
+      sv[r] = s01 + s23;
       finish(r);
     }
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(sv[0] != sv[0] || sv[1] != sv[1] || sv[2] != sv[2] || sv[3] != sv[3]) != 0, 0)) {
-      // the chunk's scores once more, a key a row of the left operand and q in all columns: product j holds this lane's keys if j = col / 4
+      // the chunk's scores once more, a key a row of the left operand and q in all columns: product j holds this lane's keys if j = ln16 / 4
 #pragma unroll 1
       for (int j = 0; j < 4; ++j) {
-        const int key = c0 + 16 * (col / 4) + 4 * j + col % 4, seen = key >= first && key <= last ? key : first;
+        const int key = c0 + (int)(16 * (ln16 / 4) + 4 * j + part), seen = is_seen(key) ? key : first;
         const char* kp = kbase + (uint64_t)(uint32_t)bt[seen >> lg] * page_bytes + (uint32_t)(2 * (seen & pmask) * D);
         floatx4 one = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
         for (int k = 0; k < DK; ++k) {
-          const int d = 32 * k + 8 * quad;
+          const int d = 32 * k + 8 * (int)ln_quad;
           uint4 kx = make_uint4(0, 0, 0, 0), qx = kx;
           if (d < D) {
             kx = *(const uint4*)(kp + 2 * d);
@@ -321,7 +336,7 @@ DEC_KERNEL(
           }
           one = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kx), __builtin_bit_cast(bf16x8_t, qx), one, 0, 0, 0);
         }
-        if (j == col / 4) {
+        if (j == (int)(ln16 / 4)) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             sv[r] = one[r];
@@ -338,7 +353,6 @@ DEC_KERNEL(
     m = m_new;
     {
       // of four neighbouring lanes the first parks the first part of their 4 weights, the others the second, the third, zeros
-      const int part = col % 4;
       uint32_t w2[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -349,7 +363,7 @@ DEC_KERNEL(
         const uint32_t p2 = pack2_bf16(a1 - __uint_as_float(p1 << 16), b1 - __uint_as_float(p1 & 0xffff0000u));
         w2[i] = part == 0 ? p0 : (part == 1 ? p1 : (part == 2 ? p2 : 0u));
       }
-      *(uint2*)&ps[wave][part][16 * quad + 4 * (col / 4)] = make_uint2(w2[0], w2[1]);
+      *(uint2*)&ps[wave][part][16 * ln_quad + ln16 / 4 * 4] = make_uint2(w2[0], w2[1]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");   // LDS only: the value loads stay in flight
     __builtin_amdgcn_wave_barrier();
@@ -366,11 +380,11 @@ DEC_KERNEL(
         __builtin_amdgcn_sched_barrier(0);               // (not moved up among the scores: the keys' registers are free only now)
         load_v(EARLY_V ? 0 : g);
       }
-      const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, *(const uint4*)&ps[wave][col < 3 ? col : 3][32 * g + 8 * quad]);
+      const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, *(const uint4*)&ps[wave][ln16 < 3 ? ln16 : 3][32 * g + 8 * ln_quad]);
       if (cut) {
         // Rows outside first..last were never written (or belong to someone else) and may hold anything:
         // their bits are cleared.  The seen rows of the lane's group are g0 + lo8 .. g0 + hi8.
-        const int g0 = c0 + 32 * g + 8 * quad;
+        const int g0 = c0 + 32 * g + 8 * (int)ln_quad;
         const int lo8 = first - g0, hi8 = last - g0;
         uint32_t msk[4];
 #pragma unroll

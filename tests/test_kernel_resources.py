@@ -1,0 +1,69 @@
+"""What the compiled kernels hold on a compute unit: registers, scratch memory and workgroups side by side, read off what the compiler
+wrote beside each kernel of the built libraries.  A change that costs a kernel a workgroup or makes it spill shows here."""
+import re
+import struct
+
+import pytest
+
+from deliverance_amd.kernels import build
+
+msgpack = pytest.importorskip("msgpack")
+
+LDS = 160 * 1024                 # bytes of a compute unit
+LANES, REGISTERS = 64, 512       # of a wavefront; vector registers of a SIMD, four SIMDs a compute unit
+
+
+def _code_objects(blob):
+    """The gfx950 code objects of a library (each a bundle of one entry a target: offset, size, name)."""
+    magic, at = b"__CLANG_OFFLOAD_BUNDLE__", -1
+    while (at := blob.find(magic, at + 1)) >= 0:
+        n, q = struct.unpack_from("<Q", blob, at + len(magic))[0], at + len(magic) + 8
+        for _ in range(n):
+            offset, size, length = struct.unpack_from("<QQQ", blob, q)
+            if b"gfx950" in blob[q + 24:q + 24 + length]:
+                yield blob[at + offset:at + offset + size]
+            q += 24 + length
+
+
+def _notes(elf):
+    """The kernels' descriptions in an ELF file's note sections."""
+    table = struct.unpack_from("<Q", elf, 40)[0]
+    entry, n = struct.unpack_from("<HH", elf, 58)
+    for i in range(n):
+        kind, = struct.unpack_from("<I", elf, table + i * entry + 4)
+        if kind == 7:
+            offset, = struct.unpack_from("<Q", elf, table + i * entry + 24)
+            name, size, _ = struct.unpack_from("<III", elf, offset)
+            yield from msgpack.unpackb(elf[offset + 12 + (name + 3) // 4 * 4:][:size])["amdhsa.kernels"]
+
+
+def resources(unit, kernel):
+    """Template arguments -> (workgroups a compute unit, scratch bytes a lane) of the kernels of this name."""
+    try:
+        build.build(only=[unit], verbose=False)
+    except build.KernelLibraryError as e:
+        pytest.skip(str(e))
+    with open(build.unit_path(unit), "rb") as f:
+        blob = f.read()
+    found = {}
+    for elf in _code_objects(blob):
+        for k in _notes(elf):
+            m = re.match(r"_Z\d+%s((?:I(?:L[a-z]\d+E)+E)?)" % kernel, k[".name"])
+            if m:
+                waves = -(-k[".max_flat_workgroup_size"] // LANES)
+                a_simd = min(8, REGISTERS // (-(-max(1, k[".vgpr_count"]) // 8) * 8))
+                fit = min(4 * a_simd // waves, LDS // max(1, k[".group_segment_fixed_size"]))
+                found[tuple(int(x) for x in re.findall(r"L[a-z](\d+)E", m[1]))] = (fit, k[".private_segment_fixed_size"])
+    assert found, f"{kernel} is not in {unit}"
+    return found
+
+
+@pytest.mark.parametrize("unit", ["attn_decode", "attn_decode_rel"])
+def test_decode_attention_fits_side_by_side_and_does_not_spill(unit):
+    """Three workgroups of 8 wavefronts a compute unit for head sizes up to 32, two up to 64; no scratch memory up to a head size of 128, and above, where two
+    pieces of keys and all results fill the registers, no more than a few numbers a lane."""
+    found = resources(unit, unit + "_kernel")
+    assert {a[:2] for a in found} == {(1, 16), (2, 16), (1, 8), (2, 8), (4, 8), (8, 8)}
+    for (dk, waves, split), (workgroups, scratch) in found.items():
+        assert workgroups >= ({1: 3, 2: 2}.get(dk, 1) if waves == 8 else 1), (dk, waves, split)
+        assert scratch <= (60 if dk == 8 else 0), (dk, waves, split)

@@ -948,7 +948,7 @@ def test_attention_decode_with_infinite_keys_and_values(ops, D):
 
 @pytest.mark.simt_quick
 @pytest.mark.parametrize("rel", [False, True])
-@pytest.mark.parametrize("D,page,window", [(64, 16, None), (64, 8, 75), (128, 64, 75), (32, 32, None)])
+@pytest.mark.parametrize("D,page,window", [(64, 16, None), (64, 8, 75), (128, 64, 75), (32, 32, None), (48, 16, 75), (80, 8, None), (16, 16, None)])
 def test_attention_decode_scores_of_an_infinite_keys_neighbours(ops, D, page, window, rel):
     """The scores of four keys that follow each other by fours are sums over all of their dimensions with zeros in the place of the
     others' (attn_decode.hip): a key of minus infinity takes its own weight and nobody else's, in each of the four places, in whole
