@@ -20,7 +20,7 @@ attn_both_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache,
   const int pairs = n_portions * Hq, id = (int)blockIdx.x - pairs * n_blocks;
   if (id < 0) {
     const int pair = (int)blockIdx.x % pairs;
-    attn_prefill_body<4, 4, 2, BT_LDS>(pair / Hq, pair % Hq, (int)blockIdx.x / pairs, n_blocks, q, cache, block_table, q_start, seq_lens, q_ld,
+    attn_prefill_body<4, 4, 2, BT_LDS, false>(pair / Hq, pair % Hq, (int)blockIdx.x / pairs, n_blocks, q, cache, block_table, q_start, seq_lens, q_ld,
                                        max_blocks, Hq, Hkv, n_decode, page, scale, window, out, out_ld);
     return;
   }

@@ -64,16 +64,15 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 // for the workgroup's keys fit its LDS copy (a table entry read from memory in front of a tile's loads
 // makes them wait for it, and for every load still in flight)
 // Included by attn_both.hip (DA_ATTN_BODIES) the kernel is a function that is told which workgroup it is.
-template <int D16, int RB, int KP, bool BT_LDS>
+// Q_LATE: the rows of q are asked for behind the first tile's keys and values (pf_q_late below says where)
+template <int D16, int RB, int KP, bool BT_LDS, bool Q_LATE>
 #ifdef DA_ATTN_BODIES
-#define PF_Q_LATE false
 #define PF_SEQ pf_seq
 #define PF_BLOCK pf_block
 #define PF_BLOCKS pf_blocks
 __device__ __forceinline__ void
 attn_prefill_body(int pf_seq, int h, int pf_block, int pf_blocks,
 #else
-#define PF_Q_LATE true
 #define PF_SEQ (int)blockIdx.y
 #define PF_BLOCK (int)blockIdx.z
 #define PF_BLOCKS (int)gridDim.z
@@ -139,18 +138,21 @@ PF_KERNEL(
   const bool q_ok = qi < T;
   const int pq = past + qi;
   const int q_lo = (window > 0 && pq - window + 1 > 0) ? pq - window + 1 : 0;
-  // Asked for behind the first tile's keys and values: a row a lane is the slow way through a compute unit's address unit (64 cycles a load), and in
-  // front of the block table's entries everything would wait for it.  Steps, in front / behind: 355M, 3 prompts of up to 701 2,797 / 2,763 us, 1.5B, 2 x
-  // 1,024 10,408 / 10,323, 37 tokens level; not beside one-token sequences in one launch (PF_Q_LATE; 355M, 512 beside 40, 1.4 % ahead of the build before
-  // with them in front, 0.6 % with them behind), nor only where the steady state runs (355M 0.3 % for 1.2).  (A column past the portion holds the last
-  // row's query; its results are never stored.)
+  static_assert(KP == 1 || !Q_LATE, "the forms with phases ask for q at once");
   bf16x8_t qf[D16];
-  auto load_q = [&]() {
+  if (!Q_LATE) {
+#pragma unroll
+    for (int kd = 0; kd < D16; ++kd) {
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (q_ok) v = *(const uint4*)(q + (size_t)(row0 + qi) * q_ld + h * D + kd * 16 + hf * 8);
+      qf[kd] = __builtin_bit_cast(bf16x8_t, v);
+    }
+  }
+  auto load_q = [&]() {                         // (a column past the portion holds the last row's query; its results are never stored)
     const bf16_t* qr = q + (size_t)(row0 + (q_ok ? qi : T - 1)) * q_ld + h * D + hf * 8;
 #pragma unroll
     for (int kd = 0; kd < D16; ++kd) qf[kd] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(qr + kd * 16));
   };
-  if (!PF_Q_LATE) load_q();
   // the wavefront's rows span positions w_first .. w_last
   const int w_first = past + i0 + wrow;
   const int w_last_row = (i0 + wrow + 31 < T - 1) ? i0 + wrow + 31 : T - 1;
@@ -467,7 +469,7 @@ PF_KERNEL(
   // loop below, which takes any tile, does all of them.
   if (b_lo == kt0 && kt0 + 4 * PF_BK - 1 <= b_last) {
     fetch_fast(rk0, rv0, kt0);
-    if (PF_Q_LATE) load_q();
+    if (Q_LATE) load_q();
     fetch_fast(rk1, rv1, kt0 + PF_BK);
     for (; kt + 4 * PF_BK - 1 <= b_last; kt += 2 * PF_BK) {
       stash(rk0, rv0, 0);
@@ -481,7 +483,7 @@ PF_KERNEL(
     }
   } else {
     fetch(rk0, rv0, kt0);
-    if (PF_Q_LATE) load_q();
+    if (Q_LATE) load_q();
     if (kt0 + PF_BK <= b_last) fetch(rk1, rv1, kt0 + PF_BK);
   }
   for (int parity = 0; kt <= b_last; kt += PF_BK, parity ^= 1) {
@@ -502,7 +504,6 @@ PF_KERNEL(
     // round: the tiles are parked before anyone reads them and read before they are replaced.
     if (b_lo == kt0 && kt0 + KP * PF_BK - 1 <= b_last) fetch_fast(rk0, rv0, kt0);     // (a first round that is whole: no clamping)
     else fetch(rk0, rv0, kt0);
-    if (PF_Q_LATE) load_q();
     for (int kt = kt0; kt <= b_last; kt += KP * PF_BK) {
       stash(rk0, rv0, 0);
       lds_barrier();
@@ -562,6 +563,26 @@ PF_KERNEL(
 }
 
 #ifndef DA_ATTN_BODIES
+// Whether q is asked for behind the first tile's keys and values: a row a lane is the slow way through a compute unit's address unit (64 cycles a load), and
+// in front of the block table's entries everything waits for it.  But its registers are then held beside the tiles': at head sizes of 48 and 64 the form
+// without phases loses the third workgroup that its LDS has room for, with a bias at 80 the second, and head sizes above 200 spill.  us, in front / behind, head
+// size 64 without phases, prompts of 1,024: 2 x 25 heads (400 workgroups) 24.8 / 23.5, 5 x 16 (640) 26.4 / 24.9, 6 x 16 (768) 28.5 / 30.3, 8 x 12 (768)
+// 28.2 / 30.9, 8 x 25 (1,600) 55.0 / 60.1; 16 x 512, 12 heads (768) 19.1 / 20.9; few long ones, whose first workgroups walk alone at the end: 6,000 x 16 (752) 124 / 110,
+// 8,192 x 12 (768) 161 / 149, but 8,192 x 25 (1,600) 311 / 323.  With a bias 8 x 1,024 x 16 at 64 43.3 / 41.4, at 112 94.2 / 88.4, at 128 95.4 / 89.1, at 80
+// 53.4 / 67.5, at 96 level.  Forms with phases: 1,024 x 12 17.2 / 17.8, 4 x 64 rows after 900 keys 15.8 / 17.6, 8 x 16 after 1,000 20.9 / 21.7, head size 48
+// 2 x 1,024 x 16 16.8 / 18.9.  Other head sizes level or behind: 160 37.6 / 38.7, 240 57.3 / 62.4, 256 65.4 / 76.8.
+#ifdef PF_REL
+static constexpr bool pf_q_late(int D) { return D == 64 || D == 112 || D == 128; }
+#define PF_LAUNCH_41(N) LAUNCH3(N, 4, 1, pf_q_late(16 * N))
+#else
+static bool pf_q_late(int D, long workgroups, int max_query_len) { return D == 64 && workgroups <= (max_query_len >= 4096 ? 800 : 640); }
+#define PF_LAUNCH_41(N)                                                        \
+  do {                                                                         \
+    if (N == 4 && pf_q_late(16 * N, per128, max_query_len)) LAUNCH3(N, 4, 1, (N == 4)); \
+    else LAUNCH3(N, 4, 1, false);                                              \
+  } while (0)
+#endif
+
 #ifdef PF_REL
 extern "C" int da_attn_prefill_rel_max_dist() { return PF_REL_MAX_DIST; }
 
@@ -632,30 +653,30 @@ extern "C" int da_attn_prefill(const void* q, int q_ld, const void* cache, const
              "attn_prefill: form %d with a head size of %d (41 for any; 22 up to 128; 42 and 14 up to 64)", chosen, D);
   // every key a workgroup can see lies within max_blocks pages
   const bool bt_lds = max_blocks <= (chosen == 41 ? PF_BT_MAX : PF_BT_MAX_PHASED);
-#define LAUNCH2(N, RB, KP, L)                                                                                  \
-  hipLaunchKernelGGL((PF_KERNEL<N, RB, KP, L>), dim3(Hq, n_here, da_ceil_div(max_query_len, 32 * RB)), \
+#define LAUNCH2(N, RB, KP, L, Q)                                                                               \
+  hipLaunchKernelGGL((PF_KERNEL<N, RB, KP, L, Q>), dim3(Hq, n_here, da_ceil_div(max_query_len, 32 * RB)), \
                      dim3(RB * KP * DA_WAVE), 0, st, (const bf16_t*)q, (const bf16_t*)cache, block_table, q_start, seq_lens, \
                      q_ld, max_blocks, Hq, Hkv, s0, page, scale, window, (bf16_t*)out, out_ld PF_REL_ARGS)
-#define LAUNCH3(N, RB, KP)                \
-  do {                                    \
-    if (bt_lds) LAUNCH2(N, RB, KP, true); \
-    else LAUNCH2(N, RB, KP, false);       \
+#define LAUNCH3(N, RB, KP, Q)                \
+  do {                                       \
+    if (bt_lds) LAUNCH2(N, RB, KP, true, Q); \
+    else LAUNCH2(N, RB, KP, false, Q);       \
   } while (0)
-#define LAUNCH_SMALL(N)                     \
-  case N:                                   \
-    if (chosen == 14) LAUNCH3(N, 1, 4);     \
-    else if (chosen == 22) LAUNCH3(N, 2, 2); \
-    else if (chosen == 42) LAUNCH3(N, 4, 2); \
-    else LAUNCH3(N, 4, 1);                  \
+#define LAUNCH_SMALL(N)                            \
+  case N:                                          \
+    if (chosen == 14) LAUNCH3(N, 1, 4, false);     \
+    else if (chosen == 22) LAUNCH3(N, 2, 2, false); \
+    else if (chosen == 42) LAUNCH3(N, 4, 2, false); \
+    else PF_LAUNCH_41(N);                          \
     break;
-#define LAUNCH_MID(N)                       \
-  case N:                                   \
-    if (chosen == 22) LAUNCH3(N, 2, 2);     \
-    else LAUNCH3(N, 4, 1);                  \
+#define LAUNCH_MID(N)                              \
+  case N:                                          \
+    if (chosen == 22) LAUNCH3(N, 2, 2, false);     \
+    else PF_LAUNCH_41(N);                          \
     break;
-#define LAUNCH(N)                           \
-  case N:                                   \
-    LAUNCH3(N, 4, 1);                       \
+#define LAUNCH(N)                                  \
+  case N:                                          \
+    PF_LAUNCH_41(N);                               \
     break;
   // (a head, a sequence and a row block a workgroup, found without a division; a launch's second size ends at 65,535)
   for (int s0 = seq0; s0 < seq0 + n_seqs; s0 += 65535) {
@@ -670,6 +691,7 @@ extern "C" int da_attn_prefill(const void* q, int q_ld, const void* cache, const
 #undef LAUNCH
 #undef LAUNCH_MID
 #undef LAUNCH_SMALL
+#undef PF_LAUNCH_41
 #undef LAUNCH3
 #undef LAUNCH2
   DA_CHECK_LAUNCH("attn_prefill");

@@ -67,3 +67,18 @@ def test_decode_attention_fits_side_by_side_and_does_not_spill(unit):
     for (dk, waves, split), (workgroups, scratch) in found.items():
         assert workgroups >= ({1: 3, 2: 2}.get(dk, 1) if waves == 8 else 1), (dk, waves, split)
         assert scratch <= (60 if dk == 8 else 0), (dk, waves, split)
+
+
+def test_prefill_attention_fits_side_by_side_and_does_not_spill():
+    """The form for long steps (4 row blocks, no phases): three workgroups a compute unit at head sizes of 48 and 64 where q is asked for first, two with a
+    bias at 80; head sizes of 240 and 256 spill what their results leave no room for and no more."""
+    found = resources("attn_prefill", "attn_prefill_kernel")
+    late = {a[:4] for a in found if a[4]}
+    assert late == {(4, 4, 1, 0), (4, 4, 1, 1)}
+    for (d16, blocks, phases, table, q_late), (workgroups, scratch) in found.items():
+        if (blocks, phases) == (4, 1):
+            assert workgroups >= (3 if d16 in (3, 4) and table and not q_late else 2 if d16 <= 4 else 1), (d16, table, q_late)
+            assert scratch <= {15: 44, 16: 208}.get(d16, 0), (d16, table, q_late)
+    for (d16, blocks, phases, table, q_late), (workgroups, scratch) in resources("attn_prefill_rel", "attn_prefill_rel_kernel").items():
+        if (blocks, phases) == (4, 1):
+            assert workgroups >= (2 if d16 <= 5 else 1) and scratch == 0, (d16, table, q_late)

@@ -1528,6 +1528,30 @@ def test_attention_of_more_sequences_than_a_launch_has_rows(ops, form):
     assert bool((out != 0).any(dim=1).all())
 
 
+@pytest.mark.parametrize("window", [None, 100])
+def test_prefill_attention_has_the_same_bits_wherever_q_is_asked_for(ops, window):
+    """Head size 64 without phases: a launch of more than 640 workgroups asks for q first, its halves behind the first tile (attn_prefill.hip); portions
+    that end inside a row block, tiles that a window or the length cuts, a sequence with no rows."""
+    helpers.skip_in_simulation_if(True)
+    g = torch.Generator().manual_seed(5)
+    n, H, page = 24, 16, 16
+    new = [0 if i == 7 else 130 + 9 * i for i in range(n)]
+    lens = [t + 13 * (i % 5) for i, t in enumerate(new)]
+    pages = [-(-max(1, l) // page) for l in lens]
+    bt = torch.zeros(n, max(pages), dtype=torch.int32)
+    for i, p in enumerate(pages):
+        bt[i, :p] = torch.arange(sum(pages[:i]), sum(pages[:i + 1]))
+    cache = bf(torch.randn(sum(pages), 2, H, page, 64, generator=g)).to(DEV)
+    at = [sum(new[:i]) for i in range(n + 1)]
+    q = bf(torch.randn(at[-1], H * 64, generator=g)).to(DEV)
+    bt, starts, sl = bt.to(DEV), torch.tensor(at, dtype=torch.int32, device=DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+    run = lambda s0, m, out: ops.attention_prefill(q, cache, bt, starts, sl, s0, m, max(new), H, 0.125, window, out, form=41)
+    assert H * n * -(-max(new) // 128) > 640 >= H * (n // 2) * -(-max(new) // 128)
+    whole = run(0, n, torch.zeros(at[-1], H * 64, dtype=torch.bfloat16, device=DEV))
+    halves = run(n // 2, n // 2, run(0, n // 2, torch.zeros_like(whole)))
+    assert torch.equal(whole, halves) and bool((whole != 0).any(dim=1).all())
+
+
 @pytest.mark.parametrize("K,F", [helpers.quick(72, 24), (128, 40), (136, 20), (1024, 344), (1376, 72), (1544, 36)])
 @pytest.mark.parametrize("gated", [True, False])
 def test_grouped_products_of_experts_with_few_rows(ops, K, F, gated):
