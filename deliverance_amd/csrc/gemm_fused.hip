@@ -7,10 +7,11 @@
 //   out[m, n] = act( sum_k a[m, k] * w[n, k] + bias[n] )
 //   columns n >= kv.q_cols of a q|k|v projection are also stored to the cache row kv.slot_map[m]
 //
-// Every block owns 16 output columns and all M <= 16*MT rows, and computes the statistics of
+// Every workgroup owns a few output columns and all rows, and computes the statistics of
 // all rows itself (M * K floats from L2: cheap while M is small; the host uses the unfused
-// kernels for larger steps).  Statistics as in rowwise.hip: mean, then the centred sum of
-// squares, one wavefront per row, the row held in registers.
+// kernels for larger steps): mean, then the centred sum of squares.  Three kernels: gemm_ln_quads (a wavefront
+// holds a part of every row, the parts' statistics are joined), gemm_ln_rows (a wavefront a row or two, held in registers) and
+// gemm_ln_skinny (any of up to 32 rows, parameters of unlike dtypes).
 // Formulas: core/src/main/java/io/teknek/deliverance/generator/LayerNorm.java:127-150,
 // CausalSelfAttention.java:266-291,315-336, MLPBlock.java:250-292.
 #include "gemm_common.h"
@@ -194,10 +195,7 @@ struct LnRest {
 // normalises: nothing passes through LDS but a wavefront's mean and squares of each row.  Wavefront v of NW has the steps v and, SW of them, v + NW of 128
 // elements of k.  A row's statistics join its wavefronts' means and squares around them (M2 = sum of M2_v + n_v (mean_v - mean)^2).
 // Bound by what a wavefront computes for each row (so as few wavefronts as hold k in two steps each: K = 768, 3,072 columns, one row 3.5 us with 6
-// of them, 2.9 with 3) and by the bytes of w.  A workgroup owns `cols` columns, 4 * NG at most: as many as give every compute unit one workgroup, or
-// two.  us, cold weights, one behind the other, the kernel below with a row a wavefront -> this:
-//   1 row  K = 768, N = 2,304 3.2 -> 2.8, 3,072 3.6 -> 2.9; K = 1,024, N = 3,072 3.9 -> 3.3; K = 1,600, N = 4,800 6.7 -> 5.7, 6,400 7.4 -> 6.8
-//   8 rows K = 768, N = 2,304 3.9 -> 3.7, 3,072 4.1 -> 3.7; K = 1,024, N = 3,072 4.6 -> 4.1; K = 1,600, N = 4,800 8.5 -> 7.0, 6,400 9.3 -> 8.4
+// of them, 2.9 with 3) and by the bytes of w.  A workgroup owns `cols` columns, 4 * NG at most.  Beside gemm_ln_rows below: ln_quads_takes.
 // (w alone, read and dropped: 2.5 at K = 768, 4.5 to 5 and 5.2 at 1,600.)
 // ---------------------------------------------------------------------------------------------
 template <int MG, int NG, int NW, int SW, bool PBF16>
@@ -266,7 +264,6 @@ gemm_ln_quads_kernel(const float* __restrict__ x, const int* __restrict__ rows, 
 
   // ---- statistics: a wavefront's own mean and squares around it, joined in the order of the wavefronts
   auto count = [&](int v) {                            // elements of a row that wavefront v holds
-
     int n = K - v * 128;
     n = n < 0 ? 0 : (n < 128 ? n : 128);
 #pragma unroll
@@ -364,7 +361,6 @@ gemm_ln_quads_kernel(const float* __restrict__ x, const int* __restrict__ rows, 
       if (lane % 4 == 0) red[wave][4 * i + r4][j * 4 + lane / 16] = v;
     }
   lds_barrier();
-  
   if (e_ok) {
     float v = red[0][em][ec];
 #pragma unroll
@@ -376,13 +372,16 @@ gemm_ln_quads_kernel(const float* __restrict__ x, const int* __restrict__ rows, 
 }
 
 // ---------------------------------------------------------------------------------------------
-// 9 to 16 rows, K <= 2048, parameters of one dtype: every load in whole cache lines.
+// Up to 8 rows and K = 1,536, up to 16 and 1,024 (and what ln_quads_takes leaves), parameters of one dtype: every load in whole cache lines.
 // Wavefront v of 8 reads rows v and v + 8 whole (RV float4 a lane), with the gain and bias at the
 // same places, computes their statistics, and writes the normalised rows as bfloat16 into LDS,
 // zeros past K.  The steps of w (64 elements of k, 8 rows x 128 bytes a load; wavefront v takes the
 // steps v, v + 8, ...) are asked for before anything else is computed and parked in the wavefront's
 // own piece of LDS; the fragments of both operands are read from LDS.  Steps past K read step 0 and
 // meet zeros.  The sum over k runs in the order of the steps, whatever M is.
+// TWO_ROWS false: M <= 8, a wavefront has one row and LDS holds 8 (the fragment's rows 8..15 read
+// rows 0..7 again and are never stored): half the LDS, so that with a wide K two workgroups still
+// share a compute unit and N / 16 workgroups run side by side.
 // ---------------------------------------------------------------------------------------------
 #define FL_LD (64 + 8)       // padded row of a parked step of w, elements
 // A workgroup owns `cols` columns, 16 * CT at most.  16 of them leave some compute units with more workgroups than others
@@ -391,7 +390,7 @@ gemm_ln_quads_kernel(const float* __restrict__ x, const int* __restrict__ rows, 
 // what the kernel takes: rows of w, the rows of x, and gain and bias once a wavefront that has a row.
 // The arguments that the loads need are the first 14 words (build.py: KERNARG_PRELOAD; M and cols, 16 and 32 at most, share one);
 // what the epilogue needs is asked for behind the operands, with the place in the cache of the thread's column.
-template <int RV, bool PBF16, int CT>
+template <int RV, bool PBF16, bool TWO_ROWS, int CT>
 __global__ void __launch_bounds__(512)
 gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, const void* __restrict__ gain, const void* __restrict__ shift,
                     const bf16_t* __restrict__ w, int ldw, int N, int K, int rows_cols, LnRest lr_, Epilogue ep, KvScatter kv) {
@@ -399,7 +398,7 @@ gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, c
   const LnPrologue ln{x, rows, gain, 0, shift, 0, lr_.eps, lr_.center, lr_.gain_offset};
   constexpr int NW = 8, KMAX = RV * 256, ALD = KMAX + 8;      // ALD: padded row of a in LDS, elements
   constexpr int SW = (RV * 4 + NW - 1) / NW;                   // steps a wavefront
-  constexpr int RPW = 2, AR = RPW * NW;                         // rows a wavefront normalises; rows in LDS
+  constexpr int RPW = TWO_ROWS ? 2 : 1, AR = RPW * NW;         // rows a wavefront normalises; rows in LDS
   __shared__ __attribute__((aligned(16))) bf16_t a_lds[AR][ALD];
   constexpr int COLS = CT * 16, WL = COLS / 8;                 // columns at most; loads of 8 rows that cover w's
   // The wavefronts' sums lie behind the parked steps, where two workgroups still share a compute unit; else they take their place once all
@@ -444,7 +443,7 @@ gemm_ln_rows_kernel(const float* __restrict__ x, const int* __restrict__ rows, c
         bq[i] = *(const uint4*)((const float*)(ln.b ? ln.b : ln.g) + cs);
       }
     }
-    if (row0 + NW < M) load_row(sv[RPW - 1], row0 + NW);
+    if (TWO_ROWS && row0 + NW < M) load_row(sv[RPW - 1], row0 + NW);
   }
   uint4 wv[SW][WL];
 #pragma unroll
@@ -575,6 +574,40 @@ static void launch_fused(int mt, dim3 grid, hipStream_t s, const LnPrologue& ln,
   else hipLaunchKernelGGL((gemm_ln_skinny_kernel<2, NW, UN>), grid, dim3(NW * 64), 0, s, ln, W, ldw, ep, kv, M, N, K);
 }
 
+// Up to 8 rows: whether they go to gemm_ln_quads, else to gemm_ln_rows.  By the rows, K and the parameters' dtype alone, so that a column has the same bits
+// among fewer columns.  us, cold weights, recorded one behind the other, gemm_ln_rows / gemm_ln_quads, parameters in bfloat16:
+//   1, 4 rows  K =   256, N = 2,304 2.6 / 2.7, 2.6 / 2.7; 6,144 3.2 / 3.0, 3.3 / 3.1
+//              K =   768, N = 2,304 3.4 / 3.2, 3.6 / 3.3; 3,072 3.6 / 3.3, 3.7 / 3.4; 8,320 5.1 / 4.8, 5.5 / 4.9; 12,800 5.8 / 5.8, 5.7 / 5.7
+//              K = 1,280, N = 4,096 4.8 / 4.9, 4.8 / 5.0; 4,800 5.2 / 5.0, 5.3 / 5.1 (six wavefronts hold up to 1,536; with 32-bit parameters 2 to 9 % behind up
+//              to 8,192 columns)
+//              K = 1,600, N = 4,800 6.3 / 5.6, 6.6 / 5.6; 6,400 7.3 / 6.9, 7.5 / 6.8; 8,320 9.2 / 7.9, 9.6 / 7.9; 12,800 12.1 / 11.2, 13.1 / 11.0
+//   5, 8 rows  every workgroup normalises all rows, here a lane 8 rows' pieces, there a wavefront a row:
+//              K =   768, N = 2,304 3.9 / 4.0, 4.1 / 4.1; 8,192 5.6 / 6.9, 5.8 / 6.9; K = 1,536, N = 4,096 5.7 / 6.4, 5.9 / 6.3; 10,240 10.2 / 12.7, 10.9 / 12.8
+//              K = 1,600, N = 2,304 - 3 %, 4,096 + 7 %, 4,800 7.4 / 7.2, 7.8 / 7.2; K = 2,048, N = 2,048 6.5 / 5.7, 6.8 / 5.8; 6,144 9.4 / 9.4, 9.9 / 9.3
+static bool ln_quads_takes(int M, int K, int params) {
+  if (M > 4) return M <= 8 && K > 1536;
+  return K > 256 && (params == DA_BF16 || K <= 1024 || K > 1280);
+}
+// Its columns a workgroup, in groups of 4: every compute unit a workgroup up to 8,192 columns, two up to 16,384 as long as they fit side by side; 16 for a
+// vocabulary.  With K above 1,024 registers let two workgroups of 28 columns run side by side, with 32-bit parameters of 20: wider ones would run one behind the other,
+// and as many as give every compute unit three are ahead.  us, 1 and 4 rows, two a unit / three:
+//   bfloat16   N = 14,400, K = 1,600 13.3 / 11.9, 13.1 / 11.7; N = 16,384, K = 1,536 12.4 / 11.8, 12.5 / 11.5; K = 2,048 15.2 / 14.3, 15.1 / 14.1
+//              (gemm_ln_rows at N = 16,384: K = 1,032 9.5, where this is 10.4, 1,536 11.4, 1,600 13.3, 2,048 14.7; 4 rows 10.0, 11.7, 14.5, 16.7)
+//   32-bit     N = 10,400, K = 1,600 10.5 / 10.1, 10.6 / 10.1; N = 12,800, K = 1,536 10.9 / 10.5, 11.1 / 10.3; K = 2,048 12.5 / 12.2, 12.6 / 12.2; N = 14,336,
+//              K = 1,600 12.7 / 11.6, 12.7 / 11.8; beyond three of 20 columns 32 or 16: N = 16,384, K = 1,536 12.5 / 13.8, 12.6 / 14.0, K = 2,048 15.0 / 14.0, 15.1 / 13.8
+static int ln_quads_columns(int M, int N, int K, int params) {
+  if (N > 64 * 256) return FZ_COLS;
+  const int most = params == DA_BF16 ? 28 : 20, two = da_ceil_div(N, 512), three = da_ceil_div(N, 768);
+  int share = N <= 32 * 256 ? da_ceil_div(N, 256) : two;
+  if (N > 32 * 256 && K > 1024 && M <= 4 && two > most) share = three <= most ? three : (K <= 1536 ? 32 : 16);
+  return share <= 16 ? da_ceil_div(share, 4) * 4 : share;
+}
+
+// The columns a workgroup of gemm_ln_quads, or 0 where the rows go to another kernel.
+extern "C" int da_gemm_bf16_ln_choice(int M, int N, int K, int params) {
+  return M > 0 && K <= 2048 && ln_quads_takes(M, K, params) ? ln_quads_columns(M, N, K, params) : 0;
+}
+
 static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_dtype, const void* b,
                           int b_dtype, float eps, float center, float gain_offset, const void* w, int ldw,
                           const void* bias, int bias_dtype, int act, void* out, int out_dtype, int ldo, int M, int N,
@@ -597,17 +630,16 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
   dim3 grid(da_ceil_div(N, FZ_COLS));
   const int mt = da_ceil_div(M, 16);
   hipStream_t s = (hipStream_t)stream;
-  // These kernels take one row tile, K up to 2048, and parameters of one dtype.
-  // Columns a workgroup, up to 8 rows: every compute unit a workgroup up to 8,192 columns, two up to 16,384 (32 columns at most, and 16
-  // for a vocabulary), whole groups of 4 where that is no matter.  9 to 16 rows: 16 up to 4,096 columns and for a vocabulary; up to 8,192 as many as
-  // give every compute unit one workgroup; up to 16,384 as many as give every one two, both only up to K = 1,024 (LDS; no step sends wider
-  // ones here).  16 columns a workgroup -> this, 16 rows, K = 768, us: N = 8,320 (17, two a unit) 10.0 -> 8.6; N = 12,800 (25) 12.2 -> 9.2.
-  const int units = N <= 32 * 256 ? 256 : 512;
-  const bool wide = N > 16 * 256 && N <= 64 * 256 && K <= 1024;
-  const int share = N <= 64 * 256 ? da_ceil_div(N, units) : FZ_COLS;
-  const int cols = M <= 8 ? (share <= 16 ? da_ceil_div(share, 4) * 4 : share) : (wide ? share : FZ_COLS);
+  // Columns a workgroup of gemm_ln_rows: 16 up to 4,096 columns and for a vocabulary; up to 8,192 as many as give every compute unit one
+  // workgroup; up to 16,384 as many as give every one two.  16 columns -> this, us:
+  //   16 rows, K =   768, N = 8,320 (17, two a unit) 10.0 -> 8.6; N = 12,800 (25) 12.2 -> 9.2
+  //    8 rows, K = 1,536, N = 8,200 (17) 10.4 -> 10.0; N = 12,800 14.3 -> 11.9; N = 16,384 (32) 15.0 -> 13.4
+  const bool wide = N > 16 * 256 && N <= 64 * 256;
   const int pdt = g_dtype;
   const bool same = (!b || b_dtype == pdt) && (!bias || bias_dtype == pdt) && (pdt == DA_BF16 || pdt == DA_F32);
+  const bool quads = same && ln_quads_takes(M, K, pdt);
+  const bool in_rows = same && !quads && (M <= 8 ? K <= 1536 : M <= 16 && K <= 1024);
+  const int cols = quads ? ln_quads_columns(M, N, K, pdt) : (wide ? da_ceil_div(N, N <= 32 * 256 ? 256 : 512) : FZ_COLS);
 #define LAUNCH_LN(KERNEL, THREADS)                                                                                 \
   hipLaunchKernelGGL(KERNEL, dim3(da_ceil_div(N, cols)), dim3(THREADS), 0, s, x, rows, g, b, (const bf16_t*)w, ldw, N, K, M | cols << 8, LnRest{eps, center, gain_offset}, ep, kv)
 #define LAUNCH_Q(MG, NG, NW, SW)                                                                                   \
@@ -617,14 +649,15 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
   } while (0)
 #define LAUNCH_Q_K(MG, NG)                                                                                         \
   do {                                                                                                            \
-    if (K <= 512) LAUNCH_Q(MG, NG, 4, 1);                                                                          \
-    else if (K <= 1024) LAUNCH_Q(MG, NG, 4, 2);                                                                    \
-    else if (K <= 1536) LAUNCH_Q(MG, NG, 6, 2);                                                                    \
+    if (MG == 1 && K <= 512) LAUNCH_Q(1, NG, 4, 1);                                                                \
+    else if (MG == 1 && K <= 1024) LAUNCH_Q(1, NG, 4, 2);                                                          \
+    else if (MG == 1 && K <= 1536) LAUNCH_Q(1, NG, 6, 2);                                                          \
     else LAUNCH_Q(MG, NG, 8, 2);                                                                                   \
   } while (0)
+  // (a width more than needed, 4 more columns' loads, takes 1 to 5 % of the launch)
 #define LAUNCH_Q_N(MG)                                                                                             \
   do {                                                                                                            \
-    switch ((cols + 3) / 4) {                                                                                     \
+    switch (da_ceil_div(cols, 4)) {                                                                               \
       case 1: LAUNCH_Q_K(MG, 1); break;                                                                            \
       case 2: LAUNCH_Q_K(MG, 2); break;                                                                            \
       case 3: LAUNCH_Q_K(MG, 3); break;                                                                            \
@@ -635,25 +668,30 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
       default: LAUNCH_Q_K(MG, 8); break;                                                                           \
     }                                                                                                             \
   } while (0)
-#define LAUNCH_LDS(RV)                                                                                            \
+#define LAUNCH_R_P(RV, TWO, CT)                                                                                    \
   do {                                                                                                            \
-    constexpr int CT = RV > 4 ? 1 : 2;                                                                            \
-    if (pdt == DA_BF16 && wide) LAUNCH_LN((gemm_ln_rows_kernel<RV, true, CT>), 512);                               \
-    else if (pdt == DA_BF16) LAUNCH_LN((gemm_ln_rows_kernel<RV, true, 1>), 512);                                   \
-    else if (wide) LAUNCH_LN((gemm_ln_rows_kernel<RV, false, CT>), 512);                                           \
-    else LAUNCH_LN((gemm_ln_rows_kernel<RV, false, 1>), 512);                                                      \
+    if (pdt == DA_BF16) LAUNCH_LN((gemm_ln_rows_kernel<RV, true, TWO, CT>), 512);                                  \
+    else LAUNCH_LN((gemm_ln_rows_kernel<RV, false, TWO, CT>), 512);                                                \
   } while (0)
-  if (same && M <= 4 && K <= 2048) LAUNCH_Q_N(1);
-  else if (same && M <= 8 && K <= 2048) LAUNCH_Q_N(2);
-  else if (mt == 1 && same && K <= 2048) {
-    if (K <= 256) LAUNCH_LDS(1);
-    else if (K <= 512) LAUNCH_LDS(2);
-    else if (K <= 768) LAUNCH_LDS(3);
-    else if (K <= 1024) LAUNCH_LDS(4);
-    else if (K <= 1280) LAUNCH_LDS(5);
-    else if (K <= 1536) LAUNCH_LDS(6);
-    else if (K <= 1792) LAUNCH_LDS(7);
-    else LAUNCH_LDS(8);
+#define LAUNCH_R(RV, TWO)                                                                                          \
+  do {                                                                                                            \
+    if (cols > 16) LAUNCH_R_P(RV, TWO, 2);                                                                         \
+    else LAUNCH_R_P(RV, TWO, 1);                                                                                   \
+  } while (0)
+  if (quads && M <= 4) LAUNCH_Q_N(1);
+  else if (quads) LAUNCH_Q_N(2);
+  else if (in_rows && M <= 8) {
+    if (K <= 256) LAUNCH_R(1, false);
+    else if (K <= 512) LAUNCH_R(2, false);
+    else if (K <= 768) LAUNCH_R(3, false);
+    else if (K <= 1024) LAUNCH_R(4, false);
+    else if (K <= 1280) LAUNCH_R(5, false);
+    else LAUNCH_R(6, false);
+  } else if (in_rows) {
+    if (K <= 256) LAUNCH_R(1, true);
+    else if (K <= 512) LAUNCH_R(2, true);
+    else if (K <= 768) LAUNCH_R(3, true);
+    else LAUNCH_R(4, true);
   } else
     // 8 wavefronts, two chunks in flight each: 125 registers, so two workgroups share a compute unit
     // (deeper unrolling needs 168 and halves that; 16 wavefronts spill)

@@ -81,6 +81,7 @@ _ARGTYPES = {
     "da_gemm_ref": [_VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_f32": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _I, _VP],
     "da_gemm_f32_rows_choice": [_I, _I, _I],
+    "da_gemm_bf16_ln_choice": [_I, _I, _I, _I],
     "da_gemm_f32_ln_takes": [_I, _I, _I],
     "da_gemm_f32_ln": [_VP, _VP, _VP, _F, _VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_bf16": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],

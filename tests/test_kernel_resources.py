@@ -82,3 +82,25 @@ def test_prefill_attention_fits_side_by_side_and_does_not_spill():
     for (d16, blocks, phases, table, q_late), (workgroups, scratch) in resources("attn_prefill_rel", "attn_prefill_rel_kernel").items():
         if (blocks, phases) == (4, 1):
             assert workgroups >= (2 if d16 <= 5 else 1) and scratch == 0, (d16, table, q_late)
+
+
+def test_norm_and_product_of_few_rows_run_side_by_side():
+    """gemm_ln_quads: steps whose launch is up to two workgroups a compute unit have them side by side (a wide workgroup alone would leave half of them for a
+    second round); no scratch memory; every kernel that is compiled is one that some call asks for.  Which kernel a row goes to does not hang on the columns."""
+    from deliverance_amd.kernels import ops
+    found = resources("gemm_fused", "gemm_ln_quads_kernel")
+    lib, asked = ops._lib(), set()
+    columns = (1, 4, 8, 256, 768, 1024, 1500, 2304, 3072, 4096, 4800, 5120, 6144, 6400, 7168, 8192, 8193, 9600, 10240, 10241, 12800, 14336, 14337, 15360, 16384, 50257)
+    for M in (1, 4, 5, 8):
+        for K in range(8, 2049, 8):
+            for dtype in (ops.F32, ops.BF16):
+                cols = [lib.da_gemm_bf16_ln_choice(M, N, K, dtype) for N in columns]
+                assert all(cols) or not any(cols)
+                for N, c in zip(columns, cols if all(cols) else ()):
+                    form = ((1 if M <= 4 else 2), -(-c // 4), *((4, 1) if K <= 512 else (4, 2) if K <= 1024 else (6, 2) if K <= 1536 else (8, 2)), int(dtype == ops.BF16))
+                    asked.add(form)
+                    workgroups, scratch = found[form]
+                    assert scratch == 0 and c <= 32
+                    if lib.da_can_fuse_ln(M, K, N) and 256 < -(-N // c) <= 512:
+                        assert workgroups >= 2, (M, K, N, c, dtype)
+    assert asked == set(found)

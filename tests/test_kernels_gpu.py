@@ -467,11 +467,11 @@ def test_fused_norm_product_one_workgroup_a_compute_unit(ops, M, N, K):
 
 @pytest.mark.parametrize("dt", [helpers.quick(torch.bfloat16, mark="simt_a"), torch.float32])
 @pytest.mark.parametrize("N,K", [helpers.quick(50, 120, mark="simt_b"), (2304, 512), (1021, 520), (4100, 1024), (4801, 1032), (8190, 1536), (8200, 1544),
-                                 helpers.quick(12, 2048, mark="simt_b"), (6401, 1600)])
+                                 helpers.quick(12, 2048, mark="simt_b"), (6401, 1600), (1030, 1792), (2304, 1600), (4801, 1920), (14400, 1536), (16383, 1040)])
 def test_norm_and_product_of_up_to_8_rows(ops, N, K, dt):
     """A wavefront holds one step of 128 k or two, 4 to 8 of them; 4 to 32 columns a workgroup, columns that end inside a group of 4; one group
-    of 4 rows or two; rows in any order.  Rows whose mean is a hundred times their spread (statistics joined from the wavefronts' own means keep it);
-    a row has the same bits beside any others, and one that is not finite leaves the others alone."""
+    of 4 rows or two; a wavefront a row (5 to 8 rows up to K = 1,536, and K up to 256); rows in any order.  Rows whose mean is a hundred times their spread;
+    a row has the same bits beside any others of its kernel, and one that is not finite leaves the others alone."""
     g = torch.Generator().manual_seed(N + K)
     R = 11
     x = (torch.randn(R, K, generator=g) * 3 + torch.arange(R).view(R, 1) * 30.0).to(DEV)
@@ -491,9 +491,35 @@ def test_norm_and_product_of_up_to_8_rows(ops, N, K, dt):
         assert (rms.double() - ref).abs().max() < 2e-2 * max(1.0, ref.abs().max().item()), M
     whole = ops.linear_ln(x, None, 8, gw, gb, 1e-5, w, bias, torch.empty(8, N, device=DEV))
     few = lambda lo, hi: ops.linear_ln(x[lo:hi].contiguous(), None, hi - lo, gw, gb, 1e-5, w, bias, torch.empty(hi - lo, N, device=DEV))
-    assert torch.equal(few(2, 3)[0], whole[2]) and torch.equal(few(1, 5), whole[1:5]) and torch.equal(few(3, 8), whole[3:])
-    x[0, K - 1] = float("inf")
-    assert torch.equal(few(0, 8)[1:], whole[1:])
+    four = few(1, 5)
+    assert torch.equal(few(2, 3)[0], four[1]) and torch.equal(few(3, 8), whole[3:])
+    if K <= 256 or K > 1536:                     # one kernel
+        assert torch.equal(four, whole[1:5])
+    x[0, K - 1] = x[1, 3] = float("inf")
+    assert torch.equal(few(0, 8)[2:], whole[2:]) and torch.equal(few(1, 5)[1:], four[1:])
+
+
+@pytest.mark.parametrize("M", [helpers.quick(1), helpers.quick(4, mark="simt_a"), 8])
+@pytest.mark.parametrize("K", [helpers.quick(264, mark="simt_b"), 512, 640, 1024, 1160, 1536, 1600, helpers.quick(2048, mark="simt_b")])
+def test_norm_statistics_of_rows_that_change_along_k(ops, M, K):
+    """Every 128 entries have a mean of their own, far apart beside what they scatter by: the variance is what lies between the parts of a row that the
+    wavefronts hold, one or two steps each.  The oracle without that term is 10 tolerances away and more, so a kernel that lost it would be too."""
+    g = torch.Generator().manual_seed(M + K)
+    part = torch.arange(K) // 128
+    x = torch.randn(M, K, generator=g) + 7.0 * ((part * 5 + torch.arange(M).view(M, 1)) % 7)
+    gw, gb = torch.randn(K, generator=g) + 2, torch.randn(K, generator=g)
+    w = bf(torch.randn(40, K, generator=g) * 0.1)
+    out = ops.linear_ln(x.to(DEV), None, M, gw.to(DEV), gb.to(DEV), 1e-5, w.to(DEV), None, torch.empty(M, 40, device=DEV)).double().cpu()
+    xd = x.double()
+    mean = xd.mean(1, keepdim=True)
+    within = sum(((xd[:, part == p] - xd[:, part == p].mean(1, keepdim=True)) ** 2).sum(1, keepdim=True) for p in range(int(part[-1]) + 1)) / K
+
+    def product(variance):
+        return ((xd - mean) / torch.sqrt(variance + 1e-5) * gw.double() + gb.double()).to(torch.bfloat16).double() @ w.double().t()
+
+    want = product(((xd - mean) ** 2).mean(1, keepdim=True))
+    tol = 2e-3 * max(1.0, want.abs().max().item())
+    assert (out - want).abs().max() < tol and (product(within) - want).abs().amax(1).min() > 10 * tol
 
 
 @pytest.mark.parametrize("M,N,K", [(1600, 2000, 200), (1555, 1999, 320), (2048, 1600, 1600), (1536, 2304, 768), (2048, 2304, 768),
