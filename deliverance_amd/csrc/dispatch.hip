@@ -15,15 +15,14 @@ extern "C" int da_decode_splits(int n_seqs, int n_heads, int max_blocks, int pag
 }
 
 // Measured on MI355X inside the model: the fused norm + product kernel wins up to 16 rows (one row tile)
-// and a width of 1,024, by 10 to 15 % of a decode step; up to 8 rows (which take half the LDS, so that the
-// workgroups still run side by side) up to a width of 2,048.  Every workgroup reads and normalises all rows again (at a
-// width of 1,600 that is 2.5 us of vector work a compute unit), so beyond a width of 1,536, where no two workgroups of more
-// than 16 columns fit on a compute unit, and beyond 8,192 columns, which are three and four rounds of 16, the norm is
-// a kernel of its own from 5 rows on: us, fused / two kernels, 5 and 8 rows, K = 1,600: N = 8,200 11.3 / 10.4 and 12.1 / 10.6, 12,800 14.5 / 13.4
-// and 15.9 / 13.7; K = 1,920, N = 10,240 13.0 / 12.3 and 14.5 / 12.7 (3 rows 11.1 / 12.3); but K = 2,048, where the product takes 12 wavefronts, N = 10,240
-// 13.4 / 14.4 and 14.9 / 14.8.  Never for a vocabulary.
+// and a width of 1,024, by 10 to 15 % of a decode step; up to 8 rows up to a width of 2,048.  Every workgroup reads and normalises all rows again, so with
+// 5 rows and more, beyond a width of 1,536 and about 5,000 columns, the norm is a kernel of its own.  us, fused / two kernels, cold weights, recorded one behind
+// the other, 5 and 8 rows: K = 1,600, N = 4,800 7.2 / 8.0, 7.2 / 8.0; N = 6,400 8.5 / 7.7, 8.6 / 7.7; N = 8,192 10.0 / 8.7, 10.1 / 8.9; N = 12,800 16.8 / 12.7,
+// 17.1 / 13.2; K = 1,920, N = 7,680 10.4 / 9.7, 10.5 / 10.1; K = 2,048, where the product takes 12 wavefronts, N = 6,144 9.2 / 9.6, 9.3 / 9.9; N = 8,192 10.6 / 10.4,
+// 10.8 / 10.6; N = 10,240 14.0 / 13.6, 14.4 / 13.7 (K = 1,536, N = 10,240 10.2 / 11.5, 10.9 / 11.7; 4 rows, K = 1,600, N = 12,800 10.4 / 12.8).  Never for a
+// vocabulary.
 extern "C" int da_can_fuse_ln(int n_rows, int K, int N) {
   const bool fits = (n_rows <= 16 && K <= 1024) || (n_rows <= 8 && K <= 2048);
-  const bool slower = n_rows > 4 && K > 1536 && K < 2048 && N > 8192;
+  const bool slower = n_rows > 4 && K > 1536 && N > (K < 1920 ? 5120 : 6144);
   return n_rows > 0 && fits && !slower && K % 8 == 0 && N <= 16384;
 }

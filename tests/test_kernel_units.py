@@ -100,3 +100,13 @@ def test_a_norm_that_writes_the_stream_promises_nothing_about_it(tmp_path):
     assert {join for join, _ in found} == {"0", "1"}
     for join, stream in found:
         assert ("noalias" in stream) == (join == "0"), (join, stream)
+
+
+def test_which_steps_norm_and_product_take_in_one_kernel():
+    """One row tile and a width of 1,024, 8 rows and 2,048; with 5 rows and more not for wide widths with many columns; never a vocabulary."""
+    from deliverance_amd.kernels import ops
+    takes = ops._lib().da_can_fuse_ln
+    for rows, K, N in ((1, 768, 2304), (16, 1024, 4096), (8, 1536, 16384), (4, 2048, 16384), (8, 1600, 4800), (5, 1912, 5120), (8, 2048, 6144), (5, 1920, 6144)):
+        assert takes(rows, K, N), (rows, K, N)
+    for rows, K, N in ((0, 768, 768), (17, 768, 768), (9, 1032, 768), (8, 2056, 768), (1, 764, 768), (1, 768, 16385), (5, 1600, 6400), (8, 1544, 5121), (8, 2048, 6145)):
+        assert not takes(rows, K, N), (rows, K, N)
