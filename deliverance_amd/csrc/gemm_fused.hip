@@ -372,7 +372,7 @@ gemm_ln_quads_kernel(const float* __restrict__ x, const int* __restrict__ rows, 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Up to 8 rows and K = 1,536, up to 16 and 1,024 (and what ln_quads_takes leaves), parameters of one dtype: every load in whole cache lines.
+// Up to 8 rows and K = 1,536, up to 16 and 1,024 (what ln_quads_takes leaves of them), parameters of one dtype: every load in whole cache lines.
 // Wavefront v of 8 reads rows v and v + 8 whole (RV float4 a lane), with the gain and bias at the
 // same places, computes their statistics, and writes the normalised rows as bfloat16 into LDS,
 // zeros past K.  The steps of w (64 elements of k, 8 rows x 128 bytes a load; wavefront v takes the
@@ -574,8 +574,8 @@ static void launch_fused(int mt, dim3 grid, hipStream_t s, const LnPrologue& ln,
   else hipLaunchKernelGGL((gemm_ln_skinny_kernel<2, NW, UN>), grid, dim3(NW * 64), 0, s, ln, W, ldw, ep, kv, M, N, K);
 }
 
-// Up to 8 rows: whether they go to gemm_ln_quads, else to gemm_ln_rows.  By the rows, K and the parameters' dtype alone, so that a column has the same bits
-// among fewer columns.  us, cold weights, recorded one behind the other, gemm_ln_rows / gemm_ln_quads, parameters in bfloat16:
+// Up to 8 rows: whether they go to gemm_ln_quads, else to gemm_ln_rows.  By the rows, K and the parameters' dtype, so that a column has the same bits
+// among fewer columns; 5 to 8 rows with K from 641 to 1,024 by the columns too.  us, cold weights, recorded one behind the other, gemm_ln_rows / gemm_ln_quads, parameters in bfloat16:
 //   1, 4 rows  K =   256, N = 2,304 2.6 / 2.7, 2.6 / 2.7; 6,144 3.2 / 3.0, 3.3 / 3.1
 //              K =   768, N = 2,304 3.4 / 3.2, 3.6 / 3.3; 3,072 3.6 / 3.3, 3.7 / 3.4; 8,320 5.1 / 4.8, 5.5 / 4.9; 12,800 5.8 / 5.8, 5.7 / 5.7
 //              K = 1,280, N = 4,096 4.8 / 4.9, 4.8 / 5.0; 4,800 5.2 / 5.0, 5.3 / 5.1 (six wavefronts hold up to 1,536; with 32-bit parameters 2 to 9 % behind up
@@ -583,9 +583,15 @@ static void launch_fused(int mt, dim3 grid, hipStream_t s, const LnPrologue& ln,
 //              K = 1,600, N = 4,800 6.3 / 5.6, 6.6 / 5.6; 6,400 7.3 / 6.9, 7.5 / 6.8; 8,320 9.2 / 7.9, 9.6 / 7.9; 12,800 12.1 / 11.2, 13.1 / 11.0
 //   5, 8 rows  every workgroup normalises all rows, here a lane 8 rows' pieces, there a wavefront a row:
 //              K =   768, N = 2,304 3.9 / 4.0, 4.1 / 4.1; 8,192 5.6 / 6.9, 5.8 / 6.9; K = 1,536, N = 4,096 5.7 / 6.4, 5.9 / 6.3; 10,240 10.2 / 12.7, 10.9 / 12.8
-//              K = 1,600, N = 2,304 - 3 %, 4,096 + 7 %, 4,800 7.4 / 7.2, 7.8 / 7.2; K = 2,048, N = 2,048 6.5 / 5.7, 6.8 / 5.8; 6,144 9.4 / 9.4, 9.9 / 9.3
-static bool ln_quads_takes(int M, int K, int params) {
-  if (M > 4) return M <= 8 && K > 1536;
+//              K = 1,600, N = 2,304 - 3 % of the time, 4,096 + 7 %, 4,800 7.4 / 7.2, 7.8 / 7.2; K = 2,048, N = 2,048 6.5 / 5.7, 6.8 / 5.8; 6,144 9.4 / 9.4, 9.9 / 9.3
+//              K = 1,024, N = 3,072 4.6 / 4.3, 4,096 + 8 %, 4,800 - 6 %, 6,144 level, 8,192 6.5 / 7.2.  So up to K = 1,024 where its columns a workgroup are 12 or fewer, or
+//              17 to 20, for which gemm_ln_rows has two groups of 16.  Recorded steps, all rows / all quads / this: 355M, 5 requests 617 / 611 / 605,
+//              8 650 / 645 / 637; 124M, 8 320 / 316 / 318; a Virudra of the 355M's sizes, 5 974 / 958 / 958
+static bool ln_quads_takes(int M, int N, int K, int params) {
+  if (M > 4) {
+    const int share = da_ceil_div(N, 256);
+    return M <= 8 && (K > 1536 || (K > 640 && K <= 1024 && (share <= 12 || (share > 16 && share <= 20))));
+  }
   return K > 256 && (params == DA_BF16 || K <= 1024 || K > 1280);
 }
 // Its columns a workgroup, in groups of 4: every compute unit a workgroup up to 8,192 columns, two up to 16,384 as long as they fit side by side; 16 for a
@@ -605,7 +611,7 @@ static int ln_quads_columns(int M, int N, int K, int params) {
 
 // The columns a workgroup of gemm_ln_quads, or 0 where the rows go to another kernel.
 extern "C" int da_gemm_bf16_ln_choice(int M, int N, int K, int params) {
-  return M > 0 && K <= 2048 && ln_quads_takes(M, K, params) ? ln_quads_columns(M, N, K, params) : 0;
+  return M > 0 && K <= 2048 && ln_quads_takes(M, N, K, params) ? ln_quads_columns(M, N, K, params) : 0;
 }
 
 static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_dtype, const void* b,
@@ -637,7 +643,7 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
   const bool wide = N > 16 * 256 && N <= 64 * 256;
   const int pdt = g_dtype;
   const bool same = (!b || b_dtype == pdt) && (!bias || bias_dtype == pdt) && (pdt == DA_BF16 || pdt == DA_F32);
-  const bool quads = same && ln_quads_takes(M, K, pdt);
+  const bool quads = same && ln_quads_takes(M, N, K, pdt);
   const bool in_rows = same && !quads && (M <= 8 ? K <= 1536 : M <= 16 && K <= 1024);
   const int cols = quads ? ln_quads_columns(M, N, K, pdt) : (wide ? da_ceil_div(N, N <= 32 * 256 ? 256 : 512) : FZ_COLS);
 #define LAUNCH_LN(KERNEL, THREADS)                                                                                 \
@@ -679,7 +685,12 @@ static int gemm_bf16_norm(const float* x, const int* rows, const void* g, int g_
     else LAUNCH_R_P(RV, TWO, 1);                                                                                   \
   } while (0)
   if (quads && M <= 4) LAUNCH_Q_N(1);
-  else if (quads) LAUNCH_Q_N(2);
+  else if (quads && K <= 1024) {                     // (the widths that ln_quads_takes leaves)
+    if (cols <= 4) LAUNCH_Q(2, 1, 4, 2);
+    else if (cols <= 8) LAUNCH_Q(2, 2, 4, 2);
+    else if (cols <= 12) LAUNCH_Q(2, 3, 4, 2);
+    else LAUNCH_Q(2, 5, 4, 2);
+  } else if (quads) LAUNCH_Q_N(2);
   else if (in_rows && M <= 8) {
     if (K <= 256) LAUNCH_R(1, false);
     else if (K <= 512) LAUNCH_R(2, false);
