@@ -826,13 +826,19 @@ gemm_skinny4_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, 
 // where that pays.  us, cold weights, recorded one behind the other, 4x4x4 with a row a lane (up to 4 rows) or gemm_skinny (8 rows) -> this:
 //   1 row   1,600 x 6,400 6.3 -> 5.7, 768 x 3,072 3.8 -> 3.2, 1,600 x 1,600 3.7 -> 3.4, 768 x 768 2.7 -> 2.6
 //   4 rows  1,600 x 6,400 7.3 -> 6.1, 768 x 3,072 4.3 -> 3.5, 1,600 x 1,600 4.0 -> 3.6, 2,048 x 8,192 9.4 -> 7.8
-//   8 rows  1,600 x 6,400 7.4 -> 7.1, 768 x 3,072 4.5 -> 4.0, 1,024 x 4,096 5.5 -> 4.4; 1,600 x 1,600 3.8 -> 3.9 (so from K = 2,048 on)
+//   8 rows  1,600 x 6,400 7.4 -> 7.1, 768 x 3,072 4.5 -> 4.0, 1,024 x 4,096 5.5 -> 4.4; 1,600 x 1,600 3.8 -> 3.9 (so from K = 2,048 on);
+//           2,048 x 2,048 4.0 -> 4.2, 2,048 x 3,072 4.5 -> 4.7, 2,048 x 4,096 5.5 -> 5.5, but 1,984 x 2,048 level (so not where every compute unit has one of its
+//           workgroups, up to K = 3,584)
 // The weights alone, read and dropped, take 5.2, 2.5 and 2.6 us (1,600 x 6,400, 768 x 3,072, 1,600 x 1,600).
 #define SK4_ROWS 4
 #define SK4_LONG_ROWS 8
 #define SK4_LONG_K 2048
 #define SK4_COLS 2048
-static bool sk4_takes(int M, int N, int K) { return N <= SK4_COLS && (M <= SK4_ROWS || (M <= SK4_LONG_ROWS && K >= SK4_LONG_K)); }
+static bool sk4_takes(int M, int N, int K) {
+  return N <= SK4_COLS && (M <= SK4_ROWS || (M <= SK4_LONG_ROWS && K >= SK4_LONG_K && (N <= 1984 || K >= 3584)));
+}
+// 1 when a product goes there
+extern "C" int da_gemm_pieces_takes(int M, int N, int K) { return M > 0 && sk4_takes(M, N, K); }
 static void launch_skinny4(hipStream_t s, const bf16_t* A, int lda, const bf16_t* W, int ldw, const Epilogue& ep, const KvScatter& kv, int M,
                            int N, int K) {
 #define DA_SK4_GO(MG, NG, NW, U) hipLaunchKernelGGL((gemm_skinny4_kernel<MG, NG, NW, U>), dim3(da_ceil_div(N, 4 * NG)), dim3(NW * 64), 0, s, A, W, ep.bias, ep.out, lda, ldw, ep.ldo, M, N, K, epilogue_rest(ep), kv)
@@ -866,7 +872,8 @@ static int gemm_bf16_launch(const void* a, int lda, const void* w, int ldw, cons
                             int K, void* stream);
 
 // 1 where the gate and up products of few rows and their activation are one kernel: where the product of both matrices' columns would go to
-// gemm_skinny with 16 columns a workgroup and all rows in it.  One rounding to bfloat16 and one launch fewer; us, the product and the
+// gemm_skinny with 16 columns a workgroup and all rows in it (or, 5 to 8 rows with a long K, to gemm_skinny4: K = 2,048, 2 x 1,024 columns the product
+// alone 3.9, this 3.7).  One rounding to bfloat16 and one launch fewer; us, the product and the
 // activation's kernel / this, cold weights: 8 rows, K = 1,024, 2 x 2,752 columns 6.7 / 4.5; K = 768, 2 x 2,048 columns 1 row 5.2 / 3.4, 64 rows
 // 7.5 / 4.5; K = 3,072, 2 x 8,192 columns 8 rows 19.9 / 17.3.
 extern "C" int da_gemm_gated_takes(int M, int inner, int K) {

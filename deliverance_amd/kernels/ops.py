@@ -86,6 +86,7 @@ _ARGTYPES = {
     "da_gemm_f32_ln": [_VP, _VP, _VP, _F, _VP, _I, _VP, _I, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_bf16": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "da_gemm_few_rows": [_I, _I],
+    "da_gemm_pieces_takes": [_I, _I, _I],
     "da_gemm_gated_takes": [_I, _I, _I],
     "da_gemm_bf16_gated": [_VP, _I, _VP, _I, _VP, _I, _I, _I, _I, _I, _F, _VP],
     "da_gemm_bf16_kv_split": [_VP, _I, _VP, _I, _VP, _I, _VP, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _I, _I, _VP],

@@ -110,3 +110,13 @@ def test_which_steps_norm_and_product_take_in_one_kernel():
         assert takes(rows, K, N), (rows, K, N)
     for rows, K, N in ((0, 768, 768), (17, 768, 768), (9, 1032, 768), (8, 2056, 768), (1, 764, 768), (1, 768, 16385), (5, 1600, 6400), (8, 1544, 5121), (8, 2048, 6145)):
         assert not takes(rows, K, N), (rows, K, N)
+
+
+def test_which_products_take_four_pieces_of_k_side_by_side():
+    """Up to 4 rows and 2,048 columns; 5 to 8 rows with a long K, where it is ahead of the kernel for more rows."""
+    from deliverance_amd.kernels import ops
+    takes = ops._lib().da_gemm_pieces_takes
+    for rows, N, K in ((1, 2048, 8), (4, 2048, 2048), (5, 1984, 2048), (8, 64, 8192), (8, 2048, 3584)):
+        assert takes(rows, N, K), (rows, N, K)
+    for rows, N, K in ((1, 2049, 768), (5, 1024, 2040), (8, 2048, 2048), (5, 1985, 3576), (9, 64, 8192)):
+        assert not takes(rows, N, K), (rows, N, K)
