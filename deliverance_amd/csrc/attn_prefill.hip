@@ -618,12 +618,10 @@ extern "C" int da_attn_prefill(const void* q, int q_ld, const void* cache, const
   // wavefronts work and share out the keys (see below for how many keys).  Longer ones take 128 rows a workgroup (smaller row blocks
   // read the keys more often, and that traffic binds), and 4 x 2, eight wavefronts, while there is no
   // more than one workgroup a compute unit; else 4 x 1.  Measured on MI355X, head size 64, microseconds
-  // 4x1 / 4x2 / 2x2 / 1x4: 2 x 1,024 rows, 12 heads 23.3 / 19.3 / 23.4 / 34.6; 2,048 rows 40.0 / 31.8 /
-  // 38.9 / 51.7; 8 x 512 rows 19.3 / 23.3 / 26.2 / 42.5; 4 x 64 rows after 900 keys 22.8 / 17.8 / 17.8 /
-  // 16.3; 16 x 2 rows after 1,000 keys 22.8 / 18.5 / 18.3 / 18.0.  With the longest workgroups of every pair launched
-  // first, 4x1 / 4x2: 2 x 1,024 rows, 12 heads 23.2 / 20.0, 25 heads 26.0 / 25.5; 8 x 1,024 rows, 12 heads 35.5 / 39.9;
-  // 2 x 4,096 rows 93.6 / 108.5 (551 TFLOP/s; 157.6 before); 8,192 rows 165.5 / 190.2; 4 x 512 rows after 512 keys,
-  // 16 heads 22.5 / 19.7.  Workgroups of 256 rows (8 x 1) were behind 4 x 1 at every one of these.  A loop that multiplies
+  // 4x1 / 4x2 / 2x2 / 1x4: 4 x 64 rows after 900 keys 19.8 / 17.0 / 15.6 / 19.3; 16 x 2 rows after 1,000 keys 20.2 / 17.6 / 16.7 / 24.2 (one
+  // sequence of 8 or 64 rows: below).  4x1 / 4x2: 2 x 1,024 rows, 12 heads 19.6 / 17.9, 25 heads 23.5 / 23.4; 2,048 rows 33.0 / 29.3; 8 x 512 rows
+  // 14.0 / 15.9; 8 x 1,024 rows, 12 heads 28.5 / 35.2 (452 TFLOP/s), 25 heads 54.5 / 69.8 (493); 2 x 4,096 rows 79.9 / 92.5 (645); 8,192 rows
+  // 145.5 / 171.2 (709); 4 x 512 rows after 512 keys, 16 heads 19.2 / 17.9.  Workgroups of 256 rows (8 x 1) were behind 4 x 1 at every one of these.  A loop that multiplies
   // the scores of tile j + 1 while tile j is weighed (keys parked one tile ahead of values) gave the same bits and
   // -8 % to +12 % of 4 x 1's time depending on the shape: with two wavefronts a SIMD the matrix cores already run under
   // the other wavefront's softmax; it is not kept.  Four key phases (2 x 4, 4 x 4) were behind 4 x 2 at every shape (2 x

@@ -812,7 +812,7 @@ extern "C" int da_moe_combine_norm(const float* out, int ldo, const int* slot_of
 // A workgroup owns a tile of 32 slots x 16 columns of one expert, and its wavefronts share out k: wavefront v takes the
 // steps of 64 number v, v + NW, ... with MFMA 16x16x32.  With few rows an expert, as in decoding, the kernel
 // streams the expert's weights once, and narrow columns mean many workgroups for that (8 experts of 512 x 768: 256).  Operands come
-// in whole cache lines, 8 rows x 128 bytes a load, of the rows of a only those that hold a pair; the wavefront parks a step in its own
+// in whole cache lines, 8 rows x 128 bytes a load, of the rows of a the first 8, the first 16 or all 32, whichever hold the pairs; the wavefront parks a step in its own
 // piece of LDS and reads the fragments from there, as gemm_skinny does.  (Straight into fragments neighbouring lanes lie in 16 rows, which
 // a compute unit takes one lane at a time.)  The
 // wavefronts' sums meet in LDS and are added in the order of the wavefronts.  GATED: the gate and up rows of the same
